@@ -8,10 +8,10 @@
 //   y[b][co][i][j] = bias[co] + sum_{ci,u,v} w[co][ci][u][v] x[b][ci][i+u-1][j+v-1]
 // Every layer is a GEMM of M = output channels, N = pixels, K = Cin 9 taps
 // (forward), or M = output channels, N = Cin 9 taps, K = pixels (weight
-// gradient), on v_mfma_f32_32x32x8_bf16: lane l supplies A[l % 32][4 (l / 32)
-// + t] and B[4 (l / 32) + t][l % 32], t < 4; accumulator register r of lane
-// l holds D[8 (r / 4) + 4 (l / 32) + r % 4][l % 32].  Operands are rounded to
-// bfloat16 (nearest, ties to even) when they are staged into LDS.
+// gradient), on v_mfma_f32_16x16x32_bf16: lane l supplies A[l % 16][8 (l / 16)
+// + t] and B[8 (l / 16) + t][l % 16], t < 8; accumulator register r of lane
+// l holds D[4 (l / 16) + r][l % 16].  Operands are rounded to bfloat16
+// (nearest, ties to even) when they are staged into LDS.
 #include "cnn.hpp"
 
 #include <algorithm>
@@ -22,337 +22,524 @@
 
 namespace bam {
 
-typedef short bf16x4 __attribute__((ext_vector_type(4)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-__device__ inline unsigned short f2bf(float f)
-{
-	unsigned u = __float_as_uint(f);
-	u += 0x7FFFu + ((u >> 16) & 1u);  // nearest, ties to even (finite values)
-	return (unsigned short)(u >> 16);
-}
-
-constexpr int CV_MAXC = 64;    // channels (in and out) per layer at most
-constexpr int CV_PIX = 64;     // forward: pixels (row segment) per work-group
-constexpr int CV_ROWS = 4;     // forward: rows per work-group of a large launch
-constexpr int CV_FWD_THREADS = 256;
-constexpr int CV_WG_THREADS = 512;
-constexpr int CV_WG_ROWS = 8;  // weight gradient: image rows per work-group
+constexpr int CV_MAXC = 64;     // channels (in and out) per layer at most
+constexpr int CV_THREADS = 512; // 8 waves
+constexpr int CV_STRIP = 256;   // forward: pixels (row segment) per work-group
+constexpr int CV_MAXROWS = 16;  // image rows per work-group at most
 constexpr int CV_WG_MAXW = 256;
 
-__host__ __device__ inline int round8(int v) { return (v + 7) / 8 * 8; }
+// two floats rounded to bfloat16 (nearest, ties to even), the first in the
+// low half
+__device__ inline unsigned bf_pack(float a, float b)
+{
+	const f32x2 v = { a, b };
+	return __builtin_bit_cast(unsigned, __builtin_convertvector(v, bf16x2));
+}
+
+// image rows per work-group: one work-group per compute unit where there
+// are rows enough (each one reads two rows of halo), down to one row
+static int conv_rows(long total_rows, int ncu)
+{
+	return (int)std::min<long>(CV_MAXROWS, std::max<long>(1, (total_rows + ncu - 1) / ncu));
+}
+
+static int conv_ncu()
+{
+	int dev = 0, n = 1;
+	BAM_HIP(hipGetDevice(&dev));
+	BAM_HIP(hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev));
+	return std::max(1, n);
+}
 
 // ---------------------------------------------------------------------------
-// Forward: work-group = 64 pixels of one row x 64 output channels, 4 waves of
-// one 32 x 32 tile each.  K is ordered (tap, channel) with the channels
-// padded to CP (a multiple of 8): the weights are first converted to
-// bfloat16 in that order ([64][9 CP], k_conv_wprep) and read from there
-// (cached), and the 3 x 66 input patch is staged in LDS channel-fastest, so
-// that a lane's 4 consecutive k of one matrix-core step -- 4 channels of one
-// tap -- are one 8-byte read for A and one LDS read for B.
+// Forward.  Bound by HBM: 48 channels of 256^2 are 2 x 100 MB per batch of 8
+// against 22 GFLOP.  A work-group takes a strip of CV_STRIP pixels and walks
+// down its image rows, so that a row is read once (and two halo rows per
+// work-group) and stays in LDS, channel-fastest, for the three output rows
+// that need it; the next row's loads are in flight while the matrix cores
+// work on the present one.  K is ordered (tap, channel) with the channels
+// padded to 8 G, in steps of 32 (four groups of 8 channels, each of one
+// tap): the B fragment of a lane is one 16-byte LDS read at its pixel and
+// tap (pixel pitch 4 x odd dwords: no bank conflicts), and the weights of
+// all steps stay in registers (A fragments, k_conv_wprep's order).  Waves
+// share the 16-pixel tiles of the row; with many channels also the output
+// channel tiles (TPW per wave, ncog groups: three tiles of 48 channels per
+// wave spill 120 registers, 124 us; two groups 81 us).  48 -> 48 channels,
+// batch 8 of 256^2: 187 -> 81 us (2.5 TB/s) against 64-pixel, 4-row blocks
+// that staged 2-byte elements.
 // ---------------------------------------------------------------------------
 
-__host__ __device__ inline int chan_pad(int c) { return (c + 7) / 8 * 8; }
+__host__ __device__ constexpr int conv_steps(int G) { return (9 * G + 3) / 4; }
+__host__ __device__ constexpr int conv_pitch(int G) { return 8 * (G | 1); }
 
-// wb[co][t CP + ci] = bf16(w[co][ci][t]), zero for padded co / ci
-__global__ void k_conv_wprep(const float* __restrict__ w, int Cin, int Cout, int CP,
+// A fragments wb[tile][step][lane][8]: w[co = 16 tile + lane % 16][k = 32 step
+// + 8 (lane / 16) + i], zero for padded channels and taps.  flip: the
+// weights of the transposed convolution (the data gradient), w'[o][i][t] =
+// w[i][o][8 - t].
+__global__ void k_conv_wprep(const float* __restrict__ w, int Cin, int Cout, int G, int ntiles, int flip,
 			     unsigned short* __restrict__ wb)
 {
-	const int KP = 9 * CP;
-	const int n = CV_MAXC * KP;
+	const int steps = conv_steps(G);
+	const int n = ntiles * steps * 512;
 
 	for (int e = blockIdx.x * blockDim.x + threadIdx.x; e < n; e += gridDim.x * blockDim.x) {
-		const int co = e / KP;
-		const int k = e - co * KP;
-		const int t = k / CP;
-		const int ci = k - t * CP;
-		wb[e] = f2bf((co < Cout && ci < Cin) ? w[(co * Cin + ci) * 9 + t] : 0.f);
+		const int lane = (e >> 3) & 63;
+		const int ts = e >> 9;
+		const int tile = ts / steps;
+		const int k8 = 4 * (ts - tile * steps) + (lane >> 4);
+		const int t = k8 / G;
+		const int ci = (k8 - t * G) * 8 + (e & 7);
+		const int co = 16 * tile + (lane & 15);
+		float v = 0.f;
+		if (co < Cout && ci < Cin && t < 9)
+			v = flip ? w[(ci * Cout + co) * 9 + (8 - t)] : w[(co * Cin + ci) * 9 + t];
+		wb[e] = (unsigned short)(bf_pack(v, 0.f) & 0xFFFFu);
 	}
 }
 
-template <int ROWS>
-__global__ __launch_bounds__(CV_FWD_THREADS) void k_conv3x3_fwd(const float* __restrict__ x, int Cin, int H, int W,
-								const unsigned short* __restrict__ wb,
-								const float* __restrict__ bias,
-								const float* __restrict__ res, int Cout, int relu,
-								float* __restrict__ y)
+template <int G, int TPW>
+__global__ __launch_bounds__(CV_THREADS) void k_conv3x3_fwd(const float* __restrict__ x, int Cin, int H, int W,
+							    const unsigned short* __restrict__ wb,
+							    const float* __restrict__ bias,
+							    const float* __restrict__ res, int Cout, int relu,
+							    float* __restrict__ y, int rows, int ncog)
 {
+	constexpr int STEPS = conv_steps(G);
+	constexpr int PITCH = conv_pitch(G);
+	constexpr int ROWSZ = (CV_STRIP + 2) * PITCH;
+	constexpr int NT = (G * CV_STRIP + CV_THREADS - 1) / CV_THREADS;
 	extern __shared__ __align__(16) unsigned char cv_smem[];
-	const int CP = chan_pad(Cin);
-	unsigned short* xl = (unsigned short*)cv_smem;          // [ROWS + 2][66][CP]
-	constexpr int PR = ROWS + 2;                          // patch rows
+	unsigned short* xl = (unsigned short*)cv_smem;  // [3][CV_STRIP + 2][PITCH]
 
-	const int x0 = blockIdx.x * CV_PIX;
-	const int y0 = blockIdx.y * ROWS;
+	const int x0 = blockIdx.x * CV_STRIP;
+	const int y0 = blockIdx.y * rows;
 	const int b = blockIdx.z;
-
-	// input patch, channel-fastest
-	for (int e = threadIdx.x; e < CP * PR * 66; e += CV_FWD_THREADS) {
-		const int ci = e / (PR * 66);
-		const int r = e - ci * (PR * 66);
-		const int u = r / 66;
-		const int xx = r - u * 66;
-		const int gx = x0 + xx - 1;
-		const int gy = y0 + u - 1;
-		float v = 0.f;
-		if (ci < Cin && gy >= 0 && gy < H && gx >= 0 && gx < W)
-			v = x[((long)(b * Cin + ci) * H + gy) * W + gx];
-		xl[(u * 66 + xx) * CP + ci] = f2bf(v);
-	}
-
-	__syncthreads();
+	const int nrow = min(rows, H - y0);
+	const long HW = (long)H * W;
+	const float* xb = x + (long)b * Cin * HW;
 
 	const int lane = threadIdx.x & 63;
 	const int wv = threadIdx.x >> 6;
-	const int cot = wv & 1;
-	const int pt = wv >> 1;
-	const int i = lane & 31;
-	const int hk = lane >> 5;
-	// A fragments straight from the prepared weights (a few KiB, cached),
-	// each used for the ROWS rows of the block
-	const unsigned short* wrow = wb + (cot * 32 + i) * (9 * CP) + 4 * hk;
-	const int px = pt * 32 + i;
+	const int l16 = lane & 15;
+	const int kg = lane >> 4;
+	const int cog = wv % ncog;
+	const int pg = wv / ncog;
+	const int npg = 8 / ncog;
 
-	f32x16 acc[ROWS];
+	bf16x8 A[TPW][STEPS];
+
 #pragma unroll
-	for (int q = 0; q < ROWS; q++)
+	for (int q = 0; q < TPW; q++)
 #pragma unroll
-		for (int r = 0; r < 16; r++)
-			acc[q][r] = 0.f;
+		for (int s = 0; s < STEPS; s++)
+			A[q][s] = *(const bf16x8*)(wb + (((long)(cog * TPW + q) * STEPS + s) * 64 + lane) * 8);
 
-	for (int t = 0; t < 9; t++) {
+	// one image row in registers: 8 channels of a pixel per task, NT tasks
+	// of the strip and one of the two halo pixels (the first 2 G threads)
+	float v[NT + 1][8];
 
-		const int u = t / 3;
-		const int v = t - 3 * u;
-		const unsigned short* xrow = xl + (u * 66 + px + v) * CP + 4 * hk;
-		const unsigned short* wt = wrow + t * CP;
-
-		for (int c0 = 0; c0 < CP; c0 += 8) {
-			const bf16x4 a = *(const bf16x4*)(wt + c0);
+	auto load8 = [&](float (&d)[8], int g, int gy, int gx) {
+		const bool ok = gy >= 0 && gy < H && gx >= 0 && gx < W;
+		const float* p = xb + (long)(8 * g) * HW + (long)gy * W;
 #pragma unroll
-			for (int q = 0; q < ROWS; q++) {
-				const bf16x4 bv = *(const bf16x4*)(xrow + q * 66 * CP + c0);
-				acc[q] = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(a, bv, acc[q], 0, 0, 0);
+		for (int i = 0; i < 8; i++)
+			d[i] = (ok && 8 * g + i < Cin) ? (p + i * HW)[gx] : 0.f;
+	};
+
+	// the strip's channel groups are wave-uniform (scalar row addresses)
+	const int g0 = __builtin_amdgcn_readfirstlane(threadIdx.x / CV_STRIP);
+
+	auto load_row = [&](int gy) {
+#pragma unroll
+		for (int i = 0; i < NT; i++)
+			load8(v[i], g0 + i * (CV_THREADS / CV_STRIP), gy, x0 + (int)threadIdx.x % CV_STRIP);
+		if (threadIdx.x < 2 * G)
+			load8(v[NT], threadIdx.x >> 1, gy, (threadIdx.x & 1) ? x0 + CV_STRIP : x0 - 1);
+	};
+
+	auto put8 = [&](const float (&d)[8], unsigned short* p) {
+		*(uint4*)p = make_uint4(bf_pack(d[0], d[1]), bf_pack(d[2], d[3]), bf_pack(d[4], d[5]),
+					bf_pack(d[6], d[7]));
+	};
+
+	auto store_row = [&](int slot) {
+		unsigned short* r = xl + slot * ROWSZ;
+#pragma unroll
+		for (int i = 0; i < NT; i++) {
+			const int e = threadIdx.x + i * CV_THREADS;
+			if (0 == (G * CV_STRIP) % CV_THREADS || e < G * CV_STRIP)
+				put8(v[i], r + (1 + e % CV_STRIP) * PITCH + 8 * (e / CV_STRIP));
+		}
+		if (threadIdx.x < 2 * G)
+			put8(v[NT], r + ((threadIdx.x & 1) ? CV_STRIP + 1 : 0) * PITCH + 8 * (threadIdx.x >> 1));
+	};
+
+	load_row(y0 - 1);
+	store_row(0);
+	load_row(y0);
+	store_row(1);
+	load_row(y0 + 1);
+
+	const int ntile = (min(CV_STRIP, W - x0) + 15) / 16;
+
+	for (int r = 0; r < nrow; r++) {
+
+		// image row y0 + r + 1; rows y0 + r - 1 + u are in slots (r + u) % 3
+		store_row((r + 2) % 3);
+		lds_barrier();
+
+		if (r + 1 < nrow)
+			load_row(y0 + r + 2);
+
+		// LDS offsets of this lane's 8 channels of every step, pixel 0
+		int off[STEPS];
+#pragma unroll
+		for (int s = 0; s < STEPS; s++) {
+			const int k8 = min(4 * s + kg, 9 * G - 1);
+			const int t = k8 / G;
+			const int u = t / 3;
+			off[s] = ((r + u) % 3) * ROWSZ + (l16 + t - 3 * u) * PITCH + (k8 - t * G) * 8;
+		}
+
+		for (int pt = pg; pt < ntile; pt += npg) {
+
+			f32x4 acc[TPW];
+#pragma unroll
+			for (int q = 0; q < TPW; q++)
+				acc[q] = f32x4{ 0.f, 0.f, 0.f, 0.f };
+
+			const unsigned short* xp = xl + pt * 16 * PITCH;
+
+#pragma unroll
+			for (int s = 0; s < STEPS; s++) {
+				uint4 raw = *(const uint4*)(xp + off[s]);
+				// the last step's groups beyond the nine taps: zero
+				if (STEPS * 4 > 9 * G && STEPS - 1 == s && 4 * s + kg >= 9 * G)
+					raw = make_uint4(0u, 0u, 0u, 0u);
+				const bf16x8 bv = __builtin_bit_cast(bf16x8, raw);
+#pragma unroll
+				for (int q = 0; q < TPW; q++)
+					acc[q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[q][s], bv, acc[q], 0, 0, 0);
+			}
+
+			const int gx = x0 + pt * 16 + l16;
+
+			if (gx < W) {
+
+				const long at0 = ((long)b * Cout + 16 * (cog * TPW) + 4 * kg) * HW + (long)(y0 + r) * W + gx;
+
+#pragma unroll
+				for (int q = 0; q < TPW; q++)
+#pragma unroll
+					for (int i = 0; i < 4; i++) {
+						const int co = 16 * (cog * TPW + q) + 4 * kg + i;
+						if (co < Cout) {
+							float o = acc[q][i] + ((nullptr != bias) ? bias[co] : 0.f);
+							if (relu)
+								o = fmaxf(o, 0.f);
+							const long at = at0 + (16 * q + i) * HW;
+							if (nullptr != res)
+								o += res[at];
+							y[at] = o;
+						}
+					}
 			}
 		}
+
+		lds_barrier();  // the oldest slot is rewritten next
 	}
+}
 
-	const int gx = x0 + px;
+// ---------------------------------------------------------------------------
+// Weight gradient.  Bound by HBM (x and dy once).  A work-group walks down
+// its image rows: the input rows y - 1, y, y + 1 and the output-gradient row
+// y are in LDS pixel-fastest, so that a lane's 8 consecutive pixels of one
+// channel (K = pixels) are one 16-byte read; the three horizontal taps of
+// an input row come from that read and the two neighbouring pixels by
+// funnel shifts in registers.  Wave (it, ks) owns input-channel tile it and
+// every output-channel tile and tap (9 NCO accumulator tiles), for the
+// pixel chunks ks, ks + KS, ...; the KS parts are summed through LDS in
+// order, and each work-group writes one partial gradient [9][16 NCO][16 NCI]
+// (k_conv_wgrad_sum adds them in order).  The bias gradient's sums of the
+// unrounded dy are taken while its rows are staged.  48 x 48 channels, batch
+// 8 of 256^2: 600 + 508 (bias) + 72 (sum) -> 52 + 7 us (3.8 TB/s) against
+// 2-byte LDS reads of the input patch, one work-group per bias channel and a
+// thread per entry of the sum.
+// ---------------------------------------------------------------------------
 
-	if (gx < W) {
+__host__ __device__ constexpr int wg_pitch(int n) { return ((n + 7) / 8 | 1) * 8; }
+__host__ __device__ constexpr int wg_pitch_x(int W) { return wg_pitch(8 + (W + 31) / 32 * 32 + 8); }
+__host__ __device__ constexpr int wg_pitch_dy(int W) { return wg_pitch((W + 31) / 32 * 32); }
+
+template <int NCO, int NCI>
+__global__ __launch_bounds__(CV_THREADS) void k_conv3x3_wgrad(const float* __restrict__ x,
+							      const float* __restrict__ dy, int Cin, int Cout, int H,
+							      int W, int rows, int aligned, float* __restrict__ part,
+							      float* __restrict__ bpart)
+{
+	constexpr int NW = CV_THREADS / 64;
+	constexpr int KS = NW / NCI;
+	constexpr int XI = 2 * NCI;  // float4 of x (of dy) per thread and row at most
+	constexpr int DI = 2 * NCO;
+	extern __shared__ __align__(16) unsigned char cv_smem[];
+	const int PX = wg_pitch_x(W), PD = wg_pitch_dy(W);
+	unsigned short* xl = (unsigned short*)cv_smem;     // [3][16 NCI][PX], pixel p at 8 + p
+	unsigned short* dl = xl + 3 * 16 * NCI * PX;       // [16 NCO][PD]
+
+	const int nrg = (H + rows - 1) / rows;
+	const int b = blockIdx.x / nrg;
+	const int y0 = (blockIdx.x - b * nrg) * rows;
+	const int nrow = min(rows, H - y0);
+	const long HW = (long)H * W;
+	const float* xb = x + (long)b * Cin * HW;
+	const float* db = dy + (long)b * Cout * HW;
+
+	const int lane = threadIdx.x & 63;
+	const int wv = threadIdx.x >> 6;
+
+	// staging: LG lanes per channel row (four pixels each), 64 / LG channels
+	// per wave and step
+	int lgl = 1;
+	while ((4 << lgl) < W)
+		lgl++;
+	const int cstep = NW << (6 - lgl);
+	const int c0 = (wv << (6 - lgl)) + (lane >> lgl);
+	const int px = 4 * (lane & ((1 << lgl) - 1));
+	const bool pin = px < W;
+
+	// zero once: padded channels, the halo pixels and the pixels beyond W
+	for (int e = threadIdx.x; e < (3 * 16 * NCI * PX + 16 * NCO * PD) / 8; e += CV_THREADS)
+		((uint4*)cv_smem)[e] = make_uint4(0u, 0u, 0u, 0u);
+
+	f32x4 xv[XI], dv[DI];
+	float bs[DI];
 #pragma unroll
-		for (int q = 0; q < ROWS; q++) {
-			const int yy = y0 + q;
-			if (yy >= H)
-				break;
+	for (int i = 0; i < DI; i++)
+		bs[i] = 0.f;
+
+	auto ld4 = [&](const float* p) {
+		if (aligned)
+			return *(const f32x4*)p;
+		return f32x4{ p[0], p[1], p[2], p[3] };
+	};
+
+	auto load_x = [&](int gy) {
 #pragma unroll
-			for (int r = 0; r < 16; r++) {
-				const int co = cot * 32 + 8 * (r / 4) + 4 * hk + (r % 4);
-				if (co < Cout) {
-					float v = acc[q][r] + ((nullptr != bias) ? bias[co] : 0.f);
-					if (relu)
-						v = fmaxf(v, 0.f);
-					const long o = ((long)(b * Cout + co) * H + yy) * W + gx;
-					if (nullptr != res)
-						v += res[o];
-					y[o] = v;
+		for (int i = 0; i < XI; i++) {
+			const int c = c0 + i * cstep;
+			xv[i] = f32x4{ 0.f, 0.f, 0.f, 0.f };
+			if (pin && c < Cin && gy >= 0 && gy < H)
+				xv[i] = ld4(xb + c * HW + (long)gy * W + px);
+		}
+	};
+
+	auto load_dy = [&](int gy) {
+#pragma unroll
+		for (int i = 0; i < DI; i++) {
+			const int c = c0 + i * cstep;
+			dv[i] = f32x4{ 0.f, 0.f, 0.f, 0.f };
+			if (pin && c < Cout)
+				dv[i] = ld4(db + c * HW + (long)gy * W + px);
+		}
+	};
+
+	auto put4 = [&](const f32x4& f, unsigned short* p) {
+		*(uint2*)p = make_uint2(bf_pack(f[0], f[1]), bf_pack(f[2], f[3]));
+	};
+
+	auto store_x = [&](int slot) {
+#pragma unroll
+		for (int i = 0; i < XI; i++) {
+			const int c = c0 + i * cstep;
+			if (pin && c < Cin)
+				put4(xv[i], xl + (slot * 16 * NCI + c) * PX + 8 + px);
+		}
+	};
+
+	auto store_dy = [&]() {
+#pragma unroll
+		for (int i = 0; i < DI; i++) {
+			const int c = c0 + i * cstep;
+			if (pin && c < Cout) {
+				bs[i] += (dv[i][0] + dv[i][1]) + (dv[i][2] + dv[i][3]);
+				put4(dv[i], dl + c * PD + px);
+			}
+		}
+	};
+
+	const int it = wv % NCI;
+	const int ks = wv / NCI;
+	const int l16 = lane & 15;
+	const int kg = lane >> 4;
+
+	f32x4 acc[9][NCO];
+#pragma unroll
+	for (int t = 0; t < 9; t++)
+#pragma unroll
+		for (int q = 0; q < NCO; q++)
+			acc[t][q] = f32x4{ 0.f, 0.f, 0.f, 0.f };
+
+	load_x(y0 - 1);
+	__syncthreads();  // the zeroes are in
+	store_x(0);
+	load_x(y0);
+	store_x(1);
+	load_x(y0 + 1);
+	load_dy(y0);
+
+	for (int r = 0; r < nrow; r++) {
+
+		store_x((r + 2) % 3);
+		store_dy();
+		lds_barrier();
+
+		if (r + 1 < nrow) {
+			load_x(y0 + r + 2);
+			load_dy(y0 + r + 1);
+		}
+
+		if (ks < KS) {
+
+			for (int p0 = 32 * ks; p0 < W; p0 += 32 * KS) {
+
+				const int p = p0 + 8 * kg;
+				bf16x8 a[NCO];
+#pragma unroll
+				for (int q = 0; q < NCO; q++)
+					a[q] = *(const bf16x8*)(dl + (16 * q + l16) * PD + p);
+
+#pragma unroll
+				for (int u = 0; u < 3; u++) {
+
+					const unsigned short* xr = xl + ((((r + u) % 3) * NCI + it) * 16 + l16) * PX + 8 + p;
+					const uint4 d = *(const uint4*)xr;
+					const unsigned pv = *(const unsigned*)(xr - 2);
+					const unsigned nx = *(const unsigned*)(xr + 8);
+					// 8 pixels from p - 1 and from p + 1
+					const unsigned m0 = __builtin_amdgcn_alignbyte(d.x, pv, 2);
+					const unsigned m1 = __builtin_amdgcn_alignbyte(d.y, d.x, 2);
+					const unsigned m2 = __builtin_amdgcn_alignbyte(d.z, d.y, 2);
+					const unsigned m3 = __builtin_amdgcn_alignbyte(d.w, d.z, 2);
+					const unsigned m4 = __builtin_amdgcn_alignbyte(nx, d.w, 2);
+					const bf16x8 bv[3] = { __builtin_bit_cast(bf16x8, make_uint4(m0, m1, m2, m3)),
+							       __builtin_bit_cast(bf16x8, d),
+							       __builtin_bit_cast(bf16x8, make_uint4(m1, m2, m3, m4)) };
+#pragma unroll
+					for (int h = 0; h < 3; h++)
+#pragma unroll
+						for (int q = 0; q < NCO; q++)
+							acc[3 * u + h][q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+								a[q], bv[h], acc[3 * u + h][q], 0, 0, 0);
 				}
 			}
 		}
-	}
-}
 
-static size_t fwd_lds(int Cin, int rows)
-{
-	return sizeof(unsigned short) * (size_t)(rows + 2) * 66 * chan_pad(Cin);
-}
-
-// w'[ci][co][u][v] = w[co][ci][2 - u][2 - v]: the weights of the transposed
-// convolution (the data gradient)
-__global__ void k_conv_flip(const float* __restrict__ w, int Cout, int Cin, float* __restrict__ wt)
-{
-	const int n = Cout * Cin * 9;
-
-	for (int e = blockIdx.x * blockDim.x + threadIdx.x; e < n; e += gridDim.x * blockDim.x) {
-		const int co = e / (Cin * 9);
-		const int r = e - co * Cin * 9;
-		const int ci = r / 9;
-		const int t = r - ci * 9;
-		wt[(ci * Cout + co) * 9 + (8 - t)] = w[e];
-	}
-}
-
-// ---------------------------------------------------------------------------
-// Weight gradient: work-group = CV_WG_ROWS rows of one image; per row the
-// output-gradient row (M = Cout x K = W pixels) and the 3 input rows around
-// it (N = Cin 9 taps) are staged in LDS; 8 waves share the
-// ceil(Cout / 32) x ceil(Cin 9 / 32) tiles.  Each work-group writes its
-// partial [64][NP] gradient; k_conv_wgrad_sum adds the partials in order.
-// ---------------------------------------------------------------------------
-
-constexpr int CV_WG_TILES = 4;  // tiles per wave at most (2 x 14 tiles over 8 waves)
-
-__global__ __launch_bounds__(CV_WG_THREADS) void k_conv3x3_wgrad(const float* __restrict__ x,
-								  const float* __restrict__ dy, int Cin, int Cout,
-								  int H, int W, float* __restrict__ part)
-{
-	extern __shared__ __align__(16) unsigned char cv_smem[];
-	const int K = Cin * 9;
-	const int NP = (K + 31) / 32 * 32;
-	const int WX = W + 2;
-	unsigned short* dyl = (unsigned short*)cv_smem;         // [64][W]
-	unsigned short* xl = dyl + CV_MAXC * W;                 // [Cin][3][W + 2]
-	int* koff = (int*)(xl + round8(Cin * 3 * WX));          // [NP]
-
-	const int nrg = (H + CV_WG_ROWS - 1) / CV_WG_ROWS;
-	const int b = blockIdx.x / nrg;
-	const int y0 = (blockIdx.x - b * nrg) * CV_WG_ROWS;
-
-	for (int k = threadIdx.x; k < NP; k += CV_WG_THREADS) {
-		const int ci = k / 9;
-		const int t = k - ci * 9;
-		koff[k] = (k < K) ? (ci * 3 + t / 3) * WX + (t % 3) : -1;
+		lds_barrier();
 	}
 
-	const int lane = threadIdx.x & 63;
-	const int wv = threadIdx.x >> 6;
-	const int i = lane & 31;
-	const int hk = lane >> 5;
-	const int ncot = (Cout + 31) / 32;
-	const int nkt = NP / 32;
-	const int ntiles = ncot * nkt;
+	// sum of the KS parts in order, through LDS (the rows are done with)
+	f32x4* sh = (f32x4*)cv_smem;  // [NCI][9 NCO][64]
 
-	f32x16 acc[CV_WG_TILES];
+	for (int k = 1; k < KS; k++) {
+
+		if (k == ks) {
 #pragma unroll
-	for (int q = 0; q < CV_WG_TILES; q++)
+			for (int t = 0; t < 9; t++)
 #pragma unroll
-		for (int r = 0; r < 16; r++)
-			acc[q][r] = 0.f;
-
-	for (int yy = y0; yy < min(H, y0 + CV_WG_ROWS); yy++) {
-
-		__syncthreads();
-
-		for (int e = threadIdx.x; e < CV_MAXC * W; e += CV_WG_THREADS) {
-			const int co = e / W;
-			const int xx = e - co * W;
-			dyl[e] = f2bf((co < Cout) ? dy[((long)(b * Cout + co) * H + yy) * W + xx] : 0.f);
+				for (int q = 0; q < NCO; q++)
+					sh[((it * 9 + t) * NCO + q) * 64 + lane] = acc[t][q];
 		}
 
-		for (int e = threadIdx.x; e < Cin * 3 * WX; e += CV_WG_THREADS) {
-			const int cu = e / WX;
-			const int ci = cu / 3;
-			const int u = cu - ci * 3;
-			const int gx = e - cu * WX - 1;
-			const int gy = yy + u - 1;
-			float v = 0.f;
-			if (gy >= 0 && gy < H && gx >= 0 && gx < W)
-				v = x[((long)(b * Cin + ci) * H + gy) * W + gx];
-			xl[e] = f2bf(v);
+		lds_barrier();
+
+		if (0 == ks) {
+#pragma unroll
+			for (int t = 0; t < 9; t++)
+#pragma unroll
+				for (int q = 0; q < NCO; q++)
+					acc[t][q] += sh[((it * 9 + t) * NCO + q) * 64 + lane];
 		}
 
-		__syncthreads();
-
-#pragma unroll
-		for (int q = 0; q < CV_WG_TILES; q++) {
-
-			const int tile = wv + 8 * q;
-
-			if (tile >= ntiles)
-				break;
-
-			const int cot = tile / nkt;
-			const int kt = tile - cot * nkt;
-			const unsigned short* arow = dyl + (cot * 32 + i) * W;
-			const int o = koff[kt * 32 + i];
-
-			for (int p0 = 0; p0 < W; p0 += 8) {
-
-				const int pb = p0 + 4 * hk;
-				const bf16x4 a = *(const bf16x4*)(arow + pb);
-				bf16x4 bv;
-#pragma unroll
-				for (int t = 0; t < 4; t++)
-					bv[t] = (o >= 0) ? (short)xl[o + pb + t] : (short)0;
-				acc[q] = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(a, bv, acc[q], 0, 0, 0);
-			}
-		}
+		lds_barrier();
 	}
 
-	// partial [64][NP] of this work-group
-	float* pp = part + (long)blockIdx.x * CV_MAXC * NP;
+	if (0 == ks) {
+
+		float* pp = part + (long)blockIdx.x * 9 * 16 * NCO * 16 * NCI;
 
 #pragma unroll
-	for (int q = 0; q < CV_WG_TILES; q++) {
-
-		const int tile = wv + 8 * q;
-
-		if (tile >= ntiles)
-			break;
-
-		const int cot = tile / nkt;
-		const int kt = tile - cot * nkt;
-
+		for (int t = 0; t < 9; t++)
 #pragma unroll
-		for (int r = 0; r < 16; r++) {
-			const int co = cot * 32 + 8 * (r / 4) + 4 * hk + (r % 4);
-			pp[co * NP + kt * 32 + i] = acc[q][r];
+			for (int q = 0; q < NCO; q++)
+#pragma unroll
+				for (int i = 0; i < 4; i++)
+					pp[((t * 16 * NCO) + 16 * q + 4 * kg + i) * 16 * NCI + 16 * it + l16] = acc[t][q][i];
+	}
+
+	if (nullptr != bpart) {
+#pragma unroll
+		for (int i = 0; i < DI; i++) {
+			float s = bs[i];
+			for (int o = (1 << lgl) >> 1; o > 0; o >>= 1)
+				s += __shfl_xor(s, o, 64);
+			const int c = c0 + i * cstep;
+			if (0 == px && c < Cout)
+				bpart[(long)blockIdx.x * CV_MAXC + c] = s;
 		}
 	}
 }
 
-// dw[co][k] = sum over the partials in work-group order
-__global__ void k_conv_wgrad_sum(const float* __restrict__ part, int nparts, int Cout, int K, int NP,
-				 float* __restrict__ dw)
-{
-	const int n = Cout * K;
-
-	for (int e = blockIdx.x * blockDim.x + threadIdx.x; e < n; e += gridDim.x * blockDim.x) {
-		const int co = e / K;
-		const int k = e - co * K;
-		float s = 0.f;
-		for (int p = 0; p < nparts; p++)
-			s += part[((long)p * CV_MAXC + co) * NP + k];
-		dw[e] = s;
-	}
-}
-
-// db[co] = sum over b, i, j of dy (one work-group per channel, fixed order)
-__global__ __launch_bounds__(256) void k_conv_bgrad(const float* __restrict__ dy, int B, int Cout, long HW,
-						     float* __restrict__ db)
+// Sums of the partials: dw[co][ci][t] (work-groups below nblk, 64 entries of a
+// partial each) and db[co] (the work-group after them): four threads per
+// entry take every fourth partial in order, their sums are added in order.
+__global__ __launch_bounds__(256) void k_conv_wgrad_sum(const float* __restrict__ part, const float* __restrict__ bpart,
+							int nparts, int Cin, int Cout, int PO, int PI, int nblk,
+							float* __restrict__ dw, float* __restrict__ db)
 {
 	__shared__ float sh[256];
-	const int co = blockIdx.x;
+	const int j = threadIdx.x & 63;
+	const int g = threadIdx.x >> 6;
+	const bool wsum = (int)blockIdx.x < nblk;
+	const long stride = wsum ? 9l * PO * PI : CV_MAXC;
+	const int e = wsum ? (int)blockIdx.x * 64 + j : j;
+	const float* p = (wsum ? part : bpart) + e;
 	float s = 0.f;
 
-	for (int b = 0; b < B; b++)
-		for (long e = threadIdx.x; e < HW; e += 256)
-			s += dy[((long)b * Cout + co) * HW + e];
+	if (wsum || e < Cout) {
+#pragma unroll 8
+		for (int k = g; k < nparts; k += 4)
+			s += p[k * stride];
+	}
 
 	sh[threadIdx.x] = s;
 	__syncthreads();
 
-	for (int h = 128; h > 0; h >>= 1) {
-		if (threadIdx.x < h)
-			sh[threadIdx.x] += sh[threadIdx.x + h];
-		__syncthreads();
+	if (0 != g)
+		return;
+
+	s = ((sh[j] + sh[64 + j]) + sh[128 + j]) + sh[192 + j];
+
+	if (wsum) {
+		const int t = e / (PO * PI);
+		const int r = e - t * (PO * PI);
+		const int co = r / PI;
+		const int ci = r - co * PI;
+		if (co < Cout && ci < Cin)
+			dw[(co * Cin + ci) * 9 + t] = s;
+	} else if (e < Cout) {
+		db[e] = s;
 	}
-
-	if (0 == threadIdx.x)
-		db[co] = sh[0];
 }
 
-static size_t wgrad_lds(int Cin, int W)
-{
-	const int NP = (Cin * 9 + 31) / 32 * 32;
-	return sizeof(unsigned short) * ((size_t)CV_MAXC * W + round8(Cin * 3 * (W + 2))) + sizeof(int) * NP;
-}
-
-// work buffers of the weight gradient and the flipped weights
+// work buffers: the weights as matrix-core fragments, the partial gradients
 struct CnnWork {
 	std::mutex mtx;
 	DevBuf<float> part;
-	DevBuf<float> wt;
 	DevBuf<unsigned short> wb;
 };
 
@@ -369,28 +556,69 @@ static void check_shape(int B, int Cin, int Cout, int H, int W)
 		  "conv3x3: 1 to %d channels in and out (got %d, %d)", CV_MAXC, Cin, Cout);
 }
 
-// the bfloat16 weights of the forward kernel, prepared per call
+template <int G>
+static void fwd_launch_g(dim3 grid, int tpw, const float* x, int Cin, int H, int W, const unsigned short* wb,
+			 const float* bias, const float* res, int Cout, bool relu, float* y, int rows, int ncog,
+			 hipStream_t st)
+{
+	const size_t lds = sizeof(unsigned short) * 3 * (CV_STRIP + 2) * conv_pitch(G);
+
+#define BAM_CONV(T)                                                                                               \
+	hipLaunchKernelGGL((k_conv3x3_fwd<G, T>), grid, dim3(CV_THREADS), lds, st, x, Cin, H, W, wb, bias, res, Cout, \
+			   relu ? 1 : 0, y, rows, ncog)
+	if (1 == tpw)
+		BAM_CONV(1);
+	else if (2 == tpw)
+		BAM_CONV(2);
+	else if constexpr (G <= 4)
+		BAM_CONV(3);
+	else
+		fail("conv3x3: no kernel for %d channel tiles", tpw);
+#undef BAM_CONV
+}
+
+// the weights as bfloat16 fragments (prepared per call), then the layer;
+// flip: w holds the forward weights of the transposed convolution
 static void fwd_launch(const float* x, int B, int Cin, int H, int W, const float* w, const float* bias,
-		       const float* res, int Cout, bool relu, float* y, hipStream_t st, DevBuf<unsigned short>& wb)
+		       const float* res, int Cout, bool relu, float* y, hipStream_t st, DevBuf<unsigned short>& wb,
+		       bool flip)
 {
 	check_shape(B, Cin, Cout, H, W);
 	BAM_CHECK(H <= 65535 && B <= 65535, "conv3x3: too many rows or images");
-	const int CP = chan_pad(Cin);
-	const long nw = (long)CV_MAXC * 9 * CP;
+
+	// a wave keeps the weights of its output-channel tiles in registers (4
+	// per tile and step of 32): all tiles while they take at most 108, else
+	// two groups of waves (144 and more spill)
+	const int G = (Cin + 7) / 8;
+	const int nco = (Cout + 15) / 16;
+	const int ncog = (4 == nco || (3 == nco && G > 4)) ? 2 : 1;
+	const int tpw = (nco + ncog - 1) / ncog;
+	const int ntiles = ncog * tpw;
+	const long nw = (long)ntiles * conv_steps(G) * 512;
 	if ((long)wb.n < nw)
 		wb.alloc(nw);
-	hipLaunchKernelGGL(k_conv_wprep, dim3((unsigned)((nw + 255) / 256)), dim3(256), 0, st, w, Cin, Cout, CP, wb.ptr);
-	// CV_ROWS rows per work-group reuse each weight fragment CV_ROWS times;
-	// a single image keeps one row per work-group so that every CU has work
-	const long big = (long)((W + CV_PIX - 1) / CV_PIX) * ((H + CV_ROWS - 1) / CV_ROWS) * B;
-	const int rows = (big >= 2048) ? CV_ROWS : 1;
-	dim3 grid((W + CV_PIX - 1) / CV_PIX, (H + rows - 1) / rows, B);
-	if (CV_ROWS == rows)
-		hipLaunchKernelGGL(k_conv3x3_fwd<CV_ROWS>, grid, dim3(CV_FWD_THREADS), fwd_lds(Cin, rows), st, x, Cin, H, W,
-				   wb.ptr, bias, res, Cout, relu ? 1 : 0, y);
-	else
-		hipLaunchKernelGGL(k_conv3x3_fwd<1>, grid, dim3(CV_FWD_THREADS), fwd_lds(Cin, rows), st, x, Cin, H, W,
-				   wb.ptr, bias, res, Cout, relu ? 1 : 0, y);
+	hipLaunchKernelGGL(k_conv_wprep, dim3((unsigned)((nw + 255) / 256)), dim3(256), 0, st, w, Cin, Cout, G, ntiles,
+			   flip ? 1 : 0, wb.ptr);
+	const int nx = (W + CV_STRIP - 1) / CV_STRIP;
+	const int rows = conv_rows((long)nx * H * B, conv_ncu());
+	dim3 grid(nx, (H + rows - 1) / rows, B);
+
+#define BAM_CONV_G(NG) \
+	case NG: fwd_launch_g<NG>(grid, tpw, x, Cin, H, W, wb.ptr, bias, res, Cout, relu, y, rows, ncog, st); break
+	switch (G) {
+		BAM_CONV_G(1);
+		BAM_CONV_G(2);
+		BAM_CONV_G(3);
+		BAM_CONV_G(4);
+		BAM_CONV_G(5);
+		BAM_CONV_G(6);
+		BAM_CONV_G(7);
+		BAM_CONV_G(8);
+	default:
+		fail("conv3x3: no kernel for %d channels", Cin);
+	}
+#undef BAM_CONV_G
+
 	BAM_HIP(hipGetLastError());
 }
 
@@ -401,7 +629,7 @@ void conv3x3_fwd(const float* x, int B, int Cin, int H, int W, const float* w, c
 	// on the one stream every layer call uses
 	CnnWork& cw = cnn_work();
 	std::lock_guard<std::mutex> lock(cw.mtx);
-	fwd_launch(x, B, Cin, H, W, w, bias, res, Cout, relu, y, st, cw.wb);
+	fwd_launch(x, B, Cin, H, W, w, bias, res, Cout, relu, y, st, cw.wb, false);
 }
 
 void conv3x3_bwd_data(const float* dy, int B, int Cout, int H, int W, const float* w, int Cin, float* dx,
@@ -410,13 +638,31 @@ void conv3x3_bwd_data(const float* dy, int B, int Cout, int H, int W, const floa
 	check_shape(B, Cin, Cout, H, W);
 	CnnWork& cw = cnn_work();
 	std::lock_guard<std::mutex> lock(cw.mtx);
-	const long n = (long)Cout * Cin * 9;
-	if ((long)cw.wt.n < n)
-		cw.wt.alloc(n);
-	hipLaunchKernelGGL(k_conv_flip, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, w, Cout, Cin, cw.wt.ptr);
-	BAM_HIP(hipGetLastError());
-	fwd_launch(dy, B, Cout, H, W, cw.wt.ptr, nullptr, nullptr, Cin, false, dx, st, cw.wb);
-	BAM_HIP(hipStreamSynchronize(st));  // the flipped weights are reused by the next call
+	fwd_launch(dy, B, Cout, H, W, w, nullptr, nullptr, Cin, false, dx, st, cw.wb, true);
+	BAM_HIP(hipStreamSynchronize(st));
+}
+
+template <int NCO>
+static void wgrad_launch(int nci, int nparts, const float* x, const float* dy, int Cin, int Cout, int H, int W,
+			 int rows, int aligned, float* part, float* bpart, hipStream_t st)
+{
+	// the rows, later the accumulator tiles of the in-order sum
+	const size_t lds = std::max(sizeof(unsigned short) * (3 * 16 * (size_t)nci * wg_pitch_x(W) +
+							      16 * (size_t)NCO * wg_pitch_dy(W)),
+				    sizeof(f32x4) * 64 * 9 * (size_t)nci * NCO);
+
+#define BAM_WGRAD(NI)                                                                                              \
+	case NI: hipLaunchKernelGGL((k_conv3x3_wgrad<NCO, NI>), dim3(nparts), dim3(CV_THREADS), lds, st, x, dy, Cin, Cout, \
+				    H, W, rows, aligned, part, bpart); break
+	switch (nci) {
+		BAM_WGRAD(1);
+		BAM_WGRAD(2);
+		BAM_WGRAD(3);
+		BAM_WGRAD(4);
+	default:
+		fail("conv3x3 weight gradient: no kernel for %d channels", Cin);
+	}
+#undef BAM_WGRAD
 }
 
 void conv3x3_bwd_weights(const float* x, const float* dy, int B, int Cin, int Cout, int H, int W, float* dw,
@@ -425,23 +671,31 @@ void conv3x3_bwd_weights(const float* x, const float* dy, int B, int Cin, int Co
 	check_shape(B, Cin, Cout, H, W);
 	BAM_CHECK(W <= CV_WG_MAXW && 0 == W % 8, "conv3x3 weight gradient: width a multiple of 8, at most %d",
 		  CV_WG_MAXW);
+	BAM_CHECK(((Cout + 31) / 32) * ((Cin * 9 + 31) / 32) <= 32, "conv3x3 weight gradient: too many tiles");
 	CnnWork& cw = cnn_work();
 	std::lock_guard<std::mutex> lock(cw.mtx);
-	const int NP = (Cin * 9 + 31) / 32 * 32;
-	BAM_CHECK(((Cout + 31) / 32) * (NP / 32) <= 8 * CV_WG_TILES, "conv3x3 weight gradient: too many tiles");
-	const int nparts = B * ((H + CV_WG_ROWS - 1) / CV_WG_ROWS);
-	const long np = (long)nparts * CV_MAXC * NP;
+	const int nco = (Cout + 15) / 16, nci = (Cin + 15) / 16;
+	const int PO = 16 * nco, PI = 16 * nci;
+	const int rows = conv_rows((long)B * H, conv_ncu());
+	const int nparts = B * ((H + rows - 1) / rows);
+	const long np = (long)nparts * (9 * PO * PI + CV_MAXC);
 	if ((long)cw.part.n < np)
 		cw.part.alloc(np);
-	hipLaunchKernelGGL(k_conv3x3_wgrad, dim3(nparts), dim3(CV_WG_THREADS), wgrad_lds(Cin, W), st, x, dy, Cin, Cout,
-			   H, W, cw.part.ptr);
-	const int n = Cout * Cin * 9;
-	hipLaunchKernelGGL(k_conv_wgrad_sum, dim3((n + 255) / 256), dim3(256), 0, st, cw.part.ptr, nparts, Cout,
-			   Cin * 9, NP, dw);
-	if (nullptr != db)
-		hipLaunchKernelGGL(k_conv_bgrad, dim3(Cout), dim3(256), 0, st, dy, B, Cout, (long)H * W, db);
+	float* bpart = (nullptr != db) ? cw.part.ptr + (long)nparts * 9 * PO * PI : nullptr;
+	const int aligned = (0 == ((uintptr_t)x | (uintptr_t)dy) % 16) ? 1 : 0;
+
+	switch (nco) {
+	case 1: wgrad_launch<1>(nci, nparts, x, dy, Cin, Cout, H, W, rows, aligned, cw.part.ptr, bpart, st); break;
+	case 2: wgrad_launch<2>(nci, nparts, x, dy, Cin, Cout, H, W, rows, aligned, cw.part.ptr, bpart, st); break;
+	case 3: wgrad_launch<3>(nci, nparts, x, dy, Cin, Cout, H, W, rows, aligned, cw.part.ptr, bpart, st); break;
+	default: wgrad_launch<4>(nci, nparts, x, dy, Cin, Cout, H, W, rows, aligned, cw.part.ptr, bpart, st); break;
+	}
+
+	const int nblk = 9 * PO * PI / 64;
+	hipLaunchKernelGGL(k_conv_wgrad_sum, dim3(nblk + (nullptr != db ? 1 : 0)), dim3(256), 0, st, cw.part.ptr, bpart,
+			   nparts, Cin, Cout, PO, PI, nblk, dw, db);
 	BAM_HIP(hipGetLastError());
-	BAM_HIP(hipStreamSynchronize(st));  // the partials are reused by the next call
+	BAM_HIP(hipStreamSynchronize(st));
 }
 
 }  // namespace bam

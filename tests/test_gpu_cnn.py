@@ -68,6 +68,38 @@ def test_conv3x3_backward_weights(B, Cin, Cout, H, W):
     assert relerr(db.cpu().numpy(), R.conv3x3_bwd_weights(x, dy)[1]) < 1e-5
 
 
+# edges of the launch: strips of 256 pixels, 16-pixel and 32-pixel tiles,
+# channel groups of 8 and 16 (and the two groups of output-channel tiles), one
+# row, more rows than a work-group takes, pointers off 16 bytes.  FP32 sums of
+# at most 9 * 64 products (forward) or B H W products (gradients).
+EDGES = [(1, 1, 1, 1, 8), (1, 64, 64, 3, 257), (2, 33, 17, 9, 24), (1, 17, 64, 2, 40), (1, 56, 48, 5, 16),
+         (3, 40, 33, 300, 8), (1, 9, 49, 2, 515)]
+
+
+@pytest.mark.parametrize("B,Cin,Cout,H,W", EDGES)
+@pytest.mark.parametrize("offset", [0, 1])
+def test_conv3x3_edges(B, Cin, Cout, H, W, offset):
+    rng = np.random.default_rng(B + 3 * Cin + 5 * Cout + 7 * W)
+    x = rng.standard_normal((B, Cin, H, W)).astype(np.float32)
+    dy = rng.standard_normal((B, Cout, H, W)).astype(np.float32)
+    w = (rng.standard_normal((Cout, Cin, 3, 3)) / np.sqrt(9 * Cin)).astype(np.float32)
+
+    def shifted(a):
+        flat = torch.zeros(a.size + offset, dtype=torch.float32, device="cuda")
+        flat[offset:] = dev(a).reshape(-1)
+        return flat[offset:].view(a.shape)
+
+    y = ba.conv3x3(shifted(x), dev(w)).cpu().numpy()
+    assert relerr(y, R.conv3x3(R.bf16(x), R.bf16(w))) < 1e-5
+    dx = ba.conv3x3_bwd_data(shifted(dy), dev(w)).cpu().numpy()
+    assert relerr(dx, R.conv3x3_bwd_data(R.bf16(dy), R.bf16(w))) < 1e-5
+    if W % 8 or W > 256 or (Cout + 31) // 32 * ((9 * Cin + 31) // 32) > 32:
+        return
+    dw, db = ba.conv3x3_bwd_weights(shifted(x), shifted(dy))
+    assert relerr(dw.cpu().numpy(), R.conv3x3_bwd_weights(R.bf16(x), R.bf16(dy))[0]) < 1e-5
+    assert relerr(db.cpu().numpy(), R.conv3x3_bwd_weights(x, dy)[1]) < 1e-5
+
+
 def test_conv3x3_rejects_bad_shapes():
     x = torch.zeros((1, 65, 4, 64), device="cuda")
     w = torch.zeros((8, 65, 3, 3), device="cuda")
