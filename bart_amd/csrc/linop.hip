@@ -1837,8 +1837,7 @@ int lsqr_conjgrad_batch(int nprob, const struct linop_s* const ops[], int maxite
 					skip.push_back(&b.st.ptr[j].done);
 				}
 
-				std::vector<int> ng;
-				gset = normal_groups_build(plans, sens, src, dst, skip, ng);
+				gset = normal_groups_build(plans, sens, src, dst, skip);
 
 				for (size_t j = 0; j < mem.size(); j++) {
 					auto pr = normal_group_partials(*plans[j], dst[j]);

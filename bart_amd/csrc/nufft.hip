@@ -190,18 +190,6 @@ static void build_tables(Nufft& p)
 	}
 }
 
-__device__ inline float2 lin_val(const SepTables& T, int s, const int c[3])
-{
-	float2 v = make_float2(1.f, 0.f);
-
-#pragma unroll
-	for (int d = 0; d < 3; d++)
-		if (T.bitpos[d] >= 0)
-			v = cmul(v, T.lin[d][(s >> T.bitpos[d]) & 1][c[d]]);
-
-	return v;
-}
-
 __device__ inline float2 fm_val(const SepTables& T, const int c[3])
 {
 	float2 v = make_float2(1.f, 0.f);
@@ -214,143 +202,9 @@ __device__ inline float2 fm_val(const SepTables& T, const int c[3])
 	return v;
 }
 
-__device__ inline float roll_val(const SepTables& T, const int c[3])
-{
-	return T.roll[0][c[0]] * T.roll[1][c[1]] * T.roll[2][c[2]];
-}
-
-__device__ inline long pix_index(const SepTables& T, const int c[3])
-{
-	return c[0] + (long)T.n[0] * (c[1] + (long)T.n[1] * c[2]);
-}
-
-// ---------------------------------------------------------------------------
-// Geometry of the first axis with the sub-grid index fastest, then the coils
-// of a coil group, so that the S x cc transforms of one image row and coil
-// group share a work-group (for the sums over sub-grids and coils).
-// t = s + S (cl + cc (g + G o)), coil c = cl + cc g;
-// grid offset = (c + C s) N + o n + k.
-// ---------------------------------------------------------------------------
-
-struct GeomS {
-
-	VolAxis va;  // first active axis, nvol = S C (grid layout [s][c])
-	int S, C, cc, G;
-	FastDiv fS, fcc, fG;
-
-	static GeomS make(const int n[3], int axis, int S, int C, int cc)
-	{
-		GeomS g;
-		g.va = VolAxis::make(n, axis, (long)S * C);
-		g.S = S;
-		g.C = C;
-		g.cc = cc;
-		g.G = C / cc;
-		g.fS = FastDiv((uint32_t)S);
-		g.fcc = FastDiv((uint32_t)cc);
-		g.fG = FastDiv((uint32_t)g.G);
-		return g;
-	}
-
-	__device__ inline void split(long t, uint32_t& s, uint32_t& o, uint32_t& c) const
-	{
-		uint32_t q, q2, cl, gi;
-		fS.divmod((uint32_t)t, q, s);
-		fcc.divmod(q, q2, cl);
-		fG.divmod(q2, o, gi);
-		c = cl + (uint32_t)cc * gi;
-	}
-
-	__device__ inline long grid_offset(uint32_t s, uint32_t o, uint32_t c, int k) const
-	{
-		return ((long)c + (long)C * s) * va.N + (long)o * va.n[va.axis] + k;
-	}
-};
-
-// coils per reduction group: a power of two dividing C with S cc n <= 4096
-static int coil_group(int S, int C, int n, bool reduce_coils)
-{
-	if (!reduce_coils)
-		return 1;
-
-	int cc = 1;
-
-	while (0 == C % (2 * cc) && (long)S * 2 * cc * n <= 4096)
-		cc *= 2;
-
-	return cc;
-}
-
 // ---------------------------------------------------------------------------
 // Pass functors
 // ---------------------------------------------------------------------------
-
-// First forward pass: image side -> grid, x roll x linphase_s
-struct LdImgLin {
-	GeomS g;
-	SepTables T;
-	const float2* src;   // coil images [C][N] or single image [N] (with sens)
-	const float2* sens;  // [C][N] or null
-	bool roll;
-
-	__device__ float2 operator()(long t, int k) const
-	{
-		uint32_t s, o, c;
-		g.split(t, s, o, c);
-		int px[3];
-		g.va.coords(0, o, k, px);
-		long pi = pix_index(T, px);
-		float2 v;
-
-		if (nullptr != sens)
-			v = cmul(src[pi], sens[(long)c * g.va.N + pi]);
-		else
-			v = src[(long)c * g.va.N + pi];
-
-		if (roll)
-			v = cscale(v, roll_val(T, px));
-
-		return cmul(v, lin_val(T, (int)s, px));
-	}
-};
-
-// Plain grid loads in S-grouped order
-struct LdGridS {
-	GeomS g;
-	const float2* grid;
-
-	__device__ float2 operator()(long t, int k) const
-	{
-		uint32_t s, o, c;
-		g.split(t, s, o, c);
-		return grid[g.grid_offset(s, o, c, k)];
-	}
-};
-
-// Grid stores in S-grouped order (optionally x fftmod)
-struct StGridS {
-	GeomS g;
-	SepTables T;
-	float2* grid;
-	bool fm;
-
-	__device__ void put(long t, int k, float2 v) const
-	{
-		uint32_t s, o, c;
-		g.split(t, s, o, c);
-		if (fm) {
-			int px[3];
-			g.va.coords(0, o, k, px);
-			v = cmul(v, fm_val(T, px));
-		}
-		grid[g.grid_offset(s, o, c, k)] = v;
-	}
-
-	__device__ void store(const float2* lds, const FftLaunch& L, long t0) const
-	{
-		store_each(lds, L, t0, [&](long t, int k, float2 v) { put(t, k, v); });
-	}
-};
 
 // Standard-order grid loads / stores for the other axes
 // Column-block access (used by the fixed-length kernel on strided axes):
@@ -491,81 +345,6 @@ struct MdPsfPair {
 	}
 
 	__device__ float2 zf(int m, int k) const { return (0 == m) ? lz0[k] : lz1[k]; }
-};
-
-// PSF multiply in the S-grouped geometry (single active axis)
-struct MdPsfS {
-	static constexpr bool active = true;
-	GeomS g;
-	const float2* psf;
-
-	__device__ float2 operator()(long t, int k, float2 x) const
-	{
-		uint32_t s, o, c;
-		g.split(t, s, o, c);
-		return cmul(x, psf[(long)s * g.va.N + (long)o * g.va.n[g.va.axis] + k]);
-	}
-};
-
-// Last pass: sum_s conj(linphase_s) x (roll) -> image side.  With coil maps
-// the block also sums conj(sens_c) x over the cc coils of its group, in a
-// fixed order, and writes the group's partial image dst[g N + pixel] (the
-// groups are summed afterwards, also in a fixed order); without maps it
-// stores coil image c (cc = 1).  No atomics: the result is deterministic.
-struct StReduceS {
-	GeomS g;
-	SepTables T;
-	float2* dst;
-	const float2* sens;
-	bool roll;
-
-	__device__ void store(const float2* lds, const FftLaunch& L, long t0) const
-	{
-		const int n = L.plan.n;
-		const int S = g.S;
-		const int SC = S * g.cc;
-		const int groups = L.P / SC;
-
-		for (int i = threadIdx.x; i < groups * n; i += FFT_THREADS) {
-
-			int gi = i / n;
-			int k = i - gi * n;
-			long t = t0 + (long)gi * SC;
-
-			if (t >= L.total)
-				continue;
-
-			uint32_t s, o, c;
-			g.split(t, s, o, c);
-			int px[3];
-			g.va.coords(0, o, k, px);
-			long pi = pix_index(T, px);
-			const float r = roll ? roll_val(T, px) : 1.f;
-
-			float2 out = make_float2(0.f, 0.f);
-
-			for (int cl = 0; cl < g.cc; cl++) {
-
-				float2 acc = make_float2(0.f, 0.f);
-
-				for (int j = 0; j < S; j++)
-					acc = cadd(acc, cmulc(lds[(gi * SC + cl * S + j) * L.pitch + k], lin_val(T, j, px)));
-
-				if (roll)
-					acc = cscale(acc, r);
-
-				if (nullptr != sens)
-					out = cadd(out, cmulc(acc, sens[(long)(c + cl) * g.va.N + pi]));
-				else
-					out = acc;
-			}
-
-			if (nullptr != sens)
-				dst[(long)(c / g.cc) * g.va.N + pi] = out;
-			else
-				dst[(long)c * g.va.N + pi] = out;
-		}
-	}
 };
 
 // ---------------------------------------------------------------------------
@@ -1098,6 +877,8 @@ void Nufft::create(const int dims[3], int C_, long M_, const float* traj, const 
 	set_traj(M_, traj, weights_host, compute_psf);
 }
 
+static int merge_group(const Nufft& p);
+
 void Nufft::create_geometry(const int dims[3], int C_, bool toeplitz_, bool periodic_, float width_, float os_)
 {
 	BAM_CHECK(2.f == os_, "only oversampling 2 is supported (got %f)", os_);
@@ -1141,8 +922,10 @@ void Nufft::create_geometry(const int dims[3], int C_, bool toeplitz_, bool peri
 
 	build_tables(*this);
 
-	for (int j = 0; j < nact; j++)
+	for (int j = 0; j < nact; j++) {
 		axis[j] = make_axis_plan(n[act[j]]);
+		pair[j] = make_pair_plan(axis[j]);
+	}
 
 	// BART_AMD_SLICE=off selects the per-axis passes also where the x-y
 	// slices fit in LDS
@@ -1157,9 +940,9 @@ void Nufft::create_geometry(const int dims[3], int C_, bool toeplitz_, bool peri
 	grid.alloc((size_t)S * C * N);
 
 	// partial images of the coil groups of S^H (allocated here so that no
-	// allocation happens inside a captured CG iteration)
-	// partial images of the S^H sum: one per coil with the slice kernels
-	const int G = slice ? C : C / coil_group(S, C, n[act[0]], true);
+	// allocation happens inside a captured CG iteration); one per coil with
+	// the slice kernels
+	const int G = slice ? C : C / merge_group(*this);
 
 	if (G > 1)
 		part.alloc((size_t)G * N);
@@ -1228,6 +1011,220 @@ void Nufft::set_traj(long M_, const float* traj, const float2* weights_host, boo
 // Forward / adjoint / normal
 // ---------------------------------------------------------------------------
 
+// ---------------------------------------------------------------------------
+// Axis passes of the decomposition (see pair.hpp).  Axis j (of the active
+// ones) doubles the volumes: split takes the C 2^j volumes c + C s of the
+// grid (axis 0: the image side) to C 2^(j + 1), merge back.  Lengths beyond
+// the pair kernels (over PF_MAXN, or no three radices) run the element-wise
+// steps and the plain transform one after the other.
+// ---------------------------------------------------------------------------
+
+// coils per partial image of the last merge: the most that leave 4096 waves
+// (16 per compute unit) to share the work; the partial images cost a pass
+// over G N values in all
+static int merge_group(const Nufft& p)
+{
+	const PairPlan& pl = p.pair[0];
+	const long lanes = (p.N / p.n[p.act[0]]) * std::max(1, pl.NJ);
+	int cc = 1;
+
+	if (0 == pl.nr)
+		return 1;
+
+	for (int c = 2; c <= p.C; c++)
+		if (0 == p.C % c && lanes * (p.C / c) >= 4096l * 64)
+			cc = c;
+
+	return cc;
+}
+
+static PairArgs pair_args(const Nufft& p, int j, const int* skip)
+{
+	PairArgs a = {};
+	a.pl = p.pair[j];
+	a.va = VolAxis::make(p.n, p.act[j], (0 == j) ? 1 : ((long)p.C << j));
+	a.skip = skip;
+	a.l[0] = p.tabs.lin[p.act[j]][0];
+	a.l[1] = p.tabs.lin[p.act[j]][1];
+	a.grid = p.grid.ptr;
+	a.half = ((long)p.C << j) * p.N;
+	a.C = p.C;
+	a.cc = 1;
+	return a;
+}
+
+static PairArgs rows_split_args(const Nufft& p, const float2* src, const float2* sens, bool roll, bool fm,
+				const int* skip)
+{
+	PairArgs a = pair_args(p, 0, skip);
+	a.src = src;
+	a.sens = sens;
+	for (int d = 0; d < 3; d++) {
+		a.roll[d] = roll ? p.tabs.roll[d] : nullptr;
+		a.fm[d] = fm ? p.tabs.fm[d] : nullptr;
+	}
+	pair_geometry(a, true, (uint32_t)p.C);
+	return a;
+}
+
+static PairArgs rows_merge_args(const Nufft& p, float2* dst, const float2* sens, bool roll, const int* skip)
+{
+	PairArgs a = pair_args(p, 0, skip);
+	a.dst = dst;
+	a.sens = sens;
+	a.cc = (nullptr != sens) ? merge_group(p) : 1;
+	for (int d = 0; d < 3; d++)
+		a.roll[d] = roll ? p.tabs.roll[d] : nullptr;
+	pair_geometry(a, true, (uint32_t)(p.C / a.cc));
+	return a;
+}
+
+static PairArgs turn_args(const Nufft& p, const int* skip)
+{
+	const int j = p.nact - 1;
+	PairArgs a = pair_args(p, j, skip);
+	a.psf = p.psf.ptr;
+	a.psf_half = (1l << j) * p.N;
+	pair_geometry(a, false, 0);
+	return a;
+}
+
+// Element-wise steps of lengths without a pair kernel; l: the two linear
+// phases of axis g.axis; member b at + b half.
+__global__ void k_long_expand(VolAxis g, SepTables T, const float2* src, const float2* sens, bool roll, long nvol,
+			      const float2* l0, const float2* l1, float2* grid, long half, const int* skip)
+{
+	if (nullptr != skip && 0 != *skip)
+		return;
+
+	const long tot = nvol * g.N;
+
+	for (long e = (long)blockIdx.x * blockDim.x + threadIdx.x; e < tot; e += (long)gridDim.x * blockDim.x) {
+
+		const long px = e % g.N;
+		const int c[3] = { (int)(px % g.n[0]), (int)((px / g.n[0]) % g.n[1]), (int)(px / ((long)g.n[0] * g.n[1])) };
+		const int k = c[g.axis];
+		float2 h = (nullptr == src) ? grid[e] : ((nullptr != sens) ? cmul(src[px], sens[e]) : src[e]);
+
+		if (roll)
+			h = cscale(h, T.roll[0][c[0]] * T.roll[1][c[1]] * T.roll[2][c[2]]);
+
+		grid[e] = cmul(h, l0[k]);
+		grid[e + half] = cmul(h, l1[k]);
+	}
+}
+
+// dst: the image side (coil images, or with sens one partial image per coil);
+// null: in place
+__global__ void k_long_reduce(VolAxis g, SepTables T, float2* dst, const float2* sens, bool roll, long nvol,
+			      const float2* l0, const float2* l1, float2* grid, long half, const int* skip)
+{
+	if (nullptr != skip && 0 != *skip)
+		return;
+
+	const long tot = nvol * g.N;
+
+	for (long e = (long)blockIdx.x * blockDim.x + threadIdx.x; e < tot; e += (long)gridDim.x * blockDim.x) {
+
+		const long px = e % g.N;
+		const int c[3] = { (int)(px % g.n[0]), (int)((px / g.n[0]) % g.n[1]), (int)(px / ((long)g.n[0] * g.n[1])) };
+		const int k = c[g.axis];
+		float2 v = cadd(cmulc(grid[e], l0[k]), cmulc(grid[e + half], l1[k]));
+
+		if (roll)
+			v = cscale(v, T.roll[0][c[0]] * T.roll[1][c[1]] * T.roll[2][c[2]]);
+
+		if (nullptr == dst)
+			grid[e] = v;
+		else
+			dst[e] = (nullptr != sens) ? cmulc(v, sens[e]) : v;
+	}
+}
+
+static void long_fft(const Nufft& p, int j, float sign, bool fm, const int* skip, const char* name)
+{
+	VolAxis va = VolAxis::make(p.n, p.act[j], (long)p.C << (j + 1));
+	FftLaunchCfg cfg = fft_config(p.axis[j], va.transforms(), va.contig(), 1, sign, sign);
+	cfg.L.skip = skip;
+	cfg.name = name;
+	LdGrid ld{ va, p.grid.ptr };
+	StGrid st{ va, p.tabs, p.grid.ptr, fm };
+	launch_fft_axis(cfg, p.stream, ld, NoMid{}, st);
+}
+
+// the image side's forms: src / dst non-null on axis 0 only
+static void axis_split(const Nufft& p, int j, const float2* src, const float2* sens, bool roll, bool fm,
+		       const int* skip, const char* name)
+{
+	if (p.pair[j].nr > 0) {
+
+		if (0 == j) {
+			pair_launch(PF_SPLIT, true, rows_split_args(p, src, sens, roll, fm, skip), name, p.stream);
+			return;
+		}
+
+		PairArgs a = pair_args(p, j, skip);
+		for (int d = 0; d < 3; d++)
+			a.fm[d] = fm ? p.tabs.fm[d] : nullptr;
+		pair_geometry(a, false, 0);
+		pair_launch(PF_SPLIT, false, a, name, p.stream);
+		return;
+	}
+
+	const PairArgs a = pair_args(p, j, skip);
+	const long nvol = (long)p.C << j;
+	hipLaunchKernelGGL(k_long_expand, dim3((unsigned)std::min<long>((nvol * p.N + 255) / 256, 65536)), dim3(256), 0,
+			   p.stream, a.va, p.tabs, src, sens, roll, nvol, a.l[0], a.l[1], a.grid, a.half, skip);
+	BAM_HIP(hipGetLastError());
+	long_fft(p, j, -1.f, fm, skip, name);
+}
+
+static void axis_merge(const Nufft& p, int j, float2* dst, const float2* sens, bool roll, const int* skip,
+		       const char* name)
+{
+	if (p.pair[j].nr > 0) {
+
+		if (0 == j) {
+			pair_launch(PF_MERGE, true, rows_merge_args(p, dst, sens, roll, skip), name, p.stream);
+			return;
+		}
+
+		PairArgs a = pair_args(p, j, skip);
+		pair_geometry(a, false, 0);
+		pair_launch(PF_MERGE, false, a, name, p.stream);
+		return;
+	}
+
+	long_fft(p, j, +1.f, false, skip, name);
+	const PairArgs a = pair_args(p, j, skip);
+	const long nvol = (long)p.C << j;
+	hipLaunchKernelGGL(k_long_reduce, dim3((unsigned)std::min<long>((nvol * p.N + 255) / 256, 65536)), dim3(256), 0,
+			   p.stream, a.va, p.tabs, dst, sens, roll, nvol, a.l[0], a.l[1], a.grid, a.half, skip);
+	BAM_HIP(hipGetLastError());
+}
+
+// the S transforms of a row of the first axis have always had to fit the
+// FFT's LDS block
+static void check_first_axis(const Nufft& p)
+{
+	BAM_CHECK((long)p.S * p.n[p.act[0]] <= FFT_MAX_ELEMS, "FFT block of %d x %d exceeds LDS budget", p.S,
+		  p.n[p.act[0]]);
+}
+
+// partial images of S^H: their number, and where the last merge writes
+static float2* merge_target(Nufft& p, float2* dst, const float2* sens, int& G)
+{
+	G = (nullptr != sens) ? p.C / merge_group(p) : 1;
+
+	if (G <= 1)
+		return dst;
+
+	if ((long)p.part.n < (long)G * p.N)
+		p.part.alloc((size_t)G * p.N);
+
+	return p.part.ptr;
+}
+
 // z axis of the sub-grid stack (slice path).  pair: the stack is read
 // (forward) or written (adjoint) as the S/2 pair volumes of the slice
 // kernels' zpair mode -- forward: volume s holds H, the x-y transform shared
@@ -1292,28 +1289,11 @@ void Nufft::forward(float2* ksp, const float2* src, const float2* sens)
 		return;
 	}
 
-	const int a0 = act[0];
+	check_first_axis(*this);
+	axis_split(*this, 0, src, sens, true, 1 == nact, nullptr, "fft_fwd_first");
 
-	// first axis: image side -> grid (x roll x linphase), FFT
-	{
-		int cc = coil_group(S, C, n[a0], nullptr != sens);
-		GeomS gs = GeomS::make(n, a0, S, C, cc);
-		FftLaunchCfg cfg = fft_config(axis[0], gs.va.transforms(), true, S * cc, -1.f, -1.f);
-		cfg.name = "fft_fwd_first";
-		LdImgLin ld{ gs, tabs, src, sens, true };
-		StGridS st{ gs, tabs, grid.ptr, 1 == nact };
-		launch_fft_axis(cfg, stream, ld, NoMid{}, st);
-	}
-
-	for (int j = 1; j < nact; j++) {
-
-		VolAxis va = VolAxis::make(n, act[j], (long)S * C);
-		FftLaunchCfg cfg = fft_config(axis[j], va.transforms(), va.contig(), 1, -1.f, -1.f);
-		cfg.name = "fft_fwd_axis";
-		LdGrid ld{ va, grid.ptr };
-		StGrid st{ va, tabs, grid.ptr, j == nact - 1 };
-		launch_fft_axis(cfg, stream, ld, NoMid{}, st);
-	}
+	for (int j = 1; j < nact; j++)
+		axis_split(*this, j, nullptr, nullptr, false, j == nact - 1, nullptr, "fft_fwd_axis");
 
 	grid_forward(gp, kb.ptr, ksp, grid.ptr, has_weights ? weights.ptr : nullptr, stream);
 }
@@ -1339,32 +1319,14 @@ void Nufft::adjoint(float2* dst, const float2* ksp, const float2* sens)
 		return;
 	}
 
-	for (int j = nact - 1; j >= 1; j--) {
+	check_first_axis(*this);
 
-		VolAxis va = VolAxis::make(n, act[j], (long)S * C);
-		FftLaunchCfg cfg = fft_config(axis[j], va.transforms(), va.contig(), 1, +1.f, +1.f);
-		cfg.name = "fft_adj_axis";
-		LdGrid ld{ va, grid.ptr };
-		StGrid st{ va, tabs, grid.ptr, false };
-		launch_fft_axis(cfg, stream, ld, NoMid{}, st);
-	}
+	for (int j = nact - 1; j >= 1; j--)
+		axis_merge(*this, j, nullptr, nullptr, false, nullptr, "fft_adj_axis");
 
-	const int cc = coil_group(S, C, n[act[0]], nullptr != sens);
-	const int G = C / cc;
-	GeomS gs = GeomS::make(n, act[0], S, C, cc);
-	FftLaunchCfg cfg = fft_config(axis[0], gs.va.transforms(), true, S * cc, +1.f, +1.f);
-	cfg.name = "fft_adj_last";
-	LdGridS ld{ gs, grid.ptr };
-	float2* out = dst;
-
-	if (nullptr != sens && G > 1) {
-		if ((long)part.n < (long)G * N)
-			part.alloc((size_t)G * N);
-		out = part.ptr;
-	}
-
-	StReduceS st{ gs, tabs, out, sens, true };
-	launch_fft_axis(cfg, stream, ld, NoMid{}, st);
+	int G;
+	float2* out = merge_target(*this, dst, sens, G);
+	axis_merge(*this, 0, out, sens, true, nullptr, "fft_adj_last");
 
 	if (out != dst)
 		sum_groups(dst, part.ptr, N, G, stream, nullptr);
@@ -1434,66 +1396,30 @@ bool Nufft::normal(float2* dst, const float2* src, const float2* sens, const int
 		return false;
 	}
 
-	const int cc = coil_group(S, C, n[act[0]], nullptr != sens);
-	const int G = C / cc;
-	GeomS gs = GeomS::make(n, act[0], S, C, cc);
-	float2* out = dst;
+	check_first_axis(*this);
+	int G;
+	float2* out = merge_target(*this, dst, sens, G);
+	const int last = nact - 1;
 
-	if (nullptr != sens && G > 1) {
-		if ((long)part.n < (long)G * N)
-			part.alloc((size_t)G * N);
-		out = part.ptr;
+	axis_split(*this, 0, src, sens, false, false, skip, "fft_toeplitz_fwd");
+
+	for (int j = 1; j < last; j++)
+		axis_split(*this, j, nullptr, nullptr, false, false, skip, "fft_toeplitz_fwd");
+
+	if (last > 0 && pair[last].nr > 0) {
+		pair_launch(PF_TURN, false, turn_args(*this, skip), "fft_toeplitz", stream);
+	} else {
+		if (last > 0)
+			axis_split(*this, last, nullptr, nullptr, false, false, skip, "fft_toeplitz_fwd");
+		basis_psf_apply(grid.ptr, psf.ptr, S, C, 1, N, stream, skip);
+		if (last > 0)
+			axis_merge(*this, last, nullptr, nullptr, false, skip, "fft_toeplitz_inv");
 	}
 
-	if (1 == nact) {
+	for (int j = last - 1; j >= 1; j--)
+		axis_merge(*this, j, nullptr, nullptr, false, skip, "fft_toeplitz_inv");
 
-		FftLaunchCfg cfg = fft_config_skip(skip, axis[0], gs.va.transforms(), true, S * cc, -1.f, +1.f);
-		LdImgLin ld{ gs, tabs, src, sens, false };
-		MdPsfS md{ gs, psf.ptr };
-		StReduceS st{ gs, tabs, out, sens, false };
-		launch_fft_axis(cfg, stream, ld, md, st);
-
-		if (out != dst)
-			return sum_groups_or_fuse(dst, part.ptr, N, G, stream, skip, fuse);
-		return false;
-	}
-
-	{
-		FftLaunchCfg cfg = fft_config_skip(skip, axis[0], gs.va.transforms(), true, S * cc, -1.f, -1.f);
-		LdImgLin ld{ gs, tabs, src, sens, false };
-		StGridS st{ gs, tabs, grid.ptr, false };
-		launch_fft_axis(cfg, stream, ld, NoMid{}, st);
-	}
-
-	for (int j = 1; j < nact; j++) {
-
-		VolAxis va = VolAxis::make(n, act[j], (long)S * C);
-		LdGrid ld{ va, grid.ptr };
-		StGrid st{ va, tabs, grid.ptr, false };
-
-		if (j == nact - 1) {
-			FftLaunchCfg cfg = fft_config_skip(skip, axis[j], va.transforms(), va.contig(), 1, -1.f, +1.f);
-			MdPsf md{ va, C, psf.ptr };
-			launch_fft_axis(cfg, stream, ld, md, st);
-		} else {
-			FftLaunchCfg cfg = fft_config_skip(skip, axis[j], va.transforms(), va.contig(), 1, -1.f, -1.f);
-			launch_fft_axis(cfg, stream, ld, NoMid{}, st);
-		}
-	}
-
-	for (int j = nact - 2; j >= 1; j--) {
-
-		VolAxis va = VolAxis::make(n, act[j], (long)S * C);
-		FftLaunchCfg cfg = fft_config_skip(skip, axis[j], va.transforms(), va.contig(), 1, +1.f, +1.f);
-		LdGrid ld{ va, grid.ptr };
-		StGrid st{ va, tabs, grid.ptr, false };
-		launch_fft_axis(cfg, stream, ld, NoMid{}, st);
-	}
-
-	FftLaunchCfg cfg = fft_config_skip(skip, axis[0], gs.va.transforms(), true, S * cc, +1.f, +1.f);
-	LdGridS ld{ gs, grid.ptr };
-	StReduceS st{ gs, tabs, out, sens, false };
-	launch_fft_axis(cfg, stream, ld, NoMid{}, st);
+	axis_merge(*this, 0, out, sens, false, skip, "fft_toeplitz_inv");
 
 	if (out != dst)
 		return sum_groups_or_fuse(dst, part.ptr, N, G, stream, skip, fuse);
@@ -1544,44 +1470,18 @@ void Nufft::normal_basis(float2* dst, const float2* src, const int* skip)
 		return;
 	}
 
-	const int cc = coil_group(S, C, n[act[0]], false);
-	GeomS gs = GeomS::make(n, act[0], S, C, cc);
+	check_first_axis(*this);
+	axis_split(*this, 0, src, nullptr, false, false, skip, "fft_toeplitz_basis_first");
 
-	{
-		FftLaunchCfg cfg = fft_config_skip(skip, axis[0], gs.va.transforms(), true, S * cc, -1.f, -1.f);
-		cfg.name = "fft_toeplitz_basis_first";
-		LdImgLin ld{ gs, tabs, src, nullptr, false };
-		StGridS st{ gs, tabs, grid.ptr, false };
-		launch_fft_axis(cfg, stream, ld, NoMid{}, st);
-	}
-
-	for (int j = 1; j < nact; j++) {
-
-		VolAxis va = VolAxis::make(n, act[j], (long)S * C);
-		FftLaunchCfg cfg = fft_config_skip(skip, axis[j], va.transforms(), va.contig(), 1, -1.f, -1.f);
-		cfg.name = "fft_toeplitz_basis_fwd";
-		LdGrid ld{ va, grid.ptr };
-		StGrid st{ va, tabs, grid.ptr, false };
-		launch_fft_axis(cfg, stream, ld, NoMid{}, st);
-	}
+	for (int j = 1; j < nact; j++)
+		axis_split(*this, j, nullptr, nullptr, false, false, skip, "fft_toeplitz_basis_fwd");
 
 	basis_psf_apply(grid.ptr, psf.ptr, S, Cc, nbasis, N, stream, skip);
 
-	for (int j = nact - 1; j >= 1; j--) {
+	for (int j = nact - 1; j >= 1; j--)
+		axis_merge(*this, j, nullptr, nullptr, false, skip, "fft_toeplitz_basis_inv");
 
-		VolAxis va = VolAxis::make(n, act[j], (long)S * C);
-		FftLaunchCfg cfg = fft_config_skip(skip, axis[j], va.transforms(), va.contig(), 1, +1.f, +1.f);
-		cfg.name = "fft_toeplitz_basis_inv";
-		LdGrid ld{ va, grid.ptr };
-		StGrid st{ va, tabs, grid.ptr, false };
-		launch_fft_axis(cfg, stream, ld, NoMid{}, st);
-	}
-
-	FftLaunchCfg cfg = fft_config_skip(skip, axis[0], gs.va.transforms(), true, S * cc, +1.f, +1.f);
-	cfg.name = "fft_toeplitz_basis_last";
-	LdGridS ld{ gs, grid.ptr };
-	StReduceS st{ gs, tabs, dst, nullptr, false };
-	launch_fft_axis(cfg, stream, ld, NoMid{}, st);
+	axis_merge(*this, 0, dst, nullptr, false, skip, "fft_toeplitz_basis_last");
 }
 
 // ---------------------------------------------------------------------------
@@ -1686,24 +1586,22 @@ void Nufft::apply_precond(const float2* pre, float2* dst, const float2* src, int
 // Normal operators of many 2-D plans in one launch per pass (batched CG)
 // ---------------------------------------------------------------------------
 
-// The three passes of Nufft::normal's 2-D path (first axis with maps and
-// linear phases; second axis, PSF, inverse; first axis back with the sums
-// over sub-grids and coil groups) for every plan of a size class, each pass
-// one launch of k_fft_axis_n_batch: the same work-groups, functors and
-// arithmetic as the plans' own launches, so the results are the same bits.
+// The three passes of Nufft::normal's 2-D path (split of the first axis with
+// maps, turn of the second, merge of the first with the sums over coil
+// groups) for every plan, each pass one launch for the lengths of at most two
+// radices and one for the others: the same work-groups and arithmetic as the
+// plans' own launches, so the results are the same bits.
 struct NormalGroupSet {
 
-	struct Group {
-		int n0, n1;      // transform lengths of the first and second axis
-		int nb[3] = { 0, 0, 0 };
-		size_t lds[3] = { 0, 0, 0 };
-		DevBuf<FftItem<LdImgLin, NoMid, StGridS>> it1;
-		DevBuf<FftItem<LdGrid, MdPsf, StGrid>> it2;
-		DevBuf<FftItem<LdGridS, NoMid, StReduceS>> it3;
-		DevBuf<int2> bt[3];
+	struct Pass {
+		int nb = 0;
+		unsigned threads = 0;
+		size_t lds = 0;
+		DevBuf<PairArgs> items;
+		DevBuf<int2> bt;
 	};
 
-	std::vector<Group> groups;
+	Pass pass[3][2];  // [pass][three radices]
 };
 
 bool normal_groupable(const Nufft& p, const float2* sens)
@@ -1711,117 +1609,80 @@ bool normal_groupable(const Nufft& p, const float2* sens)
 	if (2 != p.nact || p.slice || !p.toeplitz || !p.has_psf || nullptr == sens || p.nbasis > 0)
 		return false;
 
-	const int S = p.S, C = p.C;
-	const int cc = coil_group(S, C, p.n[p.act[0]], true);
-	GeomS gs = GeomS::make(p.n, p.act[0], S, C, cc);
-	VolAxis va = VolAxis::make(p.n, p.act[1], (long)S * C);
-	const FftLaunchCfg c1 = fft_config(p.axis[0], gs.va.transforms(), true, S * cc, -1.f, -1.f);
-	const FftLaunchCfg c2 = fft_config(p.axis[1], va.transforms(), va.contig(), 1, -1.f, +1.f);
-	return c1.fixed && c2.fixed && (C / cc <= 1 || (long)p.part.n >= (long)(C / cc) * p.N);
+	if (0 == p.pair[0].nr || 0 == p.pair[1].nr || (long)p.S * p.n[p.act[0]] > FFT_MAX_ELEMS)
+		return false;
+
+	const int G = p.C / merge_group(p);
+	return G <= 1 || (long)p.part.n >= (long)G * p.N;
 }
 
 std::shared_ptr<NormalGroupSet> normal_groups_build(const std::vector<const Nufft*>& plans,
 						    const std::vector<const float2*>& sens,
 						    const std::vector<const float2*>& src, const std::vector<float2*>& dst,
-						    const std::vector<const int*>& skip, std::vector<int>& ngroups_out)
+						    const std::vector<const int*>& skip)
 {
 	auto set = std::make_shared<NormalGroupSet>();
-	std::vector<int> key_n0, key_n1;
-	std::vector<std::vector<int>> members;
+	std::vector<PairArgs> items[3][2];
 
 	for (size_t q = 0; q < plans.size(); q++) {
+
 		const Nufft& p = *plans[q];
-		const int n0 = p.n[p.act[0]], n1 = p.n[p.act[1]];
-		size_t g = 0;
-		while (g < members.size() && !(key_n0[g] == n0 && key_n1[g] == n1))
-			g++;
-		if (g == members.size()) {
-			key_n0.push_back(n0);
-			key_n1.push_back(n1);
-			members.emplace_back();
-		}
-		members[g].push_back((int)q);
-	}
+		float2* out = (p.C / merge_group(p) > 1) ? p.part.ptr : dst[q];
+		const PairArgs a[3] = { rows_split_args(p, src[q], sens[q], false, false, skip[q]), turn_args(p, skip[q]),
+					rows_merge_args(p, out, sens[q], false, skip[q]) };
 
-	set->groups.resize(members.size());
-	ngroups_out.assign(plans.size(), -1);
-
-	for (size_t g = 0; g < members.size(); g++) {
-
-		NormalGroupSet::Group& G = set->groups[g];
-		G.n0 = key_n0[g];
-		G.n1 = key_n1[g];
-		std::vector<FftItem<LdImgLin, NoMid, StGridS>> h1;
-		std::vector<FftItem<LdGrid, MdPsf, StGrid>> h2;
-		std::vector<FftItem<LdGridS, NoMid, StReduceS>> h3;
-		std::vector<int2> b1, b2, b3;
-
-		for (int j = 0; j < (int)members[g].size(); j++) {
-
-			const int q = members[g][j];
-			const Nufft& p = *plans[q];
-			const int S = p.S, C = p.C;
-			const int cc = coil_group(S, C, p.n[p.act[0]], true);
-			const int Gc = C / cc;
-			GeomS gs = GeomS::make(p.n, p.act[0], S, C, cc);
-			float2* out = (Gc > 1) ? p.part.ptr : dst[q];
-
-			FftLaunchCfg c1 = fft_config_skip(skip[q], p.axis[0], gs.va.transforms(), true, S * cc, -1.f, -1.f);
-			h1.push_back({ c1.L, LdImgLin{ gs, p.tabs, src[q], sens[q], false }, NoMid{},
-				       StGridS{ gs, p.tabs, p.grid.ptr, false } });
-
-			VolAxis va = VolAxis::make(p.n, p.act[1], (long)S * C);
-			FftLaunchCfg c2 = fft_config_skip(skip[q], p.axis[1], va.transforms(), va.contig(), 1, -1.f, +1.f);
-			h2.push_back({ c2.L, LdGrid{ va, p.grid.ptr }, MdPsf{ va, C, p.psf.ptr },
-				       StGrid{ va, p.tabs, p.grid.ptr, false } });
-
-			FftLaunchCfg c3 = fft_config_skip(skip[q], p.axis[0], gs.va.transforms(), true, S * cc, +1.f, +1.f);
-			h3.push_back({ c3.L, LdGridS{ gs, p.grid.ptr }, NoMid{}, StReduceS{ gs, p.tabs, out, sens[q], false } });
-
-			const FftLaunchCfg* cf[3] = { &c1, &c2, &c3 };
-			std::vector<int2>* bt[3] = { &b1, &b2, &b3 };
-			for (int ph = 0; ph < 3; ph++) {
-				BAM_CHECK(cf[ph]->fixed, "grouped normal: pass without a fixed-length kernel");
-				G.lds[ph] = std::max(G.lds[ph], cf[ph]->lds_bytes);
-				for (unsigned b = 0; b < cf[ph]->blocks; b++)
-					bt[ph]->push_back(make_int2(j, (int)b));
-			}
-
-			ngroups_out[q] = (int)g;
-		}
-
-		G.it1.alloc(h1.size());
-		G.it2.alloc(h2.size());
-		G.it3.alloc(h3.size());
-		BAM_HIP(hipMemcpy(G.it1.ptr, h1.data(), sizeof(h1[0]) * h1.size(), hipMemcpyHostToDevice));
-		BAM_HIP(hipMemcpy(G.it2.ptr, h2.data(), sizeof(h2[0]) * h2.size(), hipMemcpyHostToDevice));
-		BAM_HIP(hipMemcpy(G.it3.ptr, h3.data(), sizeof(h3[0]) * h3.size(), hipMemcpyHostToDevice));
-		const std::vector<int2>* bv[3] = { &b1, &b2, &b3 };
 		for (int ph = 0; ph < 3; ph++) {
-			G.nb[ph] = (int)bv[ph]->size();
-			G.bt[ph].alloc(bv[ph]->size());
-			BAM_HIP(hipMemcpy(G.bt[ph].ptr, bv[ph]->data(), sizeof(int2) * bv[ph]->size(), hipMemcpyHostToDevice));
+			const int cl = (3 == a[ph].pl.nr) ? 1 : 0;
+			NormalGroupSet::Pass& P = set->pass[ph][cl];
+			P.threads = std::max(P.threads, pair_threads(a[ph], 1 != ph));
+			P.lds = std::max(P.lds, pair_lds_bytes(a[ph], 1 != ph));
+			items[ph][cl].push_back(a[ph]);
 		}
 	}
+
+	for (int ph = 0; ph < 3; ph++)
+		for (int cl = 0; cl < 2; cl++) {
+
+			NormalGroupSet::Pass& P = set->pass[ph][cl];
+			const std::vector<PairArgs>& it = items[ph][cl];
+			std::vector<int2> bt;
+
+			for (size_t i = 0; i < it.size(); i++)
+				for (uint32_t b = 0; b < it[i].nblk; b++)
+					bt.push_back(make_int2((int)i, (int)b));
+
+			P.nb = (int)bt.size();
+
+			if (0 == P.nb)
+				continue;
+
+			P.items.alloc(it.size());
+			P.bt.alloc(bt.size());
+			BAM_HIP(hipMemcpy(P.items.ptr, it.data(), sizeof(PairArgs) * it.size(), hipMemcpyHostToDevice));
+			BAM_HIP(hipMemcpy(P.bt.ptr, bt.data(), sizeof(int2) * bt.size(), hipMemcpyHostToDevice));
+		}
 
 	return set;
 }
 
 void normal_groups_launch(const NormalGroupSet& set, hipStream_t st)
 {
-	for (const NormalGroupSet::Group& G : set.groups) {
-		launch_fft_axis_batch(G.n0, G.it1.ptr, G.bt[0].ptr, G.nb[0], G.lds[0], st, "fft_toeplitz_fwd");
-		launch_fft_axis_batch(G.n1, G.it2.ptr, G.bt[1].ptr, G.nb[1], G.lds[1], st, "fft_toeplitz");
-		launch_fft_axis_batch(G.n0, G.it3.ptr, G.bt[2].ptr, G.nb[2], G.lds[2], st, "fft_toeplitz_inv");
-	}
+	static const char* name[3] = { "fft_toeplitz_fwd", "fft_toeplitz", "fft_toeplitz_inv" };
+	static const int mode[3] = { PF_SPLIT, PF_TURN, PF_MERGE };
+
+	for (int ph = 0; ph < 3; ph++)
+		for (int cl = 0; cl < 2; cl++) {
+			const NormalGroupSet::Pass& P = set.pass[ph][cl];
+			pair_launch_batch(mode[ph], 1 != ph, 1 == cl, P.items.ptr, P.bt.ptr, P.nb, P.threads, P.lds, name[ph],
+					  st);
+		}
 }
 
 // the partial images of a plan's grouped normal operator: (pointer, groups)
 std::pair<const float2*, int> normal_group_partials(const Nufft& p, float2* dst)
 {
-	const int cc = coil_group(p.S, p.C, p.n[p.act[0]], true);
-	const int Gc = p.C / cc;
-	return (Gc > 1) ? std::make_pair((const float2*)p.part.ptr, Gc) : std::make_pair((const float2*)dst, 1);
+	const int G = p.C / merge_group(p);
+	return (G > 1) ? std::make_pair((const float2*)p.part.ptr, G) : std::make_pair((const float2*)dst, 1);
 }
 
 // ---------------------------------------------------------------------------

@@ -3,6 +3,7 @@
 
 #include "common.hpp"
 #include "fft.hpp"
+#include "pair.hpp"
 #include "volume.hpp"
 
 #include <complex>
@@ -201,6 +202,7 @@ struct Nufft {
 	DevBuf<float2> grid;   // work [S][C][N]
 	DevBuf<float2> part;   // per-coil-group partial images [G][N]
 	AxisPlan axis[3];
+	PairPlan pair[3];      // of the active axes (nr = 0: no pair kernel)
 	bool slice = false;    // 3-D with x-y slices transformed in LDS
 	bool pair_zpass = false;  // Toeplitz z-pass over sub-grid pairs (slice path)
 
@@ -318,18 +320,18 @@ struct Chain {
 };
 
 // Normal operators of several 2-D Toeplitz plans with coil maps, one launch
-// per pass and size class (batched CG).  normal_groupable: whether plan p
-// (with maps sens) can join; normal_groups_build: device tables for
-// plans[q] applied to src[q] -> dst[q] (or its partial images), skip flags
-// per plan, ngroups[q] = its size class; normal_groups_launch: the passes;
-// normal_group_partials: the partial images a plan's passes leave and their
-// count (dst itself and 1 without coil groups), to be summed by the caller.
+// per pass for all sizes (batched CG).  normal_groupable: whether plan p (with
+// maps sens) can join; normal_groups_build: device tables for plans[q]
+// applied to src[q] -> dst[q] (or its partial images), skip flags per plan;
+// normal_groups_launch: the passes; normal_group_partials: the partial images
+// a plan's passes leave and their count (dst itself and 1 without coil
+// groups), to be summed by the caller.
 struct NormalGroupSet;
 bool normal_groupable(const Nufft& p, const float2* sens);
 std::shared_ptr<NormalGroupSet> normal_groups_build(const std::vector<const Nufft*>& plans,
 						    const std::vector<const float2*>& sens,
 						    const std::vector<const float2*>& src, const std::vector<float2*>& dst,
-						    const std::vector<const int*>& skip, std::vector<int>& ngroups);
+						    const std::vector<const int*>& skip);
 void normal_groups_launch(const NormalGroupSet& set, hipStream_t st);
 std::pair<const float2*, int> normal_group_partials(const Nufft& p, float2* dst);
 
