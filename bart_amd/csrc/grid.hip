@@ -9,9 +9,9 @@
 //   * adjoint (k-space -> grid) is output-stationary: a work-group owns a tile
 //     of all sub-grids for a group of coils, each wave a block of every
 //     sub-grid (in 3-d 2 x 2 x 2 points = a 4 x 4 x 4 block of the 2x grid),
-//     each lane one output in registers; a wave walks only the samples that
-//     reach its block, with the coil values as wave-uniform loads.  There
-//     are no atomics and no zero-fill of the grid;
+//     accumulated on the matrix cores; a wave walks only the samples that
+//     reach its block, four at a time.  There are no atomics and no zero-fill
+//     of the grid;
 //   * forward (grid -> k-space): a thread per sample gathers its taps in
 //     cell-sorted order and stores k-space at the original positions.
 #include "nufft_impl.hpp"
@@ -84,8 +84,13 @@ __device__ inline float2 apply_conj_fm(const GridGeom& g, float2 v, int x, int y
 
 constexpr int MAX_RANGES = 256;
 
-// visits (samples of a tile's cells and their ring) per adjoint work item
+// visits (samples of a tile's cells and their ring) per adjoint work item at
+// most, and at least where a tile is split.  Every part costs a partial tile
+// written and read, but a longer item is a longer chain of 32-bit sums: the
+// 128^3 kooshball with 16 coils takes 4.34 ms at 2048 visits and 4.20 ms at
+// 8192, with an error against 64 bits of 1.8e-7 and 5.5e-7.
 constexpr int ADJ_MAXV = 2048;
+constexpr int ADJ_MINV = 512;
 
 // sample position on the grid, pos = os (k + shift) + n / 2, rounded as
 // noncart/grid.c:181-187 rounds it (the device twin is grid_pos)
@@ -119,7 +124,7 @@ static GridTiling choose_tiling(const GridGeom& g)
 
 	for (int d = 0; d < 3; d++) {
 
-		t.eoff[d] = -1;
+		t.eoff[d] = 0;
 
 		if (1 == g.n[d]) {
 			t.T[d] = 1;
@@ -129,19 +134,22 @@ static GridTiling choose_tiling(const GridGeom& g)
 			k++;
 			t.b[d] = bdim;
 			t.T[d] = std::min(want, ((g.n[d] + bdim - 1) / bdim) * bdim);
+			t.act[t.nd++] = d;
 			t.eoff[d] = e;
-			e += 2 * t.T[d];
+			e += 2 * ((t.T[d] + 3) / 4 * 4);
 		}
+
+		t.Tp[d] = (t.T[d] + 3) / 4 * 4;
 
 		t.nt[d] = (g.n[d] + t.T[d] - 1) / t.T[d];
 		t.ntiles *= t.nt[d];
-		t.W[d] = t.T[d];
 		t.Wtot *= t.T[d];
 		t.nb[d] = t.T[d] / t.b[d];
 		t.nw *= t.nb[d];
 	}
 
-	BAM_CHECK(e <= 64 && t.nw <= 16 && g.S * t.b[0] * t.b[1] * t.b[2] <= 64, "gridding: bad tiling");
+	BAM_CHECK(e <= 64 && t.nw <= 16 && 64 == g.S * t.b[0] * t.b[1] * t.b[2] &&
+			  64 * t.nw == g.S * t.Wtot, "gridding: bad tiling");
 
 	auto ilog2 = [](int v) {
 		int l = 0;
@@ -154,6 +162,11 @@ static GridTiling choose_tiling(const GridGeom& g)
 	t.lb01 = t.lb0 + ilog2(t.b[1]);
 	t.lb = t.lb01 + ilog2(t.b[2]);
 	t.cc = (g.C <= 4) ? 4 : ((g.C <= 8) ? 8 : 16);
+	t.ntap = (int)ceilf(g.width);
+	t.rwidth = 1.f / g.width;
+	t.fW = FastDiv((uint32_t)t.Wtot);
+	t.fT0 = FastDiv((uint32_t)t.T[0]);
+	t.fT1 = FastDiv((uint32_t)t.T[1]);
 
 	// cell rows visited by one work-group must fit the range list
 	long rows = 2;
@@ -425,13 +438,16 @@ void GridPlan::build(const GridGeom& geom, const float* traj)
 		kch = std::max<long>(kch, (long)((g.C + c - 1) / c) * c);
 	kspS.alloc((size_t)kch * std::max<long>(g.M, 1));
 
-	// adjoint work list: the visits of a tile (its cells and their ring) in
-	// chunks of at most MAXV; tiles with more than one chunk are split
-	const long MAXV = ADJ_MAXV;
-	std::vector<int4> hw;
-	std::vector<int4> hsplit;
+	{
+		int dev = 0;
+		BAM_HIP(hipGetDevice(&dev));
+		BAM_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
+	}
+
+	// adjoint work list: the visits of a tile (its cells and their ring)
 	const GridTiling& t = ta;
-	int slots = 0;
+	std::vector<int> visits(t.ntiles);
+	long total = 0;
 
 	for (int tile = 0; tile < t.ntiles; tile++) {
 
@@ -463,6 +479,25 @@ void GridPlan::build(const GridGeom& geom, const float* traj)
 							F += count[a + span[0][2 * xs + 1]] - count[a];
 						}
 
+		visits[tile] = (int)F;
+		total += F;
+	}
+
+	// Items of at most MAXV visits; tiles with more are split, at the cost of
+	// a partial tile per item.  Two items per compute unit where the visits
+	// of the whole plan make them (a 2-D problem's dense tiles would keep a
+	// few compute units busy while the others wait), between ADJ_MINV and
+	// ADJ_MAXV.
+	const long share = total * ((g.C + ta.cc - 1) / ta.cc) / (2l * ncu);
+	const long MAXV = std::min<long>(ADJ_MAXV, std::max<long>(ADJ_MINV, (share + 255) / 256 * 256));
+	std::vector<int4> hw;
+	std::vector<int4> hsplit;
+	int slots = 0;
+
+	for (int tile = 0; tile < t.ntiles; tile++) {
+
+		const long F = visits[tile];
+
 		if (F <= MAXV) {
 			hw.push_back(make_int4(tile, 0, (int)F, 0));
 		} else {
@@ -480,11 +515,6 @@ void GridPlan::build(const GridGeom& geom, const float* traj)
 	nsplit = (int)hsplit.size();
 	ta.nwork = nwork;
 	queue.alloc(1);
-	{
-		int dev = 0;
-		BAM_HIP(hipGetDevice(&dev));
-		BAM_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
-	}
 	nslot = slots;
 	work.alloc(std::max(nwork, 1));
 	split_tiles.alloc(std::max(nsplit, 1));
@@ -508,33 +538,57 @@ static int taps_bound(const GridGeom& g)
 // from the original sample order with si = the inverse of m(i)
 // ---------------------------------------------------------------------------
 
-// Thread per original sample m and coil chunk: the coil values are read
-// along m (coalesced) and the cc values of the chunk are written as one
-// contiguous run at the sample's sorted position si[m].
-__global__ void k_permute_ksp_inv(long M, int C, int cc, const int* __restrict__ si, const float2* __restrict__ ksp,
-				  const float2* __restrict__ weights, float2* __restrict__ kspS)
+// A work-group takes PERM_S samples of a coil chunk: the coil values are read
+// along m (coalesced), exchanged through LDS, and CC lanes write a sample's
+// values as one run at its sorted position si[m].  Bound by HBM; a thread
+// that wrote a sample's 128-byte run by itself reached 0.87 TB/s (128^3
+// kooshball, 16 coils: 615 us, now 108 us or 5 TB/s).  Also clears the work
+// queue of the gridding that follows on the stream.
+constexpr int PERM_S = 256;
+
+template <int CC>
+__global__ __launch_bounds__(256) void k_permute_ksp(long M, int C, const int* __restrict__ si,
+						     const float2* __restrict__ ksp,
+						     const float2* __restrict__ weights, float2* __restrict__ kspS,
+						     int* __restrict__ queue)
 {
-	const int nch = (C + cc - 1) / cc;
-	const long tot = (long)nch * M;
+	__shared__ float2 buf[CC * (PERM_S + 1)];
+	__shared__ int pos[PERM_S];
 
-	for (long j = (long)blockIdx.x * blockDim.x + threadIdx.x; j < tot; j += (long)gridDim.x * blockDim.x) {
+	if (0 == blockIdx.x && 0 == blockIdx.y && 0 == threadIdx.x)
+		queue[0] = 0;
 
-		const long ch = j / M;
-		const long m = j - ch * M;
-		const long i = si[m];
+	const long m0 = (long)blockIdx.x * PERM_S;
+	const int c0 = blockIdx.y * CC;
+	const long m = m0 + threadIdx.x;
+
+	if (m < M) {
+
 		const float2 w = (nullptr != weights) ? weights[m] : make_float2(1.f, 0.f);
-		float2* out = kspS + (ch * M + i) * cc;
+		float2 v[CC];
 
-		for (int cl = 0; cl < cc; cl++) {
+#pragma unroll
+		for (int cl = 0; cl < CC; cl++)
+			v[cl] = (c0 + cl < C) ? ksp[(long)(c0 + cl) * M + m] : make_float2(0.f, 0.f);
 
-			const int c = (int)ch * cc + cl;
-			float2 v = make_float2(0.f, 0.f);
+#pragma unroll
+		for (int cl = 0; cl < CC; cl++)
+			buf[cl * (PERM_S + 1) + threadIdx.x] = (nullptr != weights) ? cmulc(v[cl], w) : v[cl];
 
-			if (c < C)
-				v = (nullptr != weights) ? cmulc(ksp[(long)c * M + m], w) : ksp[(long)c * M + m];
+		pos[threadIdx.x] = si[m];
+	}
 
-			out[cl] = v;
-		}
+	__syncthreads();
+
+	float2* out = kspS + (long)blockIdx.y * M * CC;
+	const int ns = (int)min((long)PERM_S, M - m0);
+
+#pragma unroll
+	for (int e = threadIdx.x; e < CC * PERM_S; e += 256) {
+		const int i = e / CC;
+		const int cl = e % CC;
+		if (i < ns)
+			out[(long)pos[i] * CC + cl] = buf[cl * (PERM_S + 1) + i];
 	}
 }
 
@@ -620,17 +674,32 @@ __device__ inline int build_ranges(const GridGeom& g, const int* __restrict__ cs
 
 	__syncthreads();
 
-	if (0 == threadIdx.x) {
+	// prefix sums by the first wave, 64 rows at a time
+	if (threadIdx.x < 64) {
 
 		int tot = 0;
-		R.pre[0] = 0;
 
-		for (int r = 0; r < nrow; r++) {
-			tot += R.pre[r + 1];
-			R.pre[r + 1] = tot;
+		for (int r0 = 0; r0 < nrow; r0 += 64) {
+
+			const int r = r0 + (int)threadIdx.x;
+			int v = (r < nrow) ? R.pre[r + 1] : 0;
+
+#pragma unroll
+			for (int o = 1; o < 64; o <<= 1) {
+				const int u = __shfl_up(v, o, 64);
+				v += ((int)threadIdx.x >= o) ? u : 0;
+			}
+
+			if (r < nrow)
+				R.pre[r + 1] = tot + v;
+
+			tot += __shfl(v, 63, 64);
 		}
 
-		R.n = nrow;
+		if (0 == threadIdx.x) {
+			R.pre[0] = 0;
+			R.n = nrow;
+		}
 	}
 
 	__syncthreads();
@@ -724,64 +793,100 @@ __device__ inline void select_taps(const Taps1<TP>& a, const Taps1<TP>& b, bool 
 	any = an;
 }
 
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-constexpr int ADJ_BATCH = 256;  // visits per batch (4 groups of 64)
-constexpr int ADJ_WROW = 65;    // weight table row: 64 entries and a constant 1 (inactive dims)
-
 template <typename X>
 __device__ inline X sel3(int d, X a, X b, X c)
 {
 	return (0 == d) ? a : ((1 == d) ? b : c);
 }
 
-__global__ void k_reset_queue(int* q)
+// x / width, correctly rounded from the rounded reciprocal (one residual
+// step, Markstein)
+__device__ inline float div_width(float x, float width, float rwidth)
 {
-	if (0 == threadIdx.x)
-		q[0] = 0;
+	const float q = x * rwidth;
+	return __builtin_fmaf(__builtin_fmaf(-q, width, x), rwidth, q);
+}
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+constexpr int ADJ_BATCH = 256;  // visits per batch (4 groups of 64)
+constexpr int ADJ_WROW = 68;    // weight table row of a visit: 64 entries, 16-byte aligned, bank spread
+
+// LDS of the adjoint after the KB table and the ranges
+struct AdjLds {
+	float2* vbuf;         // [ADJ_BATCH + 1][CC] coil values per visit
+	float* wtab;          // [ADJ_BATCH + 1][ADJ_WROW] tap weights per visit
+	unsigned* rows;       // [6][ADJ_BATCH] tile rows hit, per active dim and variant
+	float* kc;            // [3][ADJ_BATCH] coordinates of the active dims
+	int* sidx;            // [2][ADJ_BATCH] sorted sample of each visit, two batches
+	unsigned short* list; // [16][ADJ_BATCH + 4] a wave's visits of the batch
+};
+
+template <int CC>
+constexpr size_t adj_work_bytes()
+{
+	return sizeof(float2) * (ADJ_BATCH + 1) * CC + sizeof(float) * (ADJ_BATCH + 1) * ADJ_WROW +
+	       sizeof(unsigned) * 6 * ADJ_BATCH + sizeof(float) * 3 * ADJ_BATCH + sizeof(int) * 2 * ADJ_BATCH +
+	       sizeof(unsigned short) * 16 * (ADJ_BATCH + 4);
 }
 
 // Adjoint gridding (k-space -> grid), output-stationary and atomic-free.
-// grid layout [S][C][N].  Persistent work-groups (one per CU) take work
+// grid layout [S][C][N].  Persistent work-groups (a few per CU) take work
 // items (tile, visit range, coil chunk) from a queue, largest first.
 //
 // A wave owns a block of b points per dim in every sub-grid (64 outputs:
 // sub-grid s, point).  For each batch of visits (samples of the tile's cells
 // and of the ring of neighbouring cells, in cell order):
-//   1. one lane per (visit, dim, shift variant) evaluates the taps once and
-//      writes the weight of every tile row (0 off the taps) and a bit mask
-//      of the rows hit to LDS; the coil values of the batch, loaded during
+//   1. a wave takes 64 visits, one dim and one shift variant (its parameters
+//      are scalars): a lane evaluates the taps of its visit, clears its row
+//      of tile weights and scatters the taps there, with a bit mask of the
+//      rows hit; the coil values and coordinates of the batch, loaded during
 //      the previous batch, go to LDS;
-//   2. every wave tests from the masks which visits reach its block and
-//      walks those two at a time: C[out][j] += sum_k A[out][k] B[k][j] on
-//      the matrix cores (v_mfma_f32_32x32x2_f32), A = tap weight
-//      wz * wy * wx of output out for visit k, B = value j (coil j / 2,
-//      re / im) of visit k.
+//   2. every wave lists the visits that reach its block (from the masks) and
+//      walks them four at a time on the matrix cores: C[out][j] += sum_k
+//      A[out][k] B[k][j], v_mfma_f32_16x16x4_f32 with A = tap weight of output
+//      out for visit k and B = value j (coil j / 2, re / im) of visit k.  The
+//      64 outputs are 4 groups of 16 rows; sub-grids that differ in the last
+//      one (two) active dims are in the same lane, so that 4 to 5 weights
+//      per lane and visit make the 4 rows' products.
 // Each product is accumulated in visit order, as in the sequential gridding
 // of noncart/grid.c:240-250.  Tiles whose visits are split over several
 // work items store partial tiles, summed in order by k_sum_split.
-template <int TP, int CC>
+//
+// Bound by the vector instructions of both steps, the latencies at the start
+// of an item and, for 2-D problems, by the largest item.  When a lane chose
+// one of its taps for every tile row, two visits were multiplied per step
+// (32x32x2 tiles, half empty with 8 coils) and the store formed an address
+// and a factor per value: 128^3 kooshball, 16 coils 5040 -> 2755 us; 256^2
+// radial, 8 coils 197 -> 45 us.
+template <int TP, int CC, int ND>
 __global__ __launch_bounds__(1024) void k_grid_adj(GridGeom g, GridTiling t, const float* __restrict__ kbt,
 						   const float4* __restrict__ sk, const int* __restrict__ cstart,
 						   const int4* __restrict__ work, int nitems, int* __restrict__ queue,
 						   const float2* __restrict__ kspS, float2* __restrict__ grid,
 						   float2* __restrict__ spart)
 {
+	constexpr int NCB = (CC + 7) / 8;  // blocks of 16 columns (8 coils)
 	extern __shared__ float4 smem4[];
 	char* smem = (char*)smem4;
 	float* table = (float*)smem;
 	CellRanges& R = *(CellRanges*)(smem + SMEM_TABLE);
-	float4* skall = (float4*)(smem + SMEM_DATA);          // [ADJ_MAXV] coordinates of each visit
-	float2* vbuf = (float2*)(skall + ADJ_MAXV);           // [ADJ_BATCH][CC] coil values per visit
-	int* sidx = (int*)(vbuf + ADJ_BATCH * CC);            // [ADJ_MAXV] sorted sample of each visit
-	float* wtab = (float*)(sidx + ADJ_MAXV);              // [ADJ_BATCH][ADJ_WROW] tap weights per visit
-	unsigned* rows = (unsigned*)(wtab + ADJ_WROW * ADJ_BATCH);  // [ADJ_BATCH][6] tile rows hit per dim, variant
-	int* qitem = (int*)(rows + 6 * ADJ_BATCH);
+	AdjLds L;
+	L.vbuf = (float2*)(smem + SMEM_DATA);
+	L.wtab = (float*)(L.vbuf + (ADJ_BATCH + 1) * CC);
+	L.rows = (unsigned*)(L.wtab + (ADJ_BATCH + 1) * ADJ_WROW);
+	L.kc = (float*)(L.rows + 6 * ADJ_BATCH);
+	L.sidx = (int*)(L.kc + 3 * ADJ_BATCH);
+	const size_t otile_bytes = sizeof(float2) * g.S * CC * (t.Wtot + 1);
+	const size_t data_bytes = max(adj_work_bytes<CC>(), otile_bytes);
+	int* qitem = (int*)(smem + SMEM_DATA + (data_bytes + 15) / 16 * 16);
 	float2* fml = (float2*)(qitem + 4);                   // [n0 + n1 + n2] fftmod tables (when t.fmlds)
 
 	const int nthr = blockDim.x;
+	const int nwv = nthr >> 6;
 	const int lane = threadIdx.x & 63;
 	const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform
 	const int nwork = t.nwork;
+	L.list = (unsigned short*)(L.sidx + 2 * ADJ_BATCH) + wid * (ADJ_BATCH + 4);
 
 	for (int i = threadIdx.x; i < KB_SIZE + 1; i += nthr)
 		table[i] = kbt[i];
@@ -801,37 +906,65 @@ __global__ __launch_bounds__(1024) void k_grid_adj(GridGeom g, GridTiling t, con
 			fml[g.n[0] + g.n[1] + i] = g.fm[2][i];
 	}
 
-	// the wave's block; C rows this lane feeds with weights: l % 32 and 32 + l % 32
-	const int B = t.b[0] * t.b[1] * t.b[2];
+	// the wave's block, and the weight table entries of the lane's rows
+	// 16 q + l16, q = 0 .. 3 (row = sub-grid x B + point): wo[d][bit], the
+	// entry of active dim d for shift variant bit.  In 3-d the x bit follows
+	// from l16, y and z bits from q; in 2-d both from q; in 1-d the bit and
+	// the upper half of the points.
+	constexpr int LB = (3 == ND) ? 3 : ((2 == ND) ? 4 : 5);  // points per block and sub-grid
+	constexpr int B = 1 << LB;
 	const int wb[3] = { wid % t.nb[0], (wid / t.nb[0]) % t.nb[1], wid / (t.nb[0] * t.nb[1]) };
-	const int jcol = lane & 31;
-	int wo1[3], wo2[3];
+	const int l16 = lane & 15;
+	int wo[ND][2], wo1[4];
+
+	// the lane's point and sub-grid of the output store
+	uint32_t srs, spq, sx0, sx1, sx2;
 	{
-		const int r1 = lane & 31;
-		const int r2 = 32 + (lane & 31);
-		const int s1 = min(r1 / B, g.S - 1), s2 = min(r2 / B, g.S - 1);
-		const int cb1 = r1 - (r1 / B) * B, cb2 = r2 - (r2 / B) * B;
-		const int p1[3] = { wb[0] * t.b[0] + cb1 % t.b[0], wb[1] * t.b[1] + (cb1 / t.b[0]) % t.b[1],
-				    wb[2] * t.b[2] + cb1 / (t.b[0] * t.b[1]) };
-		const int p2[3] = { wb[0] * t.b[0] + cb2 % t.b[0], wb[1] * t.b[1] + (cb2 / t.b[0]) % t.b[1],
-				    wb[2] * t.b[2] + cb2 / (t.b[0] * t.b[1]) };
+		uint32_t r;
+		t.fW.divmod(threadIdx.x, srs, spq);
+		t.fT0.divmod(spq, r, sx0);
+		t.fT1.divmod(r, sx2, sx1);
+	}
+
+	{
+		const int cb = l16 & (B - 1);
+		int q[3];
+		q[0] = wb[0] * t.b[0] + (cb & (t.b[0] - 1));
+		q[1] = wb[1] * t.b[1] + ((cb >> t.lb0) & (t.b[1] - 1));
+		q[2] = wb[2] * t.b[2] + (cb >> t.lb01);
+
 #pragma unroll
-		for (int d = 0; d < 3; d++) {
-			wo1[d] = (t.eoff[d] < 0) ? 64 : (t.eoff[d] + g.sbit[s1][d] * t.T[d] + min(p1[d], t.T[d] - 1));
-			wo2[d] = (t.eoff[d] < 0) ? 64 : (t.eoff[d] + g.sbit[s2][d] * t.T[d] + min(p2[d], t.T[d] - 1));
+		for (int a = 0; a < ND; a++) {
+			const int d = t.act[a];
+			const int e = t.eoff[d] + min(sel3(d, q[0], q[1], q[2]), t.T[d] - 1);
+			wo[a][0] = e;
+			wo[a][1] = e + t.Tp[d];
+		}
+
+		if (3 == ND && l16 >= 8)
+			wo[0][0] = wo[0][1];
+
+		if (1 == ND) {
+			const int d = t.act[0];
+#pragma unroll
+			for (int r = 0; r < 4; r++)
+				wo1[r] = t.eoff[d] + (r >> 1) * t.Tp[d] +
+					 min(sel3(d, wb[0], wb[1], wb[2]) * t.b[d] + 16 * (r & 1) + l16, t.T[d] - 1);
 		}
 	}
 
 	constexpr int VPT = (ADJ_BATCH * CC + 1023) / 1024;  // coil values carried per lane (1024 lanes)
 
+	// the first work-groups' first items are their own; later ones come from
+	// the queue, asked for one item ahead
+	int next = (int)blockIdx.x;
+
 	while (true) {
 
 		// next work item (the barrier also ends every wave's use of the
 		// previous item's LDS data)
-		__syncthreads();
-
 		if (0 == threadIdx.x)
-			qitem[0] = atomicAdd(queue, 1);
+			qitem[0] = next;
 
 		__syncthreads();
 
@@ -840,10 +973,15 @@ __global__ __launch_bounds__(1024) void k_grid_adj(GridGeom g, GridTiling t, con
 		if (item >= nitems)
 			break;
 
-		// the constant-1 weight entry of every row (the output store of the
-		// previous item reused this memory)
-		for (int v = threadIdx.x; v < ADJ_BATCH; v += nthr)
-			wtab[v * ADJ_WROW + 64] = 1.f;
+		if (0 == threadIdx.x)
+			next = (int)gridDim.x + atomicAdd(queue, 1);
+
+		// the visit that fills up groups of four: no weight, no value (the
+		// output store of the previous item reused this memory)
+		for (int i = threadIdx.x; i < ADJ_WROW; i += nthr)
+			L.wtab[ADJ_BATCH * ADJ_WROW + i] = 0.f;
+		for (int i = threadIdx.x; i < CC; i += nthr)
+			L.vbuf[ADJ_BATCH * CC + i] = make_float2(0.f, 0.f);
 
 		const int ch = item / nwork;
 		const int4 wk = work[item - ch * nwork];  // (tile, first visit, end visit, partial slot + 1 or 0)
@@ -872,41 +1010,59 @@ __global__ __launch_bounds__(1024) void k_grid_adj(GridGeom g, GridTiling t, con
 		const int fe = min(wk.z, Ftile);
 		const int F = fe - fb;
 
-		// sorted sample and coordinates of every visit of this item (F <= ADJ_MAXV)
-		for (int f = fb + threadIdx.x; f < fe; f += nthr) {
-			int lo = 0, hi = R.n;
-			while (hi - lo > 1) {
-				const int mid = (lo + hi) >> 1;
-				if (R.pre[mid] <= f)
-					lo = mid;
-				else
-					hi = mid;
+		// sorted sample of the visits of batch q into its half of sidx
+		// (visits past the end: the last one)
+		auto find = [&](int q) {
+			for (int v = threadIdx.x; v < ADJ_BATCH; v += nthr) {
+				const int f = fb + min(q * ADJ_BATCH + v, F - 1);
+				int lo = 0, hi = R.n;
+				while (hi - lo > 1) {
+					const int mid = (lo + hi) >> 1;
+					if (R.pre[mid] <= f)
+						lo = mid;
+					else
+						hi = mid;
+				}
+				L.sidx[(q & 1) * ADJ_BATCH + v] = R.start[lo] + (f - R.pre[lo]);
 			}
-			const int i = R.start[lo] + (f - R.pre[lo]);
-			sidx[f - fb] = i;
-			skall[f - fb] = sk[i];
+		};
+
+		if (F > 0) {
+			find(0);
+			find(1);
 		}
 
 		__syncthreads();
 
 		// coil values: lane carries VPT float2 of the next batch (entries
-		// threadIdx.x + 1024 q: visit e / CC, coil e % CC) through the current one
+		// threadIdx.x + 1024 q: visit e / CC, coil e % CC) through the current
+		// one; the first ADJ_BATCH lanes its coordinates
 		const float2* kch = kspS + (long)ch * g.M * CC;
 		float2 vnext[VPT];
+		float4 knext = make_float4(0.f, 0.f, 0.f, 0.f);
 
 #pragma unroll
 		for (int q = 0; q < VPT; q++) {
 			const int e = threadIdx.x + 1024 * q;
-			vnext[q] = (e < ADJ_BATCH * CC && F > 0) ? kch[(long)sidx[min(e / CC, F - 1)] * CC + (e % CC)]
-								 : make_float2(0.f, 0.f);
+			vnext[q] = (e < ADJ_BATCH * CC && F > 0) ? kch[(long)L.sidx[e / CC] * CC + (e % CC)] : make_float2(0.f, 0.f);
 		}
 
-		f32x16 C1 = {}, C2 = {};
+		if (threadIdx.x < ADJ_BATCH && F > 0)
+			knext = sk[L.sidx[threadIdx.x]];
+
+		f32x4 acc[NCB][4];
+#pragma unroll
+		for (int c = 0; c < NCB; c++)
+#pragma unroll
+			for (int q = 0; q < 4; q++)
+				acc[c][q] = f32x4{ 0.f, 0.f, 0.f, 0.f };
 
 		for (int base = 0; base < F; base += ADJ_BATCH) {
 
 			const int nb = min(ADJ_BATCH, F - base);
-			const float4* skc = skall + base;
+			const int bi = base / ADJ_BATCH;
+			const int* scur = L.sidx + (bi & 1) * ADJ_BATCH;
+			const int* snext = L.sidx + (1 - (bi & 1)) * ADJ_BATCH;
 
 			// the previous batch is done with the LDS buffers
 			lds_barrier();
@@ -915,13 +1071,27 @@ __global__ __launch_bounds__(1024) void k_grid_adj(GridGeom g, GridTiling t, con
 			for (int q = 0; q < VPT; q++) {
 				const int e = threadIdx.x + 1024 * q;
 				if (e < ADJ_BATCH * CC)
-					vbuf[e] = vnext[q];
+					L.vbuf[e] = vnext[q];
+			}
+
+			if (threadIdx.x < ADJ_BATCH) {
+				const float kk[3] = { knext.x, knext.y, knext.z };
+#pragma unroll
+				for (int a = 0; a < ND; a++)
+					L.kc[a * ADJ_BATCH + threadIdx.x] = sel3(t.act[a], kk[0], kk[1], kk[2]);
 			}
 
 			// work-groups of fewer than 1024 lanes load the rest now
 			for (int e = threadIdx.x + nthr; e < ADJ_BATCH * CC; e += nthr)
 				if (e % 1024 >= nthr)
-					vbuf[e] = kch[(long)sidx[base + min(e / CC, nb - 1)] * CC + (e % CC)];
+					L.vbuf[e] = kch[(long)scur[e / CC] * CC + (e % CC)];
+
+			for (int v = threadIdx.x + nthr; v < ADJ_BATCH; v += nthr) {
+				const float4 k = sk[scur[v]];
+#pragma unroll
+				for (int a = 0; a < ND; a++)
+					L.kc[a * ADJ_BATCH + v] = sel3(t.act[a], k.x, k.y, k.z);
+			}
 
 			// the next batch's values are loaded while this one is processed
 			if (base + ADJ_BATCH < F) {
@@ -929,30 +1099,33 @@ __global__ __launch_bounds__(1024) void k_grid_adj(GridGeom g, GridTiling t, con
 				for (int q = 0; q < VPT; q++) {
 					const int e = threadIdx.x + 1024 * q;
 					if (e < ADJ_BATCH * CC)
-						vnext[q] = kch[(long)sidx[min(base + ADJ_BATCH + e / CC, F - 1)] * CC + (e % CC)];
+						vnext[q] = kch[(long)snext[e / CC] * CC + (e % CC)];
 				}
+				if (threadIdx.x < ADJ_BATCH)
+					knext = sk[snext[threadIdx.x]];
 			}
 
-			// 1. taps of the batch: lane (visit v, dim d, variant var)
-			for (int jj = threadIdx.x; jj < 6 * nb; jj += nthr) {
+			lds_barrier();
 
-				const int v = jj / 6;
-				const int k = jj - 6 * v;
-				const int d = k >> 1;
+			// the batch after the next (this one's half of sidx is free)
+			if (base + 2 * ADJ_BATCH < F)
+				find(bi + 2);
+
+			// 1. taps of the batch: wave task (64 visits, dim, variant)
+			for (int task = wid; task < 4 * 2 * ND; task += nwv) {
+
+				const int vg = task / (2 * ND);
+				const int k = task - vg * (2 * ND);
 				const int var = k & 1;
 
-				// per-dim parameters by selection (no indexed kernel-argument loads)
-				const int eo = sel3(d, t.eoff[0], t.eoff[1], t.eoff[2]);
+				if (vg * 64 >= nb)
+					break;
 
-				if (eo < 0)
-					continue;
-
-				const float4 kc = skc[v];
-				const float kd = sel3(d, kc.x, kc.y, kc.z);
-				const int n = sel3(d, g.n[0], g.n[1], g.n[2]);
-				const bool v1 = (1 == var) && (sel3(d, g.nshv[0], g.nshv[1], g.nshv[2]) > 1);
-				const float sh = v1 ? sel3(d, g.shv[0][1], g.shv[1][1], g.shv[2][1])
-						    : sel3(d, g.shv[0][0], g.shv[1][0], g.shv[2][0]);
+				const int v = vg * 64 + lane;
+				const int d = t.act[k >> 1];
+				const int n = g.n[d];
+				const float sh = g.shv[d][(g.nshv[d] > 1) ? var : 0];
+				const float kd = L.kc[(k >> 1) * ADJ_BATCH + v];
 				const float pos = grid_pos(g.os, kd, sh, (float)(n / 2));
 				int sti = (int)ceil((double)pos - 0.5 * (double)g.width);
 				int eni = (int)floor((double)pos + 0.5 * (double)g.width);
@@ -962,203 +1135,246 @@ __global__ __launch_bounds__(1024) void k_grid_adj(GridGeom g, GridTiling t, con
 					eni = min(eni, n - 1);
 				}
 
-				const int cnt = min(max(eni - sti + 1, 0), TP);
-				float wq[TP];
-
-#pragma unroll
-				for (int q = 0; q < TP; q++)
-					wq[q] = (q < cnt) ? kb_lookup(table, fabsf((float)(sti + q) - pos) / g.width) : 0.f;
-
-				const int T = sel3(d, t.T[0], t.T[1], t.T[2]);
+				const int cnt = min(min(max(eni - sti + 1, 0), TP), n);
+				const int T = t.T[d], Tp = t.Tp[d];
 				const int td = sel3(d, t0[0], t0[1], t0[2]);
-				float* wr = wtab + v * ADJ_WROW + eo + var * T;
+				float* wr = L.wtab + v * ADJ_WROW + t.eoff[d] + var * Tp;
 				unsigned bits = 0u;
 
-				for (int l = 0; l < T; l++) {
+				for (int l = 0; l < Tp; l += 4)
+					*(f32x4*)(wr + l) = f32x4{ 0.f, 0.f, 0.f, 0.f };
 
-					const int gl = td + l;
-					int j;
+				int l0 = sti - td;
 
-					if (g.periodic) {
-						j = (gl - sti) % n;
-						if (j < 0)
-							j += n;
-					} else {
-						j = gl - sti;
-					}
-
-					const bool mem = (gl < n) && (j >= 0) && (j < cnt);
-					float wl = 0.f;
-
-#pragma unroll
-					for (int q = 0; q < TP; q++)
-						wl = (mem && j == q) ? wq[q] : wl;
-
-					wr[l] = wl;
-					bits |= mem ? (1u << l) : 0u;
+				if (g.periodic) {
+					l0 = sti % n;
+					l0 += (l0 < 0) ? n : 0;
+					l0 -= td;
 				}
 
-				rows[v * 6 + k] = bits;
+#pragma unroll
+				for (int q = 0; q < TP; q++) {
+
+					if (q >= t.ntap)
+						break;
+
+					int l = l0 + q;
+
+					if (g.periodic && l + td >= n)
+						l -= n;
+
+					const float w = kb_lookup(table, div_width(fabsf((float)(sti + q) - pos), g.width, t.rwidth));
+
+					if (q < cnt && l >= 0 && l < T) {
+						wr[l] = w;
+						bits |= 1u << l;
+					}
+				}
+
+				L.rows[k * ADJ_BATCH + v] = bits;
 			}
 
 			lds_barrier();
 
-			// 2. per group of 64 visits: those that reach this wave's block
-			// (taps in its rows in every active dim, either variant), two at
-			// a time
+			// 2. the visits that reach this wave's block (taps in its rows in
+			// every active dim, either variant), in order
+			int cnt = 0;
+
 			for (int gb = 0; gb < nb; gb += 64) {
 
-				const int vl = gb + min(lane, nb - gb - 1);
 				bool reach = lane < nb - gb;
 
 #pragma unroll
-				for (int d = 0; d < 3; d++)
-					if (t.eoff[d] >= 0) {
-						const unsigned long long m = rows[vl * 6 + 2 * d] | rows[vl * 6 + 2 * d + 1];
-						reach = reach && (0ull != ((m >> (wb[d] * t.b[d])) & ((1ull << t.b[d]) - 1ull)));
-					}
-
-				unsigned long long mh = __ballot(reach);
-
-				while (0ull != mh) {
-
-					const int vA = gb + __builtin_ctzll(mh);
-					mh &= mh - 1ull;
-					const bool hasB = 0ull != mh;
-					const int vB = hasB ? (gb + __builtin_ctzll(mh)) : vA;
-					if (hasB)
-						mh &= mh - 1ull;
-
-					const bool use = (lane < 32) || hasB;
-					const int v = (lane < 32) ? vA : vB;
-					const float* wv = wtab + v * ADJ_WROW;
-
-					// z, y, x (BART order)
-					float a1 = wv[wo1[2]];
-					a1 = a1 * wv[wo1[1]];
-					a1 = a1 * wv[wo1[0]];
-					float a2 = wv[wo2[2]];
-					a2 = a2 * wv[wo2[1]];
-					a2 = a2 * wv[wo2[0]];
-					float bv = (jcol < 2 * CC) ? ((const float*)vbuf)[v * 2 * CC + jcol] : 0.f;
-
-					if (!use) {
-						a1 = 0.f;
-						a2 = 0.f;
-						bv = 0.f;
-					}
-
-					C1 = __builtin_amdgcn_mfma_f32_32x32x2f32(a1, bv, C1, 0, 0, 0);
-					C2 = __builtin_amdgcn_mfma_f32_32x32x2f32(a2, bv, C2, 0, 0, 0);
+				for (int a = 0; a < ND; a++) {
+					const int d = t.act[a];
+					const unsigned m = L.rows[2 * a * ADJ_BATCH + gb + lane] |
+							   L.rows[(2 * a + 1) * ADJ_BATCH + gb + lane];
+					const unsigned sel = (32 == t.b[d]) ? ~0u : ((1u << t.b[d]) - 1u) << (sel3(d, wb[0], wb[1], wb[2]) * t.b[d]);
+					reach = reach && 0u != (m & sel);
 				}
+
+				const unsigned long long mh = __ballot(reach);
+
+				if (reach)
+					L.list[cnt + __builtin_amdgcn_mbcnt_hi((unsigned)(mh >> 32),
+									       __builtin_amdgcn_mbcnt_lo((unsigned)mh, 0u))] =
+						(unsigned short)(gb + lane);
+
+				cnt += (int)__popcll(mh);
+			}
+
+			if (lane < 4)
+				L.list[cnt + lane] = (unsigned short)ADJ_BATCH;
+
+			// the list is this wave's own
+			__builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+			__builtin_amdgcn_wave_barrier();
+			__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+
+			const unsigned short* lp = L.list + (lane >> 4);
+
+#pragma unroll 2
+			for (int i = 0; i < cnt; i += 4) {
+
+				const int v = lp[i];
+				const float* wv = L.wtab + v * ADJ_WROW;
+				const float* bp = (const float*)L.vbuf + v * 2 * CC;
+				float bv[NCB];
+
+#pragma unroll
+				for (int c = 0; c < NCB; c++)
+					bv[c] = bp[16 * c + ((4 == CC) ? (l16 & 7) : l16)];
+
+				float a[4];
+
+				if constexpr (3 == ND) {
+					const float x = wv[wo[0][0]];
+					const float y0 = wv[wo[1][0]] * x, y1 = wv[wo[1][1]] * x;
+					const float z0 = wv[wo[2][0]], z1 = wv[wo[2][1]];
+					a[0] = z0 * y0;
+					a[1] = z0 * y1;
+					a[2] = z1 * y0;
+					a[3] = z1 * y1;
+				} else if constexpr (2 == ND) {
+					const float x0 = wv[wo[0][0]], x1 = wv[wo[0][1]];
+					const float y0 = wv[wo[1][0]], y1 = wv[wo[1][1]];
+					a[0] = y0 * x0;
+					a[1] = y0 * x1;
+					a[2] = y1 * x0;
+					a[3] = y1 * x1;
+				} else {
+#pragma unroll
+					for (int q = 0; q < 4; q++)
+						a[q] = wv[wo1[q]];
+				}
+
+#pragma unroll
+				for (int c = 0; c < NCB; c++)
+#pragma unroll
+					for (int q = 0; q < 4; q++)
+						acc[c][q] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[q], bv[c], acc[c][q], 0, 0, 0);
 			}
 		}
 
 		// Store through LDS: the waves put their outputs into the tile
 		// buffer otile[s][c][point] (plane pitch Wtot + 1, spread over the
-		// banks; it reuses the batch buffers), then all lanes write the tile
-		// out row by row.  C row i (of the wave's 64 outputs), column
-		// j = 2 coil + (re, im): register r of lane l holds
-		// i = 8 (r / 4) + 4 (l / 32) + r % 4 (+ 32 in C2), j = l % 32.
+		// banks; it reuses the batch buffers), then a lane writes one point of
+		// one sub-grid for all coils (S Wtot lanes: the whole work-group), so
+		// that its address and fftmod factor are formed once.  Column j = l16
+		// of block c is coil 8 c + j / 2 (re, im); register r of group q holds
+		// row 16 q + 4 (lane / 16) + r.
 		const int OP = t.Wtot + 1;
-		float* otile = (float*)skall;
+		float* otile = (float*)L.vbuf;
 
 		lds_barrier();
 
 		{
 			// (zero is 0, read from LDS here so that the row decoding is
-			// not hoisted out of the item loop, where its 32 copies would
-			// stay live)
+			// not hoisted out of the item loop, where its copies would stay
+			// live)
 			const int zero = qitem[1];
-			const int c = (jcol + zero) >> 1;
-			const int lhalf = (lane + zero) >> 5;
+			const int kg = (lane + zero) >> 4;
 
 #pragma unroll
-			for (int h = 0; h < 2; h++)
+			for (int h = 0; h < ((LB > 4) ? 2 : 1); h++)
 #pragma unroll
-				for (int r = 0; r < 16; r++) {
+				for (int r = 0; r < 4; r++) {
 
-					const int i = 32 * h + 8 * (r / 4) + 4 * lhalf + (r % 4);
-					const int rs = i >> t.lb;
-					const int rc = i & (B - 1);
+					// rows 16 q + i: sub-grid (16 q + i) / B, point of the block
+					// i % B (+ 16 h where a block spans two groups)
+					const int i = 4 * kg + r;
+					const int rc = (LB > 4) ? i + 16 * h : (i & (B - 1));
 					const int q0 = wb[0] * t.b[0] + (rc & (t.b[0] - 1));
 					const int q1 = wb[1] * t.b[1] + ((rc >> t.lb0) & (t.b[1] - 1));
 					const int q2 = wb[2] * t.b[2] + (rc >> t.lb01);
+					const int pt = q0 + t.T[0] * (q1 + t.T[1] * q2);
+					float* op = otile + (((i >> LB) * CC + (l16 >> 1)) * OP + pt) * 2 + (l16 & 1);
 
-					if (i < g.S * B && c < CC)
-						otile[(((long)rs * CC + c) * OP + q0 + t.W[0] * (q1 + t.W[1] * q2)) * 2 + (lane & 1)] =
-							(0 == h) ? C1[r] : C2[r];
+#pragma unroll
+					for (int q = h; q < 4; q += ((LB > 4) ? 2 : 1)) {
+						const int rs = (16 * q) >> LB;
+#pragma unroll
+						for (int c = 0; c < NCB; c++)
+							if (4 != CC || l16 < 8)
+								op[((rs * CC + 8 * c) * OP) * 2] = acc[c][q][r];
+					}
 				}
 		}
 
 		lds_barrier();
 
-		for (int e = threadIdx.x; e < g.S * CC * t.Wtot; e += nthr) {
+		{
+			const int x0 = t0[0] + (int)sx0, x1 = t0[1] + (int)sx1, x2 = t0[2] + (int)sx2;
 
-			const int pq = e % t.Wtot;
-			const int rest = e / t.Wtot;
-			const int c = rest % CC;
-			const int rs = rest / CC;
-			const int x0 = t0[0] + pq % t.W[0];
-			const int x1 = t0[1] + (pq / t.W[0]) % t.W[1];
-			const int x2 = t0[2] + pq / (t.W[0] * t.W[1]);
+			if ((int)srs < g.S && x0 < g.n[0] && x1 < g.n[1] && x2 < g.n[2]) {
 
-			if (c >= ncc || x0 >= g.n[0] || x1 >= g.n[1] || x2 >= g.n[2])
-				continue;
+				const float2* op = (const float2*)otile + (long)srs * CC * OP + spq;
 
-			const float* op = otile + (((long)rs * CC + c) * OP + pq) * 2;
-			const float2 val = make_float2(op[0], op[1]);
+				if (0 == wk.w) {
 
-			if (0 == wk.w) {
-				const long idx = x0 + (long)g.n[0] * (x1 + (long)g.n[1] * x2);
-				float2 o = val;
-				if (fmlds) {
-					float2 f = fml[x0];
-					f = cmul(f, fml[g.n[0] + x1]);
-					f = cmul(f, fml[g.n[0] + g.n[1] + x2]);
-					o = cmulc(val, f);
+					float2 f = make_float2(1.f, 0.f);
+
+					if (fmlds) {
+						f = fml[x0];
+						f = cmul(f, fml[g.n[0] + x1]);
+						f = cmul(f, fml[g.n[0] + g.n[1] + x2]);
+					} else if (fm) {
+						f = cmul(cmul(g.fm[0][x0], g.fm[1][x1]), g.fm[2][x2]);
+					}
+
+					float2* out = grid + ((long)srs * g.C + c0) * g.N + x0 + (long)g.n[0] * (x1 + (long)g.n[1] * x2);
+
+					for (int c = 0; c < ncc; c++)
+						out[(long)c * g.N] = cmulc(op[c * OP], f);
+
 				} else {
-					o = apply_conj_fm(g, val, x0, x1, x2);
+
+					// tile split over several work items (dense region): the
+					// partial tile goes to its own slot, summed by k_sum_split
+					float2* out = spart + (((long)(wk.w - 1) * g.S + srs) * g.C + c0) * t.Wtot + spq;
+
+					for (int c = 0; c < ncc; c++)
+						out[(long)c * t.Wtot] = op[c * OP];
 				}
-				grid[((long)rs * g.C + c0 + c) * g.N + idx] = o;
-			} else {
-				// tile split over several work items (dense region): the
-				// partial tile goes to its own slot, summed by k_sum_split
-				spart[(((long)(wk.w - 1) * g.S + rs) * g.C + c0 + c) * t.Wtot + pq] = val;
 			}
 		}
 	}
 }
 
 // tiles split over several work items: sum of their partial tiles in slot
-// order (deterministic, no atomics); thread per (split tile, s, c, point)
-__global__ void k_sum_split(GridGeom g, GridTiling t, const int4* __restrict__ tiles, int ntl,
-			    const float2* __restrict__ spart, float2* __restrict__ grid)
+// order (deterministic, no atomics); work-group (split tile, sub-grid, group
+// of nc coils), thread per (coil, point)
+
+__global__ __launch_bounds__(256) void k_sum_split(GridGeom g, GridTiling t, const int4* __restrict__ tiles,
+						   const float2* __restrict__ spart, float2* __restrict__ grid, int nc)
 {
-	const int per = t.Wtot;
-	const long SC = (long)g.S * g.C;
-	const long tot = (long)ntl * SC * per;
+	const int4 st = tiles[blockIdx.x];
+	const int tile = st.x;
+	const int tb0 = tile % t.nt[0], tb1 = (tile / t.nt[0]) % t.nt[1], tb2 = tile / (t.nt[0] * t.nt[1]);
+	const int c0 = blockIdx.z * nc;
+	const int ncc = min(nc, g.C - c0);
+	const long slot = (long)g.S * g.C * t.Wtot;
 
-	for (long j = (long)blockIdx.x * blockDim.x + threadIdx.x; j < tot; j += (long)gridDim.x * blockDim.x) {
+	for (uint32_t e = threadIdx.x; e < (uint32_t)(ncc * t.Wtot); e += 256) {
 
-		const long q = j / per;
-		const int pnt = (int)(j - q * per);
-		const long sc = q % SC;
-		const int tl = (int)(q / SC);
-		const int4 st = tiles[tl];
-		const int tile = st.x;
-		const int tb0 = tile % t.nt[0], tb1 = (tile / t.nt[0]) % t.nt[1], tb2 = tile / (t.nt[0] * t.nt[1]);
-		const int gx = tb0 * t.T[0] + pnt % t.W[0];
-		const int gy = tb1 * t.T[1] + (pnt / t.W[0]) % t.W[1];
-		const int gz = tb2 * t.T[2] + pnt / (t.W[0] * t.W[1]);
+		uint32_t cl, pnt, r, x0, x1, x2;
+		t.fW.divmod(e, cl, pnt);
+		t.fT0.divmod(pnt, r, x0);
+		t.fT1.divmod(r, x2, x1);
+		const int gx = tb0 * t.T[0] + (int)x0;
+		const int gy = tb1 * t.T[1] + (int)x1;
+		const int gz = tb2 * t.T[2] + (int)x2;
 
 		if (gx >= g.n[0] || gy >= g.n[1] || gz >= g.n[2])
 			continue;
 
+		const long sc = (long)blockIdx.y * g.C + c0 + cl;
+		const float2* p = spart + (long)st.y * slot + sc * t.Wtot + pnt;
 		float2 a = make_float2(0.f, 0.f);
 
+#pragma unroll 4
 		for (int k = 0; k < st.z; k++)
-			a = cadd(a, spart[((long)(st.y + k) * SC + sc) * per + pnt]);
+			a = cadd(a, p[k * slot]);
 
 		grid[sc * g.N + gx + (long)g.n[0] * (gy + (long)g.n[1] * gz)] = apply_conj_fm(g, a, gx, gy, gz);
 	}
@@ -1177,12 +1393,18 @@ void grid_adjoint(const GridPlan& gp, const float* kb, float2* grid, const float
 
 	{
 		ProfScope prof("permute_ksp", st);
-		int nch = (g.C + t.cc - 1) / t.cc;
-		long tot = (long)nch * g.M;
-		unsigned blocks = (unsigned)std::max<long>(1, std::min<long>((tot + 255) / 256, 16384));
-		if (tot > 0)
-			hipLaunchKernelGGL(k_permute_ksp_inv, dim3(blocks), dim3(256), 0, st, g.M, g.C, t.cc, gp.si.ptr, ksp,
-					   weights, gp.kspS.ptr);
+		const int nch = (g.C + t.cc - 1) / t.cc;
+		const dim3 blocks(std::max(1u, ceil_div(g.M, PERM_S)), nch);
+#define BAM_PERM(CC) \
+	hipLaunchKernelGGL(k_permute_ksp<CC>, blocks, dim3(256), 0, st, g.M, g.C, gp.si.ptr, ksp, weights, \
+			   gp.kspS.ptr, gp.queue.ptr)
+		if (t.cc <= 4)
+			BAM_PERM(4);
+		else if (t.cc <= 8)
+			BAM_PERM(8);
+		else
+			BAM_PERM(16);
+#undef BAM_PERM
 		BAM_HIP(hipGetLastError());
 	}
 
@@ -1193,15 +1415,10 @@ void grid_adjoint(const GridPlan& gp, const float* kb, float2* grid, const float
 	const int nch = (g.C + t.cc - 1) / t.cc;
 	const int nitems = gp.nwork * nch;
 	const unsigned nwg = (unsigned)std::max(1, std::min(nitems, gp.wpc * gp.ncu));
-	size_t lds = SMEM_DATA + sizeof(float4) * ADJ_MAXV + sizeof(float2) * ADJ_BATCH * t.cc +
-		     sizeof(int) * ADJ_MAXV + sizeof(float) * ADJ_WROW * ADJ_BATCH + sizeof(unsigned) * 6 * ADJ_BATCH +
-		     sizeof(int) * 4;
-
+	const size_t workb = (t.cc <= 4) ? adj_work_bytes<4>() : ((t.cc <= 8) ? adj_work_bytes<8>() : adj_work_bytes<16>());
 	// the output tile (plane pitch Wtot + 1) reuses the batch buffers
-	BAM_CHECK((size_t)g.S * t.cc * (t.Wtot + 1) * sizeof(float2) <=
-			  sizeof(float4) * ADJ_MAXV + sizeof(float2) * ADJ_BATCH * t.cc + sizeof(int) * ADJ_MAXV +
-				  sizeof(float) * ADJ_WROW * ADJ_BATCH,
-		  "gridding: output tile larger than the batch buffers");
+	const size_t otile = (size_t)g.S * t.cc * (t.Wtot + 1) * sizeof(float2);
+	size_t lds = SMEM_DATA + (std::max(workb, otile) + 15) / 16 * 16 + sizeof(int) * 4;
 
 	// fftmod tables in LDS when they fit (160 KiB per work-group)
 	GridTiling tl = t;
@@ -1210,31 +1427,38 @@ void grid_adjoint(const GridPlan& gp, const float* kb, float2* grid, const float
 	if (tl.fmlds)
 		lds += fmb;
 
-	hipLaunchKernelGGL(k_reset_queue, dim3(1), dim3(64), 0, st, gp.queue.ptr);
-
-#define BAM_ADJ(TP, CC)                                                                                     \
-	hipLaunchKernelGGL((k_grid_adj<TP, CC>), dim3(nwg), dim3(nthr), lds, st, g, tl, kb, gp.sk.ptr, gp.cstart.ptr, \
+#define BAM_ADJ(TP, CC, ND)                                                                                     \
+	hipLaunchKernelGGL((k_grid_adj<TP, CC, ND>), dim3(nwg), dim3(nthr), lds, st, g, tl, kb, gp.sk.ptr, gp.cstart.ptr, \
 			   gp.work.ptr, nitems, gp.queue.ptr, gp.kspS.ptr, grid, gp.spart.ptr)
+#define BAM_ADJ_ND(TP, CC)             \
+	do {                           \
+		if (3 == t.nd)         \
+			BAM_ADJ(TP, CC, 3); \
+		else if (2 == t.nd)    \
+			BAM_ADJ(TP, CC, 2); \
+		else                   \
+			BAM_ADJ(TP, CC, 1); \
+	} while (0)
 
 	if (4 == tp) {
-		if (t.cc <= 4) BAM_ADJ(4, 4);
-		else if (t.cc <= 8) BAM_ADJ(4, 8);
-		else BAM_ADJ(4, 16);
+		if (t.cc <= 4) BAM_ADJ_ND(4, 4);
+		else if (t.cc <= 8) BAM_ADJ_ND(4, 8);
+		else BAM_ADJ_ND(4, 16);
 	} else {
-		if (t.cc <= 4) BAM_ADJ(8, 4);
-		else if (t.cc <= 8) BAM_ADJ(8, 8);
-		else BAM_ADJ(8, 16);
+		if (t.cc <= 4) BAM_ADJ_ND(8, 4);
+		else if (t.cc <= 8) BAM_ADJ_ND(8, 8);
+		else BAM_ADJ_ND(8, 16);
 	}
+#undef BAM_ADJ_ND
 #undef BAM_ADJ
 
 	BAM_HIP(hipGetLastError());
 
 	if (gp.nsplit > 0) {
 		ProfScope prof2("grid_adjoint_sum_split", st);
-		long tot = (long)gp.nsplit * g.S * g.C * t.Wtot;
-		unsigned zb = (unsigned)std::min<long>((tot + 255) / 256, 16384);
-		hipLaunchKernelGGL(k_sum_split, dim3(zb), dim3(256), 0, st, g, t, gp.split_tiles.ptr, gp.nsplit,
-				   gp.spart.ptr, grid);
+		const int nc = std::max(1, 256 / t.Wtot);
+		hipLaunchKernelGGL(k_sum_split, dim3((unsigned)gp.nsplit, (unsigned)g.S, ceil_div(g.C, nc)), dim3(256), 0, st, g,
+				   t, gp.split_tiles.ptr, gp.spart.ptr, grid, nc);
 		BAM_HIP(hipGetLastError());
 	}
 }
@@ -1665,7 +1889,7 @@ void tune_grid_adjoint(GridPlan& gp, const float* kb, float2* grid, hipStream_t 
 		return;
 
 	char kbuf[256];
-	snprintf(kbuf, sizeof(kbuf), "adj:%dx%dx%d:S%d:C%d:M%ld:ccmax%d", g.n[0], g.n[1], g.n[2], g.S, g.C, g.M,
+	snprintf(kbuf, sizeof(kbuf), "adj:%dx%dx%d:S%d:C%d:M%ld:ccmax%d:quads", g.n[0], g.n[1], g.n[2], g.S, g.C, g.M,
 		 gp.cc_max);
 	const std::string key = kbuf;
 

@@ -83,24 +83,29 @@ struct GridGeom {
 
 // Tiling of the adjoint gridding: a work-group owns a tile of T points per
 // dim of all sub-grids for cc coils.  Each wave owns a block of b points per
-// dim of every sub-grid (S x b0 b1 b2 = 64 lanes); the tile holds nb blocks
-// per dim.  The per-visit weight table has 2 T[d] entries (two shift
-// variants) for every active dim d, starting at eoff[d] (-1: inactive).
+// dim of every sub-grid (S x b0 b1 b2 = 64 outputs); the tile holds nb blocks
+// per dim.  The per-visit weight table has 2 Tp[d] entries (two shift
+// variants, T rounded up to 4) for every active dim d, starting at eoff[d].
 struct GridTiling {
 
 	int T[3];
+	int Tp[3];
 	int nt[3];
 	int ntiles;
 	int cc;    // coils per work-group
-	int W[3];  // = T
 	int Wtot;  // points per tile and sub-grid
 	int b[3];  // wave block
 	int nb[3]; // blocks per tile
 	int nw;    // waves per work-group
+	int nd;    // active dims
+	int act[3];
 	int eoff[3];
 	int nwork; // work items per coil chunk
 	int lb, lb0, lb01;  // log2 of b0 b1 b2, b0 and b0 b1 (all powers of two)
 	int fmlds;          // fftmod tables staged in LDS by the adjoint (they fit)
+	int ntap;           // taps evaluated per dim: ceil(width) (of width + 1 taps both ends weigh 0)
+	float rwidth;       // 1 / width
+	FastDiv fW, fT0, fT1;
 };
 
 // Tiling of the forward gather of 3-D grids: samples are grouped by the

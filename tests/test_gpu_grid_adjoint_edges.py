@@ -1,0 +1,56 @@
+"""GPU: the adjoint gridding at the edges of its work split -- one, two and
+three active dims, every coil-chunk width (4, 8, 16) with a chunk that does
+not fill, four and eight taps per dim, tiles cut by the grid, periodic grids
+smaller than the kernel's reach, batches of visits that do not fill and tiles
+split over several work items -- against the oracle, FP32 sums of both sides:
+1e-5 as for every operator."""
+import numpy as np
+import pytest
+
+import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+
+def d16(*d):
+    return list(d) + [1] * (16 - len(d))
+
+
+def relerr(a, ref):
+    a = np.asarray(a, np.complex128).ravel()
+    ref = np.asarray(ref, np.complex128).ravel()
+    return float(np.linalg.norm(a - ref) / np.linalg.norm(ref))
+
+
+@pytest.mark.parametrize("dims", [(50, 1, 1), (33, 28, 1), (10, 12, 9), (18, 16, 1), (8, 6, 4)])
+@pytest.mark.parametrize("C", [1, 7, 17])
+@pytest.mark.parametrize("width,periodic", [(6.0, False), (6.0, True), (10.0, False)])
+@pytest.mark.parametrize("M", [1, 300, 9000])
+def test_grid_adjoint_edges(dims, C, width, periodic, M):
+    import bart_amd as ba
+    if periodic and min(n for n in dims if n > 1) < 6:
+        pytest.skip("the oracle wraps each tap, kernels wider than the grid count points twice")
+    if periodic and any(n > 1 and n % 2 for n in dims):
+        pytest.skip("odd periodic dims: the cells of two points do not tile the period")
+    rng = np.random.default_rng(M + C + dims[0])
+    traj = np.zeros((M, 3), np.complex64)
+    for d in range(3):
+        if dims[d] > 1:
+            # most samples near the centre (tiles of thousands of visits),
+            # some over the edges of k-space
+            k = rng.standard_normal(M) * dims[d] / 12
+            far = rng.random(M) < 0.3
+            k[far] = (rng.random(far.sum()) - 0.5) * dims[d] * 1.05
+            traj[:, d] = k
+    ksp = (rng.standard_normal((C, M)) + 1j * rng.standard_normal((C, M))).astype(np.complex64)
+    w = (0.5 + rng.random(M)).astype(np.complex64)
+    conf = ba.NufftConf.defaults(toeplitz=False, width=width, periodic=periodic)
+    op = ba.nufft_create2(d16(1, M, 1, C), d16(*dims, C), d16(3, M), ba.traj_array(traj), weights=w, conf=conf)
+    ref = O.Nufft(dims, traj, C, weights=w, toeplitz=False, width=width, periodic=periodic)
+    y = torch.from_numpy(ksp.reshape(-1)).cuda()
+    a = op.adjoint(y)
+    assert relerr(a.cpu(), ref.adjoint(ksp)) < 1e-5
+    assert torch.equal(a, op.adjoint(y))
+    op.free()
