@@ -260,7 +260,7 @@ void GridPlan::build_forward_tiles(const GridGeom& gg, const std::vector<int>& h
 		return;
 
 	// the staged region of FW_CC coils and the KB table fit into 64 KiB
-	if ((size_t)ft.Etot * FW_CC * sizeof(float2) + (KB_SIZE + 4) * sizeof(float) > 64 * 1024)
+	if (((size_t)ft.Etot + 2 * FW_E + 4) * FW_CC * sizeof(float2) + (KB_SIZE + 4) * sizeof(float) > 64 * 1024)
 		return;
 
 	const int cpt = FW_T / gg.CS[0];  // cells per tile edge (CS is equal in every dim)
@@ -706,93 +706,6 @@ __device__ inline int build_ranges(const GridGeom& g, const int* __restrict__ cs
 	return R.pre[R.n];
 }
 
-// ---------------------------------------------------------------------------
-// Taps of one sample along one dim (noncart/grid.c:415-457), computed once
-// per sample and shift variant and reused by every sub-grid and coil.
-// ---------------------------------------------------------------------------
-
-__device__ inline float sample_pos_v(const GridGeom& g, int d, int v, float k)
-{
-	return grid_pos(g.os, k, g.shv[d][v], (float)(g.n[d] / 2));
-}
-
-template <int TP> struct Taps1 {
-	int start;  // first tap (grid index before wrapping; clamped when not periodic)
-	int cnt;    // number of taps
-	float w[TP];
-};
-
-template <int TP>
-__device__ inline void taps_raw(const GridGeom& g, int d, int v, float k, const float* table, Taps1<TP>& t)
-{
-	if (1 == g.n[d]) {
-		t.start = 0;
-		t.cnt = 1;
-#pragma unroll
-		for (int j = 0; j < TP; j++)
-			t.w[j] = (0 == j) ? 1.f : 0.f;
-		return;
-	}
-
-	const float pos = sample_pos_v(g, d, v, k);
-	int sti = (int)ceil((double)pos - 0.5 * (double)g.width);
-	int eni = (int)floor((double)pos + 0.5 * (double)g.width);
-
-	if (!g.periodic) {
-		sti = max(sti, 0);
-		eni = min(eni, g.n[d] - 1);
-	}
-
-	t.start = sti;
-	t.cnt = min(max(eni - sti + 1, 0), TP);
-
-#pragma unroll
-	for (int j = 0; j < TP; j++)
-		t.w[j] = (j < t.cnt) ? kb_lookup(table, fabsf((float)(sti + j) - pos) / g.width) : 0.f;
-}
-
-// local index of tap j relative to a tile or window starting at org with
-// extent range, or -1 (periodic grids: modulo n)
-__device__ inline int tap_local(const GridGeom& g, int d, int w, int org, int range)
-{
-	int l;
-
-	if (g.periodic) {
-		const int nn = g.n[d];
-		int gw = w % nn;
-		if (gw < 0)
-			gw += nn;
-		l = gw - org;
-		if (l < 0)
-			l += nn;
-		else if (l >= nn)
-			l -= nn;
-	} else {
-		l = w - org;
-	}
-
-	return (l >= 0 && l < range) ? l : -1;
-}
-
-template <int TP>
-__device__ inline void select_taps(const Taps1<TP>& a, const Taps1<TP>& b, bool useb, const GridGeom& g, int d,
-				   int org, int range, int (&li)[TP], float (&wt)[TP], bool& any)
-{
-	const int start = useb ? b.start : a.start;
-	const int cnt = useb ? b.cnt : a.cnt;
-	bool an = false;
-
-#pragma unroll
-	for (int j = 0; j < TP; j++) {
-		int l = (j < cnt) ? tap_local(g, d, start + j, org, range) : -1;
-		li[j] = l;
-		wt[j] = useb ? b.w[j] : a.w[j];
-		an = an || (l >= 0);
-	}
-
-	any = an;
-}
-
 template <typename X>
 __device__ inline X sel3(int d, X a, X b, X c)
 {
@@ -805,6 +718,59 @@ __device__ inline float div_width(float x, float width, float rwidth)
 {
 	const float q = x * rwidth;
 	return __builtin_fmaf(__builtin_fmaf(-q, width, x), rwidth, q);
+}
+
+// ---------------------------------------------------------------------------
+// Taps of one sample along one dim (noncart/grid.c:415-457): NT = ceil(width)
+// of them -- of the width + 1 taps of a sample half way between grid points
+// both ends weigh 0 -- with weight 0 for those the grid's edge cuts off.
+// ---------------------------------------------------------------------------
+
+__device__ inline float sample_pos_v(const GridGeom& g, int d, int v, float k)
+{
+	return grid_pos(g.os, k, g.shv[d][v], (float)(g.n[d] / 2));
+}
+
+template <int NT>
+__device__ inline void taps_of(const GridGeom& g, int d, int v, float k, const float* table, float rwidth, int& start,
+			       float (&w)[NT])
+{
+	if (1 == g.n[d]) {
+		start = 0;
+#pragma unroll
+		for (int j = 0; j < NT; j++)
+			w[j] = (0 == j) ? 1.f : 0.f;
+		return;
+	}
+
+	const float pos = sample_pos_v(g, d, v, k);
+	int sti = (int)ceil((double)pos - 0.5 * (double)g.width);
+	int eni = (int)floor((double)pos + 0.5 * (double)g.width);
+
+	if (!g.periodic) {
+		sti = max(sti, 0);
+		eni = min(eni, g.n[d] - 1);
+	}
+
+	start = sti;
+
+#pragma unroll
+	for (int j = 0; j < NT; j++)
+		w[j] = (sti + j <= eni) ? kb_lookup(table, div_width(fabsf((float)(sti + j) - pos), g.width, rwidth)) : 0.f;
+}
+
+// grid index of tap w: wrapped, or kept on the grid (where a tap off it has
+// weight 0)
+__device__ inline int tap_index(const GridGeom& g, int d, int w)
+{
+	const int n = g.n[d];
+
+	if (g.periodic) {
+		w %= n;
+		return w + ((w < 0) ? n : 0);
+	}
+
+	return min(max(w, 0), n - 1);
 }
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -1471,15 +1437,20 @@ void grid_adjoint(const GridPlan& gp, const float* kb, float2* grid, const float
 // multiplied by the weights (:1456-1457).  Samples are taken in cell-sorted
 // order, so that the lanes of a wave read neighbouring grid lines (in the
 // original order a 3-d readout crosses many lines: measured 8x slower on a
-// 128^3 kooshball); the k-space stores go to the original positions.
+// 128^3 kooshball); the k-space stores go to the original positions.  Small
+// problems are bound by a thread's chain of loads, so the dims and taps are
+// constants and every load of a sample (sub-grids x taps) is in flight before
+// the first is used, without branches around taps cut off at the edge; with
+// run-time dims and taps the loads went one by one (64^2, 4 coils: 38 us; now
+// 6.2.  320^2 spiral, 32 coils: 155; now 112).
 // Launch (ceil(M / 256), ceil(C / CC)).
 // ---------------------------------------------------------------------------
 
-template <int TP, int CC>
+template <int NT, int CC, int ND>
 __global__ __launch_bounds__(256) void k_grid_fwd(GridGeom g, const float* __restrict__ kbt,
 						  const int* __restrict__ sm, const float4* __restrict__ sk,
 						  const float2* __restrict__ grid, const float2* __restrict__ weights,
-						  float2* __restrict__ ksp)
+						  float2* __restrict__ ksp, int a0, int a1, int a2, float rwidth)
 {
 	__shared__ float table[KB_SIZE + 1];
 
@@ -1496,17 +1467,39 @@ __global__ __launch_bounds__(256) void k_grid_fwd(GridGeom g, const float* __res
 	const int c0 = blockIdx.y * CC;
 	const int ncc = min(CC, g.C - c0);
 	const float4 kc = sk[i];
-	const float kk[3] = { kc.x, kc.y, kc.z };
+	const int act[3] = { a0, a1, a2 };  // active dims, x first
 
-	Taps1<TP> tv[3][2];
+	// taps of the active dims and shift variants: weights, and offsets of the
+	// grid points in a coil plane
+	float w[ND][2][NT];
+	int off[ND][2][NT];
 
 #pragma unroll
-	for (int d = 0; d < 3; d++) {
-		taps_raw<TP>(g, d, 0, kk[d], table, tv[d][0]);
-		if (g.nshv[d] > 1)
-			taps_raw<TP>(g, d, 1, kk[d], table, tv[d][1]);
-		else
-			tv[d][1] = tv[d][0];
+	for (int a = 0; a < ND; a++) {
+
+		const int d = act[a];
+		const int str = (0 == d) ? 1 : ((1 == d) ? g.n[0] : g.n[0] * g.n[1]);
+		const float k = sel3(d, kc.x, kc.y, kc.z);
+
+#pragma unroll
+		for (int v = 0; v < 2; v++) {
+
+			if (v > 0 && g.nshv[d] < 2) {
+#pragma unroll
+				for (int j = 0; j < NT; j++) {
+					w[a][1][j] = w[a][0][j];
+					off[a][1][j] = off[a][0][j];
+				}
+				continue;
+			}
+
+			int start;
+			taps_of<NT>(g, d, v, k, table, rwidth, start, w[a][v]);
+
+#pragma unroll
+			for (int j = 0; j < NT; j++)
+				off[a][v][j] = str * tap_index(g, d, start + j);
+		}
 	}
 
 	float2 acc[CC];
@@ -1514,18 +1507,23 @@ __global__ __launch_bounds__(256) void k_grid_fwd(GridGeom g, const float* __res
 	for (int cl = 0; cl < CC; cl++)
 		acc[cl] = make_float2(0.f, 0.f);
 
-	for (int s = 0; s < g.S; s++) {
+	// sub-grids: one bit per active dim (unrolled, with all their loads in
+	// flight, while the registers last)
+	constexpr int UNROLL = (ND <= 2 && NT <= 4) ? (1 << ND) : 1;
 
-		int li0[TP], li1[TP], li2[TP];
-		float wt0[TP], wt1[TP], wt2[TP];
-		bool a0, a1, a2;
+#pragma unroll UNROLL
+	for (int s = 0; s < (1 << ND); s++) {
 
-		select_taps<TP>(tv[0][0], tv[0][1], 0 != g.sbit[s][0], g, 0, 0, g.n[0], li0, wt0, a0);
-		select_taps<TP>(tv[1][0], tv[1][1], 0 != g.sbit[s][1], g, 1, 0, g.n[1], li1, wt1, a1);
-		select_taps<TP>(tv[2][0], tv[2][1], 0 != g.sbit[s][2], g, 2, 0, g.n[2], li2, wt2, a2);
+		float ws[ND][NT];
+		int os[ND][NT];
 
-		if (!(a0 && a1 && a2))
-			continue;
+#pragma unroll
+		for (int a = 0; a < ND; a++)
+#pragma unroll
+			for (int j = 0; j < NT; j++) {
+				ws[a][j] = ((s >> a) & 1) ? w[a][1][j] : w[a][0][j];
+				os[a][j] = ((s >> a) & 1) ? off[a][1][j] : off[a][0][j];
+			}
 
 		float2 val[CC];
 #pragma unroll
@@ -1533,36 +1531,29 @@ __global__ __launch_bounds__(256) void k_grid_fwd(GridGeom g, const float* __res
 			val[cl] = make_float2(0.f, 0.f);
 
 		const float2* gs = grid + ((long)s * g.C + c0) * g.N;
+		constexpr int NZ = (ND > 2) ? NT : 1, NY = (ND > 1) ? NT : 1;
 
 #pragma unroll
-		for (int iz = 0; iz < TP; iz++) {
+		for (int iz = 0; iz < NZ; iz++) {
 
-			if (li2[iz] < 0)
-				continue;
-
-			float dz = 1.f * wt2[iz];
+			const float dz = (ND > 2) ? ws[ND - 1][iz] : 1.f;
+			const int oz = (ND > 2) ? os[ND - 1][iz] : 0;
 
 #pragma unroll
-			for (int iy = 0; iy < TP; iy++) {
+			for (int iy = 0; iy < NY; iy++) {
 
-				if (li1[iy] < 0)
-					continue;
-
-				float dy = dz * wt1[iy];
-				const float2* row = gs + (long)g.n[0] * (li1[iy] + (long)g.n[1] * li2[iz]);
+				const float dy = (ND > 1) ? dz * ws[(ND > 1) ? 1 : 0][iy] : dz;
+				const int oy = oz + ((ND > 1) ? os[(ND > 1) ? 1 : 0][iy] : 0);
 
 #pragma unroll
-				for (int ix = 0; ix < TP; ix++) {
+				for (int ix = 0; ix < NT; ix++) {
 
-					if (li0[ix] < 0)
-						continue;
-
-					float dd = dy * wt0[ix];
-					const float2* p = row + li0[ix];
+					const float dd = dy * ws[0][ix];
+					const float2* p = gs + (oy + os[0][ix]);
 
 #pragma unroll
 					for (int cl = 0; cl < CC; cl++) {
-						if (cl < ncc) {
+						if (CC == 1 || cl < ncc) {
 							float2 x = p[(long)cl * g.N];
 							val[cl].x += x.x * dd;
 							val[cl].y += x.y * dd;
@@ -1578,12 +1569,12 @@ __global__ __launch_bounds__(256) void k_grid_fwd(GridGeom g, const float* __res
 	}
 
 	const int m = sm[i];
-	const float2 w = (nullptr != weights) ? weights[m] : make_float2(1.f, 0.f);
+	const float2 wm = (nullptr != weights) ? weights[m] : make_float2(1.f, 0.f);
 
 #pragma unroll
 	for (int cl = 0; cl < CC; cl++)
 		if (cl < ncc)
-			ksp[(long)(c0 + cl) * g.M + m] = (nullptr != weights) ? cmul(acc[cl], w) : acc[cl];
+			ksp[(long)(c0 + cl) * g.M + m] = (nullptr != weights) ? cmul(acc[cl], wm) : acc[cl];
 }
 
 // ---------------------------------------------------------------------------
@@ -1593,20 +1584,35 @@ __global__ __launch_bounds__(256) void k_grid_fwd(GridGeom g, const float* __res
 // outside the grid -- in LDS with row-wise coalesced loads, and each thread
 // gathers the taps of its samples from there.  The arithmetic is that of
 // k_grid_fwd, term by term in the same order, so both give the same bits.
+// A wave's samples come from the same or neighbouring cells, so that its
+// lanes read points up to one apart in every dim: a point is 8 banks, a row
+// 12 points and a plane 2 points more than its rows, which puts the 8 points
+// of such a cube into 8 different bank groups.  All taps are taken (weight 0
+// beyond an edge) instead of branching around the ones that are cut off.
+// Bound by LDS reads (27 float2 per sample, coil and sub-grid) and the waits of
+// the staging: 128^3 kooshball, 16 coils, 3.31 -> 2.85 ms with constant taps
+// and the padded planes (39.6 thousand vector instructions per wave, 47.6
+// before).
 // ---------------------------------------------------------------------------
 
 constexpr size_t FW_TABLE_BYTES = ((KB_SIZE + 4) * sizeof(float) + 15) / 16 * 16;
+constexpr int FW_ZPAD = 2;
+
+// points of the staged region: planes with their padding, and the taps past
+// the last row's end
+constexpr int fw_region(int E) { return E * (E * E + FW_ZPAD) + 4; }
 
 // E: staged region edge (tile + halo); LDS region layout [z][y][x][coil]
-template <int CCH, int E>
+template <int CCH, int E, int NT>
 __global__ __launch_bounds__(FW_THREADS) void k_grid_fwd_tile(GridGeom g, FwdTiling ft, const float* __restrict__ kbt,
 							      const int4* __restrict__ work,
 							      const int* __restrict__ fsm,
 							      const float4* __restrict__ fsk,
 							      const float2* __restrict__ grid,
 							      const float2* __restrict__ weights,
-							      float2* __restrict__ ksp)
+							      float2* __restrict__ ksp, float rwidth)
 {
+	constexpr int ZS = E * E + FW_ZPAD;
 	static_assert(CCH == 4 && E <= 16 && 0 == E % 2, "region rows are loaded by 8 lanes, 4 coils per point");
 
 	extern __shared__ __align__(16) unsigned char fw_smem[];
@@ -1615,6 +1621,10 @@ __global__ __launch_bounds__(FW_THREADS) void k_grid_fwd_tile(GridGeom g, FwdTil
 
 	for (int i = threadIdx.x; i < KB_SIZE + 1; i += FW_THREADS)
 		table[i] = kbt[i];
+
+	// the padding is read with weight 0
+	for (int i = threadIdx.x; i < fw_region(E) * CCH; i += FW_THREADS)
+		reg[i] = make_float2(0.f, 0.f);
 
 	const int4 it = work[blockIdx.x];
 	const int tile = it.x;
@@ -1675,7 +1685,7 @@ __global__ __launch_bounds__(FW_THREADS) void k_grid_fwd_tile(GridGeom g, FwdTil
 					v = *(const float4*)(gs + cl * Ni + gx + n0 * (gy + n1 * gz));
 
 				if (lx2 < E) {
-					float2* d = reg + (zy * E + lx2) * CCH + cl;
+					float2* d = reg + (z * ZS + (zy - z * E) * E + lx2) * CCH + cl;
 					d[0] = make_float2(v.x, v.y);
 					d[CCH] = make_float2(v.z, v.w);
 				}
@@ -1691,30 +1701,16 @@ __global__ __launch_bounds__(FW_THREADS) void k_grid_fwd_tile(GridGeom g, FwdTil
 				if (!valid[q])
 					continue;
 
-				Taps1<4> t0, t1, t2;
-				taps_raw<4>(g, 0, v0, kc[q].x, table, t0);
-				taps_raw<4>(g, 1, v1, kc[q].y, table, t1);
-				taps_raw<4>(g, 2, v2, kc[q].z, table, t2);
+				int b0, b1, b2;
+				float w0[NT], w1[NT], w2[NT];
+				taps_of<NT>(g, 0, v0, kc[q].x, table, rwidth, b0, w0);
+				taps_of<NT>(g, 1, v1, kc[q].y, table, rwidth, b1, w1);
+				taps_of<NT>(g, 2, v2, kc[q].z, table, rwidth, b2, w2);
 
-				// local tap indices (-1: no tap); taps outside the staged
-				// region cannot occur for a sample of this tile
-				int l0[4], l1[4], l2[4];
-				bool a0 = false, a1 = false, a2 = false;
-
-#pragma unroll
-				for (int j = 0; j < 4; j++) {
-					int w0 = t0.start + j, w1 = t1.start + j, w2 = t2.start + j;
-					int q0 = w0 - o0, q1 = w1 - o1, q2 = w2 - o2;
-					l0[j] = (j < t0.cnt && w0 >= 0 && w0 < n0 && q0 >= 0 && q0 < E) ? q0 : -1;
-					l1[j] = (j < t1.cnt && w1 >= 0 && w1 < n1 && q1 >= 0 && q1 < E) ? q1 : -1;
-					l2[j] = (j < t2.cnt && w2 >= 0 && w2 < n2 && q2 >= 0 && q2 < E) ? q2 : -1;
-					a0 = a0 || (l0[j] >= 0);
-					a1 = a1 || (l1[j] >= 0);
-					a2 = a2 || (l2[j] >= 0);
-				}
-
-				if (!(a0 && a1 && a2))
-					continue;
+				// in the staged region (a tap outside it has weight 0)
+				b0 = min(max(b0 - o0, 0), E - 1);
+				b1 -= o1;
+				b2 -= o2;
 
 				float2 val[CCH];
 #pragma unroll
@@ -1722,32 +1718,23 @@ __global__ __launch_bounds__(FW_THREADS) void k_grid_fwd_tile(GridGeom g, FwdTil
 					val[cl] = make_float2(0.f, 0.f);
 
 #pragma unroll
-				for (int iz = 0; iz < 4; iz++) {
+				for (int iz = 0; iz < NT; iz++) {
 
-					if (l2[iz] < 0)
-						continue;
-
-					float dz = 1.f * t2.w[iz];
+					const float dz = w2[iz];
+					const int lz = min(max(b2 + iz, 0), E - 1) * ZS + b0;
 
 #pragma unroll
-					for (int iy = 0; iy < 4; iy++) {
+					for (int iy = 0; iy < NT; iy++) {
 
-						if (l1[iy] < 0)
-							continue;
-
-						float dy = dz * t1.w[iy];
-						const float2* row = reg + (l2[iz] * E + l1[iy]) * E * CCH;
+						const float dy = dz * w1[iy];
+						const float4* row = (const float4*)(reg + (lz + min(max(b1 + iy, 0), E - 1) * E) * CCH);
 
 #pragma unroll
-						for (int ix = 0; ix < 4; ix++) {
+						for (int ix = 0; ix < NT; ix++) {
 
-							if (l0[ix] < 0)
-								continue;
-
-							float dd = dy * t0.w[ix];
-							const float4* pp = (const float4*)(row + l0[ix] * CCH);
-							const float4 x01 = pp[0];
-							const float4 x23 = pp[1];
+							const float dd = dy * w0[ix];
+							const float4 x01 = row[2 * ix];
+							const float4 x23 = row[2 * ix + 1];
 							val[0].x += x01.x * dd;
 							val[0].y += x01.y * dd;
 							val[1].x += x01.z * dd;
@@ -1796,29 +1783,64 @@ void grid_forward(const GridPlan& gp, const float* kb, float2* ksp, const float2
 	if (gp.ft.on) {
 
 		const FwdTiling& ft = gp.ft;
-		const size_t lds = FW_TABLE_BYTES + (size_t)FW_CC * ft.Etot * sizeof(float2);
+		const size_t lds = FW_TABLE_BYTES + (size_t)FW_CC * fw_region(FW_E) * sizeof(float2);
 		BAM_CHECK(4 == taps_bound(g) && !g.periodic && lds <= 64 * 1024 && FW_E == ft.E[0] &&
 			  FW_E == ft.E[1] && FW_E == ft.E[2], "grid_forward: bad tiling");
-		hipLaunchKernelGGL((k_grid_fwd_tile<FW_CC, FW_E>), dim3(ft.nitems), dim3(FW_THREADS), lds, st, g, ft,
-				   kb, gp.fwork.ptr, gp.fsm.ptr, gp.fsk.ptr, grid, weights, ksp);
+#define BAM_FWT(NT)                                                                                              \
+	hipLaunchKernelGGL((k_grid_fwd_tile<FW_CC, FW_E, NT>), dim3(ft.nitems), dim3(FW_THREADS), lds, st, g, ft, kb, \
+			   gp.fwork.ptr, gp.fsm.ptr, gp.fsk.ptr, grid, weights, ksp, gp.ta.rwidth)
+		if (gp.ta.ntap <= 3)
+			BAM_FWT(3);
+		else
+			BAM_FWT(4);
+#undef BAM_FWT
 		BAM_HIP(hipGetLastError());
 		return;
 	}
 
 	const int tp = taps_bound(g);
+	const GridTiling& t = gp.ta;
+
 	// 4 coils per thread: the launch walks the samples chunk by chunk, so the
 	// grid planes in use at a time are those of 4 coils (measured on a 128^3,
 	// 16-coil kooshball: 7.7 ms at 4 coils, 12.4 ms at 16; 1 or 2 coils gain
-	// nothing more)
-	constexpr int CC = 4;
-	dim3 blocks(ceil_div(g.M, 256), ceil_div(g.C, CC));
+	// nothing more).  One coil per thread in 2-D, where the taps cost little
+	// beside the loads and all of a sample's loads fit in flight (320^2 spiral,
+	// 32 coils: 112 us against 121), and where 4 would leave less than 8 waves
+	// per compute unit: a thread's chain of loads is then what the launch waits
+	// for (64^2, 4 coils, 3968 samples: 38 -> 6 us).
+	const bool one = t.ntap <= 3 && (t.nd < 3 || (long)g.M * ceil_div(g.C, 4) < 8l * 64 * gp.ncu);
+	const dim3 blocks(ceil_div(g.M, 256), one ? (unsigned)g.C : ceil_div(g.C, 4));
 
-	if (4 == tp)
-		hipLaunchKernelGGL((k_grid_fwd<4, CC>), blocks, dim3(256), 0, st, g, kb, gp.sm.ptr, gp.sk.ptr, grid,
-				   weights, ksp);
+#define BAM_FWD(NT, CC, ND)                                                                                      \
+	hipLaunchKernelGGL((k_grid_fwd<NT, CC, ND>), blocks, dim3(256), 0, st, g, kb, gp.sm.ptr, gp.sk.ptr, grid, \
+			   weights, ksp, t.act[0], t.act[1], t.act[2], t.rwidth)
+#define BAM_FWD_CC(NT, ND)               \
+	do {                             \
+		if (one)                 \
+			BAM_FWD(3, 1, ND); \
+		else                     \
+			BAM_FWD(NT, 4, ND); \
+	} while (0)
+#define BAM_FWD_ND(NT)                \
+	do {                          \
+		if (3 == t.nd)        \
+			BAM_FWD_CC(NT, 3); \
+		else if (2 == t.nd)   \
+			BAM_FWD_CC(NT, 2); \
+		else                  \
+			BAM_FWD_CC(NT, 1); \
+	} while (0)
+
+	if (t.ntap <= 3)
+		BAM_FWD_ND(3);
+	else if (4 == tp)
+		BAM_FWD_ND(4);
 	else
-		hipLaunchKernelGGL((k_grid_fwd<8, CC>), blocks, dim3(256), 0, st, g, kb, gp.sm.ptr, gp.sk.ptr, grid,
-				   weights, ksp);
+		BAM_FWD_ND(8);
+#undef BAM_FWD_ND
+#undef BAM_FWD_CC
+#undef BAM_FWD
 
 	BAM_HIP(hipGetLastError());
 }
