@@ -84,7 +84,7 @@ AxisPlan make_axis_plan(int n)
 	return p;
 }
 
-FftLaunchCfg fft_config(const AxisPlan& plan, long total, bool contig, int P_min, float sign1, float sign2)
+FftLaunchCfg fft_config(const AxisPlan& plan, long total, bool contig, int P_min, float sign)
 {
 	FftLaunchCfg c;
 	const int n = plan.n;
@@ -107,8 +107,7 @@ FftLaunchCfg fft_config(const AxisPlan& plan, long total, bool contig, int P_min
 		c.L.logP = logP;
 		c.L.contig = contig;
 		c.L.total = total;
-		c.L.sign1 = sign1;
-		c.L.sign2 = sign2;
+		c.L.sign = sign;
 		c.L.pitch = n + 1;
 		c.blocks = (unsigned)((total + P - 1) / P);
 		c.lds_bytes = (size_t)(P * (n + 1) + n) * sizeof(float2);
@@ -143,8 +142,7 @@ FftLaunchCfg fft_config(const AxisPlan& plan, long total, bool contig, int P_min
 	c.L.logP = logP;
 	c.L.contig = contig;
 	c.L.total = total;
-	c.L.sign1 = sign1;
-	c.L.sign2 = sign2;
+	c.L.sign = sign;
 	c.blocks = (unsigned)((total + P - 1) / P);
 	c.L.pitch = n;
 	c.lds_bytes = (size_t)P * n * sizeof(float2);
@@ -241,10 +239,10 @@ void fft_nd(const int dims[3], long batch, unsigned flags, float sign, float2* d
 
 		VolAxis g = VolAxis::make(dims, 2, batch);
 		AxisPlan pz = make_axis_plan(dims[2]);
-		FftLaunchCfg cfg = fft_config(pz, g.transforms(), g.contig(), 1, sign, sign);
+		FftLaunchCfg cfg = fft_config(pz, g.transforms(), g.contig(), 1, sign);
 		LdPlain ld{ g, dst };
 		StPlain st{ g, dst, scale };
-		launch_fft_axis(cfg, stream, ld, NoMid{}, st);
+		launch_fft_axis(cfg, stream, ld, st);
 		return;
 	}
 
@@ -270,12 +268,12 @@ void fft_nd(const int dims[3], long batch, unsigned flags, float sign, float2* d
 
 		VolAxis g = VolAxis::make(dims, a, batch);
 		AxisPlan plan = make_axis_plan(dims[a]);
-		FftLaunchCfg cfg = fft_config(plan, g.transforms(), g.contig(), 1, sign, sign);
+		FftLaunchCfg cfg = fft_config(plan, g.transforms(), g.contig(), 1, sign);
 
 		LdPlain ld{ g, first ? src : dst };
 		StPlain st{ g, dst, (a == last) ? scale : 1.f };
 
-		launch_fft_axis(cfg, stream, ld, NoMid{}, st);
+		launch_fft_axis(cfg, stream, ld, st);
 		first = false;
 	}
 }

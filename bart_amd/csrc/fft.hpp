@@ -52,8 +52,7 @@ struct FftLaunch {
 	int pitch = 0;       // LDS distance of consecutive transforms (n or n + 1)
 	bool contig = true;
 	long total = 0;      // number of transforms
-	float sign1 = -1.f;  // first transform
-	float sign2 = +1.f;  // second transform (only when a middle stage is present)
+	float sign = -1.f;  // first transform
 	const int* skip = nullptr;  // device flag: when set (non-zero) the launch does nothing
 };
 
@@ -304,16 +303,6 @@ __device__ inline void run_passes(float2* lds, const AxisPlan& plan, int P, floa
 	}
 }
 
-// Identity middle stage.
-struct NoMid {
-	static constexpr bool active = false;
-	static constexpr bool colblock = true;
-	__device__ float2 operator()(long, int, float2 v) const { return v; }
-	__device__ bool cb_ok(int) const { return true; }
-	__device__ int base(long) const { return 0; }
-	__device__ float2 at(int, int, int, float2 v) const { return v; }
-};
-
 // functors with column-block access (static constexpr bool colblock = true;
 // cb_ok(P), base(t0), at(base, p, k [, v]))
 template <class F, class = void>
@@ -328,13 +317,12 @@ struct colblock_of<F, std::void_t<decltype(F::colblock)>> {
 
 // ---------------------------------------------------------------------------
 // The axis kernel.  Ld: float2 operator()(long t, int k) const.
-// Md: float2 operator()(long t, int k, float2 v) const (when active).
 // St: void store(const float2* lds, const FftLaunch&, long t0) const -- runs
 //     the block's whole store loop so that it may reduce over transforms.
 // ---------------------------------------------------------------------------
 
-template <int EPT, bool GEN, class Ld, class Md, class St>
-__global__ __launch_bounds__(FFT_THREADS) void k_fft_axis(FftLaunch L, Ld ld, Md md, St st)
+template <int EPT, bool GEN, class Ld, class St>
+__global__ __launch_bounds__(FFT_THREADS) void k_fft_axis(FftLaunch L, Ld ld, St st)
 {
 	extern __shared__ float2 lds[];
 
@@ -378,32 +366,7 @@ __global__ __launch_bounds__(FFT_THREADS) void k_fft_axis(FftLaunch L, Ld ld, Md
 
 	lds_barrier();
 
-	run_passes<EPT, GEN>(lds, L.plan, P, L.sign1);
-
-	if constexpr (Md::active) {
-
-		for (int i = threadIdx.x; i < tot; i += FFT_THREADS) {
-
-			int p, k;
-
-			if (L.contig) {
-				p = i / n;
-				k = i - p * n;
-			} else {
-				p = i & (P - 1);
-				k = i >> L.logP;
-			}
-
-			long t = t0 + p;
-
-			if (t < L.total)
-				lds[p * n + k] = md(t, k, lds[p * n + k]);
-		}
-
-		lds_barrier();
-
-		run_passes<EPT, GEN>(lds, L.plan, P, L.sign2);
-	}
+	run_passes<EPT, GEN>(lds, L.plan, P, L.sign);
 
 	st.store(lds, L, t0);
 }
@@ -548,13 +511,11 @@ __device__ inline void ct_passes_between(float2* lds, const float2* tw, float sg
 	}
 }
 
-// Transform of a column block (strided axis) -- or forward transform,
-// pointwise multiply and inverse transform -- with the first and last passes
+// Transform of a column block (strided axis) with the first and last passes
 // in registers: a thread's E = P N / FFT_THREADS points k0 + j N / E are the
 // inputs of one butterfly of the first radix-E pass and the outputs of one
-// butterfly of the last radix-E pass, so the loads, the stores and (with a
-// multiply) the forward's last pass, the multiply and the inverse's first
-// pass need no LDS round trip.
+// butterfly of the last radix-E pass, so the loads and the stores need no LDS
+// round trip.
 template <int N>
 constexpr int ct_edge_radix()
 {
@@ -569,8 +530,8 @@ constexpr bool ct_edges_in_regs()
 	       0 == N % (E * E) && 0 == FFT_THREADS % ct_block_p(N);
 }
 
-template <int N, int E, class Ld, class Md, class St>
-__device__ inline void fft_mul_ifft_regs(const FftLaunch& L, const Ld& ld, const Md& md, const St& st, float2* lds,
+template <int N, int E, class Ld, class St>
+__device__ inline void fft_cols_regs(const FftLaunch& L, const Ld& ld, const St& st, float2* lds,
 					 const float2* tw, long t0)
 {
 	constexpr int P = ct_block_p(N);
@@ -591,7 +552,7 @@ __device__ inline void fft_mul_ifft_regs(const FftLaunch& L, const Ld& ld, const
 			v[j] = in ? ld.at(lb, p, k0 + j * NE) : make_float2(0.f, 0.f);
 	}
 
-	dft_any<E>(v, L.sign1, tw, N);
+	dft_any<E>(v, L.sign, tw, N);
 
 #pragma unroll
 	for (int q = 0; q < E; q++)
@@ -599,50 +560,22 @@ __device__ inline void fft_mul_ifft_regs(const FftLaunch& L, const Ld& ld, const
 
 	lds_barrier();
 
-	ct_passes_between<N, P, E, NE>(lds, tw, L.sign1);
+	ct_passes_between<N, P, E, NE>(lds, tw, L.sign);
 
-	// last forward pass (radix E, sub-transforms of length N / E)
-	auto last_pass = [&](float sgn) {
+	// last pass (radix E, sub-transforms of length N / E)
 #pragma unroll
-		for (int r = 0; r < E; r++) {
-			float2 x = lds[p * PN + k0 + r * NE];
-			if (r > 0) {
-				float2 w = tw[r * k0];
-				if (sgn > 0.f)
-					w.y = -w.y;
-				x = cmul(x, w);
-			}
-			v[r] = x;
+	for (int r = 0; r < E; r++) {
+		float2 x = lds[p * PN + k0 + r * NE];
+		if (r > 0) {
+			float2 w = tw[r * k0];
+			if (L.sign > 0.f)
+				w.y = -w.y;
+			x = cmul(x, w);
 		}
-		dft_any<E>(v, sgn, tw, N);
-	};
-
-	last_pass(L.sign1);
-
-	if constexpr (Md::active) {
-
-		// pointwise multiply of the points k0 + q N / E; first inverse pass
-		if (in) {
-			const auto mb = md.base(t0);
-#pragma unroll
-			for (int q = 0; q < E; q++)
-				v[q] = md.at(mb, p, k0 + q * NE, v[q]);
-		}
-
-		dft_any<E>(v, L.sign2, tw, N);
-
-		lds_barrier();
-
-#pragma unroll
-		for (int q = 0; q < E; q++)
-			lds[p * PN + k0 * E + q] = v[q];
-
-		lds_barrier();
-
-		ct_passes_between<N, P, E, NE>(lds, tw, L.sign2);
-
-		last_pass(L.sign2);
+		v[r] = x;
 	}
+
+	dft_any<E>(v, L.sign, tw, N);
 
 	if (in) {
 		const auto sb = st.base(t0);
@@ -652,19 +585,9 @@ __device__ inline void fft_mul_ifft_regs(const FftLaunch& L, const Ld& ld, const
 	}
 }
 
-// store functors that take single elements: put(t, k, value)
-template <class F, class = void>
-struct has_put : std::false_type {
-};
-template <class F>
-struct has_put<F, std::void_t<decltype(std::declval<const F&>().put(0l, 0, float2{}))>> : std::true_type {
-};
-
 // Contiguous axis (transforms along rows): a thread takes the E points
 // k0 + j N / E of one transform -- coalesced loads along k0 -- runs the
-// first radix-E pass on them, the middle passes in LDS, and, when the store
-// takes single elements, the last radix-E pass into registers and stores
-// from there.
+// first radix-E pass on them and the other passes in LDS.
 template <int N, int E, class Ld, class St>
 __device__ inline void fft_contig_regs(const FftLaunch& L, const Ld& ld, const St& st, float2* lds, const float2* tw,
 				       long t0)
@@ -683,7 +606,7 @@ __device__ inline void fft_contig_regs(const FftLaunch& L, const Ld& ld, const S
 	for (int j = 0; j < E; j++)
 		v[j] = in ? ld(t, k0 + j * NE) : make_float2(0.f, 0.f);
 
-	dft_any<E>(v, L.sign1, tw, N);
+	dft_any<E>(v, L.sign, tw, N);
 
 #pragma unroll
 	for (int q = 0; q < E; q++)
@@ -691,40 +614,13 @@ __device__ inline void fft_contig_regs(const FftLaunch& L, const Ld& ld, const S
 
 	lds_barrier();
 
-	if constexpr (has_put<St>::value) {
-
-		ct_passes_between<N, P, E, NE>(lds, tw, L.sign1);
-
-#pragma unroll
-		for (int r = 0; r < E; r++) {
-			float2 x = lds[p * PN + k0 + r * NE];
-			if (r > 0) {
-				float2 w = tw[r * k0];
-				if (L.sign1 > 0.f)
-					w.y = -w.y;
-				x = cmul(x, w);
-			}
-			v[r] = x;
-		}
-
-		dft_any<E>(v, L.sign1, tw, N);
-
-		if (in)
-#pragma unroll
-			for (int q = 0; q < E; q++)
-				st.put(t, k0 + q * NE, v[q]);
-
-	} else {
-
-		ct_passes_between<N, P, E, N>(lds, tw, L.sign1);
-		st.store(lds, L, t0);
-	}
+	ct_passes_between<N, P, E, N>(lds, tw, L.sign);
+	st.store(lds, L, t0);
 }
 
-// The transforms [t0, t0 + P) of one launch (the body of k_fft_axis_n and of
-// its batched form k_fft_axis_n_batch).
-template <int N, class Ld, class Md, class St>
-__device__ inline void fft_axis_block(const FftLaunch& L, const Ld& ld, const Md& md, const St& st, long t0,
+// The transforms [t0, t0 + P) of one launch (the body of k_fft_axis_n).
+template <int N, class Ld, class St>
+__device__ inline void fft_axis_block(const FftLaunch& L, const Ld& ld, const St& st, long t0,
 				      float2* lds)
 {
 	constexpr int P = ct_block_p(N);
@@ -736,23 +632,23 @@ __device__ inline void fft_axis_block(const FftLaunch& L, const Ld& ld, const Md
 	float2* tw = lds + P * PN;
 
 	// strided axis with column-block functors: per-block base addresses
-	constexpr bool CBF = colblock_of<Ld>::value && colblock_of<Md>::value && colblock_of<St>::value;
+	constexpr bool CBF = colblock_of<Ld>::value && colblock_of<St>::value;
 	bool cb = false;
 
 	if constexpr (CBF)
-		cb = !L.contig && ld.cb_ok(P) && md.cb_ok(P) && st.cb_ok(P);
+		cb = !L.contig && ld.cb_ok(P) && st.cb_ok(P);
 
 	for (int i = threadIdx.x; i < N; i += FFT_THREADS)
 		tw[i] = L.plan.tw[i];
 
 	if constexpr (CBF && ct_edges_in_regs<N>()) {
 		if (cb) {
-			fft_mul_ifft_regs<N, ct_edge_radix<N>()>(L, ld, md, st, lds, tw, t0);
+			fft_cols_regs<N, ct_edge_radix<N>()>(L, ld, st, lds, tw, t0);
 			return;
 		}
 	}
 
-	if constexpr (!Md::active && ct_edges_in_regs<N>()) {
+	if constexpr (ct_edges_in_regs<N>()) {
 		if (L.contig) {
 			fft_contig_regs<N, ct_edge_radix<N>()>(L, ld, st, lds, tw, t0);
 			return;
@@ -801,52 +697,7 @@ __device__ inline void fft_axis_block(const FftLaunch& L, const Ld& ld, const Md
 
 	lds_barrier();
 
-	ct_passes<N, P, 0, 1>(lds, tw, L.sign1);
-
-	if constexpr (Md::active) {
-
-		bool done = false;
-
-		if constexpr (CBF) {
-			if (cb) {
-				const auto mb = md.base(t0);
-
-				for (int i = threadIdx.x; i < TOT; i += FFT_THREADS) {
-					const int p = i & (P - 1);
-					const int k = i >> LOGP;
-					if (t0 + p < L.total)
-						lds[p * PN + k] = md.at(mb, p, k, lds[p * PN + k]);
-				}
-
-				done = true;
-			}
-		}
-
-		if (!done) {
-
-			for (int i = threadIdx.x; i < TOT; i += FFT_THREADS) {
-
-				int p, k;
-
-				if (L.contig) {
-					p = i / N;
-					k = i - p * N;
-				} else {
-					p = i & (P - 1);
-					k = i >> LOGP;
-				}
-
-				const long t = t0 + p;
-
-				if (t < L.total)
-					lds[p * PN + k] = md(t, k, lds[p * PN + k]);
-			}
-		}
-
-		lds_barrier();
-
-		ct_passes<N, P, 0, 1>(lds, tw, L.sign2);
-	}
+	ct_passes<N, P, 0, 1>(lds, tw, L.sign);
 
 	if constexpr (CBF) {
 		if (cb) {
@@ -866,281 +717,15 @@ __device__ inline void fft_axis_block(const FftLaunch& L, const Ld& ld, const Md
 	st.store(lds, L, t0);
 }
 
-template <int N, class Ld, class Md, class St>
-__global__ __launch_bounds__(FFT_THREADS) void k_fft_axis_n(FftLaunch L, Ld ld, Md md, St st)
+template <int N, class Ld, class St>
+__global__ __launch_bounds__(FFT_THREADS) void k_fft_axis_n(FftLaunch L, Ld ld, St st)
 {
 	extern __shared__ float2 lds[];
 
 	if (nullptr != L.skip && 0 != *L.skip)
 		return;
 
-	fft_axis_block<N>(L, ld, md, st, (long)blockIdx.x * ct_block_p(N), lds);
-}
-
-// One pass of many problems of the same transform length in one launch:
-// items[q] holds problem q's launch and functors, btab[b] = (q, block of
-// problem q) for work-group b.
-template <class Ld, class Md, class St>
-struct FftItem {
-	FftLaunch L;
-	Ld ld;
-	Md md;
-	St st;
-};
-
-template <int N, class Ld, class Md, class St>
-__global__ __launch_bounds__(FFT_THREADS) void k_fft_axis_n_batch(const FftItem<Ld, Md, St>* __restrict__ items,
-								  const int2* __restrict__ btab)
-{
-	extern __shared__ float2 lds[];
-	const int2 e = btab[blockIdx.x];
-	const FftItem<Ld, Md, St>& it = items[e.x];
-
-	if (nullptr != it.L.skip && 0 != *it.L.skip)
-		return;
-
-	fft_axis_block<N>(it.L, it.ld, it.md, it.st, (long)e.y * ct_block_p(N), lds);
-}
-
-// Lengths whose pair kernel exists (k_fft_axis_pair needs the register-edge
-// geometry of the column-block path).
-inline bool fft_pair_len_ok(int n)
-{
-	return 64 == n || 128 == n || 256 == n || 512 == n;
-}
-
-// columns per block of the pair kernel: 2048 elements up to n = 128 (for
-// n = 128, 16 columns of 4 points per thread need 63 registers and allow
-// 8 waves per SIMD, against 112 and 4 for 32 columns: 0.94 against 1.05 ms
-// per kooshball z-pass)
-constexpr int pair_block_p(int n)
-{
-	return (n <= 128) ? 2048 / n : ct_block_p(n);
-}
-
-// the register-edge geometry for P columns of length N
-template <int N, int P>
-constexpr bool edges_in_regs_p()
-{
-	constexpr int E = P * N / FFT_THREADS;
-	return 0 == (P * N) % FFT_THREADS && (2 == E || 4 == E || 8 == E || 16 == E) && 0 == N % (E * E) &&
-	       0 == FFT_THREADS % P;
-}
-
-// Strided-axis transform, pointwise multiply and inverse transform for a
-// pair of inputs that differ only by a factor along the axis: the column h
-// (held in registers) is multiplied by zf(b, k), transformed, multiplied by
-// the pair member's factor table at(b, ...), inverse-transformed, and
-// conj(zf(b, k)) x result is summed over b = 0, 1 into the store.  One read
-// and one write of the column serve both members.  Md provides base(t0),
-// at(base, b, p, k, x), zf(b, k) and cb_ok(P); the host launches it only
-// where the column-block geometry holds (cb_ok for every functor, strided).
-template <int N, class Ld, class Md, class St>
-__global__ __launch_bounds__(FFT_THREADS) void k_fft_axis_pair(FftLaunch L, Ld ld, Md md, St st)
-{
-	constexpr int P = pair_block_p(N);
-	static_assert(edges_in_regs_p<N, P>(), "pair kernel needs the register-edge geometry");
-	constexpr int LOGP = ct_log2(P);
-	constexpr int PN = N + 1;
-	constexpr int E = P * N / FFT_THREADS;
-	constexpr int NE = N / E;
-
-	extern __shared__ float2 lds[];
-	float2* tw = lds + P * PN;
-
-	if (nullptr != L.skip && 0 != *L.skip)
-		return;
-
-	const long t0 = (long)blockIdx.x * P;
-
-	for (int i = threadIdx.x; i < N; i += FFT_THREADS)
-		tw[i] = L.plan.tw[i];
-
-	const int p = threadIdx.x & (P - 1);
-	const int k0 = threadIdx.x >> LOGP;
-	const bool in = t0 + p < L.total;
-	float2 h[E], acc[E], v[E];
-
-	{
-		const auto lb = ld.base(t0);
-#pragma unroll
-		for (int j = 0; j < E; j++) {
-			h[j] = in ? ld.at(lb, p, k0 + j * NE) : make_float2(0.f, 0.f);
-			acc[j] = make_float2(0.f, 0.f);
-		}
-	}
-
-	const auto mb = md.base(t0);
-
-	// last radix-E pass of a transform (sub-transforms of length N / E) from
-	// LDS into registers
-	auto last_pass = [&](float sgn) {
-#pragma unroll
-		for (int r = 0; r < E; r++) {
-			float2 x = lds[p * PN + k0 + r * NE];
-			if (r > 0) {
-				float2 w = tw[r * k0];
-				if (sgn > 0.f)
-					w.y = -w.y;
-				x = cmul(x, w);
-			}
-			v[r] = x;
-		}
-		dft_any<E>(v, sgn, tw, N);
-	};
-
-	for (int b = 0; b < 2; b++) {
-
-		// factor along the axis; first forward pass in registers
-#pragma unroll
-		for (int j = 0; j < E; j++)
-			v[j] = cmul(h[j], md.zf(b, k0 + j * NE));
-
-		dft_any<E>(v, L.sign1, tw, N);
-
-		if (b > 0)
-			lds_barrier();  // the previous member's last pass has read LDS
-
-#pragma unroll
-		for (int q = 0; q < E; q++)
-			lds[p * PN + k0 * E + q] = v[q];
-
-		lds_barrier();
-		ct_passes_between<N, P, E, NE>(lds, tw, L.sign1);
-		last_pass(L.sign1);
-
-		// pointwise multiply; first inverse pass
-		if (in) {
-#pragma unroll
-			for (int q = 0; q < E; q++)
-				v[q] = md.at(mb, b, p, k0 + q * NE, v[q]);
-		}
-
-		dft_any<E>(v, L.sign2, tw, N);
-
-		lds_barrier();
-
-#pragma unroll
-		for (int q = 0; q < E; q++)
-			lds[p * PN + k0 * E + q] = v[q];
-
-		lds_barrier();
-		ct_passes_between<N, P, E, NE>(lds, tw, L.sign2);
-		last_pass(L.sign2);
-
-#pragma unroll
-		for (int q = 0; q < E; q++)
-			acc[q] = cadd(acc[q], cmulc(v[q], md.zf(b, k0 + q * NE)));
-	}
-
-	if (in) {
-		const auto sb = st.base(t0);
-#pragma unroll
-		for (int q = 0; q < E; q++)
-			st.at(sb, p, k0 + q * NE, acc[q]);
-	}
-}
-
-// Strided-axis transform for a pair of volumes that differ only by a
-// factor along the axis, without a pointwise multiply.  Split (forward): the
-// column h of volume v is multiplied by zf_b(k) and transformed, for b = 0, 1,
-// into volumes v and v + pair_off.  Merge (adjoint): the columns of volumes
-// v and v + pair_off are transformed and conj(zf_b(k)) x result is summed
-// over b into volume v.  Same launch geometry as k_fft_axis_pair.
-template <int N, bool MERGE, class Ld, class St>
-__global__ __launch_bounds__(FFT_THREADS) void k_fft_axis_pair_io(FftLaunch L, Ld ld, St st, const float2* zf0,
-								  const float2* zf1, long pair_off)
-{
-	constexpr int P = pair_block_p(N);
-	static_assert(edges_in_regs_p<N, P>(), "pair kernel needs the register-edge geometry");
-	constexpr int LOGP = ct_log2(P);
-	constexpr int PN = N + 1;
-	constexpr int E = P * N / FFT_THREADS;
-	constexpr int NE = N / E;
-
-	extern __shared__ float2 lds[];
-	float2* tw = lds + P * PN;
-
-	if (nullptr != L.skip && 0 != *L.skip)
-		return;
-
-	const long t0 = (long)blockIdx.x * P;
-
-	for (int i = threadIdx.x; i < N; i += FFT_THREADS)
-		tw[i] = L.plan.tw[i];
-
-	const int p = threadIdx.x & (P - 1);
-	const int k0 = threadIdx.x >> LOGP;
-	const bool in = t0 + p < L.total;
-	float2 h[E], v[E];  // split: the input column; merge: the sum
-
-	const auto lb = ld.base(t0);
-	const auto sb = st.base(t0);
-
-#pragma unroll
-	for (int j = 0; j < E; j++)
-		h[j] = (!MERGE && in) ? ld.at(lb, p, k0 + j * NE) : make_float2(0.f, 0.f);
-
-	for (int b = 0; b < 2; b++) {
-
-		const float2* zf = (0 == b) ? zf0 : zf1;
-
-		if constexpr (MERGE) {
-			auto lbb = lb;
-			lbb.off += b * pair_off;
-#pragma unroll
-			for (int j = 0; j < E; j++)
-				v[j] = in ? ld.at(lbb, p, k0 + j * NE) : make_float2(0.f, 0.f);
-		} else {
-#pragma unroll
-			for (int j = 0; j < E; j++)
-				v[j] = cmul(h[j], zf[k0 + j * NE]);
-		}
-
-		dft_any<E>(v, L.sign1, tw, N);
-
-		if (b > 0)
-			lds_barrier();  // the previous member's last pass has read LDS
-
-#pragma unroll
-		for (int q = 0; q < E; q++)
-			lds[p * PN + k0 * E + q] = v[q];
-
-		lds_barrier();
-		ct_passes_between<N, P, E, NE>(lds, tw, L.sign1);
-
-		// last radix-E pass into registers
-#pragma unroll
-		for (int r = 0; r < E; r++) {
-			float2 x = lds[p * PN + k0 + r * NE];
-			if (r > 0) {
-				float2 w = tw[r * k0];
-				if (L.sign1 > 0.f)
-					w.y = -w.y;
-				x = cmul(x, w);
-			}
-			v[r] = x;
-		}
-		dft_any<E>(v, L.sign1, tw, N);
-
-		if constexpr (MERGE) {
-#pragma unroll
-			for (int q = 0; q < E; q++)
-				h[q] = cadd(h[q], cmulc(v[q], zf[k0 + q * NE]));
-		} else if (in) {
-			auto sbb = sb;
-			sbb.off += b * pair_off;
-#pragma unroll
-			for (int q = 0; q < E; q++)
-				st.at(sbb, p, k0 + q * NE, v[q]);
-		}
-	}
-
-	if (MERGE && in) {
-#pragma unroll
-		for (int q = 0; q < E; q++)
-			st.at(sb, p, k0 + q * NE, h[q]);
-	}
+	fft_axis_block<N>(L, ld, st, (long)blockIdx.x * ct_block_p(N), lds);
 }
 
 // ---------------------------------------------------------------------------
@@ -1225,85 +810,6 @@ __device__ inline void slice_passes(float2* lds, const float2* tw, float sgn)
 	}
 }
 
-// The passes of a length-N transform after its first passes have built
-// sub-transforms of length NS in place (M = N / NS still to combine).
-template <int N, int M, int NS, int P, int ES, int TS, int NTH>
-__device__ inline void slice_passes_rest(float2* lds, const float2* tw, float sgn)
-{
-	if constexpr (M > 1) {
-		constexpr int R = SLICE_R16 ? ct_next_radix16(M) : ct_next_radix(M);
-		slice_pass<N, R, NS, P, ES, TS, NTH>(lds, tw, sgn);
-		slice_passes_rest<N, M / R, NS * R, P, ES, TS, NTH>(lds, tw, sgn);
-	}
-}
-
-// the passes from sub-transforms of length NS up to (not including) length
-// NSEND, radices as slice_passes chooses them
-template <int N, int NS, int NSEND, int P, int ES, int TS, int NTH>
-__device__ inline void slice_passes_range(float2* lds, const float2* tw, float sgn)
-{
-	if constexpr (NS < NSEND) {
-		constexpr int R = SLICE_R16 ? ct_next_radix16(N / NS) : ct_next_radix(N / NS);
-		slice_pass<N, R, NS, P, ES, TS, NTH>(lds, tw, sgn);
-		slice_passes_range<N, NS * R, NSEND, P, ES, TS, NTH>(lds, tw, sgn);
-	}
-}
-
-// radix of the last pass of slice_passes for length n
-constexpr int slice_last_radix(int n)
-{
-	int m = n, r = n;
-	while (m > 1) {
-		r = SLICE_R16 ? ct_next_radix16(m) : ct_next_radix(m);
-		m /= r;
-	}
-	return r;
-}
-
-// The last (radix R) pass of P length-N transforms stored as rows (element
-// stride 1, row pitch LD) with the lanes along the butterfly index j of a
-// row: butterfly (p, j) reads j + r N / R and yields the outputs x = j +
-// q N / R of row p, handed to f(m, q, p, x, value) (m: the thread's
-// butterfly count) instead of being written back.
-template <int N, int R, int P, int LD, int NTH, class F>
-__device__ inline void slice_last_pass_rows(const float2* lds, const float2* tw, float sgn, F&& f)
-{
-	constexpr int NS = N / R;
-	constexpr int NB = P * NS;
-	constexpr int PER = (NB + NTH - 1) / NTH;
-
-#pragma unroll
-	for (int m = 0; m < PER; m++) {
-
-		const int b = threadIdx.x + m * NTH;
-
-		if (0 != NB % NTH && b >= NB)
-			break;
-
-		const int p = b / NS;
-		const int j = b - p * NS;
-		float2 v[R];
-
-#pragma unroll
-		for (int r = 0; r < R; r++) {
-			float2 x = lds[p * LD + j + r * NS];
-			if (r > 0) {
-				float2 w = tw[r * j];
-				if (sgn > 0.f)
-					w.y = -w.y;
-				x = cmul(x, w);
-			}
-			v[r] = x;
-		}
-
-		dft_any<R>(v, sgn, tw, N);
-
-#pragma unroll
-		for (int q = 0; q < R; q++)
-			f(m, q, p, j + q * NS, v[q]);
-	}
-}
-
 // lengths with a compile-time kernel
 inline bool ct_supported(int n)
 {
@@ -1355,57 +861,10 @@ struct FftLaunchCfg {
 	const char* name = "fft_axis";
 };
 
-FftLaunchCfg fft_config(const AxisPlan& plan, long total, bool contig, int P_min, float sign1, float sign2);
+FftLaunchCfg fft_config(const AxisPlan& plan, long total, bool contig, int P_min, float sign);
 
-// the launch geometry of k_fft_axis_pair (its own columns per block)
-inline void fft_config_pair(FftLaunchCfg& c)
-{
-	const int n = c.L.plan.n;
-	const int P = pair_block_p(n);
-	int logP = 0;
-	while ((1 << logP) < P)
-		logP++;
-	c.L.P = P;
-	c.L.logP = logP;
-	c.blocks = (unsigned)((c.L.total + P - 1) / P);
-	c.lds_bytes = (size_t)(P * (n + 1) + n) * sizeof(float2);
-}
-
-// k_fft_axis_n_batch over nblocks work-groups for transforms of length n
-// (a compile-time length); items and btab device arrays
-template <class Ld, class Md, class St>
-void launch_fft_axis_batch(int n, const FftItem<Ld, Md, St>* items, const int2* btab, int nblocks, size_t lds_bytes,
-			   hipStream_t stream, const char* name)
-{
-	if (nblocks <= 0)
-		return;
-
-	ProfScope prof(name, stream);
-	const dim3 gb((unsigned)nblocks), tb(FFT_THREADS);
-
-#define BAM_FFT_N(NN) case NN: hipLaunchKernelGGL((k_fft_axis_n_batch<NN, Ld, Md, St>), gb, tb, lds_bytes, stream, items, btab); break
-	switch (n) {
-		BAM_FFT_N(16);
-		BAM_FFT_N(32);
-		BAM_FFT_N(64);
-		BAM_FFT_N(128);
-		BAM_FFT_N(192);
-		BAM_FFT_N(256);
-		BAM_FFT_N(320);
-		BAM_FFT_N(384);
-		BAM_FFT_N(512);
-		BAM_FFT_N(640);
-		BAM_FFT_N(768);
-	default:
-		fail("batched FFT: no kernel for n = %d", n);
-	}
-#undef BAM_FFT_N
-
-	BAM_HIP(hipGetLastError());
-}
-
-template <class Ld, class Md, class St>
-void launch_fft_axis(const FftLaunchCfg& cfg, hipStream_t stream, const Ld& ld, const Md& md, const St& st)
+template <class Ld, class St>
+void launch_fft_axis(const FftLaunchCfg& cfg, hipStream_t stream, const Ld& ld, const St& st)
 {
 	if (0 == cfg.blocks)
 		return;
@@ -1417,7 +876,7 @@ void launch_fft_axis(const FftLaunchCfg& cfg, hipStream_t stream, const Ld& ld, 
 		const dim3 gb(cfg.blocks), tb(FFT_THREADS);
 		const size_t lds = cfg.lds_bytes;
 
-#define BAM_FFT_N(NN) case NN: hipLaunchKernelGGL((k_fft_axis_n<NN, Ld, Md, St>), gb, tb, lds, stream, cfg.L, ld, md, st); break
+#define BAM_FFT_N(NN) case NN: hipLaunchKernelGGL((k_fft_axis_n<NN, Ld, St>), gb, tb, lds, stream, cfg.L, ld, st); break
 		switch (cfg.L.plan.n) {
 			BAM_FFT_N(16);
 			BAM_FFT_N(32);
@@ -1448,72 +907,17 @@ void launch_fft_axis(const FftLaunchCfg& cfg, hipStream_t stream, const Ld& ld, 
 
 	if (gen) {
 		switch (cfg.ept) {
-		case 8: hipLaunchKernelGGL((k_fft_axis<8, true, Ld, Md, St>), gb, tb, cfg.lds_bytes, stream, cfg.L, ld, md, st); break;
-		case 16: hipLaunchKernelGGL((k_fft_axis<16, true, Ld, Md, St>), gb, tb, cfg.lds_bytes, stream, cfg.L, ld, md, st); break;
-		default: hipLaunchKernelGGL((k_fft_axis<32, true, Ld, Md, St>), gb, tb, cfg.lds_bytes, stream, cfg.L, ld, md, st); break;
+		case 8: hipLaunchKernelGGL((k_fft_axis<8, true, Ld, St>), gb, tb, cfg.lds_bytes, stream, cfg.L, ld, st); break;
+		case 16: hipLaunchKernelGGL((k_fft_axis<16, true, Ld, St>), gb, tb, cfg.lds_bytes, stream, cfg.L, ld, st); break;
+		default: hipLaunchKernelGGL((k_fft_axis<32, true, Ld, St>), gb, tb, cfg.lds_bytes, stream, cfg.L, ld, st); break;
 		}
 	} else {
 		switch (cfg.ept) {
-		case 8: hipLaunchKernelGGL((k_fft_axis<8, false, Ld, Md, St>), gb, tb, cfg.lds_bytes, stream, cfg.L, ld, md, st); break;
-		case 16: hipLaunchKernelGGL((k_fft_axis<16, false, Ld, Md, St>), gb, tb, cfg.lds_bytes, stream, cfg.L, ld, md, st); break;
-		default: hipLaunchKernelGGL((k_fft_axis<32, false, Ld, Md, St>), gb, tb, cfg.lds_bytes, stream, cfg.L, ld, md, st); break;
+		case 8: hipLaunchKernelGGL((k_fft_axis<8, false, Ld, St>), gb, tb, cfg.lds_bytes, stream, cfg.L, ld, st); break;
+		case 16: hipLaunchKernelGGL((k_fft_axis<16, false, Ld, St>), gb, tb, cfg.lds_bytes, stream, cfg.L, ld, st); break;
+		default: hipLaunchKernelGGL((k_fft_axis<32, false, Ld, St>), gb, tb, cfg.lds_bytes, stream, cfg.L, ld, st); break;
 		}
 	}
-
-	BAM_HIP(hipGetLastError());
-}
-
-template <class Ld, class Md, class St>
-void launch_fft_axis_pair(const FftLaunchCfg& cfg, hipStream_t stream, const Ld& ld, const Md& md, const St& st)
-{
-	BAM_CHECK(cfg.fixed && !cfg.L.contig && fft_pair_len_ok(cfg.L.plan.n) &&
-			  cfg.L.P == pair_block_p(cfg.L.plan.n),
-		  "pair transform: unsupported geometry (n = %d, P = %d)", cfg.L.plan.n, cfg.L.P);
-
-	if (0 == cfg.blocks)
-		return;
-
-	ProfScope prof(cfg.name, stream);
-	const dim3 gb(cfg.blocks), tb(FFT_THREADS);
-
-#define BAM_FFT_N(NN) case NN: hipLaunchKernelGGL((k_fft_axis_pair<NN, Ld, Md, St>), gb, tb, cfg.lds_bytes, stream, cfg.L, ld, md, st); break
-	switch (cfg.L.plan.n) {
-		BAM_FFT_N(64);
-		BAM_FFT_N(128);
-		BAM_FFT_N(256);
-		BAM_FFT_N(512);
-	default:
-		fail("pair transform: no kernel for n = %d", cfg.L.plan.n);
-	}
-#undef BAM_FFT_N
-
-	BAM_HIP(hipGetLastError());
-}
-
-template <bool MERGE, class Ld, class St>
-void launch_fft_axis_pair_io(const FftLaunchCfg& cfg, hipStream_t stream, const Ld& ld, const St& st,
-			     const float2* zf0, const float2* zf1, long pair_off)
-{
-	BAM_CHECK(cfg.fixed && !cfg.L.contig && fft_pair_len_ok(cfg.L.plan.n) &&
-			  cfg.L.P == pair_block_p(cfg.L.plan.n),
-		  "pair transform: unsupported geometry (n = %d, P = %d)", cfg.L.plan.n, cfg.L.P);
-
-	if (0 == cfg.blocks)
-		return;
-
-	ProfScope prof(cfg.name, stream);
-	const dim3 gb(cfg.blocks), tb(FFT_THREADS);
-
-#define BAM_FFT_N(NN) case NN: hipLaunchKernelGGL((k_fft_axis_pair_io<NN, MERGE, Ld, St>), gb, tb, cfg.lds_bytes, stream, cfg.L, ld, st, zf0, zf1, pair_off); break
-	switch (cfg.L.plan.n) {
-		BAM_FFT_N(64);
-		BAM_FFT_N(128);
-		BAM_FFT_N(256);
-		BAM_FFT_N(512);
-	default:
-		fail("pair transform: no kernel for n = %d", cfg.L.plan.n);
-	}
-#undef BAM_FFT_N
 
 	BAM_HIP(hipGetLastError());
 }

@@ -87,24 +87,6 @@ double rolloff_1d(int d, int i, float os, double beta, double width)
 	return 1. / ft / width;
 }
 
-// x-y product tables, computed on the device with the same cmul as the
-// per-element products they replace (bitwise equal)
-__global__ void k_xy_tables(SepTables T, float2* out)
-{
-	const long nxy = (long)T.n[0] * T.n[1];
-
-	for (long e = (long)blockIdx.x * blockDim.x + threadIdx.x; e < nxy; e += (long)gridDim.x * blockDim.x) {
-
-		const int x = (int)(e % T.n[0]);
-		const int y = (int)(e / T.n[0]);
-
-		for (int b = 0; b < 4; b++)
-			out[b * nxy + e] = cmul(T.lin[0][b & 1][x], T.lin[1][b >> 1][y]);
-
-		out[4 * nxy + e] = cmul(T.fm[0][x], T.fm[1][y]);
-	}
-}
-
 static void build_tables(Nufft& p)
 {
 	long tot = 0;
@@ -169,24 +151,6 @@ static void build_tables(Nufft& p)
 		p.tabs.lin[d][1] = p.tab2.ptr + o2[d] + p.n[d];
 		p.tabs.fm[d] = p.tab2.ptr + o2[d] + 2 * p.n[d];
 		p.tabs.roll[d] = p.tabr.ptr + orr[d];
-	}
-
-	for (int b = 0; b < 4; b++)
-		p.tabs.linxy[b] = nullptr;
-	p.tabs.fmxy = nullptr;
-
-	if (p.n[0] > 1 && p.n[1] > 1 && p.n[2] > 1) {
-
-		const long nxy = (long)p.n[0] * p.n[1];
-		p.tabxy.alloc(5 * nxy);
-		hipLaunchKernelGGL(k_xy_tables, dim3((unsigned)std::min<long>((nxy + 255) / 256, 4096)), dim3(256), 0,
-				   p.stream, p.tabs, p.tabxy.ptr);
-		BAM_HIP(hipGetLastError());
-		BAM_HIP(hipStreamSynchronize(p.stream));
-
-		for (int b = 0; b < 4; b++)
-			p.tabs.linxy[b] = p.tabxy.ptr + b * nxy;
-		p.tabs.fmxy = p.tabxy.ptr + 4 * nxy;
 	}
 }
 
@@ -271,519 +235,14 @@ struct StGrid {
 	__device__ void at(const ColBase& b, int p, int k, float2 x) const
 	{
 		if (fm) {
-			if (2 == g.axis && nullptr != T.fmxy) {
-				// fm_val = ((fm0 fm1) fm2), the x-y product from its table
-				x = cmul(x, cmul(T.fmxy[b.i0 + p], T.fm[2][k]));
-			} else {
-				int px[3];
-				g.coords(b.i0 + p, b.o, k, px);
-				x = cmul(x, fm_val(T, px));
-			}
+			int px[3];
+			g.coords(b.i0 + p, b.o, k, px);
+			x = cmul(x, fm_val(T, px));
 		}
 
 		grid[b.off + p + (long)g.inner * k] = x;
 	}
 };
-
-// PSF multiply between forward and inverse transform (standard order,
-// volumes v = c + C s)
-struct MdPsf {
-	static constexpr bool active = true;
-	static constexpr bool colblock = true;
-	VolAxis g;
-	int C;
-	const float2* psf;
-
-	__device__ float2 operator()(long t, int k, float2 x) const
-	{
-		uint32_t i, o, v;
-		g.split(t, i, o, v);
-		uint32_t s = v / (uint32_t)C;
-		long off = g.offset_iov(i, o, 0, k);
-		return cmul(x, psf[(long)s * g.N + off]);
-	}
-
-	__device__ bool cb_ok(int P) const { return 0 == g.inner % (uint32_t)P; }
-
-	// base: the PSF offset of element (0, 0) (sub-grid v / C)
-	__device__ ColBase base(long t0) const
-	{
-		ColBase b = col_base(g, t0);
-		b.off = (long)(b.v / (uint32_t)C) * g.N + g.offset_iov(b.i0, b.o, 0, 0);
-		return b;
-	}
-
-	__device__ float2 at(const ColBase& b, int p, int k, float2 x) const
-	{
-		return cmul(x, psf[b.off + p + (long)g.inner * k]);
-	}
-};
-
-// Toeplitz z-pass over pairs of sub-grids s, s + S/2 (the same x-y
-// transform H, z factors lz_0 and lz_1): the stack holds the volumes
-// v = c + C s, s < S/2, the PSF all S sub-grids
-struct MdPsfPair {
-	VolAxis g;
-	int C;
-	long half;  // PSF offset of sub-grid s + S/2 from sub-grid s: (S/2) N
-	const float2* psf;
-	const float2* lz0;
-	const float2* lz1;
-
-	__device__ bool cb_ok(int P) const { return 0 == g.inner % (uint32_t)P; }
-
-	__device__ ColBase base(long t0) const
-	{
-		ColBase b = col_base(g, t0);
-		b.off = (long)(b.v / (uint32_t)C) * g.N + g.offset_iov(b.i0, b.o, 0, 0);
-		return b;
-	}
-
-	__device__ float2 at(const ColBase& b, int m, int p, int k, float2 x) const
-	{
-		return cmul(x, psf[b.off + m * half + p + (long)g.inner * k]);
-	}
-
-	__device__ float2 zf(int m, int k) const { return (0 == m) ? lz0[k] : lz1[k]; }
-};
-
-// ---------------------------------------------------------------------------
-// Slice kernels for 3-D grids whose x-y slice fits in LDS (NX x NY <= 128 x
-// 128): one work-group transforms whole slices along x and y, so that the
-// sub-grid stack makes one round trip through HBM for both in-plane axes.
-// LDS holds the slice row-major with a row pitch of NX + 1 (bank spread of
-// the column transforms) and the two twiddle tables.
-//
-// Sub-grids s and s + S/2 differ only in the z shift (the z decomposition
-// bit is the top bit of s), and the z factor of linphase, lz_s(z), is one
-// scalar per slice.  The x-y transform is linear, so
-//   FFT_xy(v linxy_s lz_s(z)) = lz_s(z) FFT_xy(v linxy_s)
-// and one transform serves both sub-grids of a pair; likewise the inverse
-// transforms the combination conj(lz_s) g_s + conj(lz_s') g_s' once.
-//
-// k_slice_fwd: work-group (z, c).  The image-side values of slice z (coil
-// image c, or image x map c; x rolloff when roll) are read once into
-// registers; for every pair (s, s + S/2) they are multiplied by the x-y
-// factor linxy_s, transformed along x and y, and stored to grid[s][c][z]
-// times lz_s(z) and to grid[s + S/2][c][z] times lz_{s+S/2}(z).
-//
-// k_slice_inv: work-group (z, c).  For every pair, conj(lz_s) grid[s][c][z]
-// + conj(lz_{s+S/2}) grid[s + S/2][c][z] is inverse-transformed along y and
-// x, and conj(linxy_s) x value is summed over the pairs in order; the sum is
-// scaled by the rolloff (when roll) and, with maps, multiplied by
-// conj(map_c) into partial image c (the coils are summed in order by
-// sum_groups), else stored as coil image c.  No atomics.
-// ---------------------------------------------------------------------------
-
-// threads of a slice work-group: a multiple of NX (every lane keeps its x)
-template <int NX>
-constexpr int slice_threads()
-{
-	return (1024 / NX) * NX;
-}
-
-template <int NX, int NY>
-constexpr int slice_threads_inv()
-{
-	return slice_threads<NX>();
-}
-
-struct SliceGeom {
-	int nz, S, C;
-	long N;
-};
-
-// the first pass along y runs in registers when a lane's points y0 + i DY
-// (i < EPT) are exactly the inputs of one radix-EPT butterfly
-template <int NX, int NY>
-constexpr bool slice_regpass()
-{
-	constexpr int DY = slice_threads<NX>() / NX;
-	constexpr int EPT = NY / DY;
-	return 0 == NY % DY && (2 == EPT || 4 == EPT || 8 == EPT || 16 == EPT);
-}
-
-template <int NX, int NY>
-constexpr size_t slice_lds_bytes()
-{
-	return sizeof(float2) * ((size_t)NY * (NX + 1) + NX + NY);
-}
-
-// separable factors of one lane: x and z fixed, y = y0 + i dy
-struct SliceLane {
-	int x, y0, dy;
-};
-
-// x-y factor of sub-grid s's linphase, lin_x lin_y, from its table
-__device__ inline float2 lin_xy(const SepTables& T, int s, int x, int y)
-{
-	const int bx = (s >> T.bitpos[0]) & 1, by = (s >> T.bitpos[1]) & 1;
-	return T.linxy[bx + 2 * by][x + T.n[0] * y];
-}
-
-__device__ inline float roll_xyz(const SepTables& T, int x, int y, int z)
-{
-	return T.roll[0][x] * T.roll[1][y] * T.roll[2][z];
-}
-
-template <int NX, int NY>
-__global__ __launch_bounds__(slice_threads<NX>()) void k_slice_fwd(SliceGeom sg, SepTables T,
-								    const float2* __restrict__ src,
-								    const float2* __restrict__ sens, bool roll,
-								    float2* __restrict__ grid,
-								    const float2* __restrict__ twx_g,
-								    const float2* __restrict__ twy_g, const int* skip,
-								    bool zpair)
-{
-	constexpr int NTH = slice_threads<NX>();
-	constexpr int DY = NTH / NX;
-	constexpr int EPT = (NY + DY - 1) / DY;
-	constexpr int NP = NX * NY;
-	constexpr int LD = NX + 1;
-
-	extern __shared__ float2 lds[];
-	float2* twx = lds + NY * LD;
-	float2* twy = twx + NX;
-
-	if (nullptr != skip && 0 != *skip)
-		return;
-
-	const int z = blockIdx.x;
-	const int c = blockIdx.y;
-	const int x = threadIdx.x % NX;
-	const int y0 = threadIdx.x / NX;
-
-	for (int i = threadIdx.x; i < NX; i += NTH)
-		twx[i] = twx_g[i];
-
-	for (int i = threadIdx.x; i < NY; i += NTH)
-		twy[i] = twy_g[i];
-
-	const long zoff = (long)z * NP;
-	const float2* img = (nullptr != sens) ? src + zoff : src + (long)c * sg.N + zoff;
-	const float2* map = (nullptr != sens) ? sens + (long)c * sg.N + zoff : nullptr;
-
-	// image-side values of this lane's points, held across the sub-grids
-	float2 vin[EPT];
-
-#pragma unroll
-	for (int i = 0; i < EPT; i++) {
-
-		const int y = y0 + i * DY;
-		vin[i] = make_float2(0.f, 0.f);
-
-		if (0 == NY % DY || y < NY) {
-
-			const int e = y * NX + x;
-			float2 v = (nullptr != map) ? cmul(img[e], map[e]) : img[e];
-
-			if (roll)
-				v = cscale(v, roll_xyz(T, x, y, z));
-
-			vin[i] = v;
-		}
-	}
-
-	// z factors of the two sub-grids of a pair; sub-grid s + SH is s shifted in z
-	const float2 lz0 = T.lin[2][0][z], lz1 = T.lin[2][1][z];
-	const int SH = sg.S / 2;
-	const long pair_off = (long)sg.C * SH * sg.N;
-
-	for (int s = 0; s < SH; s++) {
-
-		// per-iteration copies of the lane coordinates (keeps the element
-		// addresses out of registers across the loop)
-		int xs = x, ys = y0;
-		asm volatile("" : "+v"(xs), "+v"(ys));
-
-		if constexpr (slice_regpass<NX, NY>()) {
-
-			// the lane's points y0 + i DY are the inputs of one butterfly of
-			// the first radix-EPT pass along y: that pass runs in registers,
-			// then the rest of y and the x passes in LDS
-			float2 v[EPT];
-
-#pragma unroll
-			for (int i = 0; i < EPT; i++)
-				v[i] = cmul(vin[i], lin_xy(T, s, xs, ys + i * DY));
-
-			dft_any<EPT>(v, -1.f, twy, NY);
-
-			lds_barrier();
-
-#pragma unroll
-			for (int q = 0; q < EPT; q++)
-				lds[(ys * EPT + q) * LD + xs] = v[q];
-
-			lds_barrier();
-
-			slice_passes_rest<NY, NY / EPT, EPT, NX, LD, 1, NTH>(lds, twy, -1.f);
-
-			// x passes; the last one stores its outputs straight to the grid
-			// (16 lanes per row: 128-byte runs)
-			constexpr int RLX = slice_last_radix(NX);
-			slice_passes_range<NX, 1, NX / RLX, NY, 1, LD, NTH>(lds, twx, -1.f);
-			float2* out = grid + ((long)c + (long)sg.C * s) * sg.N + zoff;
-			slice_last_pass_rows<NX, RLX, NY, LD, NTH>(lds, twx, -1.f, [&](int, int, int p, int xo, float2 v) {
-				if (zpair) {
-					out[p * NX + xo] = v;
-				} else {
-					out[p * NX + xo] = cmul(v, lz0);
-					out[pair_off + p * NX + xo] = cmul(v, lz1);
-				}
-			});
-			continue;
-
-		} else {
-
-			lds_barrier();
-
-#pragma unroll
-			for (int i = 0; i < EPT; i++) {
-
-				const int y = ys + i * DY;
-
-				if (0 == NY % DY || y < NY)
-					lds[y * LD + xs] = cmul(vin[i], lin_xy(T, s, xs, y));
-			}
-
-			lds_barrier();
-
-			slice_passes<NX, NY, 1, LD, NTH>(lds, twx, -1.f);
-			slice_passes<NY, NX, LD, 1, NTH>(lds, twy, -1.f);
-		}
-
-		float2* out = grid + ((long)c + (long)sg.C * s) * sg.N + zoff;
-
-		xs = x;
-		ys = y0;
-		asm volatile("" : "+v"(xs), "+v"(ys));
-
-#pragma unroll 4
-		for (int i = 0; i < EPT; i++) {
-
-			const int y = ys + i * DY;
-
-			if (0 == NY % DY || y < NY) {
-				const float2 l = lds[y * LD + xs];
-				if (zpair) {
-					out[y * NX + xs] = l;
-				} else {
-					out[y * NX + xs] = cmul(l, lz0);
-					out[pair_off + y * NX + xs] = cmul(l, lz1);
-				}
-			}
-		}
-	}
-}
-
-template <int NX, int NY>
-__global__ __launch_bounds__((slice_threads_inv<NX, NY>())) void k_slice_inv(SliceGeom sg, SepTables T,
-								    const float2* __restrict__ grid,
-								    const float2* __restrict__ sens, bool roll,
-								    float2* __restrict__ dst,
-								    const float2* __restrict__ twx_g,
-								    const float2* __restrict__ twy_g, const int* skip,
-								    bool zpair)
-{
-	constexpr int NTH = slice_threads_inv<NX, NY>();
-	constexpr int DY = NTH / NX;
-	constexpr int EPT = (NY + DY - 1) / DY;
-	constexpr int NP = NX * NY;
-	constexpr int LD = NX + 1;
-
-	extern __shared__ float2 lds[];
-	float2* twx = lds + NY * LD;
-	float2* twy = twx + NX;
-
-	if (nullptr != skip && 0 != *skip)
-		return;
-
-	const int z = blockIdx.x;
-	const int c = blockIdx.y;
-	const long zoff = (long)z * NP;
-	const int x = threadIdx.x % NX;
-	const int y0 = threadIdx.x / NX;
-
-	for (int i = threadIdx.x; i < NX; i += NTH)
-		twx[i] = twx_g[i];
-
-	for (int i = threadIdx.x; i < NY; i += NTH)
-		twy[i] = twy_g[i];
-
-	float2 acc[EPT];
-
-#pragma unroll
-	for (int i = 0; i < EPT; i++)
-		acc[i] = make_float2(0.f, 0.f);
-
-	// z factors of the two sub-grids of a pair; sub-grid s + SH is s shifted in z
-	const float2 lz0 = T.lin[2][0][z], lz1 = T.lin[2][1][z];
-	const int SH = sg.S / 2;
-	const long pair_off = (long)sg.C * SH * sg.N;
-
-	for (int s = 0; s < SH; s++) {
-
-		const float2* in = grid + ((long)c + (long)sg.C * s) * sg.N + zoff;
-
-		// per-iteration copies of the lane coordinates (keeps the element
-		// addresses out of registers across the loop)
-		int xs = x, ys = y0;
-		asm volatile("" : "+v"(xs), "+v"(ys));
-
-		if constexpr (slice_regpass<NX, NY>()) {
-
-			// first radix-EPT pass along y in registers (see k_slice_fwd)
-			float2 v[EPT];
-
-#pragma unroll
-			for (int i = 0; i < EPT; i++) {
-				const int e = (ys + i * DY) * NX + xs;
-				v[i] = zpair ? in[e] : cadd(cmulc(in[e], lz0), cmulc(in[pair_off + e], lz1));
-			}
-
-			dft_any<EPT>(v, +1.f, twy, NY);
-
-			lds_barrier();
-
-#pragma unroll
-			for (int q = 0; q < EPT; q++)
-				lds[(ys * EPT + q) * LD + xs] = v[q];
-
-			lds_barrier();
-
-			slice_passes_rest<NY, NY / EPT, EPT, NX, LD, 1, NTH>(lds, twy, +1.f);
-
-		} else {
-
-			lds_barrier();
-
-#pragma unroll 4
-			for (int i = 0; i < EPT; i++) {
-
-				const int y = ys + i * DY;
-
-				if (0 == NY % DY || y < NY)
-					lds[y * LD + xs] = zpair ? in[y * NX + xs]
-								 : cadd(cmulc(in[y * NX + xs], lz0),
-									cmulc(in[pair_off + y * NX + xs], lz1));
-			}
-
-			lds_barrier();
-
-			slice_passes<NY, NX, LD, 1, NTH>(lds, twy, +1.f);
-		}
-
-		slice_passes<NX, NY, 1, LD, NTH>(lds, twx, +1.f);
-
-		// sum over the pairs of conj(linxy_s) x value
-		xs = x;
-		ys = y0;
-		asm volatile("" : "+v"(xs), "+v"(ys));
-
-#pragma unroll
-		for (int i = 0; i < EPT; i++) {
-
-			const int y = ys + i * DY;
-
-			if (0 == NY % DY || y < NY)
-				acc[i] = cadd(acc[i], cmulc(lds[y * LD + xs], lin_xy(T, s, xs, y)));
-		}
-	}
-
-	// rolloff, then conj(map_c) into partial image c, or coil image c
-	const float2* map = (nullptr != sens) ? sens + (long)c * sg.N + zoff : nullptr;
-	int xs = x, ys = y0;
-	asm volatile("" : "+v"(xs), "+v"(ys));
-
-#pragma unroll
-	for (int i = 0; i < EPT; i++) {
-
-		const int y = ys + i * DY;
-
-		if (0 == NY % DY || y < NY) {
-
-			float2 v = roll ? cscale(acc[i], roll_xyz(T, xs, y, z)) : acc[i];
-
-			if (nullptr != map)
-				v = cmulc(v, map[y * NX + xs]);
-
-			dst[(long)c * sg.N + zoff + y * NX + xs] = v;
-		}
-	}
-}
-
-// slice sizes with a kernel (square slices)
-static bool slice_supported(const int n[3])
-{
-	if (n[0] != n[1] || n[2] < 2)
-		return false;
-
-	switch (n[0]) {
-	case 32: case 64: case 96: case 128:
-		return true;
-	default:
-		return false;
-	}
-}
-
-// the slice kernels pair sub-grid s with s + S/2: the z decomposition bit
-// must be the top bit of s
-static void check_slice_pairs(const Nufft& p)
-{
-	if (8 != p.S || 0 != p.tabs.bitpos[0] || 1 != p.tabs.bitpos[1] || 2 != p.tabs.bitpos[2])
-		fail("slice FFT: needs the 3-D decomposition into 8 sub-grids (S = %d)", p.S);
-}
-
-// zpair: store only the x-y transform H of each pair (volumes s < S/2),
-// without the z factors, for the pair z-pass of the Toeplitz operator
-static void launch_slice_fwd(const Nufft& p, const float2* src, const float2* sens, bool roll, const int* skip,
-			     const char* name, bool zpair = false)
-{
-	ProfScope prof(name, p.stream);
-	SliceGeom sg{ p.n[2], p.S, p.C, p.N };
-	dim3 blocks(p.n[2], p.C);
-	check_slice_pairs(p);
-
-#define BAM_SLICE(NN)                                                                                           	case NN:                                                                                                		hipLaunchKernelGGL((k_slice_fwd<NN, NN>), blocks, dim3(slice_threads<NN>()), (slice_lds_bytes<NN, NN>()), 				   p.stream, sg, p.tabs, src, sens, roll, p.grid.ptr, p.axis[0].tw, p.axis[1].tw,   				   skip, zpair);                                                                       		break
-
-	switch (p.n[0]) {
-		BAM_SLICE(32);
-		BAM_SLICE(64);
-		BAM_SLICE(96);
-		BAM_SLICE(128);
-	default:
-		fail("slice FFT: unsupported size %d", p.n[0]);
-	}
-#undef BAM_SLICE
-
-	BAM_HIP(hipGetLastError());
-}
-
-// zpair: the volumes s < S/2 already hold conj(lz_s) g_s + conj(lz_s') g_s'
-// (pair z-pass output)
-static void launch_slice_inv(const Nufft& p, float2* dst, const float2* sens, bool roll, const int* skip,
-			     const char* name, bool zpair = false)
-{
-	ProfScope prof(name, p.stream);
-	SliceGeom sg{ p.n[2], p.S, p.C, p.N };
-	dim3 blocks(p.n[2], p.C);
-	check_slice_pairs(p);
-
-#define BAM_SLICE(NN)                                                                                           	case NN:                                                                                                		hipLaunchKernelGGL((k_slice_inv<NN, NN>), blocks, dim3(slice_threads_inv<NN, NN>()), (slice_lds_bytes<NN, NN>()), 				   p.stream, sg, p.tabs, p.grid.ptr, sens, roll, dst, p.axis[0].tw,                 				   p.axis[1].tw, skip, zpair);                                                         		break
-
-	switch (p.n[0]) {
-		BAM_SLICE(32);
-		BAM_SLICE(64);
-		BAM_SLICE(96);
-		BAM_SLICE(128);
-	default:
-		fail("slice FFT: unsupported size %d", p.n[0]);
-	}
-#undef BAM_SLICE
-
-	BAM_HIP(hipGetLastError());
-}
 
 // ---------------------------------------------------------------------------
 // Small element-wise kernels
@@ -857,15 +316,6 @@ void fill(float2* p, long n, float2 v, hipStream_t st, const int* skip)
 	BAM_HIP(hipGetLastError());
 }
 
-static FftLaunchCfg fft_config_skip(const int* skip, const AxisPlan& plan, long total, bool contig, int P_min,
-				   float sign1, float sign2)
-{
-	FftLaunchCfg c = fft_config(plan, total, contig, P_min, sign1, sign2);
-	c.L.skip = skip;
-	c.name = "fft_toeplitz";
-	return c;
-}
-
 // ---------------------------------------------------------------------------
 // Plan creation
 // ---------------------------------------------------------------------------
@@ -927,22 +377,11 @@ void Nufft::create_geometry(const int dims[3], int C_, bool toeplitz_, bool peri
 		pair[j] = make_pair_plan(axis[j]);
 	}
 
-	// BART_AMD_SLICE=off selects the per-axis passes also where the x-y
-	// slices fit in LDS
-	const char* sl = getenv("BART_AMD_SLICE");
-	slice = (3 == nact) && slice_supported(n) && !(nullptr != sl && 0 == strcmp(sl, "off"));
-
-	// BART_AMD_PAIRZ=off: Toeplitz z-pass over all S sub-grids instead of
-	// over the pairs that share an x-y transform
-	const char* pz = getenv("BART_AMD_PAIRZ");
-	pair_zpass = slice && fft_pair_len_ok(n[2]) && !(nullptr != pz && 0 == strcmp(pz, "off"));
-
 	grid.alloc((size_t)S * C * N);
 
 	// partial images of the coil groups of S^H (allocated here so that no
-	// allocation happens inside a captured CG iteration); one per coil with
-	// the slice kernels
-	const int G = slice ? C : C / merge_group(*this);
+	// allocation happens inside a captured CG iteration)
+	const int G = C / merge_group(*this);
 
 	if (G > 1)
 		part.alloc((size_t)G * N);
@@ -1144,12 +583,12 @@ __global__ void k_long_reduce(VolAxis g, SepTables T, float2* dst, const float2*
 static void long_fft(const Nufft& p, int j, float sign, bool fm, const int* skip, const char* name)
 {
 	VolAxis va = VolAxis::make(p.n, p.act[j], (long)p.C << (j + 1));
-	FftLaunchCfg cfg = fft_config(p.axis[j], va.transforms(), va.contig(), 1, sign, sign);
+	FftLaunchCfg cfg = fft_config(p.axis[j], va.transforms(), va.contig(), 1, sign);
 	cfg.L.skip = skip;
 	cfg.name = name;
 	LdGrid ld{ va, p.grid.ptr };
 	StGrid st{ va, p.tabs, p.grid.ptr, fm };
-	launch_fft_axis(cfg, p.stream, ld, NoMid{}, st);
+	launch_fft_axis(cfg, p.stream, ld, st);
 }
 
 // the image side's forms: src / dst non-null on axis 0 only
@@ -1225,70 +664,8 @@ static float2* merge_target(Nufft& p, float2* dst, const float2* sens, int& G)
 	return p.part.ptr;
 }
 
-// z axis of the sub-grid stack (slice path).  pair: the stack is read
-// (forward) or written (adjoint) as the S/2 pair volumes of the slice
-// kernels' zpair mode -- forward: volume s holds H, the x-y transform shared
-// by sub-grids s and s + S/2, and both are written; adjoint: sub-grids s and
-// s + S/2 are read and conj(lz_s) Z_s + conj(lz_{s+S/2}) Z_{s+S/2} is
-// written to volume s.  Returns whether the pair form was used.
-static bool z_pass(const Nufft& p, float sign, bool fm, const char* name)
-{
-	if (p.pair_zpass) {
-		VolAxis va = VolAxis::make(p.n, 2, (long)(p.S / 2) * p.C);
-		FftLaunchCfg cfg = fft_config(p.axis[2], va.transforms(), va.contig(), 1, sign, sign);
-
-		if (cfg.fixed) {
-			fft_config_pair(cfg);
-
-			if (!cfg.L.contig && 0 == va.inner % (uint32_t)cfg.L.P) {
-				cfg.name = name;
-				LdGrid ld{ va, p.grid.ptr };
-				StGrid st{ va, p.tabs, p.grid.ptr, fm };
-				const long pair_off = (long)(p.S / 2) * p.C * p.N;
-				if (sign < 0.f)
-					launch_fft_axis_pair_io<false>(cfg, p.stream, ld, st, p.tabs.lin[2][0], p.tabs.lin[2][1],
-								       pair_off);
-				else
-					launch_fft_axis_pair_io<true>(cfg, p.stream, ld, st, p.tabs.lin[2][0], p.tabs.lin[2][1],
-								      pair_off);
-				return true;
-			}
-		}
-	}
-
-	VolAxis va = VolAxis::make(p.n, 2, (long)p.S * p.C);
-	FftLaunchCfg cfg = fft_config(p.axis[2], va.transforms(), va.contig(), 1, sign, sign);
-	cfg.name = name;
-	LdGrid ld{ va, p.grid.ptr };
-	StGrid st{ va, p.tabs, p.grid.ptr, fm };
-	launch_fft_axis(cfg, p.stream, ld, NoMid{}, st);
-	return false;
-}
-
-// whether z_pass takes the pair form (same conditions)
-static bool z_pass_pairs(const Nufft& p)
-{
-	if (!p.pair_zpass)
-		return false;
-	VolAxis va = VolAxis::make(p.n, 2, (long)(p.S / 2) * p.C);
-	FftLaunchCfg cfg = fft_config(p.axis[2], va.transforms(), va.contig(), 1, -1.f, -1.f);
-	if (!cfg.fixed)
-		return false;
-	fft_config_pair(cfg);
-	return !cfg.L.contig && 0 == va.inner % (uint32_t)cfg.L.P;
-}
-
 void Nufft::forward(float2* ksp, const float2* src, const float2* sens)
 {
-	if (slice) {
-		const bool pz = z_pass_pairs(*this);
-		launch_slice_fwd(*this, src, sens, true, nullptr, "fft_fwd_slice", pz);
-		const bool used = z_pass(*this, -1.f, true, "fft_fwd_axis");
-		BAM_CHECK(used == pz, "z-pass form mismatch");
-		grid_forward(gp, kb.ptr, ksp, grid.ptr, has_weights ? weights.ptr : nullptr, stream);
-		return;
-	}
-
 	check_first_axis(*this);
 	axis_split(*this, 0, src, sens, true, 1 == nact, nullptr, "fft_fwd_first");
 
@@ -1302,22 +679,6 @@ void Nufft::adjoint(float2* dst, const float2* ksp, const float2* sens)
 {
 	// the output-stationary adjoint gridding writes every grid point
 	grid_adjoint(gp, kb.ptr, grid.ptr, ksp, has_weights ? weights.ptr : nullptr, stream);
-
-	if (slice) {
-
-		const bool pz = z_pass(*this, +1.f, false, "fft_adj_axis");
-
-		// with maps: one partial image per coil, summed in coil order
-		const int G = C;
-		float2* out = (nullptr != sens && G > 1) ? part.ptr : dst;
-
-		launch_slice_inv(*this, out, sens, true, nullptr, "fft_adj_slice", pz);
-
-		if (out != dst)
-			sum_groups(dst, part.ptr, N, G, stream, nullptr);
-
-		return;
-	}
 
 	check_first_axis(*this);
 
@@ -1351,50 +712,6 @@ bool Nufft::normal(float2* dst, const float2* src, const float2* sens, const int
 {
 	BAM_CHECK(has_psf, "Toeplitz normal operator without PSF");
 	BAM_CHECK(0 == nbasis, "normal: a plan with a subspace basis takes normal_basis");
-
-	if (slice) {
-
-		// sub-grids s and s + S/2 share the x-y transform H: the slice
-		// kernels store and read H once per pair, and the z-pass applies both
-		// members' z factors and PSFs to it (pair_z)
-		VolAxis va = VolAxis::make(n, 2, (long)(S / 2) * C);
-		FftLaunchCfg cfg = fft_config_skip(skip, axis[2], va.transforms(), va.contig(), 1, -1.f, +1.f);
-		if (cfg.fixed)
-			fft_config_pair(cfg);
-		const bool pair_z = pair_zpass && cfg.fixed && !cfg.L.contig && 0 == va.inner % (uint32_t)cfg.L.P;
-
-		if (!pair_z) {
-			va = VolAxis::make(n, 2, (long)S * C);
-			cfg = fft_config_skip(skip, axis[2], va.transforms(), va.contig(), 1, -1.f, +1.f);
-		}
-
-		launch_slice_fwd(*this, src, sens, false, skip, "fft_toeplitz_slice_fwd", pair_z);
-
-		// the C coil volumes of a sub-grid share its PSF: launch order
-		// column group -> volume, so that the PSF columns come from cache
-		va.group_volumes(cfg.L.P);
-		LdGrid ld{ va, grid.ptr };
-		StGrid st{ va, tabs, grid.ptr, false };
-
-		if (pair_z) {
-			MdPsfPair md{ va, C, (long)(S / 2) * N, psf.ptr, tabs.lin[2][0], tabs.lin[2][1] };
-			launch_fft_axis_pair(cfg, stream, ld, md, st);
-		} else {
-			MdPsf md{ va, C, psf.ptr };
-			launch_fft_axis(cfg, stream, ld, md, st);
-		}
-
-		// with maps: one partial image per coil, summed in coil order
-		const int G = C;
-		float2* out = (nullptr != sens && G > 1) ? part.ptr : dst;
-
-		launch_slice_inv(*this, out, sens, false, skip, "fft_toeplitz_slice_inv", pair_z);
-
-		if (out != dst)
-			return sum_groups_or_fuse(dst, part.ptr, N, G, stream, skip, fuse);
-
-		return false;
-	}
 
 	check_first_axis(*this);
 	int G;
@@ -1448,27 +765,6 @@ void Nufft::normal_basis(float2* dst, const float2* src, const int* skip)
 	BAM_CHECK(has_psf && nbasis > 0, "normal_basis: no subspace PSF");
 	BAM_CHECK(0 == C % nbasis, "normal_basis: channels %d not a multiple of %d coefficients", C, nbasis);
 	const int Cc = C / nbasis;
-
-	if (slice) {
-
-		VolAxis va = VolAxis::make(n, 2, (long)S * C);
-		launch_slice_fwd(*this, src, nullptr, false, skip, "fft_toeplitz_slice_fwd", false);
-
-		FftLaunchCfg cf = fft_config_skip(skip, axis[2], va.transforms(), va.contig(), 1, -1.f, -1.f);
-		cf.name = "fft_toeplitz_basis_fwd";
-		LdGrid ld{ va, grid.ptr };
-		StGrid st{ va, tabs, grid.ptr, false };
-		launch_fft_axis(cf, stream, ld, NoMid{}, st);
-
-		basis_psf_apply(grid.ptr, psf.ptr, S, Cc, nbasis, N, stream, skip);
-
-		FftLaunchCfg ci = fft_config_skip(skip, axis[2], va.transforms(), va.contig(), 1, +1.f, +1.f);
-		ci.name = "fft_toeplitz_basis_inv";
-		launch_fft_axis(ci, stream, ld, NoMid{}, st);
-
-		launch_slice_inv(*this, dst, nullptr, false, skip, "fft_toeplitz_slice_inv", false);
-		return;
-	}
 
 	check_first_axis(*this);
 	axis_split(*this, 0, src, nullptr, false, false, skip, "fft_toeplitz_basis_first");
@@ -1588,9 +884,9 @@ void Nufft::apply_precond(const float2* pre, float2* dst, const float2* src, int
 
 // The three passes of Nufft::normal's 2-D path (split of the first axis with
 // maps, turn of the second, merge of the first with the sums over coil
-// groups) for every plan, each pass one launch for the lengths of at most two
-// radices and one for the others: the same work-groups and arithmetic as the
-// plans' own launches, so the results are the same bits.
+// groups) for every plan, each pass one launch per kernel that its lengths
+// take: the same work-groups and arithmetic as the plans' own launches, so the
+// results are the same bits.
 struct NormalGroupSet {
 
 	struct Pass {
@@ -1601,12 +897,12 @@ struct NormalGroupSet {
 		DevBuf<int2> bt;
 	};
 
-	Pass pass[3][2];  // [pass][three radices]
+	Pass pass[3][PF_CLASSES];
 };
 
 bool normal_groupable(const Nufft& p, const float2* sens)
 {
-	if (2 != p.nact || p.slice || !p.toeplitz || !p.has_psf || nullptr == sens || p.nbasis > 0)
+	if (2 != p.nact || !p.toeplitz || !p.has_psf || nullptr == sens || p.nbasis > 0)
 		return false;
 
 	if (0 == p.pair[0].nr || 0 == p.pair[1].nr || (long)p.S * p.n[p.act[0]] > FFT_MAX_ELEMS)
@@ -1622,7 +918,7 @@ std::shared_ptr<NormalGroupSet> normal_groups_build(const std::vector<const Nuff
 						    const std::vector<const int*>& skip)
 {
 	auto set = std::make_shared<NormalGroupSet>();
-	std::vector<PairArgs> items[3][2];
+	std::vector<PairArgs> items[3][PF_CLASSES];
 
 	for (size_t q = 0; q < plans.size(); q++) {
 
@@ -1632,7 +928,7 @@ std::shared_ptr<NormalGroupSet> normal_groups_build(const std::vector<const Nuff
 					rows_merge_args(p, out, sens[q], false, skip[q]) };
 
 		for (int ph = 0; ph < 3; ph++) {
-			const int cl = (3 == a[ph].pl.nr) ? 1 : 0;
+			const int cl = a[ph].cl;
 			NormalGroupSet::Pass& P = set->pass[ph][cl];
 			P.threads = std::max(P.threads, pair_threads(a[ph], 1 != ph));
 			P.lds = std::max(P.lds, pair_lds_bytes(a[ph], 1 != ph));
@@ -1641,7 +937,7 @@ std::shared_ptr<NormalGroupSet> normal_groups_build(const std::vector<const Nuff
 	}
 
 	for (int ph = 0; ph < 3; ph++)
-		for (int cl = 0; cl < 2; cl++) {
+		for (int cl = 0; cl < PF_CLASSES; cl++) {
 
 			NormalGroupSet::Pass& P = set->pass[ph][cl];
 			const std::vector<PairArgs>& it = items[ph][cl];
@@ -1671,9 +967,9 @@ void normal_groups_launch(const NormalGroupSet& set, hipStream_t st)
 	static const int mode[3] = { PF_SPLIT, PF_TURN, PF_MERGE };
 
 	for (int ph = 0; ph < 3; ph++)
-		for (int cl = 0; cl < 2; cl++) {
+		for (int cl = 0; cl < PF_CLASSES; cl++) {
 			const NormalGroupSet::Pass& P = set.pass[ph][cl];
-			pair_launch_batch(mode[ph], 1 != ph, 1 == cl, P.items.ptr, P.bt.ptr, P.nb, P.threads, P.lds, name[ph],
+			pair_launch_batch(mode[ph], 1 != ph, cl, P.items.ptr, P.bt.ptr, P.nb, P.threads, P.lds, name[ph],
 					  st);
 		}
 }
@@ -1813,12 +1109,12 @@ void Nufft::compute_psf_from_traj(const float* traj, const float2* weights_host,
 
 		int a = p2.act[j];
 		VolAxis va = VolAxis::make(n2, a, J);
-		FftLaunchCfg cfg = fft_config(p2.axis[j], va.transforms(), va.contig(), 1, -1.f, -1.f);
+		FftLaunchCfg cfg = fft_config(p2.axis[j], va.transforms(), va.contig(), 1, -1.f);
 		cfg.name = "fft_psf";
 		LdFm2 ld{ va, p2.tabs, psft.ptr, 0 == j };
 		StDecomp st{ va, p2.tabs, (a == last) ? psf.ptr : psft.ptr, a == last, false, scale,
 			     { n[0], n[1], n[2] }, N, (long)S * N };
-		launch_fft_axis(cfg, stream, ld, NoMid{}, st);
+		launch_fft_axis(cfg, stream, ld, st);
 	}
 
 	apply_real_psf();

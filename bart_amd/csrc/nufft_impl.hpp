@@ -168,11 +168,6 @@ struct SepTables {
 	const float* roll[3];
 	int bitpos[3];  // decomposition bit of each dim, -1 if the dim is trivial
 	int n[3];
-
-	// x-y products for 3-D grids (null otherwise), each [n1][n0]:
-	// linxy[bx + 2 by] = lin[0][bx] x lin[1][by], fmxy = fm[0] x fm[1]
-	const float2* linxy[4];
-	const float2* fmxy;
 };
 
 struct CgApFuse;
@@ -195,7 +190,6 @@ struct Nufft {
 	DevBuf<float> kb;
 	DevBuf<float2> tab2;   // separable complex tables
 	DevBuf<float> tabr;    // separable rolloff
-	DevBuf<float2> tabxy;  // x-y product tables (3-D)
 	SepTables tabs;
 	DevBuf<float2> weights;
 	bool has_weights = false;
@@ -208,8 +202,6 @@ struct Nufft {
 	DevBuf<float2> part;   // per-coil-group partial images [G][N]
 	AxisPlan axis[3];
 	PairPlan pair[3];      // of the active axes (nr = 0: no pair kernel)
-	bool slice = false;    // 3-D with x-y slices transformed in LDS
-	bool pair_zpass = false;  // Toeplitz z-pass over sub-grid pairs (slice path)
 
 	hipStream_t stream = 0;
 

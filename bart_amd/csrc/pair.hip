@@ -81,7 +81,24 @@ void pair_geometry(PairArgs& a, bool rows, uint32_t units)
 	const uint32_t count = rows ? a.va.outer : a.va.inner;
 	int P = 1;
 
-	if (rows) {
+	a.cl = pf_class(n, a.pl.nr);
+
+	if (a.cl >= PF_32) {
+		const int RB = pf_fixed_lanes(a.cl);
+		P = PF_FP;
+		a.group = P * RB;
+
+		if (rows) {
+			// both members of a row in one wave; four waves per work-group,
+			// one where that would leave compute units without a work-group
+			// (CG of 256^2, 8 coils, 30 iterations: 1.611 ms at four, 1.640
+			// at one)
+			const int rw = 32 / RB;
+			const int waves = ((long)units * count / (4 * rw) >= 256) ? 4 : 1;
+			P = rw * waves;
+			a.group = 32 * waves;
+		}
+	} else if (rows) {
 		// whole waves, twice as many once there are enough work-groups
 		while (P * a.pl.NJ < 64 && 2 * P * a.pl.NJ <= lim)
 			P *= 2;
@@ -98,9 +115,10 @@ void pair_geometry(PairArgs& a, bool rows, uint32_t units)
 	a.logP = 0;
 	while ((1 << a.logP) < P)
 		a.logP++;
-	a.group = (P * a.pl.NJ + 63) / 64 * 64;
-	a.pitch = n + n / 8 + 1;
-	a.pitch |= 1;
+	if (a.cl < PF_32)
+		a.group = (P * a.pl.NJ + 63) / 64 * 64;
+
+	a.pitch = pf_row_pitch(n);
 	a.ncg = (count + P - 1) / P;
 	a.f_ncg = FastDiv(a.ncg);
 	a.f_outer = FastDiv(a.va.outer);
@@ -111,16 +129,38 @@ void pair_geometry(PairArgs& a, bool rows, uint32_t units)
 	a.nblk = (uint32_t)nblk;
 }
 
+#define BAM_PF_CLASSES(cl, F)    \
+	switch (cl) {            \
+	case PF_32:              \
+		F(8, 4);         \
+		break;           \
+	case PF_64:              \
+		F(8, 8);         \
+		break;           \
+	case PF_128:             \
+		F(16, 8);        \
+		break;           \
+	case PF_256:             \
+		F(16, 16);       \
+		break;           \
+	default:                 \
+		break;           \
+	}
+
 template <int MODE, bool ROWS>
 static void launch_m(const PairArgs& a, hipStream_t st)
 {
 	const dim3 gb(a.nblk), tb(pair_threads(a, ROWS));
 	const size_t lds = pair_lds_bytes(a, ROWS);
 
-	if (3 == a.pl.nr)
+#define BAM_PF_FIXED(RA, RB) hipLaunchKernelGGL((k_pair_fixed<MODE, ROWS, RA, RB>), gb, tb, lds, st, a)
+	if (a.cl >= PF_32)
+		BAM_PF_CLASSES(a.cl, BAM_PF_FIXED)
+	else if (PF_THREE == a.cl)
 		hipLaunchKernelGGL((k_pair<MODE, ROWS, true>), gb, tb, lds, st, a);
 	else
 		hipLaunchKernelGGL((k_pair<MODE, ROWS, false>), gb, tb, lds, st, a);
+#undef BAM_PF_FIXED
 }
 
 void pair_launch(int mode, bool rows, const PairArgs& a, const char* name, hipStream_t st)
@@ -150,7 +190,21 @@ void pair_launch(int mode, bool rows, const PairArgs& a, const char* name, hipSt
 	BAM_HIP(hipGetLastError());
 }
 
-void pair_launch_batch(int mode, bool rows, bool three, const PairArgs* items, const int2* btab, int nblk,
+template <int MODE, bool ROWS>
+static void launch_b(int cl, const PairArgs* items, const int2* btab, dim3 gb, dim3 tb, size_t lds, hipStream_t st)
+{
+#define BAM_PF_FIXED(RA, RB) \
+	hipLaunchKernelGGL((k_pair_fixed_batch<MODE, ROWS, RA, RB>), gb, tb, lds, st, items, btab)
+	if (cl >= PF_32)
+		BAM_PF_CLASSES(cl, BAM_PF_FIXED)
+	else if (PF_THREE == cl)
+		hipLaunchKernelGGL((k_pair_batch<MODE, ROWS, true>), gb, tb, lds, st, items, btab);
+	else
+		hipLaunchKernelGGL((k_pair_batch<MODE, ROWS, false>), gb, tb, lds, st, items, btab);
+#undef BAM_PF_FIXED
+}
+
+void pair_launch_batch(int mode, bool rows, int cl, const PairArgs* items, const int2* btab, int nblk,
 		       unsigned threads, size_t lds, const char* name, hipStream_t st)
 {
 	if (nblk <= 0)
@@ -159,21 +213,12 @@ void pair_launch_batch(int mode, bool rows, bool three, const PairArgs* items, c
 	ProfScope prof(name, st);
 	const dim3 gb((unsigned)nblk), tb(threads);
 
-#define BAM_PB(M, ROWS)                                                                                 \
-	do {                                                                                            \
-		if (three)                                                                              \
-			hipLaunchKernelGGL((k_pair_batch<M, ROWS, true>), gb, tb, lds, st, items, btab);  \
-		else                                                                                    \
-			hipLaunchKernelGGL((k_pair_batch<M, ROWS, false>), gb, tb, lds, st, items, btab); \
-	} while (0)
-
 	if (rows && PF_SPLIT == mode)
-		BAM_PB(PF_SPLIT, true);
+		launch_b<PF_SPLIT, true>(cl, items, btab, gb, tb, lds, st);
 	else if (rows)
-		BAM_PB(PF_MERGE, true);
+		launch_b<PF_MERGE, true>(cl, items, btab, gb, tb, lds, st);
 	else
-		BAM_PB(PF_TURN, false);
-#undef BAM_PB
+		launch_b<PF_TURN, false>(cl, items, btab, gb, tb, lds, st);
 
 	BAM_HIP(hipGetLastError());
 }

@@ -64,6 +64,7 @@ struct PairArgs {
 	const float2* l[2];      // linear phase of the axis per bit
 	float2* grid;
 	long half;               // from a volume to its second member
+	int cl;                  // kernel
 	int P, logP, pitch;      // transforms per work-group; rows: LDS pitch
 	int group;               // rows: threads per member (whole waves), twice as many in all
 	int C;
@@ -83,6 +84,23 @@ struct PairArgs {
 	const float2* psf;
 	long psf_half;
 };
+
+// kernel of a length: general with two radices, with three, or with the radices
+// in the code
+enum { PF_TWO = 0, PF_THREE, PF_32, PF_64, PF_128, PF_256, PF_CLASSES };
+
+constexpr int pf_class(int n, int nr)
+{
+	return (32 == n) ? PF_32 : (64 == n) ? PF_64 : (128 == n) ? PF_128 : (256 == n) ? PF_256 : (3 == nr) ? PF_THREE : PF_TWO;
+}
+
+constexpr int PF_FP = 16;  // columns per work-group of the latter: 128-byte rows
+
+// the last of their two radices: the lanes of a transform
+constexpr int pf_fixed_lanes(int cl) { return (PF_256 == cl) ? 16 : (PF_32 == cl) ? 4 : 8; }
+
+// LDS pitch of a row
+constexpr int pf_row_pitch(int n) { return (n + n / 8 + 1) | 1; }
 
 size_t pair_lds_bytes(const PairArgs& a, bool rows);
 unsigned pair_threads(const PairArgs& a, bool rows);
@@ -384,6 +402,23 @@ enum { PF_SPLIT = 0, PF_MERGE = 1, PF_TURN = 2 };
 // Strided axis: P adjacent columns of a volume per work-group, in place
 // ---------------------------------------------------------------------------
 
+// work-group -> column group, outer index, volume.  Turn: the volumes of a
+// column group one after the other (coils share its PSF columns); otherwise
+// neighbouring column groups
+__device__ __forceinline__ void pf_column(int mode, const PairArgs& a, uint32_t w, uint32_t& cg, uint32_t& o,
+					  uint32_t& v)
+{
+	uint32_t r;
+
+	if (PF_TURN == mode) {
+		a.f_nvol.divmod(w, r, v);
+		a.f_ncg.divmod(r, o, cg);
+	} else {
+		a.f_ncg.divmod(w, r, cg);
+		a.f_outer.divmod(r, v, o);
+	}
+}
+
 template <int MODE, bool MID>
 __device__ __forceinline__ void pair_cols_block(const PairArgs& a, uint32_t w, float2* lds)
 {
@@ -392,19 +427,8 @@ __device__ __forceinline__ void pair_cols_block(const PairArgs& a, uint32_t w, f
 	float2* tw = lds + size;
 	float2* lin = tw + n;
 
-	// turn: the volumes of a column group one after the other (coils share
-	// its PSF columns); otherwise neighbouring column groups
 	uint32_t cg, o, v;
-
-	if (PF_TURN == MODE) {
-		uint32_t r;
-		a.f_nvol.divmod(w, r, v);
-		a.f_ncg.divmod(r, o, cg);
-	} else {
-		uint32_t r;
-		a.f_ncg.divmod(w, r, cg);
-		a.f_outer.divmod(r, v, o);
-	}
+	pf_column(MODE, a, w, cg, o, v);
 
 	const uint32_t inner = a.va.inner;
 	const int p = threadIdx.x & (a.P - 1);
@@ -645,11 +669,230 @@ __device__ __forceinline__ void pair_cols_block(const PairArgs& a, uint32_t w, f
 }
 
 // ---------------------------------------------------------------------------
+// Strided axis of a length n = RA RB with RB | RA (32, 64, 128, 256): RB lanes
+// hold a column, RA points j + r RB each.  These are the inputs of one radix-RA
+// butterfly of the first pass and, for the RA / RB radix-RB butterflies of the
+// last pass, its outputs: every lane works in both passes, the points of a
+// forward transform are those that the backward one starts from, and nothing
+// but the exchange between the two passes goes through LDS.  With the radix in
+// the code: the general kernel above switches on it around every pass, and n =
+// 128 = 8 x 16 leaves half of its lanes idle in one of the two.
+// Split and merge are bound by HBM (128^3, 16 coils, between 2 and 4 volumes
+// per coil: 1.6 GB in 290 us), the turn by its vector instructions (4
+// transforms per point: 999 us in the general kernel, 914 with the passes of
+// the strided FFT, 665 here); 256^2, 8 coils: 16 -> 13.6 us.  One Toeplitz
+// operator on coil images, against whole x-y slices in LDS (the z axis after
+// them) for 128^3, 16 coils: 1842 -> 1665 us; 64^3: 232 -> 172; 32^3: 73 -> 68.
+// ---------------------------------------------------------------------------
+
+template <int MODE, int RA, int RB>
+__device__ __forceinline__ void pair_cols_fixed(const PairArgs& a, uint32_t w, float2* lds)
+{
+	constexpr int N = RA * RB, K = RA / RB;
+	static_assert(0 == RA % RB, "the last pass takes whole lanes");
+	float2* tw = lds + PF_FP * N;
+	float2* lin = tw + N;
+
+	uint32_t cg, o, v;
+	pf_column(MODE, a, w, cg, o, v);
+
+	const uint32_t inner = a.va.inner;
+	const int p = threadIdx.x & (PF_FP - 1);
+	const int j = threadIdx.x / PF_FP;
+	const uint32_t i = cg * PF_FP + p;
+	const bool in = i < inner;
+	float2* ls = lds + p;
+	const long vol0 = (long)inner * N * o + i + (long)inner * j;  // the lane's first point
+	float2* col = a.grid + (long)v * a.va.N + vol0;
+	const long step = (long)inner * RB;
+
+	auto load = [&](float2 (&x)[RA], const float2* q) BAM_INLINE {
+#pragma unroll
+		for (int r = 0; r < RA; r++)
+			x[r] = in ? q[r * step] : make_float2(0.f, 0.f);
+	};
+
+	auto put = [&](const float2 (&x)[RA]) BAM_INLINE {
+#pragma unroll
+		for (int q = 0; q < RA; q++)
+			ls[(j * RA + q) * PF_FP] = x[q];
+	};
+
+	// butterfly m of the last pass: f(r, point j + r RB)
+	auto last = [&](auto sg, auto&& f) BAM_INLINE {
+		constexpr int SG = decltype(sg)::value;
+#pragma unroll
+		for (int m = 0; m < K; m++) {
+			const int jb = j + m * RB;
+			float2 y[RB];
+#pragma unroll
+			for (int r = 0; r < RB; r++) {
+				y[r] = ls[(jb + r * RA) * PF_FP];
+				if (r > 0)
+					y[r] = (SG > 0) ? cmulc(y[r], tw[r * jb]) : cmul(y[r], tw[r * jb]);
+			}
+			PfDft<RB, SG>::run(y);
+#pragma unroll
+			for (int q = 0; q < RB; q++)
+				f(m + K * q, y[q]);
+		}
+	};
+
+	using Fwd = std::integral_constant<int, -1>;
+	using Bwd = std::integral_constant<int, 1>;
+
+	if constexpr (PF_SPLIT == MODE) {
+
+		float2 h[RA];
+		load(h, col);
+		pf_tables(a, tw, lin, nullptr);
+
+		// fftmod of the other axes of this column
+		float2 fo = make_float2(1.f, 0.f);
+		const float2* fma = nullptr;
+
+		if (nullptr != a.fm[0]) {
+			int c[3];
+			a.va.coords(in ? i : 0, o, 0, c);
+#pragma unroll
+			for (int d = 0; d < 3; d++) {
+				if (d == a.va.axis)
+					fma = a.fm[d];
+				else
+					fo = cmul(fo, a.fm[d][c[d]]);
+			}
+		}
+
+		lds_barrier();
+
+#pragma unroll 1
+		for (int b = 0; b < 2; b++) {
+
+			const float2* lb = lin + b * N + j;
+			float2 x[RA];
+#pragma unroll
+			for (int r = 0; r < RA; r++)
+				x[r] = cmul(h[r], lb[r * RB]);
+			PfDft<RA, -1>::run(x);
+
+			if (b > 0)
+				lds_barrier();  // the first member's last pass has read LDS
+
+			put(x);
+			lds_barrier();
+
+			float2* out = col + b * a.half;
+
+			last(Fwd{}, [&](int r, float2 y) BAM_INLINE {
+				if (nullptr != fma)
+					y = cmul(y, cmul(fo, fma[j + r * RB]));
+				if (in)
+					out[r * step] = y;
+			});
+		}
+
+	} else if constexpr (PF_MERGE == MODE) {
+
+		// both members' loads in flight
+		float2 x[RA], x1[RA];
+		load(x, col);
+		load(x1, col + a.half);
+		pf_tables(a, tw, lin, nullptr);
+		PfDft<RA, 1>::run(x);
+		put(x);
+		lds_barrier();
+
+		const float2* lb = lin + j;
+		float2 acc[RA];
+		last(Bwd{}, [&](int r, float2 y) BAM_INLINE { acc[r] = cmulc(y, lb[r * RB]); });
+
+		PfDft<RA, 1>::run(x1);
+		lds_barrier();
+		put(x1);
+		lds_barrier();
+
+		last(Bwd{}, [&](int r, float2 y) BAM_INLINE {
+			if (in)
+				col[r * step] = cadd(acc[r], cmulc(y, lb[N + r * RB]));
+		});
+
+	} else {
+
+		float2 h[RA], acc[RA];
+		load(h, col);
+		pf_tables(a, tw, lin, nullptr);
+#pragma unroll
+		for (int r = 0; r < RA; r++)
+			acc[r] = make_float2(0.f, 0.f);
+		lds_barrier();
+
+		const float2* psf = a.psf + (long)a.f_C.div(v) * a.va.N + vol0;
+
+#pragma unroll 1
+		for (int b = 0; b < 2; b++) {
+
+			const float2* lb = lin + b * N + j;
+			float2 x[RA];
+#pragma unroll
+			for (int r = 0; r < RA; r++)
+				x[r] = cmul(h[r], lb[r * RB]);
+			PfDft<RA, -1>::run(x);
+
+			if (b > 0)
+				lds_barrier();
+
+			put(x);
+			float2 ps[RA];
+			load(ps, psf + b * a.psf_half);  // in flight across the exchange
+			lds_barrier();
+			last(Fwd{}, [&](int r, float2 y) BAM_INLINE { x[r] = cmul(y, ps[r]); });
+			PfDft<RA, 1>::run(x);
+			lds_barrier();
+			put(x);
+			lds_barrier();
+			last(Bwd{}, [&](int r, float2 y) BAM_INLINE { acc[r] = cadd(acc[r], cmulc(y, lb[r * RB])); });
+		}
+
+#pragma unroll
+		for (int r = 0; r < RA; r++)
+			if (in)
+				col[r * step] = acc[r];
+	}
+}
+
+// ---------------------------------------------------------------------------
 // First axis: P rows of the image per work-group.  Split: coil image c (or
 // image x map c) x rolloff into volumes c and c + C; merge: the volumes of the
 // coils of a group back to the coil image, or conj(map) x summed over the
 // group into its partial image (no atomics, fixed order).
 // ---------------------------------------------------------------------------
+
+// rolloff and fftmod of the other axes of a row, fftmod table along it (null:
+// no fftmod)
+__device__ __forceinline__ void pf_row_factors(const PairArgs& a, uint32_t row, float& rr, float2& fo,
+					       const float2*& fma)
+{
+	rr = 1.f;
+	fo = make_float2(1.f, 0.f);
+	fma = nullptr;
+
+	if (nullptr == a.roll[0] && nullptr == a.fm[0])
+		return;
+
+	int c[3];
+	a.va.coords(0, row, 0, c);
+#pragma unroll
+	for (int d = 0; d < 3; d++) {
+		if (nullptr != a.roll[0] && d != a.va.axis)
+			rr *= a.roll[d][c[d]];
+		if (nullptr != a.fm[0]) {
+			if (d == a.va.axis)
+				fma = a.fm[d];
+			else
+				fo = cmul(fo, a.fm[d][c[d]]);
+		}
+	}
+}
 
 template <int MODE, bool MID>
 __device__ __forceinline__ void pair_rows_block(const PairArgs& a, uint32_t w, float2* lds)
@@ -706,26 +949,10 @@ __device__ __forceinline__ void pair_rows_block(const PairArgs& a, uint32_t w, f
 
 	pf_tables(a, tw, lin, a.roll[a.va.axis]);
 
-	// rolloff and fftmod of the other axes of this row
-	float rr = 1.f;
-	float2 fo = make_float2(1.f, 0.f);
-	const float2* fma = nullptr;
-
-	if (nullptr != a.roll[0] || nullptr != a.fm[0]) {
-		int c[3];
-		a.va.coords(0, t.in ? row : 0, 0, c);
-#pragma unroll
-		for (int d = 0; d < 3; d++) {
-			if (nullptr != a.roll[0] && d != a.va.axis)
-				rr *= a.roll[d][c[d]];
-			if (nullptr != a.fm[0]) {
-				if (d == a.va.axis)
-					fma = a.fm[d];
-				else
-					fo = cmul(fo, a.fm[d][c[d]]);
-			}
-		}
-	}
+	float rr;
+	float2 fo;
+	const float2* fma;
+	pf_row_factors(a, t.in ? row : 0, rr, fo, fma);
 
 	lds_barrier();
 
@@ -861,6 +1088,168 @@ __device__ __forceinline__ void pair_rows_block(const PairArgs& a, uint32_t w, f
 	}
 }
 
+// ---------------------------------------------------------------------------
+// First axis of such a length: RB lanes per row and member, the two members of
+// a row in the same wave.  A row never leaves its wave, so its exchange needs
+// no barrier, and a merge's next coil is loaded while the present one is
+// transformed (the coils of a group follow one another in the same lanes).
+// 128^3, 16 coils with maps: merge 444 us in the general kernel, 180 here (0.8
+// GB); split 235 -> 212.  CG of 256^2, 8 coils, 30 iterations: rows and columns
+// together 1.96 -> 1.61 ms.
+// ---------------------------------------------------------------------------
+
+// LDS of a wave's own rows, written and read by its lanes
+__device__ __forceinline__ void pf_wave_sync()
+{
+	__builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+	__builtin_amdgcn_wave_barrier();
+	__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+template <int MODE, int RA, int RB>
+__device__ __forceinline__ void pair_rows_fixed(const PairArgs& a, uint32_t w, float2* lds)
+{
+	constexpr int n = RA * RB, K = RA / RB;
+	constexpr int PITCH = pf_row_pitch(n);
+	const int P = a.P;  // of a batch's work-group maybe not all waves
+	float2* tw = lds + 2 * P * PITCH;
+	float2* lin = tw + n;
+
+	uint32_t rg, u;
+	a.f_ncg.divmod(w, u, rg);  // u: coil, or coil group
+	const int tr = threadIdx.x / RB;  // transform of the work-group: row, member
+	const int j = threadIdx.x % RB;
+	const int b = tr & 1;
+	const uint32_t row = rg * P + (tr >> 1);
+	const bool in = tr < 2 * P && row < a.va.outer;
+	const long N = a.va.N;
+	const long ro = (long)(in ? row : 0) * n + j;
+	float2* ls = lds + tr * PITCH;
+	const float2* lb = lin + b * n + j;
+
+	auto load = [&](float2 (&x)[RA], const float2* q) BAM_INLINE {
+#pragma unroll
+		for (int r = 0; r < RA; r++)
+			x[r] = q[r * RB];
+	};
+
+	auto at = [](int k) BAM_INLINE { return k + (k >> 3); };
+
+	// DFT of x, exchange, last pass: f(r, point j + r RB)
+	auto transform = [&](auto sg, float2 (&x)[RA], auto&& f) BAM_INLINE {
+		constexpr int SG = decltype(sg)::value;
+		PfDft<RA, SG>::run(x);
+		pf_wave_sync();
+#pragma unroll
+		for (int q = 0; q < RA; q++)
+			ls[at(j * RA + q)] = x[q];
+		pf_wave_sync();
+#pragma unroll
+		for (int m = 0; m < K; m++) {
+			const int jb = j + m * RB;
+			float2 y[RB];
+#pragma unroll
+			for (int r = 0; r < RB; r++) {
+				y[r] = ls[at(jb + r * RA)];
+				if (r > 0)
+					y[r] = (SG > 0) ? cmulc(y[r], tw[r * jb]) : cmul(y[r], tw[r * jb]);
+			}
+			PfDft<RB, SG>::run(y);
+#pragma unroll
+			for (int q = 0; q < RB; q++)
+				f(m + K * q, y[q]);
+		}
+	};
+
+	float2 x[RA];
+
+	if constexpr (PF_SPLIT == MODE) {
+
+		load(x, ((nullptr != a.sens) ? a.src : a.src + (long)u * N) + ro);
+
+		if (nullptr != a.sens) {
+			float2 m[RA];
+			load(m, a.sens + (long)u * N + ro);
+#pragma unroll
+			for (int r = 0; r < RA; r++)
+				x[r] = cmul(x[r], m[r]);
+		}
+	} else {
+		load(x, a.grid + (long)u * a.cc * N + b * a.half + ro);
+	}
+
+	pf_tables(a, tw, lin, a.roll[a.va.axis]);
+
+	float rr;
+	float2 fo;
+	const float2* fma;
+	pf_row_factors(a, in ? row : 0, rr, fo, fma);
+	lds_barrier();
+
+	if (tr >= 2 * P)
+		return;  // a whole wave
+
+	if constexpr (PF_SPLIT == MODE) {
+
+#pragma unroll
+		for (int r = 0; r < RA; r++)
+			x[r] = cscale(cmul(x[r], lb[r * RB]), rr);
+
+		float2* out = a.grid + (long)u * N + ro + b * a.half;
+
+		transform(std::integral_constant<int, -1>{}, x, [&](int r, float2 y) BAM_INLINE {
+			if (nullptr != fma)
+				y = cmul(y, cmul(fo, fma[j + r * RB]));
+			if (in)
+				out[r * RB] = y;
+		});
+
+	} else {
+
+		float2 acc[RA];
+#pragma unroll
+		for (int r = 0; r < RA; r++)
+			acc[r] = make_float2(0.f, 0.f);
+
+#pragma unroll 1
+		for (int m = 0; m < a.cc; m++) {
+
+			const long c = (long)u * a.cc + m;
+			float2 xn[RA], mp[RA];
+
+			if (nullptr != a.sens)
+				load(mp, a.sens + c * N + ro);
+
+			if (m + 1 < a.cc)
+				load(xn, a.grid + (c + 1) * N + b * a.half + ro);
+
+			transform(std::integral_constant<int, 1>{}, x, [&](int r, float2 y) BAM_INLINE {
+				y = cmulc(y, lb[r * RB]);
+				if (nullptr != a.sens)
+					y = cmulc(y, mp[r]);
+				acc[r] = cadd(acc[r], y);
+			});
+
+			if (m + 1 < a.cc)
+#pragma unroll
+				for (int r = 0; r < RA; r++)
+					x[r] = xn[r];
+		}
+
+		// sum of the members: each takes half of the points
+		float2* out = a.dst + (long)u * N + ro + b * (n / 2);
+
+#pragma unroll
+		for (int r = 0; r < RA / 2; r++) {
+			const float2 own = (b > 0) ? acc[r + RA / 2] : acc[r];
+			const float2 oth = (b > 0) ? acc[r] : acc[r + RA / 2];
+			const float2 rec = make_float2(__shfl_xor(oth.x, RB), __shfl_xor(oth.y, RB));
+			if (in)
+				out[r * RB] = cscale(cadd(own, rec), rr);
+		}
+	}
+}
+
 #undef BAM_PF_PASS
 #undef BAM_PF_END
 
@@ -891,6 +1280,25 @@ __global__ __launch_bounds__(pf_threads(ROWS, MID)) void k_pair(PairArgs a)
 	pair_block<MODE, ROWS, MID>(a, pf_xcd_order(blockIdx.x, gridDim.x), pf_lds);
 }
 
+template <int MODE, bool ROWS, int RA, int RB>
+__device__ __forceinline__ void pair_fixed_block(const PairArgs& a, uint32_t w, float2* lds)
+{
+	if (nullptr != a.skip && 0 != *a.skip)
+		return;
+
+	if constexpr (ROWS)
+		pair_rows_fixed<MODE, RA, RB>(a, w, lds);
+	else
+		pair_cols_fixed<MODE, RA, RB>(a, w, lds);
+}
+
+template <int MODE, bool ROWS, int RA, int RB>
+__global__ __launch_bounds__(ROWS ? 256 : PF_FP * RB) void k_pair_fixed(PairArgs a)
+{
+	extern __shared__ float2 pf_lds[];
+	pair_fixed_block<MODE, ROWS, RA, RB>(a, pf_xcd_order(blockIdx.x, gridDim.x), pf_lds);
+}
+
 // one pass of many plans in one launch: btab[b] = (plan, its work-group)
 template <int MODE, bool ROWS, bool MID>
 __global__ __launch_bounds__(pf_threads(ROWS, MID)) void k_pair_batch(const PairArgs* __restrict__ items,
@@ -901,9 +1309,18 @@ __global__ __launch_bounds__(pf_threads(ROWS, MID)) void k_pair_batch(const Pair
 	pair_block<MODE, ROWS, MID>(items[e.x], (uint32_t)e.y, pf_lds);
 }
 
+template <int MODE, bool ROWS, int RA, int RB>
+__global__ __launch_bounds__(ROWS ? 256 : PF_FP * RB) void k_pair_fixed_batch(const PairArgs* __restrict__ items,
+									     const int2* __restrict__ btab)
+{
+	extern __shared__ float2 pf_lds[];
+	const int2 e = btab[blockIdx.x];
+	pair_fixed_block<MODE, ROWS, RA, RB>(items[e.x], (uint32_t)e.y, pf_lds);
+}
+
 // launches (pair.hip)
 void pair_launch(int mode, bool rows, const PairArgs& a, const char* name, hipStream_t st);
-void pair_launch_batch(int mode, bool rows, bool three, const PairArgs* items, const int2* btab, int nblk,
+void pair_launch_batch(int mode, bool rows, int cl, const PairArgs* items, const int2* btab, int nblk,
 		       unsigned threads, size_t lds, const char* name, hipStream_t st);
 
 }  // namespace bam

@@ -1,6 +1,6 @@
 """GPU: the FFT passes over sub-grid pairs at the lengths where their plan
-changes -- one, two and three radices, every odd radix, column groups that do
-not fill, coil groups of more than one coil, and lengths without a pair
+changes -- one, two and three radices, every odd radix, the lengths with a
+kernel of their own, column groups that do not fill, coil groups of more than one coil, and lengths without a pair
 kernel (over 1024, or no three radices of at most 16) -- against the oracle:
 forward, adjoint and the Toeplitz normal operator with coil maps.  FP32
 transforms of both sides: 1e-5, as for every operator."""
@@ -43,6 +43,22 @@ CASES = [
     ((625, 12, 1), 2),      # 5^4: no three radices
     ((12, 1040, 1), 2),     # over 1024
     ((1040, 1, 1), 2),
+    # 32, 64, 128 and 256 (a kernel of their own): rows and columns, rows that do
+    # not fill a wave or a work-group, ragged column groups, one and four waves
+    ((32, 33, 1), 2),
+    ((64, 3, 1), 1),
+    ((128, 18, 1), 3),
+    ((256, 7, 1), 2),
+    ((18, 64, 1), 2),
+    ((33, 32, 1), 2),
+    ((1, 32, 1), 2),
+    ((5, 128, 1), 2),
+    ((22, 256, 1), 2),
+    ((1, 64, 1), 3),
+    ((256, 128, 1), 17),
+    ((64, 10, 128), 5),
+    ((6, 128, 64), 2),
+    ((32, 32, 32), 3),
 ]
 
 
