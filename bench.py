@@ -73,11 +73,10 @@ def survey_bytes(w):
 # per Toeplitz CG iteration is charged with the whole iteration's
 # compulsory bytes, a kernel of the NUFFT with the whole application's
 UNIT_OF = {
-    "fft_toeplitz": "iteration", "fft_toeplitz_slice_fwd": "iteration", "fft_toeplitz_slice_inv": "iteration",
-    "sum_coil_groups": "iteration", "fft_toeplitz_fwd": "iteration", "fft_toeplitz_inv": "iteration",
+    "fft_toeplitz": "iteration", "sum_coil_groups": "iteration",
+    "fft_toeplitz_fwd": "iteration", "fft_toeplitz_inv": "iteration",
     "grid_adjoint": "nufft", "grid_forward": "nufft", "permute_ksp": "nufft", "fft_fwd_axis": "nufft",
-    "fft_adj_axis": "nufft", "fft_fwd_first": "nufft", "fft_adj_last": "nufft", "fft_fwd_slice": "nufft",
-    "fft_adj_slice": "nufft",
+    "fft_adj_axis": "nufft", "fft_fwd_first": "nufft", "fft_adj_last": "nufft",
 }
 
 
@@ -86,10 +85,10 @@ def algorithmic_bytes(kernel, w):
     once, each output written once (complex64 = 8 B, coordinates 4 B/dim).
     The NUFFT operator of the step works on coil images (no maps); the
     Toeplitz classes belong to the SENSE normal operator (maps read, one
-    image in and out, coil-group partial images).  Where the x-y slices fit
-    in LDS and the z length has a pair kernel, the Toeplitz stack holds one
-    x-y transform per pair of sub-grids that differ only in the z shift
-    (S/2 volumes per coil), and the z-pass reads the PSF of all S."""
+    image in and out, coil-group partial images).  The passes work on
+    pairs of sub-grids that differ in the shift of one axis: after j axes the
+    stack holds 2^j volumes per coil, and the last axis of the Toeplitz
+    operator reads and writes S/2 of them and the PSF of all S."""
     X, Y, Z = w["img"]
     N = X * Y * Z
     C = w["C"]
@@ -98,8 +97,9 @@ def algorithmic_bytes(kernel, w):
     S = 2 ** d
     grid = 8 * S * C * N
     G = w.get("groups", 1)
-    pair = d == 3 and X == Y and X in (32, 64, 96, 128) and Z in (64, 128, 256, 512)
-    tgrid = grid // 2 if pair else grid
+    vol = 8 * C * N
+    cols = sum(3 * 2 ** j for j in range(1, d)) / max(d - 1, 1)
+    mid = sum(3 * 2 ** j for j in range(1, d - 1))
     table = {
         # k-space (x conj(weights)) -> sorted, coil-interleaved copy
         "permute_ksp": 8 * C * M + 8 * C * M,
@@ -107,23 +107,20 @@ def algorithmic_bytes(kernel, w):
         "grid_adjoint": 8 * C * M + 4 * d * M + grid,
         # sub-grid stack + coordinates in, k-space out
         "grid_forward": grid + 4 * d * M + 8 * C * M,
-        # one axis of the sub-grid stack: read + write (z-pass with pairs:
-        # the pair stack on one side)
-        "fft_fwd_axis": tgrid + grid,
-        "fft_adj_axis": grid + tgrid,
-        # coil images in, sub-grid stack out / back
-        "fft_fwd_first": 8 * C * N + grid,
-        "fft_adj_last": grid + 8 * C * N,
-        # (3-D slice path with pairs: the slice kernels store / read one
-        # x-y transform per pair, the z-pass writes / reads all S sub-grids)
-        "fft_fwd_slice": 8 * C * N + tgrid,
-        "fft_adj_slice": tgrid + 8 * C * N,
-        # SENSE normal operator: image + maps in, stack out
-        "fft_toeplitz_slice_fwd": 8 * N + 8 * C * N + tgrid,
-        # z axis forward, x PSF, inverse: stack read + write, PSF read
-        "fft_toeplitz": 2 * tgrid + 8 * S * N,
-        # stack + maps in, coil-group partial images out
-        "fft_toeplitz_slice_inv": tgrid + 8 * C * N + 8 * G * N,
+        # passes over sub-grid pairs: axis j takes 2^j volumes per coil to
+        # 2^(j + 1) and back (mean over the axes that share a name)
+        "fft_fwd_axis": cols * vol,
+        "fft_adj_axis": cols * vol,
+        "fft_fwd_first": 3 * vol,
+        "fft_adj_last": 3 * vol,
+        # SENSE normal operator: image + maps in, 2 volumes per coil out, then
+        # the axes between the first and the last
+        "fft_toeplitz_fwd": (8 * N + 3 * vol + mid * vol) / max(d - 1, 1),
+        # last axis forward, x PSF, inverse: half of the stack read + written,
+        # PSF read
+        "fft_toeplitz": grid + 8 * S * N,
+        # 2 volumes and the map of every coil in, coil-group partial images out
+        "fft_toeplitz_inv": (3 * vol + 8 * G * N + mid * vol) / max(d - 1, 1),
         "sum_coil_groups": 8 * G * N + 8 * N,
     }
     return table.get(kernel)
