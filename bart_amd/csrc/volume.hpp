@@ -102,26 +102,19 @@ struct VolAxis {
 		return offset_iov(i, o, v, k);
 	}
 
-	// pixel coordinates (x, y, z) of element k of transform (i, o)
+	// pixel coordinates (x, y, z) of element k of transform (i, o).  Selects
+	// instead of a branch per axis: from the three-way branch the compiler
+	// (ROCm 7.2, gfx950) made code that took c[2] = o for axis 2 in the PSF's
+	// kernels of 64, 128 and 256 points.
 	__host__ __device__ inline void coords(uint32_t i, uint32_t o, int k, int c[3]) const
 	{
-		uint32_t q, r;
-
-		if (0 == axis) {
-			c[0] = k;
-			f_n1.divmod(o, q, r);
-			c[1] = (int)r;
-			c[2] = (int)q;
-		} else if (1 == axis) {
-			c[0] = (int)i;
-			c[1] = k;
-			c[2] = (int)o;
-		} else {
-			f_n0.divmod(i, q, r);
-			c[0] = (int)r;
-			c[1] = (int)q;
-			c[2] = k;
-		}
+		const bool a0 = 0 == axis, a2 = 2 == axis;
+		const uint32_t x = a0 ? o : i;
+		const uint32_t q = a0 ? f_n1.div(x) : f_n0.div(x);
+		const uint32_t r = x - q * (uint32_t)(a0 ? n[1] : n[0]);
+		c[0] = a0 ? k : (a2 ? (int)r : (int)i);
+		c[1] = a0 ? (int)r : (a2 ? (int)q : k);
+		c[2] = a0 ? (int)q : (a2 ? k : (int)o);
 	}
 };
 
