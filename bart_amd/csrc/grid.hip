@@ -178,6 +178,23 @@ static GridTiling choose_tiling(const GridGeom& g)
 	return t;
 }
 
+// cell that holds position x on the axis of dim d.  The cells of a periodic
+// grid continue beyond both ends, where the last cell of an odd dim, which
+// holds one point, takes the place of a whole one.
+__host__ __device__ inline int cell_at(const GridGeom& g, int d, float x)
+{
+	const float n = (float)g.n[d];
+	const float cs = (float)g.CS[d];
+
+	if (g.periodic && x < 0.f)
+		return (int)floorf((x + n) / cs) - g.ncell[d];
+
+	if (g.periodic && x >= n)
+		return (int)floorf((x - n) / cs) + g.ncell[d];
+
+	return (int)floorf(x / cs);
+}
+
 // cells [clo, chi] of one dim as up to two spans {a0, n0, a1, n1} (wrapped
 // for periodic grids, clamped otherwise, every cell at most once); the
 // device twin is cell_span()
@@ -460,8 +477,8 @@ void GridPlan::build(const GridGeom& geom, const float* traj)
 
 			if (g.n[d] > 1) {
 				int t0 = tb[d] * t.T[d];
-				clo = (int)floorf(((float)t0 - g.reach_hi) / (float)g.CS[d]);
-				chi = (int)floorf(((float)(t0 + t.T[d] - 1) + g.reach_lo) / (float)g.CS[d]);
+				clo = cell_at(g, d, (float)t0 - g.reach_hi);
+				chi = cell_at(g, d, (float)(t0 + t.T[d] - 1) + g.reach_lo);
 			}
 
 			host_cell_span(g, d, clo, chi, span[d]);
@@ -966,8 +983,8 @@ __global__ __launch_bounds__(1024) void k_grid_adj(GridGeom g, GridTiling t, con
 				clo[d] = 0;
 				chi[d] = 0;
 			} else {
-				clo[d] = (int)floorf(((float)t0[d] - g.reach_hi) / (float)g.CS[d]);
-				chi[d] = (int)floorf(((float)(t0[d] + t.T[d] - 1) + g.reach_lo) / (float)g.CS[d]);
+				clo[d] = cell_at(g, d, (float)t0[d] - g.reach_hi);
+				chi[d] = cell_at(g, d, (float)(t0[d] + t.T[d] - 1) + g.reach_lo);
 			}
 		}
 
@@ -1101,7 +1118,9 @@ __global__ __launch_bounds__(1024) void k_grid_adj(GridGeom g, GridTiling t, con
 					eni = min(eni, n - 1);
 				}
 
-				const int cnt = min(min(max(eni - sti + 1, 0), TP), n);
+				const int cnt = min(max(eni - sti + 1, 0), TP);
+				// more taps than points of the period: a point gets several
+				const bool twice = g.periodic && n < t.ntap;
 				const int T = t.T[d], Tp = t.Tp[d];
 				const int td = sel3(d, t0[0], t0[1], t0[2]);
 				float* wr = L.wtab + v * ADJ_WROW + t.eoff[d] + var * Tp;
@@ -1129,10 +1148,14 @@ __global__ __launch_bounds__(1024) void k_grid_adj(GridGeom g, GridTiling t, con
 					if (g.periodic && l + td >= n)
 						l -= n;
 
+					if (twice)
+						while (l + td >= n)
+							l -= n;
+
 					const float w = kb_lookup(table, div_width(fabsf((float)(sti + q) - pos), g.width, t.rwidth));
 
 					if (q < cnt && l >= 0 && l < T) {
-						wr[l] = w;
+						wr[l] = twice ? wr[l] + w : w;
 						bits |= 1u << l;
 					}
 				}

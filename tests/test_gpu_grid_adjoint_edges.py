@@ -1,7 +1,8 @@
 """GPU: the adjoint gridding at the edges of its work split -- one, two and
 three active dims, every coil-chunk width (4, 8, 16) with a chunk that does
-not fill, four and eight taps per dim, tiles cut by the grid, periodic grids
-smaller than the kernel's reach, batches of visits that do not fill and tiles
+not fill, four and eight taps per dim, tiles cut by the grid, periodic grids of
+even and odd dims, among them some smaller than the kernel's reach and some with
+fewer points than taps, batches of visits that do not fill and tiles
 split over several work items -- against the oracle, FP32 sums of both sides:
 1e-5 as for every operator."""
 import numpy as np
@@ -24,16 +25,12 @@ def relerr(a, ref):
     return float(np.linalg.norm(a - ref) / np.linalg.norm(ref))
 
 
-@pytest.mark.parametrize("dims", [(50, 1, 1), (33, 28, 1), (10, 12, 9), (18, 16, 1), (8, 6, 4)])
+@pytest.mark.parametrize("dims", [(50, 1, 1), (33, 28, 1), (10, 12, 9), (18, 16, 1), (8, 6, 4), (5, 3, 2), (2, 1, 1)])
 @pytest.mark.parametrize("C", [1, 7, 17])
-@pytest.mark.parametrize("width,periodic", [(6.0, False), (6.0, True), (10.0, False)])
+@pytest.mark.parametrize("width,periodic", [(6.0, False), (6.0, True), (10.0, False), (10.0, True)])
 @pytest.mark.parametrize("M", [1, 300, 9000])
 def test_grid_adjoint_edges(dims, C, width, periodic, M):
     import bart_amd as ba
-    if periodic and min(n for n in dims if n > 1) < 6:
-        pytest.skip("the oracle wraps each tap, kernels wider than the grid count points twice")
-    if periodic and any(n > 1 and n % 2 for n in dims):
-        pytest.skip("odd periodic dims: the cells of two points do not tile the period")
     rng = np.random.default_rng(M + C + dims[0])
     traj = np.zeros((M, 3), np.complex64)
     for d in range(3):
