@@ -239,6 +239,7 @@ constexpr int FW_THREADS = 512;
 constexpr int FW_MAXS = FW_SPT * FW_THREADS;
 constexpr int FW_CC = 4;         // coils per staged region
 constexpr int FW_E = 12;         // staged region edge: tile + halo of a kernel of width 3
+constexpr int FW_NT = 3;         // taps of such a kernel (an edge of 12 means a width over 2, up to 3)
 
 static int taps_bound(const GridGeom& g);
 
@@ -277,7 +278,7 @@ void GridPlan::build_forward_tiles(const GridGeom& gg, const std::vector<int>& h
 		return;
 
 	// the staged region of FW_CC coils and the KB table fit into 64 KiB
-	if (((size_t)ft.Etot + 2 * FW_E + 4) * FW_CC * sizeof(float2) + (KB_SIZE + 4) * sizeof(float) > 64 * 1024)
+	if (((size_t)ft.Etot + 2 * FW_E) * FW_CC * sizeof(float2) + (KB_SIZE + 4) * sizeof(float) > 64 * 1024)
 		return;
 
 	const int cpt = FW_T / gg.CS[0];  // cells per tile edge (CS is equal in every dim)
@@ -741,6 +742,7 @@ __device__ inline float div_width(float x, float width, float rwidth)
 // Taps of one sample along one dim (noncart/grid.c:415-457): NT = ceil(width)
 // of them -- of the width + 1 taps of a sample half way between grid points
 // both ends weigh 0 -- with weight 0 for those the grid's edge cuts off.
+// last: the last tap with a weight.  Returns whether there is one.
 // ---------------------------------------------------------------------------
 
 __device__ inline float sample_pos_v(const GridGeom& g, int d, int v, float k)
@@ -749,15 +751,16 @@ __device__ inline float sample_pos_v(const GridGeom& g, int d, int v, float k)
 }
 
 template <int NT>
-__device__ inline void taps_of(const GridGeom& g, int d, int v, float k, const float* table, float rwidth, int& start,
-			       float (&w)[NT])
+__device__ inline bool taps_of(const GridGeom& g, int d, int v, float k, const float* table, float rwidth, int& start,
+			       int& last, float (&w)[NT])
 {
 	if (1 == g.n[d]) {
 		start = 0;
+		last = 0;
 #pragma unroll
 		for (int j = 0; j < NT; j++)
 			w[j] = (0 == j) ? 1.f : 0.f;
-		return;
+		return true;
 	}
 
 	const float pos = sample_pos_v(g, d, v, k);
@@ -769,15 +772,54 @@ __device__ inline void taps_of(const GridGeom& g, int d, int v, float k, const f
 		eni = min(eni, g.n[d] - 1);
 	}
 
+	// (positions beyond the range of int saturate: taps are counted first)
+	const int cnt = max(eni - sti + 1, 0);
 	start = sti;
+	last = max(min(cnt, NT), 1) - 1;
 
 #pragma unroll
 	for (int j = 0; j < NT; j++)
-		w[j] = (sti + j <= eni) ? kb_lookup(table, div_width(fabsf((float)(sti + j) - pos), g.width, rwidth)) : 0.f;
+		w[j] = (j < cnt) ? kb_lookup(table, div_width(fabsf((float)(int)((unsigned)sti + j) - pos), g.width, rwidth)) : 0.f;
+
+	return cnt > 0;
 }
 
-// grid index of tap w: wrapped, or kept on the grid (where a tap off it has
-// weight 0)
+// The same in a staged region whose points off the grid are 0, so that no tap
+// has to be cut off: start is tap 0 of an unbounded grid, and a tap beyond the
+// kernel (width < NT) weighs 0 by its distance.
+template <int NT>
+__device__ inline bool taps_staged(const GridGeom& g, int d, int v, float k, const float* table, float rwidth,
+				   int& start, int& last, float (&w)[NT])
+{
+	const float pos = sample_pos_v(g, d, v, k);
+	start = (int)ceil((double)pos - 0.5 * (double)g.width);
+	last = min(max((int)floor((double)pos + 0.5 * (double)g.width) - start, 0), NT - 1);
+
+#pragma unroll
+	for (int j = 0; j < NT; j++)
+		w[j] = kb_lookup(table, div_width(fabsf((float)(int)((unsigned)start + j) - pos), g.width, rwidth));
+
+	// a tap on the grid: start in (-NT, n)
+	return (unsigned)start + (NT - 1) < (unsigned)(g.n[d] + NT - 1);
+}
+
+// acc += val where `in`, whatever val holds elsewhere.  The mask goes through an
+// empty asm: given a select or a branch the compiler moves the loads behind val
+// around (those of all samples of a thread come at once and spill 140 registers).
+template <int CC>
+__device__ inline void acc_where(float2 (&acc)[CC], const float2 (&val)[CC], bool in)
+{
+	unsigned m = in ? ~0u : 0u;
+	asm("" : "+v"(m));
+
+#pragma unroll
+	for (int cl = 0; cl < CC; cl++) {
+		acc[cl].x += __uint_as_float(__float_as_uint(val[cl].x) & m);
+		acc[cl].y += __uint_as_float(__float_as_uint(val[cl].y) & m);
+	}
+}
+
+// grid index of tap w: wrapped, or kept on the grid (of a sample without taps)
 __device__ inline int tap_index(const GridGeom& g, int d, int w)
 {
 	const int n = g.n[d];
@@ -1493,15 +1535,19 @@ __global__ __launch_bounds__(256) void k_grid_fwd(GridGeom g, const float* __res
 	const int act[3] = { a0, a1, a2 };  // active dims, x first
 
 	// taps of the active dims and shift variants: weights, and offsets of the
-	// grid points in a coil plane
+	// grid points in a coil plane (unsigned: a plane of 2^31 points and more
+	// fits the memory).  A tap without a weight takes the last one's point, and
+	// a sub-grid where the sample has no taps adds nothing, so that a non-finite
+	// grid point reaches only the samples next to it.
 	float w[ND][2][NT];
-	int off[ND][2][NT];
+	unsigned off[ND][2][NT];
+	bool any[ND][2];
 
 #pragma unroll
 	for (int a = 0; a < ND; a++) {
 
 		const int d = act[a];
-		const int str = (0 == d) ? 1 : ((1 == d) ? g.n[0] : g.n[0] * g.n[1]);
+		const unsigned str = (0 == d) ? 1u : ((1 == d) ? (unsigned)g.n[0] : (unsigned)g.n[0] * (unsigned)g.n[1]);
 		const float k = sel3(d, kc.x, kc.y, kc.z);
 
 #pragma unroll
@@ -1513,15 +1559,16 @@ __global__ __launch_bounds__(256) void k_grid_fwd(GridGeom g, const float* __res
 					w[a][1][j] = w[a][0][j];
 					off[a][1][j] = off[a][0][j];
 				}
+				any[a][1] = any[a][0];
 				continue;
 			}
 
-			int start;
-			taps_of<NT>(g, d, v, k, table, rwidth, start, w[a][v]);
+			int start, last;
+			any[a][v] = taps_of<NT>(g, d, v, k, table, rwidth, start, last, w[a][v]);
 
 #pragma unroll
 			for (int j = 0; j < NT; j++)
-				off[a][v][j] = str * tap_index(g, d, start + j);
+				off[a][v][j] = str * (unsigned)tap_index(g, d, (int)((unsigned)start + min(j, last)));
 		}
 	}
 
@@ -1530,23 +1577,21 @@ __global__ __launch_bounds__(256) void k_grid_fwd(GridGeom g, const float* __res
 	for (int cl = 0; cl < CC; cl++)
 		acc[cl] = make_float2(0.f, 0.f);
 
-	// sub-grids: one bit per active dim (unrolled, with all their loads in
-	// flight, while the registers last)
-	constexpr int UNROLL = (ND <= 2 && NT <= 4) ? (1 << ND) : 1;
-
-#pragma unroll UNROLL
-	for (int s = 0; s < (1 << ND); s++) {
+	auto subgrid = [&](int s, auto checked) {
 
 		float ws[ND][NT];
-		int os[ND][NT];
+		unsigned os[ND][NT];
+		bool in = true;
 
 #pragma unroll
-		for (int a = 0; a < ND; a++)
+		for (int a = 0; a < ND; a++) {
 #pragma unroll
 			for (int j = 0; j < NT; j++) {
 				ws[a][j] = ((s >> a) & 1) ? w[a][1][j] : w[a][0][j];
 				os[a][j] = ((s >> a) & 1) ? off[a][1][j] : off[a][0][j];
 			}
+			in = in && (((s >> a) & 1) ? any[a][1] : any[a][0]);
+		}
 
 		float2 val[CC];
 #pragma unroll
@@ -1560,13 +1605,13 @@ __global__ __launch_bounds__(256) void k_grid_fwd(GridGeom g, const float* __res
 		for (int iz = 0; iz < NZ; iz++) {
 
 			const float dz = (ND > 2) ? ws[ND - 1][iz] : 1.f;
-			const int oz = (ND > 2) ? os[ND - 1][iz] : 0;
+			const unsigned oz = (ND > 2) ? os[ND - 1][iz] : 0u;
 
 #pragma unroll
 			for (int iy = 0; iy < NY; iy++) {
 
 				const float dy = (ND > 1) ? dz * ws[(ND > 1) ? 1 : 0][iy] : dz;
-				const int oy = oz + ((ND > 1) ? os[(ND > 1) ? 1 : 0][iy] : 0);
+				const unsigned oy = oz + ((ND > 1) ? os[(ND > 1) ? 1 : 0][iy] : 0u);
 
 #pragma unroll
 				for (int ix = 0; ix < NT; ix++) {
@@ -1586,9 +1631,34 @@ __global__ __launch_bounds__(256) void k_grid_fwd(GridGeom g, const float* __res
 			}
 		}
 
+		if (!decltype(checked)::value || in)
 #pragma unroll
-		for (int cl = 0; cl < CC; cl++)
-			acc[cl] = cadd(acc[cl], val[cl]);
+			for (int cl = 0; cl < CC; cl++)
+				acc[cl] = cadd(acc[cl], val[cl]);
+	};
+
+	// sub-grids: one bit per active dim (unrolled, with all their loads in
+	// flight, while the registers last; a check per sub-grid would keep the
+	// loads apart)
+	bool all = true;
+
+#pragma unroll
+	for (int a = 0; a < ND; a++)
+		all = all && any[a][0] && any[a][1];
+
+	if (__all(all)) {
+
+		constexpr int UNROLL = (ND <= 2 && NT <= 4) ? (1 << ND) : 1;
+
+#pragma unroll UNROLL
+		for (int s = 0; s < (1 << ND); s++)
+			subgrid(s, std::false_type{});
+
+	} else {
+
+#pragma unroll 1
+		for (int s = 0; s < (1 << ND); s++)
+			subgrid(s, std::true_type{});
 	}
 
 	const int m = sm[i];
@@ -1611,7 +1681,8 @@ __global__ __launch_bounds__(256) void k_grid_fwd(GridGeom g, const float* __res
 // lanes read points up to one apart in every dim: a point is 8 banks, a row
 // 12 points and a plane 2 points more than its rows, which puts the 8 points
 // of such a cube into 8 different bank groups.  All taps are taken (weight 0
-// beyond an edge) instead of branching around the ones that are cut off.
+// beyond an edge) instead of branching around the ones that are cut off.  Plans
+// with such tiles have kernels of more than 2 and at most 3 points.
 // Bound by LDS reads (27 float2 per sample, coil and sub-grid) and the waits of
 // the staging: 128^3 kooshball, 16 coils, 3.31 -> 2.85 ms with constant taps
 // and the padded planes (39.6 thousand vector instructions per wave, 47.6
@@ -1621,12 +1692,14 @@ __global__ __launch_bounds__(256) void k_grid_fwd(GridGeom g, const float* __res
 constexpr size_t FW_TABLE_BYTES = ((KB_SIZE + 4) * sizeof(float) + 15) / 16 * 16;
 constexpr int FW_ZPAD = 2;
 
-// points of the staged region: planes with their padding, and the taps past
-// the last row's end
-constexpr int fw_region(int E) { return E * (E * E + FW_ZPAD) + 4; }
+// points of the staged region: planes with their padding
+constexpr int fw_region(int E) { return E * (E * E + FW_ZPAD); }
 
-// E: staged region edge (tile + halo); LDS region layout [z][y][x][coil]
-template <int CCH, int E, int NT>
+// E: staged region edge (tile + halo); LDS region layout [z][y][x][coil].
+// FULL: the kernel width is NT, so that only a grid's edge takes taps away and
+// the taps off the grid are points of the halo, which is 0 there; otherwise a
+// tap without a weight takes the last one's point.
+template <int CCH, int E, int NT, bool FULL>
 __global__ __launch_bounds__(FW_THREADS) void k_grid_fwd_tile(GridGeom g, FwdTiling ft, const float* __restrict__ kbt,
 							      const int4* __restrict__ work,
 							      const int* __restrict__ fsm,
@@ -1644,10 +1717,6 @@ __global__ __launch_bounds__(FW_THREADS) void k_grid_fwd_tile(GridGeom g, FwdTil
 
 	for (int i = threadIdx.x; i < KB_SIZE + 1; i += FW_THREADS)
 		table[i] = kbt[i];
-
-	// the padding is read with weight 0
-	for (int i = threadIdx.x; i < fw_region(E) * CCH; i += FW_THREADS)
-		reg[i] = make_float2(0.f, 0.f);
 
 	const int4 it = work[blockIdx.x];
 	const int tile = it.x;
@@ -1724,16 +1793,17 @@ __global__ __launch_bounds__(FW_THREADS) void k_grid_fwd_tile(GridGeom g, FwdTil
 				if (!valid[q])
 					continue;
 
-				int b0, b1, b2;
+				int b0, b1, b2, e0, e1, e2;
 				float w0[NT], w1[NT], w2[NT];
-				taps_of<NT>(g, 0, v0, kc[q].x, table, rwidth, b0, w0);
-				taps_of<NT>(g, 1, v1, kc[q].y, table, rwidth, b1, w1);
-				taps_of<NT>(g, 2, v2, kc[q].z, table, rwidth, b2, w2);
+				const bool a0 = taps_staged<NT>(g, 0, v0, kc[q].x, table, rwidth, b0, e0, w0);
+				const bool a1 = taps_staged<NT>(g, 1, v1, kc[q].y, table, rwidth, b1, e1, w1);
+				const bool a2 = taps_staged<NT>(g, 2, v2, kc[q].z, table, rwidth, b2, e2, w2);
 
-				// in the staged region (a tap outside it has weight 0)
-				b0 = min(max(b0 - o0, 0), E - 1);
-				b1 -= o1;
-				b2 -= o2;
+				// in the staged region (outside it: a sample without taps)
+				b0 = min(max(b0, o0) - o0, E - NT);
+				b1 = min(max(b1, o1) - o1, E - NT);
+				b2 = min(max(b2, o2) - o2, E - NT);
+				const float2* pt = reg + (b0 + E * b1 + ZS * b2) * CCH;
 
 				float2 val[CCH];
 #pragma unroll
@@ -1744,20 +1814,21 @@ __global__ __launch_bounds__(FW_THREADS) void k_grid_fwd_tile(GridGeom g, FwdTil
 				for (int iz = 0; iz < NT; iz++) {
 
 					const float dz = w2[iz];
-					const int lz = min(max(b2 + iz, 0), E - 1) * ZS + b0;
+					const int lz = (FULL ? iz : min(iz, e2)) * ZS;
 
 #pragma unroll
 					for (int iy = 0; iy < NT; iy++) {
 
 						const float dy = dz * w1[iy];
-						const float4* row = (const float4*)(reg + (lz + min(max(b1 + iy, 0), E - 1) * E) * CCH);
+						const int ly = lz + (FULL ? iy : min(iy, e1)) * E;
 
 #pragma unroll
 						for (int ix = 0; ix < NT; ix++) {
 
 							const float dd = dy * w0[ix];
-							const float4 x01 = row[2 * ix];
-							const float4 x23 = row[2 * ix + 1];
+							const float4* p = (const float4*)(pt + (ly + (FULL ? ix : min(ix, e0))) * CCH);
+							const float4 x01 = p[0];
+							const float4 x23 = p[1];
 							val[0].x += x01.x * dd;
 							val[0].y += x01.y * dd;
 							val[1].x += x01.z * dd;
@@ -1770,9 +1841,7 @@ __global__ __launch_bounds__(FW_THREADS) void k_grid_fwd_tile(GridGeom g, FwdTil
 					}
 				}
 
-#pragma unroll
-				for (int cl = 0; cl < CCH; cl++)
-					acc[q][cl] = cadd(acc[q][cl], val[cl]);
+				acc_where<CCH>(acc[q], val, a0 && a1 && a2);
 			}
 		}
 
@@ -1807,15 +1876,15 @@ void grid_forward(const GridPlan& gp, const float* kb, float2* ksp, const float2
 
 		const FwdTiling& ft = gp.ft;
 		const size_t lds = FW_TABLE_BYTES + (size_t)FW_CC * fw_region(FW_E) * sizeof(float2);
-		BAM_CHECK(4 == taps_bound(g) && !g.periodic && lds <= 64 * 1024 && FW_E == ft.E[0] &&
+		BAM_CHECK(FW_NT == gp.ta.ntap && !g.periodic && lds <= 64 * 1024 && FW_E == ft.E[0] &&
 			  FW_E == ft.E[1] && FW_E == ft.E[2], "grid_forward: bad tiling");
-#define BAM_FWT(NT)                                                                                              \
-	hipLaunchKernelGGL((k_grid_fwd_tile<FW_CC, FW_E, NT>), dim3(ft.nitems), dim3(FW_THREADS), lds, st, g, ft, kb, \
-			   gp.fwork.ptr, gp.fsm.ptr, gp.fsk.ptr, grid, weights, ksp, gp.ta.rwidth)
-		if (gp.ta.ntap <= 3)
-			BAM_FWT(3);
+#define BAM_FWT(FULL)                                                                                               \
+	hipLaunchKernelGGL((k_grid_fwd_tile<FW_CC, FW_E, FW_NT, FULL>), dim3(ft.nitems), dim3(FW_THREADS), lds, st, g, ft, \
+			   kb, gp.fwork.ptr, gp.fsm.ptr, gp.fsk.ptr, grid, weights, ksp, gp.ta.rwidth)
+		if ((float)FW_NT == g.width)
+			BAM_FWT(true);
 		else
-			BAM_FWT(4);
+			BAM_FWT(false);
 #undef BAM_FWT
 		BAM_HIP(hipGetLastError());
 		return;
