@@ -418,7 +418,9 @@ __global__ __launch_bounds__(CV_THREADS) void k_conv3x3_wgrad(const float* __res
 
 					const unsigned short* xr = xl + ((((r + u) % 3) * NCI + it) * 16 + l16) * PX + 8 + p;
 					const uint4 d = *(const uint4*)xr;
-					const unsigned pv = *(const unsigned*)(xr - 2);
+					// (beyond the row dy is 0, and a 0 of dy must not
+					// meet the row's last pixel, which may be infinite)
+					const unsigned pv = (p < W) ? *(const unsigned*)(xr - 2) : 0u;
 					const unsigned nx = *(const unsigned*)(xr + 8);
 					// 8 pixels from p - 1 and from p + 1
 					const unsigned m0 = __builtin_amdgcn_alignbyte(d.x, pv, 2);

@@ -109,3 +109,19 @@ def test_conv3x3_rejects_bad_shapes():
     dy = torch.zeros((1, 4, 4, 100), device="cuda")
     with pytest.raises(ba.BartError, match="multiple of 8"):
         ba.conv3x3_bwd_weights(x, dy)
+
+
+# A row is padded to 32 pixels for the matrix cores: the last pixel has no left
+# tap in the image and must not reach that tap's gradient through the padding.
+@pytest.mark.parametrize("W", [8, 24, 32, 40])
+def test_conv3x3_backward_weights_nonfinite_last_pixel(W):
+    rng = np.random.default_rng(W)
+    x = rng.standard_normal((2, 17, 5, W)).astype(np.float32)
+    dy = rng.standard_normal((2, 3, 5, W)).astype(np.float32)
+    x[1, 4, 2, W - 1] = np.inf
+    dw = ba.conv3x3_bwd_weights(dev(x), dev(dy))[0].cpu().numpy()
+    x[1, 4, 2, W - 1] = 0
+    ref = R.conv3x3_bwd_weights(R.bf16(x), R.bf16(dy))[0]
+    assert not np.any(np.isfinite(dw[:, 4, :, 1:]))
+    dw[:, 4, :, 1:] = ref[:, 4, :, 1:]
+    assert relerr(dw, ref) < 1e-5
