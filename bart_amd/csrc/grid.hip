@@ -183,16 +183,12 @@ static GridTiling choose_tiling(const GridGeom& g)
 // holds one point, takes the place of a whole one.
 __host__ __device__ inline int cell_at(const GridGeom& g, int d, float x)
 {
-	const float n = (float)g.n[d];
-	const float cs = (float)g.CS[d];
+	int turns = 0;
 
-	if (g.periodic && x < 0.f)
-		return (int)floorf((x + n) / cs) - g.ncell[d];
+	if (g.periodic)
+		turns = (x < 0.f) ? -1 : ((x >= (float)g.n[d]) ? 1 : 0);
 
-	if (g.periodic && x >= n)
-		return (int)floorf((x - n) / cs) + g.ncell[d];
-
-	return (int)floorf(x / cs);
+	return (int)floorf((x - (float)(turns * g.n[d])) / (float)g.CS[d]) + turns * g.ncell[d];
 }
 
 // cells [clo, chi] of one dim as up to two spans {a0, n0, a1, n1} (wrapped
@@ -1161,8 +1157,6 @@ __global__ __launch_bounds__(1024) void k_grid_adj(GridGeom g, GridTiling t, con
 				}
 
 				const int cnt = min(max(eni - sti + 1, 0), TP);
-				// more taps than points of the period: a point gets several
-				const bool twice = g.periodic && n < t.ntap;
 				const int T = t.T[d], Tp = t.Tp[d];
 				const int td = sel3(d, t0[0], t0[1], t0[2]);
 				float* wr = L.wtab + v * ADJ_WROW + t.eoff[d] + var * Tp;
@@ -1190,17 +1184,24 @@ __global__ __launch_bounds__(1024) void k_grid_adj(GridGeom g, GridTiling t, con
 					if (g.periodic && l + td >= n)
 						l -= n;
 
-					if (twice)
-						while (l + td >= n)
-							l -= n;
-
 					const float w = kb_lookup(table, div_width(fabsf((float)(sti + q) - pos), g.width, t.rwidth));
 
-					if (q < cnt && l >= 0 && l < T) {
-						wr[l] = twice ? wr[l] + w : w;
+					if (q < min(cnt, n) && l >= 0 && l < T) {
+						wr[l] = w;
 						bits |= 1u << l;
 					}
 				}
+
+				// more taps than points of the period: a point gets several, the
+				// first ones are in
+				if (g.periodic && n < t.ntap)
+					for (int q = n; q < cnt; q++) {
+
+						const int l = (l0 + td + q) % n - td;
+
+						if (l >= 0 && l < T)
+							wr[l] += kb_lookup(table, div_width(fabsf((float)(sti + q) - pos), g.width, t.rwidth));
+					}
 
 				L.rows[k * ADJ_BATCH + v] = bits;
 			}
