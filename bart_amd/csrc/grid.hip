@@ -770,8 +770,9 @@ __device__ inline bool taps_of(const GridGeom& g, int d, int v, float k, const f
 
 	// (positions beyond the range of int saturate: taps are counted first)
 	const int cnt = max(eni - sti + 1, 0);
-	start = sti;
 	last = max(min(cnt, NT), 1) - 1;
+	// (of a sample without taps: some point of the grid)
+	start = g.periodic ? sti : min(sti, g.n[d] - 1);
 
 #pragma unroll
 	for (int j = 0; j < NT; j++)
@@ -815,17 +816,15 @@ __device__ inline void acc_where(float2 (&acc)[CC], const float2 (&val)[CC], boo
 	}
 }
 
-// grid index of tap w: wrapped, or kept on the grid (of a sample without taps)
-__device__ inline int tap_index(const GridGeom& g, int d, int w)
+// grid index of tap start + j, wrapped on a periodic grid
+__device__ inline int tap_index(const GridGeom& g, int d, int start, int j)
 {
+	if (!g.periodic)
+		return start + j;
+
 	const int n = g.n[d];
-
-	if (g.periodic) {
-		w %= n;
-		return w + ((w < 0) ? n : 0);
-	}
-
-	return min(max(w, 0), n - 1);
+	const int w = (int)((unsigned)start + j) % n;
+	return w + ((w < 0) ? n : 0);
 }
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -1569,7 +1568,7 @@ __global__ __launch_bounds__(256) void k_grid_fwd(GridGeom g, const float* __res
 
 #pragma unroll
 			for (int j = 0; j < NT; j++)
-				off[a][v][j] = str * (unsigned)tap_index(g, d, (int)((unsigned)start + min(j, last)));
+				off[a][v][j] = str * (unsigned)tap_index(g, d, start, min(j, last));
 		}
 	}
 

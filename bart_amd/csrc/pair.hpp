@@ -879,8 +879,11 @@ __device__ __forceinline__ void pf_row_factors(const PairArgs& a, uint32_t row, 
 	if (nullptr == a.roll[0] && nullptr == a.fm[0])
 		return;
 
-	int c[3];
-	a.va.coords(0, row, 0, c);
+	// along x: (y, z); along y: z (along z there is one row)
+	uint32_t c1 = row, c2 = row;
+	if (0 == a.va.axis)
+		a.va.f_n1.divmod(row, c2, c1);
+	const int c[3] = { 0, (int)c1, (int)c2 };
 #pragma unroll
 	for (int d = 0; d < 3; d++) {
 		if (nullptr != a.roll[0] && d != a.va.axis)
