@@ -48,14 +48,6 @@ static int conv_rows(long total_rows, int ncu)
 	return (int)std::min<long>(CV_MAXROWS, std::max<long>(1, (total_rows + ncu - 1) / ncu));
 }
 
-static int conv_ncu()
-{
-	int dev = 0, n = 1;
-	BAM_HIP(hipGetDevice(&dev));
-	BAM_HIP(hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev));
-	return std::max(1, n);
-}
-
 // ---------------------------------------------------------------------------
 // Forward.  Bound by HBM: 48 channels of 256^2 are 2 x 100 MB per batch of 8
 // against 22 GFLOP.  A work-group takes a strip of CV_STRIP pixels and walks
@@ -602,7 +594,7 @@ static void fwd_launch(const float* x, int B, int Cin, int H, int W, const float
 	hipLaunchKernelGGL(k_conv_wprep, dim3((unsigned)((nw + 255) / 256)), dim3(256), 0, st, w, Cin, Cout, G, ntiles,
 			   flip ? 1 : 0, wb.ptr);
 	const int nx = (W + CV_STRIP - 1) / CV_STRIP;
-	const int rows = conv_rows((long)nx * H * B, conv_ncu());
+	const int rows = conv_rows((long)nx * H * B, device_cus());
 	dim3 grid(nx, (H + rows - 1) / rows, B);
 
 #define BAM_CONV_G(NG) \
@@ -678,7 +670,7 @@ void conv3x3_bwd_weights(const float* x, const float* dy, int B, int Cin, int Co
 	std::lock_guard<std::mutex> lock(cw.mtx);
 	const int nco = (Cout + 15) / 16, nci = (Cin + 15) / 16;
 	const int PO = 16 * nco, PI = 16 * nci;
-	const int rows = conv_rows((long)B * H, conv_ncu());
+	const int rows = conv_rows((long)B * H, device_cus());
 	const int nparts = B * ((H + rows - 1) / rows);
 	const long np = (long)nparts * (9 * PO * PI + CV_MAXC);
 	if ((long)cw.part.n < np)

@@ -134,6 +134,9 @@ __device__ inline void lds_barrier()
 	__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+// compute units of the current device
+int device_cus();
+
 // Streams: the library launches on one stream per handle; default = 0.
 hipStream_t default_stream();
 

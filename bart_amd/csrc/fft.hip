@@ -51,6 +51,14 @@ bool fft_size_supported(int n)
 	return (n >= 1) && (n <= FFT_MAX_ELEMS) && factorize(n, p);
 }
 
+int device_cus()
+{
+	int dev = 0, n = 1;
+	BAM_HIP(hipGetDevice(&dev));
+	BAM_HIP(hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev));
+	return std::max(1, n);
+}
+
 AxisPlan make_axis_plan(int n)
 {
 	AxisPlan p;

@@ -303,26 +303,22 @@ __device__ inline void run_passes(float2* lds, const AxisPlan& plan, int P, floa
 	}
 }
 
-// functors with column-block access (static constexpr bool colblock = true;
-// cb_ok(P), base(t0), at(base, p, k [, v]))
-template <class F, class = void>
-struct colblock_of {
-	static constexpr bool value = false;
-};
-
-template <class F>
-struct colblock_of<F, std::void_t<decltype(F::colblock)>> {
-	static constexpr bool value = F::colblock;
+// no middle stage
+struct NoMid {
+	static constexpr bool active = false;
+	__device__ float2 operator()(long, int, float2 v) const { return v; }
 };
 
 // ---------------------------------------------------------------------------
 // The axis kernel.  Ld: float2 operator()(long t, int k) const.
+// Md (active): float2 operator()(long t, int k, float2 v) const, between the
+//     transform and a second one of the other sign.
 // St: void store(const float2* lds, const FftLaunch&, long t0) const -- runs
 //     the block's whole store loop so that it may reduce over transforms.
 // ---------------------------------------------------------------------------
 
-template <int EPT, bool GEN, class Ld, class St>
-__global__ __launch_bounds__(FFT_THREADS) void k_fft_axis(FftLaunch L, Ld ld, St st)
+template <int EPT, bool GEN, class Ld, class Md, class St>
+__global__ __launch_bounds__(FFT_THREADS) void k_fft_axis(FftLaunch L, Ld ld, Md md, St st)
 {
 	extern __shared__ float2 lds[];
 
@@ -367,6 +363,20 @@ __global__ __launch_bounds__(FFT_THREADS) void k_fft_axis(FftLaunch L, Ld ld, St
 	lds_barrier();
 
 	run_passes<EPT, GEN>(lds, L.plan, P, L.sign);
+
+	if constexpr (Md::active) {
+
+		for (int i = threadIdx.x; i < tot; i += FFT_THREADS) {
+
+			const int p = L.contig ? i / n : i & (P - 1);
+			const int k = L.contig ? i - p * n : i >> L.logP;
+			lds[p * n + k] = md(t0 + p, k, lds[p * n + k]);
+		}
+
+		lds_barrier();
+
+		run_passes<EPT, GEN>(lds, L.plan, P, -L.sign);
+	}
 
 	st.store(lds, L, t0);
 }
@@ -511,11 +521,8 @@ __device__ inline void ct_passes_between(float2* lds, const float2* tw, float sg
 	}
 }
 
-// Transform of a column block (strided axis) with the first and last passes
-// in registers: a thread's E = P N / FFT_THREADS points k0 + j N / E are the
-// inputs of one butterfly of the first radix-E pass and the outputs of one
-// butterfly of the last radix-E pass, so the loads and the stores need no LDS
-// round trip.
+// elements per thread of a block, and whether one butterfly of that radix holds
+// them (fft_contig_regs)
 template <int N>
 constexpr int ct_edge_radix()
 {
@@ -528,61 +535,6 @@ constexpr bool ct_edges_in_regs()
 	constexpr int E = ct_edge_radix<N>();
 	return 0 == (ct_block_p(N) * N) % FFT_THREADS && (2 == E || 4 == E || 8 == E || 16 == E) &&
 	       0 == N % (E * E) && 0 == FFT_THREADS % ct_block_p(N);
-}
-
-template <int N, int E, class Ld, class St>
-__device__ inline void fft_cols_regs(const FftLaunch& L, const Ld& ld, const St& st, float2* lds,
-					 const float2* tw, long t0)
-{
-	constexpr int P = ct_block_p(N);
-	constexpr int LOGP = ct_log2(P);
-	constexpr int PN = N + 1;
-	constexpr int NE = N / E;
-
-	const int p = threadIdx.x & (P - 1);
-	const int k0 = threadIdx.x >> LOGP;
-	const bool in = t0 + p < L.total;
-	float2 v[E];
-
-	// loads; first forward pass (radix E, no twiddles)
-	{
-		const auto lb = ld.base(t0);
-#pragma unroll
-		for (int j = 0; j < E; j++)
-			v[j] = in ? ld.at(lb, p, k0 + j * NE) : make_float2(0.f, 0.f);
-	}
-
-	dft_any<E>(v, L.sign, tw, N);
-
-#pragma unroll
-	for (int q = 0; q < E; q++)
-		lds[p * PN + k0 * E + q] = v[q];
-
-	lds_barrier();
-
-	ct_passes_between<N, P, E, NE>(lds, tw, L.sign);
-
-	// last pass (radix E, sub-transforms of length N / E)
-#pragma unroll
-	for (int r = 0; r < E; r++) {
-		float2 x = lds[p * PN + k0 + r * NE];
-		if (r > 0) {
-			float2 w = tw[r * k0];
-			if (L.sign > 0.f)
-				w.y = -w.y;
-			x = cmul(x, w);
-		}
-		v[r] = x;
-	}
-
-	dft_any<E>(v, L.sign, tw, N);
-
-	if (in) {
-		const auto sb = st.base(t0);
-#pragma unroll
-		for (int q = 0; q < E; q++)
-			st.at(sb, p, k0 + q * NE, v[q]);
-	}
 }
 
 // Contiguous axis (transforms along rows): a thread takes the E points
@@ -620,8 +572,7 @@ __device__ inline void fft_contig_regs(const FftLaunch& L, const Ld& ld, const S
 
 // The transforms [t0, t0 + P) of one launch (the body of k_fft_axis_n).
 template <int N, class Ld, class St>
-__device__ inline void fft_axis_block(const FftLaunch& L, const Ld& ld, const St& st, long t0,
-				      float2* lds)
+__device__ inline void fft_axis_block(const FftLaunch& L, const Ld& ld, const St& st, long t0, float2* lds)
 {
 	constexpr int P = ct_block_p(N);
 	constexpr int TOT = P * N;
@@ -631,22 +582,8 @@ __device__ inline void fft_axis_block(const FftLaunch& L, const Ld& ld, const St
 
 	float2* tw = lds + P * PN;
 
-	// strided axis with column-block functors: per-block base addresses
-	constexpr bool CBF = colblock_of<Ld>::value && colblock_of<St>::value;
-	bool cb = false;
-
-	if constexpr (CBF)
-		cb = !L.contig && ld.cb_ok(P) && st.cb_ok(P);
-
 	for (int i = threadIdx.x; i < N; i += FFT_THREADS)
 		tw[i] = L.plan.tw[i];
-
-	if constexpr (CBF && ct_edges_in_regs<N>()) {
-		if (cb) {
-			fft_cols_regs<N, ct_edge_radix<N>()>(L, ld, st, lds, tw, t0);
-			return;
-		}
-	}
 
 	if constexpr (ct_edges_in_regs<N>()) {
 		if (L.contig) {
@@ -667,52 +604,18 @@ __device__ inline void fft_axis_block(const FftLaunch& L, const Ld& ld, const St
 
 	} else {
 
-		bool done = false;
-
-		if constexpr (CBF) {
-			if (cb) {
-				const auto lb = ld.base(t0);
-
 #pragma unroll 4
-				for (int i = threadIdx.x; i < TOT; i += FFT_THREADS) {
-					const int p = i & (P - 1);
-					const int k = i >> LOGP;
-					lds[p * PN + k] = (t0 + p < L.total) ? ld.at(lb, p, k) : make_float2(0.f, 0.f);
-				}
-
-				done = true;
-			}
-		}
-
-		if (!done) {
-#pragma unroll 4
-			for (int i = threadIdx.x; i < TOT; i += FFT_THREADS) {
-				const int p = i & (P - 1);
-				const int k = i >> LOGP;
-				const long t = t0 + p;
-				lds[p * PN + k] = (t < L.total) ? ld(t, k) : make_float2(0.f, 0.f);
-			}
+		for (int i = threadIdx.x; i < TOT; i += FFT_THREADS) {
+			const int p = i & (P - 1);
+			const int k = i >> LOGP;
+			const long t = t0 + p;
+			lds[p * PN + k] = (t < L.total) ? ld(t, k) : make_float2(0.f, 0.f);
 		}
 	}
 
 	lds_barrier();
 
 	ct_passes<N, P, 0, 1>(lds, tw, L.sign);
-
-	if constexpr (CBF) {
-		if (cb) {
-			const auto sb = st.base(t0);
-
-			for (int i = threadIdx.x; i < TOT; i += FFT_THREADS) {
-				const int p = i & (P - 1);
-				const int k = i >> LOGP;
-				if (t0 + p < L.total)
-					st.at(sb, p, k, lds[p * PN + k]);
-			}
-
-			return;
-		}
-	}
 
 	st.store(lds, L, t0);
 }
@@ -863,61 +766,72 @@ struct FftLaunchCfg {
 
 FftLaunchCfg fft_config(const AxisPlan& plan, long total, bool contig, int P_min, float sign);
 
-template <class Ld, class St>
-void launch_fft_axis(const FftLaunchCfg& cfg, hipStream_t stream, const Ld& ld, const St& st)
+// the run-time kernel
+template <class Ld, class Md, class St>
+void launch_fft_any(const FftLaunchCfg& cfg, hipStream_t stream, const Ld& ld, const Md& md, const St& st)
 {
 	if (0 == cfg.blocks)
 		return;
 
 	ProfScope prof(cfg.name, stream);
-
-	if (cfg.fixed) {
-
-		const dim3 gb(cfg.blocks), tb(FFT_THREADS);
-		const size_t lds = cfg.lds_bytes;
-
-#define BAM_FFT_N(NN) case NN: hipLaunchKernelGGL((k_fft_axis_n<NN, Ld, St>), gb, tb, lds, stream, cfg.L, ld, st); break
-		switch (cfg.L.plan.n) {
-			BAM_FFT_N(16);
-			BAM_FFT_N(32);
-			BAM_FFT_N(64);
-			BAM_FFT_N(128);
-			BAM_FFT_N(192);
-			BAM_FFT_N(256);
-			BAM_FFT_N(320);
-			BAM_FFT_N(384);
-			BAM_FFT_N(512);
-			BAM_FFT_N(640);
-			BAM_FFT_N(768);
-		default:
-			break;
-		}
-#undef BAM_FFT_N
-
-		BAM_HIP(hipGetLastError());
-		return;
-	}
-
+	const dim3 gb(cfg.blocks), tb(FFT_THREADS);
 	bool gen = false;
 
 	for (int i = 0; i < cfg.L.plan.nr; i++)
 		gen = gen || (cfg.L.plan.radix[i] > 8 || 7 == cfg.L.plan.radix[i]);
 
-	const dim3 gb(cfg.blocks), tb(FFT_THREADS);
-
+#define BAM_FFT_ANY(EPT, GEN) \
+	hipLaunchKernelGGL((k_fft_axis<EPT, GEN, Ld, Md, St>), gb, tb, cfg.lds_bytes, stream, cfg.L, ld, md, st)
 	if (gen) {
 		switch (cfg.ept) {
-		case 8: hipLaunchKernelGGL((k_fft_axis<8, true, Ld, St>), gb, tb, cfg.lds_bytes, stream, cfg.L, ld, st); break;
-		case 16: hipLaunchKernelGGL((k_fft_axis<16, true, Ld, St>), gb, tb, cfg.lds_bytes, stream, cfg.L, ld, st); break;
-		default: hipLaunchKernelGGL((k_fft_axis<32, true, Ld, St>), gb, tb, cfg.lds_bytes, stream, cfg.L, ld, st); break;
+		case 8: BAM_FFT_ANY(8, true); break;
+		case 16: BAM_FFT_ANY(16, true); break;
+		default: BAM_FFT_ANY(32, true); break;
 		}
 	} else {
 		switch (cfg.ept) {
-		case 8: hipLaunchKernelGGL((k_fft_axis<8, false, Ld, St>), gb, tb, cfg.lds_bytes, stream, cfg.L, ld, st); break;
-		case 16: hipLaunchKernelGGL((k_fft_axis<16, false, Ld, St>), gb, tb, cfg.lds_bytes, stream, cfg.L, ld, st); break;
-		default: hipLaunchKernelGGL((k_fft_axis<32, false, Ld, St>), gb, tb, cfg.lds_bytes, stream, cfg.L, ld, st); break;
+		case 8: BAM_FFT_ANY(8, false); break;
+		case 16: BAM_FFT_ANY(16, false); break;
+		default: BAM_FFT_ANY(32, false); break;
 		}
 	}
+#undef BAM_FFT_ANY
+
+	BAM_HIP(hipGetLastError());
+}
+
+template <class Ld, class St>
+void launch_fft_axis(const FftLaunchCfg& cfg, hipStream_t stream, const Ld& ld, const St& st)
+{
+	if (!cfg.fixed) {
+		launch_fft_any(cfg, stream, ld, NoMid{}, st);
+		return;
+	}
+
+	if (0 == cfg.blocks)
+		return;
+
+	ProfScope prof(cfg.name, stream);
+	const dim3 gb(cfg.blocks), tb(FFT_THREADS);
+
+#define BAM_FFT_N(NN) \
+	case NN: hipLaunchKernelGGL((k_fft_axis_n<NN, Ld, St>), gb, tb, cfg.lds_bytes, stream, cfg.L, ld, st); break
+	switch (cfg.L.plan.n) {
+		BAM_FFT_N(16);
+		BAM_FFT_N(32);
+		BAM_FFT_N(64);
+		BAM_FFT_N(128);
+		BAM_FFT_N(192);
+		BAM_FFT_N(256);
+		BAM_FFT_N(320);
+		BAM_FFT_N(384);
+		BAM_FFT_N(512);
+		BAM_FFT_N(640);
+		BAM_FFT_N(768);
+	default:
+		break;
+	}
+#undef BAM_FFT_N
 
 	BAM_HIP(hipGetLastError());
 }

@@ -452,11 +452,7 @@ void GridPlan::build(const GridGeom& geom, const float* traj)
 		kch = std::max<long>(kch, (long)((g.C + c - 1) / c) * c);
 	kspS.alloc((size_t)kch * std::max<long>(g.M, 1));
 
-	{
-		int dev = 0;
-		BAM_HIP(hipGetDevice(&dev));
-		BAM_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
-	}
+	ncu = device_cus();
 
 	// adjoint work list: the visits of a tile (its cells and their ring)
 	const GridTiling& t = ta;

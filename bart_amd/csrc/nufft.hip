@@ -170,77 +170,202 @@ __device__ inline float2 fm_val(const SepTables& T, const int c[3])
 // Pass functors
 // ---------------------------------------------------------------------------
 
-// Standard-order grid loads / stores for the other axes
-// Column-block access (used by the fixed-length kernel on strided axes):
-// the P transforms of a block are P adjacent columns of one volume when P
-// divides the transforms below the axis, so element (p, k) of the block is
-// at base + p + inner k.
-struct ColBase {
-	long off;     // offset of element (0, 0)
-	uint32_t i0;  // index below the axis of transform 0
-	uint32_t o;   // index above the axis
-	uint32_t v;   // volume
+// Passes of the run-time FFT kernel over the members of sub-grid pairs (see
+// pair.hpp): a block holds nm members of Q = P / nm columns, transform p of it
+// member b0 + p / Q of the block's column p % Q.  Both members (nm = 2) share
+// the loads of a split and the stores of a merge; where two do not fit (over
+// FFT_MAX_ELEMS / 2 points) a launch takes one.
+struct MemberGeom {
+
+	VolAxis va;       // nvol: volumes split or merged
+	int nm, b0;
+	int logP, logQ;
+	uint32_t nblk;
+	long ncol;        // columns in all
+	int cc;           // rows: coils per group, neighbours in a block
+	FastDiv f_cc;
+
+	// column of transform t: false beyond the last one
+	__device__ bool column(long t, uint32_t& i, uint32_t& o, uint32_t& v, int& b) const
+	{
+		const uint32_t p = (uint32_t)t & ((1u << logP) - 1u);
+		uint32_t blk = (uint32_t)(t >> logP);
+
+		// neighbouring columns share cache lines
+		if (1 != va.inner)
+			blk = pf_xcd_order(blk, nblk);
+
+		const long q = ((long)blk << logQ) + (p & ((1u << logQ) - 1u));
+		b = b0 + (int)(p >> logQ);
+
+		if (q >= ncol)
+			return false;
+
+		if (1 == cc) {
+			va.split(q, i, o, v);
+		} else {
+			uint32_t r, cl, g;
+			f_cc.divmod((uint32_t)q, r, cl);
+			i = 0;
+			va.f_outer.divmod(r, g, o);
+			v = g * cc + cl;
+		}
+
+		return true;
+	}
 };
 
-__device__ inline ColBase col_base(const VolAxis& g, long t0)
-{
-	ColBase b;
-	g.split(t0, b.i0, b.o, b.v);
-	b.off = g.offset_iov(b.i0, b.o, b.v, 0);
-	return b;
-}
+// split: the image side (src, with maps sens; x rolloff) or the grid, x the
+// linear phases l; merge (no l): the members
+struct LdMember {
 
-struct LdGrid {
-	static constexpr bool colblock = true;
-	VolAxis g;
+	MemberGeom m;
+	SepTables T;
+	const float2* src;
+	const float2* sens;
+	bool roll;
+	const float2* l[2];
 	const float2* grid;
+	long half;
 
 	__device__ float2 operator()(long t, int k) const
 	{
 		uint32_t i, o, v;
-		g.split(t, i, o, v);
-		return grid[g.offset_iov(i, o, v, k)];
+		int b;
+
+		if (!m.column(t, i, o, v, b))
+			return make_float2(0.f, 0.f);
+
+		const long at = m.va.offset_iov(i, o, v, k);
+
+		if (nullptr == l[0])
+			return grid[at + b * half];
+
+		float2 x;
+
+		if (nullptr == src)
+			x = grid[at];
+		else if (nullptr != sens)
+			x = cmul(src[at - (long)v * m.va.N], sens[at]);
+		else
+			x = src[at];
+
+		if (roll) {
+			int c[3];
+			m.va.coords(i, o, k, c);
+			x = cscale(x, T.roll[0][c[0]] * T.roll[1][c[1]] * T.roll[2][c[2]]);
+		}
+
+		return cmul(x, l[b][k]);
 	}
-
-	__device__ bool cb_ok(int P) const { return 0 == g.inner % (uint32_t)P; }
-	__device__ ColBase base(long t0) const { return col_base(g, t0); }
-
-	__device__ float2 at(const ColBase& b, int p, int k) const { return grid[b.off + p + (long)g.inner * k]; }
 };
 
-struct StGrid {
-	static constexpr bool colblock = true;
-	VolAxis g;
+// PSFs of the members
+struct MdMember {
+	static constexpr bool active = true;
+	MemberGeom m;
+	FastDiv f_C;
+	const float2* psf;
+	long half;
+
+	__device__ float2 operator()(long t, int k, float2 x) const
+	{
+		uint32_t i, o, v;
+		int b;
+
+		if (!m.column(t, i, o, v, b))
+			return x;
+
+		return cmul(x, psf[m.va.offset_iov(i, o, f_C.div(v), k) + b * half]);
+	}
+};
+
+struct StSplit {
+
+	MemberGeom m;
 	SepTables T;
 	float2* grid;
+	long half;
 	bool fm;
 
 	__device__ void store(const float2* lds, const FftLaunch& L, long t0) const
 	{
 		store_each(lds, L, t0, [&](long t, int k, float2 x) {
 			uint32_t i, o, v;
-			g.split(t, i, o, v);
+			int b;
+
+			if (!m.column(t, i, o, v, b))
+				return;
+
 			if (fm) {
 				int px[3];
-				g.coords(i, o, k, px);
+				m.va.coords(i, o, k, px);
 				x = cmul(x, fm_val(T, px));
 			}
-			grid[g.offset_iov(i, o, v, k)] = x;
+
+			grid[m.va.offset_iov(i, o, v, k) + b * half] = x;
 		});
 	}
+};
 
-	__device__ bool cb_ok(int P) const { return 0 == g.inner % (uint32_t)P; }
-	__device__ ColBase base(long t0) const { return col_base(g, t0); }
+// Sum over the members (and with maps over the coils of a group, into its
+// partial image) into dst, without dst into the grid in place; the second
+// launch of single members adds to what the first has left there.
+struct StMerge {
 
-	__device__ void at(const ColBase& b, int p, int k, float2 x) const
+	MemberGeom m;
+	SepTables T;
+	float2* dst;
+	const float2* sens;
+	bool roll;
+	const float2* l[2];
+	float2* grid;
+
+	__device__ void store(const float2* lds, const FftLaunch& L, long t0) const
 	{
-		if (fm) {
-			int px[3];
-			g.coords(b.i0 + p, b.o, k, px);
-			x = cmul(x, fm_val(T, px));
-		}
+		const int n = L.plan.n;
+		const int Q = 1 << m.logQ;
+		const int ng = Q / m.cc;  // sums per block and point
 
-		grid[b.off + p + (long)g.inner * k] = x;
+		for (int e = threadIdx.x; e < ng * n; e += FFT_THREADS) {
+
+			// rows: points next to each other; columns: columns
+			const int g = L.contig ? e / n : e & (Q - 1);
+			const int k = L.contig ? e - g * n : e >> m.logQ;
+			float2 a = make_float2(0.f, 0.f);
+			uint32_t i, o, v = 0;
+			int b;
+
+			if (!m.column(t0 + g * m.cc, i, o, v, b))
+				continue;
+
+			const long at = m.va.offset_iov(i, o, v, k);
+
+			for (int c = 0; c < m.cc; c++) {
+
+				const float2* x = lds + (g * m.cc + c) * L.pitch + k;
+				float2 s = cmulc(x[0], l[m.b0][k]);
+
+				if (2 == m.nm)
+					s = cadd(s, cmulc(x[Q * L.pitch], l[1][k]));
+
+				if (nullptr != sens)
+					s = cmulc(s, sens[at + c * m.va.N]);
+
+				a = cadd(a, s);
+			}
+
+			if (roll) {
+				int px[3];
+				m.va.coords(i, o, k, px);
+				a = cscale(a, T.roll[0][px[0]] * T.roll[1][px[1]] * T.roll[2][px[2]]);
+			}
+
+			if (nullptr == dst)
+				grid[at] = (m.b0 > 0) ? cadd(grid[at], a) : a;
+			else
+				dst[m.va.offset_iov(i, o, v / (uint32_t)m.cc, k)] = a;
+		}
 	}
 };
 
@@ -334,6 +459,7 @@ void Nufft::create_geometry(const int dims[3], int C_, bool toeplitz_, bool peri
 	BAM_CHECK(2.f == os_, "only oversampling 2 is supported (got %f)", os_);
 	BAM_CHECK(width_ > 0.f && width_ / 2.f <= (float)(MAX_TAPS - 1), "kernel width %f not supported", width_);
 
+	ncu = device_cus();
 	N = 1;
 	nact = 0;
 	S = 1;
@@ -454,9 +580,20 @@ void Nufft::set_traj(long M_, const float* traj, const float2* weights_host, boo
 // Axis passes of the decomposition (see pair.hpp).  Axis j (of the active
 // ones) doubles the volumes: split takes the C 2^j volumes c + C s of the
 // grid (axis 0: the image side) to C 2^(j + 1), merge back.  Lengths beyond
-// the pair kernels (over PF_MAXN, or no three radices) run the element-wise
-// steps and the plain transform one after the other.
+// the pair kernels (over PF_MAXN, or no three radices) run on the run-time FFT
+// kernel (LdMember, ...).
 // ---------------------------------------------------------------------------
+
+// its coils per partial image: a block of at most 4096 points
+static int member_group(const Nufft& p)
+{
+	int cc = 1;
+
+	while (0 == p.C % (2 * cc) && 4l * cc * p.n[p.act[0]] <= FFT_MAX_ELEMS / 2)
+		cc *= 2;
+
+	return cc;
+}
 
 // coils per partial image of the last merge: the most that leave 4096 waves
 // (16 per compute unit) to share the work; the partial images cost a pass
@@ -468,7 +605,7 @@ static int merge_group(const Nufft& p)
 	int cc = 1;
 
 	if (0 == pl.nr)
-		return 1;
+		return member_group(p);
 
 	for (int c = 2; c <= p.C; c++)
 		if (0 == p.C % c && lanes * (p.C / c) >= 4096l * 64)
@@ -528,118 +665,150 @@ static PairArgs turn_args(const Nufft& p, const int* skip)
 	return a;
 }
 
-// Element-wise steps of lengths without a pair kernel; l: the two linear
-// phases of axis g.axis; member b at + b half.
-__global__ void k_long_expand(VolAxis g, SepTables T, const float2* src, const float2* sens, bool roll, long nvol,
-			      const float2* l0, const float2* l1, float2* grid, long half, const int* skip)
+// Members of axis j on the run-time kernel: geometry.  Rows: blocks of 2048 points
+// and more; columns: 16 next to each other (128 bytes), as far as 128 KB of LDS
+// hold them and no compute unit is left without a block (12 x 1040, 2 coils,
+// normal: 98 us with four columns per block, 62 with one).
+static FftLaunchCfg member_config(const Nufft& p, int j, int nm, int b0, int cc, float sign, MemberGeom& m)
 {
-	if (nullptr != skip && 0 != *skip)
-		return;
+	const int n = p.n[p.act[j]];
+	m.va = VolAxis::make(p.n, p.act[j], (long)p.C << j);
+	m.nm = nm;
+	m.b0 = b0;
+	m.cc = cc;
+	m.f_cc = FastDiv((uint32_t)cc);
+	m.ncol = m.va.transforms();
 
-	const long tot = nvol * g.N;
+	const bool contig = m.va.contig();
+	int Q = contig ? cc : 1;
 
-	for (long e = (long)blockIdx.x * blockDim.x + threadIdx.x; e < tot; e += (long)gridDim.x * blockDim.x) {
+	if (contig)
+		while (nm * Q * n < 2048)
+			Q *= 2;
+	else
+		while (Q < 16 && 2l * nm * Q * n <= 2 * FFT_MAX_ELEMS && m.ncol >= 2l * Q * p.ncu)
+			Q *= 2;
 
-		const long px = e % g.N;
-		const int c[3] = { (int)(px % g.n[0]), (int)((px / g.n[0]) % g.n[1]), (int)(px / ((long)g.n[0] * g.n[1])) };
-		const int k = c[g.axis];
-		float2 h = (nullptr == src) ? grid[e] : ((nullptr != sens) ? cmul(src[px], sens[e]) : src[e]);
+	BAM_CHECK((long)nm * Q * n <= 2 * FFT_MAX_ELEMS, "FFT block of %d x %d exceeds LDS budget", nm * Q, n);
 
-		if (roll)
-			h = cscale(h, T.roll[0][c[0]] * T.roll[1][c[1]] * T.roll[2][c[2]]);
+	m.logQ = 0;
+	while ((1 << m.logQ) < Q)
+		m.logQ++;
+	m.logP = m.logQ + (nm - 1);
+	m.nblk = (uint32_t)((m.ncol + Q - 1) / Q);
 
-		grid[e] = cmul(h, l0[k]);
-		grid[e + half] = cmul(h, l1[k]);
+	FftLaunchCfg c;
+	c.L.plan = p.axis[j];
+	c.L.P = nm * Q;
+	c.L.logP = m.logP;
+	c.L.contig = contig;
+	c.L.total = (long)m.nblk * c.L.P;
+	c.L.sign = sign;
+	c.L.pitch = n;
+	c.blocks = m.nblk;
+	c.lds_bytes = (size_t)nm * Q * n * sizeof(float2);
+	c.ept = (nm * Q * n <= 4096) ? 8 : ((nm * Q * n <= 8192) ? 16 : 32);
+	return c;
+}
+
+// members per block: both, as far as they fit
+static int members(const Nufft& p, int j) { return (2 * p.n[p.act[j]] <= FFT_MAX_ELEMS) ? 2 : 1; }
+
+static LdMember member_load(const Nufft& p, int j, const MemberGeom& m, const float2* src, const float2* sens, bool roll,
+			    bool phase)
+{
+	const int d = p.act[j];
+	return LdMember{ m, p.tabs, src, sens, roll, { phase ? p.tabs.lin[d][0] : nullptr, phase ? p.tabs.lin[d][1] : nullptr },
+			 p.grid.ptr, m.va.nvol * p.N };
+}
+
+static StMerge member_sum(const Nufft& p, int j, const MemberGeom& m, float2* dst, const float2* sens, bool roll)
+{
+	const int d = p.act[j];
+	return StMerge{ m, p.tabs, dst, sens, roll, { p.tabs.lin[d][0], p.tabs.lin[d][1] }, p.grid.ptr };
+}
+
+static void member_split(const Nufft& p, int j, const float2* src, const float2* sens, bool roll, bool fm,
+			 const int* skip, const char* name)
+{
+	const int nm = members(p, j);
+
+	// single members: the second first, as the first takes the source's place
+	for (int b0 = 2 - nm; b0 >= 0; b0--) {
+		MemberGeom m;
+		FftLaunchCfg cfg = member_config(p, j, nm, b0, 1, -1.f, m);
+		cfg.L.skip = skip;
+		cfg.name = name;
+		launch_fft_any(cfg, p.stream, member_load(p, j, m, src, sens, roll, true), NoMid{},
+			       StSplit{ m, p.tabs, p.grid.ptr, m.va.nvol * p.N, fm });
 	}
 }
 
-// dst: the image side (coil images, or with sens one partial image per coil);
-// null: in place
-__global__ void k_long_reduce(VolAxis g, SepTables T, float2* dst, const float2* sens, bool roll, long nvol,
-			      const float2* l0, const float2* l1, float2* grid, long half, const int* skip)
+static void member_merge(const Nufft& p, int j, float2* dst, const float2* sens, bool roll, int cc, const int* skip,
+			 const char* name)
 {
-	if (nullptr != skip && 0 != *skip)
-		return;
+	const int nm = members(p, j);
 
-	const long tot = nvol * g.N;
-
-	for (long e = (long)blockIdx.x * blockDim.x + threadIdx.x; e < tot; e += (long)gridDim.x * blockDim.x) {
-
-		const long px = e % g.N;
-		const int c[3] = { (int)(px % g.n[0]), (int)((px / g.n[0]) % g.n[1]), (int)(px / ((long)g.n[0] * g.n[1])) };
-		const int k = c[g.axis];
-		float2 v = cadd(cmulc(grid[e], l0[k]), cmulc(grid[e + half], l1[k]));
-
-		if (roll)
-			v = cscale(v, T.roll[0][c[0]] * T.roll[1][c[1]] * T.roll[2][c[2]]);
-
-		if (nullptr == dst)
-			grid[e] = v;
-		else
-			dst[e] = (nullptr != sens) ? cmulc(v, sens[e]) : v;
+	for (int b0 = 0; b0 <= 2 - nm; b0++) {
+		MemberGeom m;
+		FftLaunchCfg cfg = member_config(p, j, nm, b0, cc, +1.f, m);
+		cfg.L.skip = skip;
+		cfg.name = name;
+		launch_fft_any(cfg, p.stream, member_load(p, j, m, nullptr, nullptr, false, false), NoMid{},
+			       member_sum(p, j, m, dst, sens, roll));
 	}
 }
 
-static void long_fft(const Nufft& p, int j, float sign, bool fm, const int* skip, const char* name)
+// split, PSFs and merge of the last axis
+static void member_turn(const Nufft& p, int j, float2* dst, const float2* src, const float2* sens, int cc,
+			const int* skip, const char* name)
 {
-	VolAxis va = VolAxis::make(p.n, p.act[j], (long)p.C << (j + 1));
-	FftLaunchCfg cfg = fft_config(p.axis[j], va.transforms(), va.contig(), 1, sign);
+	MemberGeom m;
+	FftLaunchCfg cfg = member_config(p, j, 2, 0, cc, -1.f, m);
 	cfg.L.skip = skip;
 	cfg.name = name;
-	LdGrid ld{ va, p.grid.ptr };
-	StGrid st{ va, p.tabs, p.grid.ptr, fm };
-	launch_fft_axis(cfg, p.stream, ld, st);
+	launch_fft_any(cfg, p.stream, member_load(p, j, m, src, sens, false, true),
+		       MdMember{ m, FastDiv((uint32_t)p.C), p.psf.ptr, (1l << j) * p.N },
+		       member_sum(p, j, m, dst, sens, false));
 }
 
 // the image side's forms: src / dst non-null on axis 0 only
 static void axis_split(const Nufft& p, int j, const float2* src, const float2* sens, bool roll, bool fm,
 		       const int* skip, const char* name)
 {
-	if (p.pair[j].nr > 0) {
-
-		if (0 == j) {
-			pair_launch(PF_SPLIT, true, rows_split_args(p, src, sens, roll, fm, skip), name, p.stream);
-			return;
-		}
-
-		PairArgs a = pair_args(p, j, skip);
-		for (int d = 0; d < 3; d++)
-			a.fm[d] = fm ? p.tabs.fm[d] : nullptr;
-		pair_geometry(a, false, 0);
-		pair_launch(PF_SPLIT, false, a, name, p.stream);
+	if (0 == p.pair[j].nr) {
+		member_split(p, j, src, sens, roll, fm, skip, name);
 		return;
 	}
 
-	const PairArgs a = pair_args(p, j, skip);
-	const long nvol = (long)p.C << j;
-	hipLaunchKernelGGL(k_long_expand, dim3((unsigned)std::min<long>((nvol * p.N + 255) / 256, 65536)), dim3(256), 0,
-			   p.stream, a.va, p.tabs, src, sens, roll, nvol, a.l[0], a.l[1], a.grid, a.half, skip);
-	BAM_HIP(hipGetLastError());
-	long_fft(p, j, -1.f, fm, skip, name);
+	if (0 == j) {
+		pair_launch(PF_SPLIT, true, rows_split_args(p, src, sens, roll, fm, skip), name, p.stream);
+		return;
+	}
+
+	PairArgs a = pair_args(p, j, skip);
+	for (int d = 0; d < 3; d++)
+		a.fm[d] = fm ? p.tabs.fm[d] : nullptr;
+	pair_geometry(a, false, 0);
+	pair_launch(PF_SPLIT, false, a, name, p.stream);
 }
 
 static void axis_merge(const Nufft& p, int j, float2* dst, const float2* sens, bool roll, const int* skip,
 		       const char* name)
 {
-	if (p.pair[j].nr > 0) {
-
-		if (0 == j) {
-			pair_launch(PF_MERGE, true, rows_merge_args(p, dst, sens, roll, skip), name, p.stream);
-			return;
-		}
-
-		PairArgs a = pair_args(p, j, skip);
-		pair_geometry(a, false, 0);
-		pair_launch(PF_MERGE, false, a, name, p.stream);
+	if (0 == p.pair[j].nr) {
+		member_merge(p, j, dst, sens, roll, (nullptr != sens) ? member_group(p) : 1, skip, name);
 		return;
 	}
 
-	long_fft(p, j, +1.f, false, skip, name);
-	const PairArgs a = pair_args(p, j, skip);
-	const long nvol = (long)p.C << j;
-	hipLaunchKernelGGL(k_long_reduce, dim3((unsigned)std::min<long>((nvol * p.N + 255) / 256, 65536)), dim3(256), 0,
-			   p.stream, a.va, p.tabs, dst, sens, roll, nvol, a.l[0], a.l[1], a.grid, a.half, skip);
-	BAM_HIP(hipGetLastError());
+	if (0 == j) {
+		pair_launch(PF_MERGE, true, rows_merge_args(p, dst, sens, roll, skip), name, p.stream);
+		return;
+	}
+
+	PairArgs a = pair_args(p, j, skip);
+	pair_geometry(a, false, 0);
+	pair_launch(PF_MERGE, false, a, name, p.stream);
 }
 
 // the S transforms of a row of the first axis have always had to fit the
@@ -650,10 +819,11 @@ static void check_first_axis(const Nufft& p)
 		  p.n[p.act[0]]);
 }
 
-// partial images of S^H: their number, and where the last merge writes
-static float2* merge_target(Nufft& p, float2* dst, const float2* sens, int& G)
+// partial images of S^H of cc coils each: their number, and where the last merge
+// writes
+static float2* merge_target(Nufft& p, float2* dst, const float2* sens, int cc, int& G)
 {
-	G = (nullptr != sens) ? p.C / merge_group(p) : 1;
+	G = (nullptr != sens) ? p.C / cc : 1;
 
 	if (G <= 1)
 		return dst;
@@ -686,7 +856,7 @@ void Nufft::adjoint(float2* dst, const float2* ksp, const float2* sens)
 		axis_merge(*this, j, nullptr, nullptr, false, nullptr, "fft_adj_axis");
 
 	int G;
-	float2* out = merge_target(*this, dst, sens, G);
+	float2* out = merge_target(*this, dst, sens, merge_group(*this), G);
 	axis_merge(*this, 0, out, sens, true, nullptr, "fft_adj_last");
 
 	if (out != dst)
@@ -714,29 +884,43 @@ bool Nufft::normal(float2* dst, const float2* src, const float2* sens, const int
 	BAM_CHECK(0 == nbasis, "normal: a plan with a subspace basis takes normal_basis");
 
 	check_first_axis(*this);
-	int G;
-	float2* out = merge_target(*this, dst, sens, G);
 	const int last = nact - 1;
+	const int cc = merge_group(*this);
+	int G;
+	float2* out = merge_target(*this, dst, sens, cc, G);
 
-	axis_split(*this, 0, src, sens, false, false, skip, "fft_toeplitz_fwd");
+	if (0 == last) {
 
-	for (int j = 1; j < last; j++)
-		axis_split(*this, j, nullptr, nullptr, false, false, skip, "fft_toeplitz_fwd");
+		if (pair[0].nr > 0) {
+			axis_split(*this, 0, src, sens, false, false, skip, "fft_toeplitz_fwd");
+			basis_psf_apply(grid.ptr, psf.ptr, S, C, 1, N, stream, skip);
+			axis_merge(*this, 0, out, sens, false, skip, "fft_toeplitz_inv");
+		} else {
+			member_turn(*this, 0, out, src, sens, (nullptr != sens) ? cc : 1, skip, "fft_toeplitz");
+		}
 
-	if (last > 0 && pair[last].nr > 0) {
-		pair_launch(PF_TURN, false, turn_args(*this, skip), "fft_toeplitz", stream);
 	} else {
-		if (last > 0)
+
+		axis_split(*this, 0, src, sens, false, false, skip, "fft_toeplitz_fwd");
+
+		for (int j = 1; j < last; j++)
+			axis_split(*this, j, nullptr, nullptr, false, false, skip, "fft_toeplitz_fwd");
+
+		if (pair[last].nr > 0) {
+			pair_launch(PF_TURN, false, turn_args(*this, skip), "fft_toeplitz", stream);
+		} else if (2 == members(*this, last)) {
+			member_turn(*this, last, nullptr, nullptr, nullptr, 1, skip, "fft_toeplitz");
+		} else {
 			axis_split(*this, last, nullptr, nullptr, false, false, skip, "fft_toeplitz_fwd");
-		basis_psf_apply(grid.ptr, psf.ptr, S, C, 1, N, stream, skip);
-		if (last > 0)
+			basis_psf_apply(grid.ptr, psf.ptr, S, C, 1, N, stream, skip);
 			axis_merge(*this, last, nullptr, nullptr, false, skip, "fft_toeplitz_inv");
+		}
+
+		for (int j = last - 1; j >= 1; j--)
+			axis_merge(*this, j, nullptr, nullptr, false, skip, "fft_toeplitz_inv");
+
+		axis_merge(*this, 0, out, sens, false, skip, "fft_toeplitz_inv");
 	}
-
-	for (int j = last - 1; j >= 1; j--)
-		axis_merge(*this, j, nullptr, nullptr, false, skip, "fft_toeplitz_inv");
-
-	axis_merge(*this, 0, out, sens, false, skip, "fft_toeplitz_inv");
 
 	if (out != dst)
 		return sum_groups_or_fuse(dst, part.ptr, N, G, stream, skip, fuse);

@@ -202,6 +202,7 @@ struct Nufft {
 	DevBuf<float2> part;   // per-coil-group partial images [G][N]
 	AxisPlan axis[3];
 	PairPlan pair[3];      // of the active axes (nr = 0: no pair kernel)
+	int ncu = 1;           // compute units of the device
 
 	hipStream_t stream = 0;
 

@@ -2,7 +2,8 @@
 changes -- one, two and three radices, every odd radix, the lengths with a
 kernel of their own, column groups that do not fill, coil groups of more than one coil, and lengths without a pair
 kernel (over 1024, or no three radices of at most 16) -- against the oracle:
-forward, adjoint and the Toeplitz normal operator with coil maps.  FP32
+forward, adjoint and the Toeplitz normal operator with coil maps, and over 4096
+points without them.  FP32
 transforms of both sides: 1e-5, as for every operator."""
 import numpy as np
 import pytest
@@ -43,6 +44,13 @@ CASES = [
     ((625, 12, 1), 2),      # 5^4: no three radices
     ((12, 1040, 1), 2),     # over 1024
     ((1040, 1, 1), 2),
+    ((625, 12, 1), 6),      # coil groups of two
+    ((9, 1250, 1), 1),      # columns that do not fill a block of four
+    ((10, 7, 1040), 2),     # 3-D, over 1024 along the last axis
+    ((6, 1040, 5), 2),      # ... and along one in between
+    ((1, 18, 1), 48),       # one-dimensional: groups of 16 coils
+    ((24, 1, 1), 7),
+    ((1, 1, 2048), 4),
     # 32, 64, 128 and 256 (a kernel of their own): rows and columns, rows that do
     # not fill a wave or a work-group, ragged column groups, one and four waves
     ((32, 33, 1), 2),
@@ -92,6 +100,58 @@ def test_pair_lengths(dims, C):
     assert relerr(nu.normal(cim).cpu(), ref.normal(maps * img)) < 1e-5
     nu.free()
     op.free()
+
+
+# over 4096 points a block holds one member of a pair
+def test_single_members():
+    import bart_amd as ba
+    dims, C, M = (3, 4400, 1), 2, 500
+    rng = np.random.default_rng(1)
+    traj = np.zeros((M, 3), np.complex64)
+    for d in range(2):
+        traj[:, d] = (rng.random(M) - 0.5) * dims[d] * 0.98
+
+    def crandn(*s):
+        return (rng.standard_normal(s) + 1j * rng.standard_normal(s)).astype(np.complex64)
+
+    img, ksp = crandn(C, 1, dims[1], dims[0]), crandn(C, M)
+    ref = O.Nufft(dims, traj, C, toeplitz=False)
+    op = ba.nufft_create2(d16(1, M, 1, C), d16(*dims, C), d16(3, M), ba.traj_array(traj),
+                          conf=ba.NufftConf.defaults(toeplitz=False))
+    assert relerr(op.forward(torch.from_numpy(img.reshape(-1)).cuda()).cpu(), ref.forward(img)) < 1e-5
+    assert relerr(op.adjoint(torch.from_numpy(ksp.reshape(-1)).cuda()).cpu(), ref.adjoint(ksp)) < 1e-5
+    op.free()
+
+
+# ... and so the normal operator of a given PSF, against its definition in 64
+# bits (12 points: the definition itself, on the pair kernels)
+@pytest.mark.parametrize("n", [12, 4400])
+def test_single_members_normal(n):
+    import bart_amd as ba
+    dims, C = (3, n, 1), 2
+    rng = np.random.default_rng(n)
+
+    def crandn(*s):
+        return (rng.standard_normal(s) + 1j * rng.standard_normal(s)).astype(np.complex64)
+
+    img, psf = crandn(C, n, 3), crandn(4, n, 3)
+    conf = ba.NufftConf.defaults(toeplitz=True)
+    op = ba.nufft_create_normal(d16(*dims, C), list(dims) + [1] * 13 + [4], psf.reshape(-1), conf=conf)
+    y = op.normal(torch.from_numpy(img.reshape(-1)).cuda()).cpu()
+    op.free()
+
+    def phase(m, b):
+        j = np.arange(m)
+        c = m // 2
+        fm = np.exp(2j * np.pi * (j - c / 2) * c / m)
+        shift = -0.5 * b + m / 2 - m // 2
+        return np.exp(2j * np.pi * shift / m * (j - m / 2)) * fm
+
+    ref = 0
+    for s in range(4):
+        l = phase(n, s >> 1)[:, None] * phase(3, s & 1)[None, :]
+        ref = ref + np.conj(l) * np.fft.ifft2(psf[s] * np.fft.fft2(l * img.astype(np.complex128)))
+    assert relerr(y, ref) < 1e-5
 
 
 def test_first_axis_limit():
