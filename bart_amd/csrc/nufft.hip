@@ -891,9 +891,13 @@ bool Nufft::normal(float2* dst, const float2* src, const float2* sens, const int
 
 	if (0 == last) {
 
+		// one axis: the PSFs are multiplied where the split stores, or the
+		// run-time kernel takes both directions
 		if (pair[0].nr > 0) {
-			axis_split(*this, 0, src, sens, false, false, skip, "fft_toeplitz_fwd");
-			basis_psf_apply(grid.ptr, psf.ptr, S, C, 1, N, stream, skip);
+			PairArgs a = rows_split_args(*this, src, sens, false, false, skip);
+			a.psf = psf.ptr;
+			a.psf_half = N;
+			pair_launch(PF_SPLIT_PSF, true, a, "fft_toeplitz_fwd", stream);
 			axis_merge(*this, 0, out, sens, false, skip, "fft_toeplitz_inv");
 		} else {
 			member_turn(*this, 0, out, src, sens, (nullptr != sens) ? cc : 1, skip, "fft_toeplitz");

@@ -176,6 +176,8 @@ void pair_launch(int mode, bool rows, const PairArgs& a, const char* name, hipSt
 	if (rows) {
 		if (PF_SPLIT == mode)
 			launch_m<PF_SPLIT, true>(a, st);
+		else if (PF_SPLIT_PSF == mode)
+			launch_m<PF_SPLIT_PSF, true>(a, st);
 		else
 			launch_m<PF_MERGE, true>(a, st);
 	} else {

@@ -80,7 +80,7 @@ struct PairArgs {
 	const float* roll[3];    // null: no rolloff
 	// split of the last axis: fftmod tables (null: none)
 	const float2* fm[3];
-	// turn
+	// turn, split with PSFs
 	const float2* psf;
 	long psf_half;
 };
@@ -377,7 +377,13 @@ __device__ __forceinline__ void pf_tables(const PairArgs& a, float2* tw, float2*
 	}
 }
 
-enum { PF_SPLIT = 0, PF_MERGE = 1, PF_TURN = 2 };
+// PF_SPLIT_PSF: the split of a plan's only axis, x the PSFs (rows; a mode of its
+// own: with the product as a branch in the split, the split of 128^3, 16 coils
+// took 196 instead of 211 us but the two passes after it 327 and 305 instead of
+// 310 and 294)
+enum { PF_SPLIT = 0, PF_MERGE = 1, PF_TURN = 2, PF_SPLIT_PSF = 3 };
+
+constexpr bool pf_is_split(int mode) { return PF_SPLIT == mode || PF_SPLIT_PSF == mode; }
 
 // Rows: half of a work-group's waves take member b = 0, the other half b = 1,
 // and a merge's second member hands its points over through LDS, at the
@@ -926,7 +932,7 @@ __device__ __forceinline__ void pair_rows_block(const PairArgs& a, uint32_t w, f
 	const float2* lb = lin + b * n;
 	float2 h[PF_MAXR];
 
-	if constexpr (PF_SPLIT == MODE) {
+	if constexpr (pf_is_split(MODE)) {
 
 		const float2* im = (nullptr != a.sens) ? a.src + ro : a.src + (long)u * N + ro;
 		const float2* mp = (nullptr != a.sens) ? a.sens + (long)u * N + ro : nullptr;
@@ -959,13 +965,16 @@ __device__ __forceinline__ void pair_rows_block(const PairArgs& a, uint32_t w, f
 
 	lds_barrier();
 
-	if constexpr (PF_SPLIT == MODE) {
+	if constexpr (pf_is_split(MODE)) {
 
 		float2* out = a.grid + (long)u * N + ro + b * a.half;
+		const float2* psf = a.psf + ro + b * a.psf_half;
 
 		auto store = [&](int k, float2 x) BAM_INLINE {
 			if (nullptr != fma)
 				x = cmul(x, cmul(fo, fma[k]));
+			if constexpr (PF_SPLIT_PSF == MODE)
+				x = cmul(x, psf[k]);
 			out[k] = x;
 		};
 
@@ -1166,7 +1175,7 @@ __device__ __forceinline__ void pair_rows_fixed(const PairArgs& a, uint32_t w, f
 
 	float2 x[RA];
 
-	if constexpr (PF_SPLIT == MODE) {
+	if constexpr (pf_is_split(MODE)) {
 
 		load(x, ((nullptr != a.sens) ? a.src : a.src + (long)u * N) + ro);
 
@@ -1192,17 +1201,20 @@ __device__ __forceinline__ void pair_rows_fixed(const PairArgs& a, uint32_t w, f
 	if (tr >= 2 * P)
 		return;  // a whole wave
 
-	if constexpr (PF_SPLIT == MODE) {
+	if constexpr (pf_is_split(MODE)) {
 
 #pragma unroll
 		for (int r = 0; r < RA; r++)
 			x[r] = cscale(cmul(x[r], lb[r * RB]), rr);
 
 		float2* out = a.grid + (long)u * N + ro + b * a.half;
+		const float2* psf = a.psf + ro + b * a.psf_half;
 
 		transform(std::integral_constant<int, -1>{}, x, [&](int r, float2 y) BAM_INLINE {
 			if (nullptr != fma)
 				y = cmul(y, cmul(fo, fma[j + r * RB]));
+			if constexpr (PF_SPLIT_PSF == MODE)
+				y = cmul(y, psf[r * RB]);
 			if (in)
 				out[r * RB] = y;
 		});
