@@ -147,6 +147,7 @@ __global__ __launch_bounds__(CG_THREADS) void k_cg_apdot_groups(CgApFuse f, cons
 
 		float a = grp[i];
 
+#pragma unroll 8
 		for (int g = 1; g < G; g++)
 			a = a + grp[(long)g * gstride + i];
 
@@ -187,6 +188,7 @@ __global__ __launch_bounds__(CG_THREADS) void k_cg_apdot_sum_batch(const int* __
 
 		float a = it.grp[i];
 
+#pragma unroll 8
 		for (int g = 1; g < it.G; g++)
 			a = a + it.grp[(long)g * it.gstride + i];
 

@@ -393,6 +393,8 @@ __global__ void k_sum_groups(float2* __restrict__ dst, const float2* __restrict_
 
 		float2 a = part[i];
 
+		// (loads of several groups in flight)
+#pragma unroll 8
 		for (int g = 1; g < G; g++)
 			a = cadd(a, part[(long)g * N + i]);
 
@@ -595,9 +597,13 @@ static int member_group(const Nufft& p)
 	return cc;
 }
 
-// coils per partial image of the last merge: the most that leave 4096 waves
-// (16 per compute unit) to share the work; the partial images cost a pass
-// over G N values in all
+// coils per partial image of the last merge: the most that leave 16 waves per
+// compute unit to share the work (the partial images cost a pass over G N
+// values in all), but not more than MERGE_IMAGES partial images, each of which
+// a point of the sum waits for (256 points, 1024 coils, normal with maps: 260 us
+// with 1024 of them, 64 with 64)
+constexpr int MERGE_IMAGES = 64;
+
 static int merge_group(const Nufft& p)
 {
 	const PairPlan& pl = p.pair[0];
@@ -608,7 +614,7 @@ static int merge_group(const Nufft& p)
 		return member_group(p);
 
 	for (int c = 2; c <= p.C; c++)
-		if (0 == p.C % c && lanes * (p.C / c) >= 4096l * 64)
+		if (0 == p.C % c && (lanes * (p.C / c) >= 16l * 64 * p.ncu || p.C / cc > MERGE_IMAGES))
 			cc = c;
 
 	return cc;

@@ -162,3 +162,10 @@ def test_first_axis_limit():
                           conf=ba.NufftConf.defaults(toeplitz=False))
     with pytest.raises(ba.BartError, match="exceeds LDS budget"):
         op.forward(torch.zeros(2560 * 4, dtype=torch.complex64, device="cuda"))
+
+
+# more partial images of the sum over coils than one sum takes: 64 of several
+# coils each, and a number of coils without a divisor that gives 64 (67, 130)
+@pytest.mark.parametrize("dims,C", [((12, 10, 1), 128), ((14, 1, 1), 130), ((32, 6, 1), 67), ((16, 12, 1), 96)])
+def test_many_coils(dims, C):
+    test_pair_lengths(dims, C)
