@@ -29,7 +29,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int CV_MAXC = 64;     // channels (in and out) per layer at most
 constexpr int CV_THREADS = 512; // 8 waves
-constexpr int CV_STRIP = 256;   // forward: pixels (row segment) per work-group
+constexpr int CV_STRIP = 256;   // forward: pixels (row segment) per work-group at most
 constexpr int CV_MAXROWS = 16;  // image rows per work-group at most
 constexpr int CV_WG_MAXW = 256;
 
@@ -41,11 +41,11 @@ __device__ inline unsigned bf_pack(float a, float b)
 	return __builtin_bit_cast(unsigned, __builtin_convertvector(v, bf16x2));
 }
 
-// image rows per work-group: one work-group per compute unit where there
-// are rows enough (each one reads two rows of halo), down to one row
-static int conv_rows(long total_rows, int ncu)
+// image rows per work-group: nwg work-groups where there are rows enough (each
+// one reads two rows of halo), down to one row
+static int conv_rows(long total_rows, int nwg)
 {
-	return (int)std::min<long>(CV_MAXROWS, std::max<long>(1, (total_rows + ncu - 1) / ncu));
+	return (int)std::min<long>(CV_MAXROWS, std::max<long>(1, (total_rows + nwg - 1) / nwg));
 }
 
 // ---------------------------------------------------------------------------
@@ -99,7 +99,7 @@ __global__ __launch_bounds__(CV_THREADS) void k_conv3x3_fwd(const float* __restr
 							    const unsigned short* __restrict__ wb,
 							    const float* __restrict__ bias,
 							    const float* __restrict__ res, int Cout, int relu,
-							    float* __restrict__ y, int rows, int ncog)
+							    float* __restrict__ y, int strip, int rows, int ncog)
 {
 	constexpr int STEPS = conv_steps(G);
 	constexpr int PITCH = conv_pitch(G);
@@ -108,7 +108,7 @@ __global__ __launch_bounds__(CV_THREADS) void k_conv3x3_fwd(const float* __restr
 	extern __shared__ __align__(16) unsigned char cv_smem[];
 	unsigned short* xl = (unsigned short*)cv_smem;  // [3][CV_STRIP + 2][PITCH]
 
-	const int x0 = blockIdx.x * CV_STRIP;
+	const int x0 = blockIdx.x * strip;
 	const int y0 = blockIdx.y * rows;
 	const int b = blockIdx.z;
 	const int nrow = min(rows, H - y0);
@@ -135,8 +135,12 @@ __global__ __launch_bounds__(CV_THREADS) void k_conv3x3_fwd(const float* __restr
 	// of the strip and one of the two halo pixels (the first 2 G threads)
 	float v[NT + 1][8];
 
+	// (a strip's right halo pixel included; it is the extra task's where the
+	// strip takes all of CV_STRIP)
+	const int xe = min(W, x0 + strip + 1);
+
 	auto load8 = [&](float (&d)[8], int g, int gy, int gx) {
-		const bool ok = gy >= 0 && gy < H && gx >= 0 && gx < W;
+		const bool ok = gy >= 0 && gy < H && gx >= 0 && gx < xe;
 		const float* p = xb + (long)(8 * g) * HW + (long)gy * W;
 #pragma unroll
 		for (int i = 0; i < 8; i++)
@@ -177,7 +181,7 @@ __global__ __launch_bounds__(CV_THREADS) void k_conv3x3_fwd(const float* __restr
 	store_row(1);
 	load_row(y0 + 1);
 
-	const int ntile = (min(CV_STRIP, W - x0) + 15) / 16;
+	const int ntile = (min(strip, W - x0) + 15) / 16;
 
 	for (int r = 0; r < nrow; r++) {
 
@@ -400,6 +404,9 @@ __global__ __launch_bounds__(CV_THREADS) void k_conv3x3_wgrad(const float* __res
 			for (int p0 = 32 * ks; p0 < W; p0 += 32 * KS) {
 
 				const int p = p0 + 8 * kg;
+				// beyond the row dy is 0, and a 0 of dy must not meet the
+				// row's last pixel, which may be infinite
+				const unsigned pm = (p < W) ? ~0u : 0u;
 				bf16x8 a[NCO];
 #pragma unroll
 				for (int q = 0; q < NCO; q++)
@@ -410,9 +417,7 @@ __global__ __launch_bounds__(CV_THREADS) void k_conv3x3_wgrad(const float* __res
 
 					const unsigned short* xr = xl + ((((r + u) % 3) * NCI + it) * 16 + l16) * PX + 8 + p;
 					const uint4 d = *(const uint4*)xr;
-					// (beyond the row dy is 0, and a 0 of dy must not
-					// meet the row's last pixel, which may be infinite)
-					const unsigned pv = (p < W) ? *(const unsigned*)(xr - 2) : 0u;
+					const unsigned pv = *(const unsigned*)(xr - 2) & pm;
 					const unsigned nx = *(const unsigned*)(xr + 8);
 					// 8 pixels from p - 1 and from p + 1
 					const unsigned m0 = __builtin_amdgcn_alignbyte(d.x, pv, 2);
@@ -552,14 +557,14 @@ static void check_shape(int B, int Cin, int Cout, int H, int W)
 
 template <int G>
 static void fwd_launch_g(dim3 grid, int tpw, const float* x, int Cin, int H, int W, const unsigned short* wb,
-			 const float* bias, const float* res, int Cout, bool relu, float* y, int rows, int ncog,
-			 hipStream_t st)
+			 const float* bias, const float* res, int Cout, bool relu, float* y, int strip, int rows,
+			 int ncog, hipStream_t st)
 {
 	const size_t lds = sizeof(unsigned short) * 3 * (CV_STRIP + 2) * conv_pitch(G);
 
 #define BAM_CONV(T)                                                                                               \
 	hipLaunchKernelGGL((k_conv3x3_fwd<G, T>), grid, dim3(CV_THREADS), lds, st, x, Cin, H, W, wb, bias, res, Cout, \
-			   relu ? 1 : 0, y, rows, ncog)
+			   relu ? 1 : 0, y, strip, rows, ncog)
 	if (1 == tpw)
 		BAM_CONV(1);
 	else if (2 == tpw)
@@ -581,8 +586,9 @@ static void fwd_launch(const float* x, int B, int Cin, int H, int W, const float
 	BAM_CHECK(H <= 65535 && B <= 65535, "conv3x3: too many rows or images");
 
 	// a wave keeps the weights of its output-channel tiles in registers (4
-	// per tile and step of 32): all tiles while they take at most 108, else
-	// two groups of waves (144 and more spill)
+	// per tile and step of 32): three tiles up to 32 input channels, two above
+	// (208 to 244 registers in all at 48 to 64 channels, none spilled; three
+	// tiles of 48 channels spill 120)
 	const int G = (Cin + 7) / 8;
 	const int nco = (Cout + 15) / 16;
 	const int ncog = (4 == nco || (3 == nco && G > 4)) ? 2 : 1;
@@ -593,12 +599,22 @@ static void fwd_launch(const float* x, int B, int Cin, int H, int W, const float
 		wb.alloc(nw);
 	hipLaunchKernelGGL(k_conv_wprep, dim3((unsigned)((nw + 255) / 256)), dim3(256), 0, st, w, Cin, Cout, G, ntiles,
 			   flip ? 1 : 0, wb.ptr);
-	const int nx = (W + CV_STRIP - 1) / CV_STRIP;
-	const int rows = conv_rows((long)nx * H * B, device_cus());
+	// Strips of equal width (320 as 256 + 64: 286 us for 48 channels, batch 8 of
+	// 320^2, as 160 + 160: 225).  A work-group per compute unit, or two where the
+	// weights of a lane and the rows in LDS are few (2 -> 48 channels, batch 8 of
+	// 320^2: 88 -> 59 us; four: 61), in halves of a strip where these would walk
+	// down less than two rows (one image of 320^2: 17.9 -> 14.4; 512^2, 16
+	// channels, with two rows: 14.8 and 15.2).
+	int nx = (W + CV_STRIP - 1) / CV_STRIP;
+	const int nwg = device_cus() * ((G <= 2) ? 2 : 1);
+	if (G <= 2 && (long)nx * H * B < 2l * nwg)
+		nx = (W + CV_STRIP / 2 - 1) / (CV_STRIP / 2);
+	const int strip = ((W + nx - 1) / nx + 15) / 16 * 16;
+	const int rows = conv_rows((long)nx * H * B, nwg);
 	dim3 grid(nx, (H + rows - 1) / rows, B);
 
 #define BAM_CONV_G(NG) \
-	case NG: fwd_launch_g<NG>(grid, tpw, x, Cin, H, W, wb.ptr, bias, res, Cout, relu, y, rows, ncog, st); break
+	case NG: fwd_launch_g<NG>(grid, tpw, x, Cin, H, W, wb.ptr, bias, res, Cout, relu, y, strip, rows, ncog, st); break
 	switch (G) {
 		BAM_CONV_G(1);
 		BAM_CONV_G(2);
@@ -665,6 +681,8 @@ void conv3x3_bwd_weights(const float* x, const float* dy, int B, int Cin, int Co
 	check_shape(B, Cin, Cout, H, W);
 	BAM_CHECK(W <= CV_WG_MAXW && 0 == W % 8, "conv3x3 weight gradient: width a multiple of 8, at most %d",
 		  CV_WG_MAXW);
+	// the entry point's range (57 to 64 channels in with more than 32 out stay
+	// outside of it), not a limit of the kernel
 	BAM_CHECK(((Cout + 31) / 32) * ((Cin * 9 + 31) / 32) <= 32, "conv3x3 weight gradient: too many tiles");
 	CnnWork& cw = cnn_work();
 	std::lock_guard<std::mutex> lock(cw.mtx);

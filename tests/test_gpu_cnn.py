@@ -73,7 +73,10 @@ def test_conv3x3_backward_weights(B, Cin, Cout, H, W):
 # row, more rows than a work-group takes, pointers off 16 bytes.  FP32 sums of
 # at most 9 * 64 products (forward) or B H W products (gradients).
 EDGES = [(1, 1, 1, 1, 8), (1, 64, 64, 3, 257), (2, 33, 17, 9, 24), (1, 17, 64, 2, 40), (1, 56, 48, 5, 16),
-         (3, 40, 33, 300, 8), (1, 9, 49, 2, 515)]
+         (3, 40, 33, 300, 8), (1, 9, 49, 2, 515),
+         # strips of equal width, and halves of a strip for few rows; the weight
+         # gradient's largest LDS layout and all its tiles
+         (1, 48, 48, 2, 320), (1, 2, 48, 5, 320), (2, 16, 16, 700, 272), (1, 56, 64, 3, 256)]
 
 
 @pytest.mark.parametrize("B,Cin,Cout,H,W", EDGES)
