@@ -1894,7 +1894,8 @@ void grid_forward(const GridPlan& gp, const float* kb, float2* ksp, const float2
 	// 16-coil kooshball: 7.7 ms at 4 coils, 12.4 ms at 16; 1 or 2 coils gain
 	// nothing more).  One coil per thread in 2-D, where the taps cost little
 	// beside the loads and all of a sample's loads fit in flight (320^2 spiral,
-	// 32 coils: 112 us against 121), and where 4 would leave less than 8 waves
+	// 32 coils: 112 us against 121; forward of 256^2, 98304 samples: 8 coils 82
+	// against 97, 16 coils 113 against 115, 32 coils 179 against 187), and where 4 would leave less than 8 waves
 	// per compute unit: a thread's chain of loads is then what the launch waits
 	// for (64^2, 4 coils, 3968 samples: 38 -> 6 us).
 	const bool one = t.ntap <= 3 && (t.nd < 3 || (long)g.M * ceil_div(g.C, 4) < 8l * 64 * gp.ncu);

@@ -645,7 +645,7 @@ static PairArgs rows_split_args(const Nufft& p, const float2* src, const float2*
 		a.roll[d] = roll ? p.tabs.roll[d] : nullptr;
 		a.fm[d] = fm ? p.tabs.fm[d] : nullptr;
 	}
-	pair_geometry(a, true, (uint32_t)p.C);
+	pair_geometry(a, true, (uint32_t)p.C, p.ncu);
 	return a;
 }
 
@@ -657,7 +657,7 @@ static PairArgs rows_merge_args(const Nufft& p, float2* dst, const float2* sens,
 	a.cc = (nullptr != sens) ? merge_group(p) : 1;
 	for (int d = 0; d < 3; d++)
 		a.roll[d] = roll ? p.tabs.roll[d] : nullptr;
-	pair_geometry(a, true, (uint32_t)(p.C / a.cc));
+	pair_geometry(a, true, (uint32_t)(p.C / a.cc), p.ncu);
 	return a;
 }
 
@@ -667,7 +667,7 @@ static PairArgs turn_args(const Nufft& p, const int* skip)
 	PairArgs a = pair_args(p, j, skip);
 	a.psf = p.psf.ptr;
 	a.psf_half = (1l << j) * p.N;
-	pair_geometry(a, false, 0);
+	pair_geometry(a, false, 0, p.ncu);
 	return a;
 }
 
@@ -795,7 +795,7 @@ static void axis_split(const Nufft& p, int j, const float2* src, const float2* s
 	PairArgs a = pair_args(p, j, skip);
 	for (int d = 0; d < 3; d++)
 		a.fm[d] = fm ? p.tabs.fm[d] : nullptr;
-	pair_geometry(a, false, 0);
+	pair_geometry(a, false, 0, p.ncu);
 	pair_launch(PF_SPLIT, false, a, name, p.stream);
 }
 
@@ -813,7 +813,7 @@ static void axis_merge(const Nufft& p, int j, float2* dst, const float2* sens, b
 	}
 
 	PairArgs a = pair_args(p, j, skip);
-	pair_geometry(a, false, 0);
+	pair_geometry(a, false, 0, p.ncu);
 	pair_launch(PF_MERGE, false, a, name, p.stream);
 }
 

@@ -74,7 +74,7 @@ size_t pair_lds_bytes(const PairArgs& a, bool rows)
 
 unsigned pair_threads(const PairArgs& a, bool rows) { return (rows ? 2 : 1) * (unsigned)a.group; }
 
-void pair_geometry(PairArgs& a, bool rows, uint32_t units)
+void pair_geometry(PairArgs& a, bool rows, uint32_t units, int ncu)
 {
 	const int n = a.pl.n;
 	const int lim = pf_threads(rows, 3 == a.pl.nr) / (rows ? 2 : 1);  // lanes of a member
@@ -91,10 +91,12 @@ void pair_geometry(PairArgs& a, bool rows, uint32_t units)
 		if (rows) {
 			// both members of a row in one wave; four waves per work-group,
 			// one where that would leave compute units without a work-group
-			// (CG of 256^2, 8 coils, 30 iterations: 1.611 ms at four, 1.640
-			// at one)
+			// (Toeplitz normal, one and four: 64^2, 8 coils 31.1 and 31.9 us;
+			// 128^2, 4 coils 36.5 and 37.7, 16 coils 39.5 and 39.8; from there
+			// on four: 256^2, 8 coils 47.5 and 46.4, 32 coils 80.5 and 76.4;
+			// 128^3, 4 coils 416 and 413)
 			const int rw = 32 / RB;
-			const int waves = ((long)units * count / (4 * rw) >= 256) ? 4 : 1;
+			const int waves = ((long)units * count / (4 * rw) >= ncu) ? 4 : 1;
 			P = rw * waves;
 			a.group = 32 * waves;
 		}
@@ -102,7 +104,7 @@ void pair_geometry(PairArgs& a, bool rows, uint32_t units)
 		// whole waves, twice as many once there are enough work-groups
 		while (P * a.pl.NJ < 64 && 2 * P * a.pl.NJ <= lim)
 			P *= 2;
-		if ((long)units * (count / P) > 4096 && 2 * P * a.pl.NJ <= lim)
+		if ((long)units * (count / P) > 16l * ncu && 2 * P * a.pl.NJ <= lim)
 			P *= 2;
 	} else {
 		// 16 columns (128-byte rows); 64 where a lane holds a whole transform

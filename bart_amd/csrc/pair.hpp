@@ -19,8 +19,8 @@
 // A transform of length n = R0 R1 (R0 R1 R2) is held by NJ = max n / Ri lanes;
 // a lane's R points j + r n / R are one butterfly of the first pass (inputs)
 // and of the last (outputs), so the first pass runs on the loaded registers,
-// the last one stores from registers, and up to n = 256 one exchange through
-// LDS lies between them (two for three radices).  Columns sit in LDS
+// the last one stores from registers, and one exchange through LDS lies between
+// them (two with three radices).  Columns sit in LDS
 // transform-fastest ([k][P], P adjacent columns: 128-byte global rows, no
 // bank conflicts in any pass), rows point-fastest with one element of
 // padding after eight.
@@ -105,8 +105,8 @@ constexpr int pf_row_pitch(int n) { return (n + n / 8 + 1) | 1; }
 size_t pair_lds_bytes(const PairArgs& a, bool rows);
 unsigned pair_threads(const PairArgs& a, bool rows);
 // fills P, logP, pitch, the block count and the divisions; `units`: row
-// kernels only, the coils (or coil groups)
-void pair_geometry(PairArgs& a, bool rows, uint32_t units);
+// kernels only, the coils (or coil groups); `ncu`: the device's compute units
+void pair_geometry(PairArgs& a, bool rows, uint32_t units, int ncu);
 
 // ---------------------------------------------------------------------------
 // DFTs of radix 2 .. 16 in registers, w = exp(SG 2 pi i / R)
