@@ -144,23 +144,17 @@ def test_nufft_3d_slice_path(n, C, S):
     assert relerr(op.adjoint(ksp).reshape(C, n, n, n), ref.adjoint(ksp)) < 1e-5
 
 
-def test_nufft_3d_slice_vs_axis_passes(monkeypatch):
-    # the same 32^3 operator with the slice kernels and with per-axis passes
+def test_nufft_3d_32_points():
+    # 32^3: every axis on the kernels of that length
     n, C, R, S = 32, 2, 64, 60
     traj = I.phyllotaxis_kooshball(spokes=S, readout=R)
     cim = crandn((C, n, n, n), 66)
     ksp = crandn((C, R * S), 67)
-    a = make_nufft((n, n, n), C, traj, R, S, toeplitz=False)
-    monkeypatch.setenv("BART_AMD_SLICE", "off")
-    b = make_nufft((n, n, n), C, traj, R, S, toeplitz=False)
+    op = make_nufft((n, n, n), C, traj, R, S, toeplitz=False)
     ref = O.Nufft((n, n, n), traj, C, toeplitz=False)
-    fa, fb = a.forward(cim), b.forward(cim)
-    aa, ab = a.adjoint(ksp), b.adjoint(ksp)
-    print(f"forward slice vs axis {relerr(fa, fb):.2e}, adjoint slice vs axis {relerr(aa, ab):.2e}, "
-          f"axis vs oracle {relerr(ab.reshape(C, -1), ref.adjoint(ksp).reshape(C, -1)):.2e}")
-    assert relerr(fa, fb) < 1e-5
-    assert relerr(ab.reshape(C, -1), ref.adjoint(ksp).reshape(C, -1)) < 1e-5
-    assert relerr(aa, ab) < 1e-5
+    assert relerr(op.forward(cim).reshape(C, -1), ref.forward(cim).reshape(C, -1)) < 1e-5
+    assert relerr(op.adjoint(ksp).reshape(C, -1), ref.adjoint(ksp).reshape(C, -1)) < 1e-5
+    op.free()
 
 
 def test_nufft_2d_dense_adjoint():
@@ -285,52 +279,36 @@ def test_psf_and_toeplitz_normal(img, R, S, C, weighted):
 
 
 @pytest.mark.parametrize("Z", [64, 128, 256, 512])
-def test_nufft_pair_zpass_vs_all_subgrids(monkeypatch, Z):
-    # forward / adjoint NUFFT with the pair z-pass (the slice kernels store
-    # and read one x-y transform per pair of sub-grids that differ only in
-    # the z shift) against the z-pass over all 8 sub-grids and the oracle;
-    # every z length with a pair kernel
+def test_nufft_3d_z_lengths(Z):
+    # forward, adjoint and the Toeplitz normal operator at the power-of-two
+    # lengths of the last axis: three with kernels of their own, and three
+    # radices (512)
     img, R, S, C = (32, 32, Z), 64, 90, 2
     X, Y, Z = img
     traj = I.phyllotaxis_kooshball(spokes=S, readout=R)
     w = (0.5 + np.random.default_rng(5).random(R * S)).astype(np.complex64)
-    a = make_nufft(img, C, traj, R, S, weights=w, toeplitz=False)
-    monkeypatch.setenv("BART_AMD_PAIRZ", "off")
-    b = make_nufft(img, C, traj, R, S, weights=w, toeplitz=False)
+    op = make_nufft(img, C, traj, R, S, weights=w, toeplitz=False)
     ref = O.Nufft(img, traj, C, weights=w, toeplitz=False)
     cim = crandn((C, Z, Y, X), 18)
     ksp = crandn((C, R * S), 19)
-    fa, fb = a.forward(cim).reshape(C, -1), b.forward(cim).reshape(C, -1)
-    aa, ab = a.adjoint(ksp).reshape(C, Z, Y, X), b.adjoint(ksp).reshape(C, Z, Y, X)
-    fr, ar = ref.forward(cim), ref.adjoint(ksp)
-    print(f"forward pair vs all {relerr(fa, fb):.2e}, vs oracle {relerr(fa, fr):.2e}; "
-          f"adjoint pair vs all {relerr(aa, ab):.2e}, vs oracle {relerr(aa, ar):.2e}")
-    assert relerr(fa, fb) < 1e-5 and relerr(aa, ab) < 1e-5
-    assert relerr(fa, fr) < 1e-5 and relerr(aa, ar) < 1e-5
-    # the Toeplitz normal of the same geometry (pair z-pass with the PSF)
-    monkeypatch.delenv("BART_AMD_PAIRZ")
+    assert relerr(op.forward(cim).reshape(C, -1), ref.forward(cim)) < 1e-5
+    assert relerr(op.adjoint(ksp).reshape(C, Z, Y, X), ref.adjoint(ksp)) < 1e-5
+    op.free()
     t = make_nufft(img, C, traj, R, S, weights=w, toeplitz=True)
     reft = O.Nufft(img, traj, C, weights=w, toeplitz=True)
     assert relerr(t.normal(cim).reshape(C, Z, Y, X), reft.normal(cim)) < 1e-5
     t.free()
 
 
-def test_toeplitz_pair_zpass_vs_all_subgrids(monkeypatch):
-    # the Toeplitz normal with the pair z-pass (one x-y transform per pair of
-    # sub-grids that differ only in the z shift) against the z-pass over all
-    # 8 sub-grids, and both against the oracle
+def test_toeplitz_3d_64_points():
+    # 64^3, three coils: split, turn and merge of every axis at that length
     img, R, S, C = (64, 64, 64), 128, 80, 3
     traj = I.phyllotaxis_kooshball(spokes=S, readout=R)
-    a = make_nufft(img, C, traj, R, S, toeplitz=True)
-    monkeypatch.setenv("BART_AMD_PAIRZ", "off")
-    b = make_nufft(img, C, traj, R, S, toeplitz=True)
+    op = make_nufft(img, C, traj, R, S, toeplitz=True)
     ref = O.Nufft(img, traj, C, toeplitz=True)
     x = crandn((C, 64, 64, 64), 17)
-    ya, yb = a.normal(x).reshape(C, 64, 64, 64), b.normal(x).reshape(C, 64, 64, 64)
-    yr = ref.normal(x)
-    print(f"pair vs all {relerr(ya, yb):.2e}, pair vs oracle {relerr(ya, yr):.2e}, all vs oracle {relerr(yb, yr):.2e}")
-    assert relerr(ya, yb) < 1e-5
-    assert relerr(ya, yr) < 1e-5 and relerr(yb, yr) < 1e-5
+    assert relerr(op.normal(x).reshape(C, 64, 64, 64), ref.normal(x)) < 1e-5
+    op.free()
 
 
 def test_psf_update_roundtrip():
