@@ -38,9 +38,9 @@ HBM_PEAK_GBS = 8000.0
 # scaled by 2 and WRITE_SIZE by 1: the factors at which the same counters
 # read 1 GiB for a 1 GiB device copy.
 TRAFFIC = {
-    ("3d_radial_kooshball_128^3_16coils_8192x256", "fft_toeplitz"): 3_222_000_000,
-    ("3d_radial_kooshball_128^3_16coils_8192x256", "grid_adjoint"): 4_277_000_000,
-    ("3d_radial_kooshball_128^3_16coils_8192x256", "grid_forward"): 12_900_000_000,
+    ("3d_radial_kooshball_128^3_16coils_8192x256", "fft_toeplitz"): 2_324_000_000,
+    ("3d_radial_kooshball_128^3_16coils_8192x256", "grid_adjoint"): 4_310_000_000,
+    ("3d_radial_kooshball_128^3_16coils_8192x256", "grid_forward"): 13_189_000_000,
 }
 
 
