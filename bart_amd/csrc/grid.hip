@@ -366,41 +366,31 @@ void GridPlan::build(const GridGeom& geom, const float* traj)
 	}
 
 	std::vector<int> cell(g.M);
-	std::vector<int> wraps(g.M);
 	std::vector<int> count(ncells + 1, 0);
 
 	for (long m = 0; m < g.M; m++) {
 
 		int cb[3];
-		int code = 0;
 
 		for (int d = 0; d < 3; d++) {
 
 			if (1 == g.n[d]) {
 				cb[d] = 0;
-				code |= 8 << (4 * d);
 				continue;
 			}
 
 			float p = host_pos(g, 0, d, traj[3 * m + d]);
-			int q = 0;
 
 			if (!std::isfinite(p))
 				p = 0.f;
 
-			if (g.periodic) {
-				q = (int)floorf(p / (float)g.n[d]);
-				q = std::min(std::max(q, -7), 7);
-				p = p - (float)g.n[d] * (float)q;
-			}
-
-			code |= (q + 8) << (4 * d);
+			if (g.periodic)
+				p = p - (float)g.n[d] * floorf(p / (float)g.n[d]);
 
 			int b = (int)floorf(p / (float)g.CS[d]);
 			cb[d] = std::min(std::max(b, 0), g.ncell[d] - 1);
 		}
 
-		wraps[m] = code;
 		cell[m] = cb[0] + g.ncell[0] * (cb[1] + g.ncell[1] * cb[2]);
 		count[cell[m] + 1]++;
 	}
@@ -416,10 +406,7 @@ void GridPlan::build(const GridGeom& geom, const float* traj)
 
 		long i = pos[cell[m]]++;
 		hsm[i] = (int)m;
-		int code = wraps[m];
-		float fcode;
-		memcpy(&fcode, &code, sizeof(float));
-		hsk[i] = make_float4(traj[3 * m + 0], traj[3 * m + 1], traj[3 * m + 2], fcode);
+		hsk[i] = make_float4(traj[3 * m + 0], traj[3 * m + 1], traj[3 * m + 2], 0.f);
 	}
 
 	BAM_CHECK(g.M < (1l << 31), "too many samples");

@@ -128,7 +128,7 @@ struct GridPlan {
 	GridGeom g;
 	DevBuf<int> sm;          // sorted sample -> original sample index
 	DevBuf<int> si;          // original sample -> sorted position
-	DevBuf<float4> sk;       // sorted coordinates (kx, ky, kz) + wrap code
+	DevBuf<float4> sk;       // sorted coordinates (kx, ky, kz, 0)
 	DevBuf<int> cstart;      // cell -> first sorted sample (ncells + 1)
 	GridTiling ta;           // adjoint tiling
 	DevBuf<float2> kspS;     // adjoint input permuted to sorted order, coil chunks interleaved

@@ -51,3 +51,29 @@ def test_grid_adjoint_edges(dims, C, width, periodic, M):
     assert relerr(a.cpu(), ref.adjoint(ksp)) < 1e-5
     assert torch.equal(a, op.adjoint(y))
     op.free()
+
+
+# samples many periods away (coordinates of 1/64: exact in FP32) are those of the
+# first period, at the ends of the grid too
+@pytest.mark.parametrize("dims", [(32, 1, 1), (20, 33, 1), (12, 10, 9)])
+@pytest.mark.parametrize("periods", [5, 9, -11])
+def test_grid_periods_away(dims, periods):
+    import bart_amd as ba
+    C, M = 3, 2000
+    rng = np.random.default_rng(7)
+    traj = np.zeros((M, 3), np.complex64)
+    for d in range(3):
+        if dims[d] > 1:
+            traj[:, d] = np.round((rng.random(M) - 0.5) * dims[d] * 64) / 64
+    far = traj + np.array([n * periods if n > 1 else 0 for n in dims])
+    ksp = (rng.standard_normal((C, M)) + 1j * rng.standard_normal((C, M))).astype(np.complex64)
+    y = torch.from_numpy(ksp.reshape(-1)).cuda()
+    conf = ba.NufftConf.defaults(toeplitz=False, periodic=True)
+    out = []
+    for t in (traj, far):
+        op = ba.nufft_create2(d16(1, M, 1, C), d16(*dims, C), d16(3, M), ba.traj_array(t.astype(np.complex64)), conf=conf)
+        a = op.adjoint(y)
+        out.append((a.cpu(), op.forward(a).cpu()))
+        op.free()
+    assert relerr(out[1][0], out[0][0]) < 1e-6
+    assert relerr(out[1][1], out[0][1]) < 1e-6
