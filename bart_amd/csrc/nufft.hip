@@ -817,8 +817,9 @@ static void axis_merge(const Nufft& p, int j, float2* dst, const float2* sens, b
 	pair_launch(PF_MERGE, false, a, name, p.stream);
 }
 
-// the S transforms of a row of the first axis have always had to fit the
-// FFT's LDS block
+// The range of the entry points: the S transforms of a row of the first axis in
+// one LDS block of the FFT.  (No pass needs it any more; a plan beyond it stays
+// refused.)
 static void check_first_axis(const Nufft& p)
 {
 	BAM_CHECK((long)p.S * p.n[p.act[0]] <= FFT_MAX_ELEMS, "FFT block of %d x %d exceeds LDS budget", p.S,

@@ -155,7 +155,7 @@ def test_single_members_normal(n):
 
 
 def test_first_axis_limit():
-    """2^d transforms of the first axis have to fit the FFT's LDS block."""
+    """The entry points take 2^d transforms of the first axis up to 8192 points."""
     import bart_amd as ba
     traj = np.zeros((8, 3), np.complex64)
     op = ba.nufft_create2(d16(1, 8, 1, 1), d16(2560, 4, 1, 1), d16(3, 8, 1), ba.traj_array(traj),
