@@ -357,9 +357,9 @@ def test_sense_forward_adjoint_normal():
 
 
 @pytest.mark.parametrize("n,C", [(32, 4), (32, 6), (64, 3)])
-def test_sense_3d_slice_path(n, C):
-    # slice kernels with the coil sum of S^H over coil groups (64^3: the
-    # Toeplitz normal with the pair z-pass)
+def test_sense_3d_square(n, C):
+    # square 3-D plans on the kernels of 32 and 64 points, with the coil sum of
+    # S^H over coil groups
     R, S = 2 * n, 120
     op, ref, maps, img, traj = make_sense(n, C, R, S, Z=n, seed=25)
     k = op.forward(img).reshape(C, -1)
